@@ -123,9 +123,16 @@ struct OrbitArgs {
   int nfrag;
   double u[kMaxFrag];
   double *part_u;       // [G][kMaxFrag] per-workgroup dE/du_f sums (projected adjoint)
+  // kOrbitBatch: triple b = tri[b] (i | j << 10 | k << 20), b < nb, in place of
+  // i, j, k and omega: W and Vb hold one v^3 block per triple, part_t and
+  // part_mo G rows per triple; wt: occupied weights of a diagonal projector or null
+  const int *tri;
+  int nb;
+  long long ws;  // element stride of W's first index (v^2 otherwise)
+  const double *wt;
 };
 
-enum OrbitMode { kOrbitPlain = 0, kOrbitProjAcc = 1, kOrbitProjVjp = 2 };
+enum OrbitMode { kOrbitPlain = 0, kOrbitProjAcc = 1, kOrbitProjVjp = 2, kOrbitBatch = 3 };
 
 // V-bar reductions: the sums over one virtual index are split into kVRS parts
 // (more workgroups in flight), and the last virtual index is processed in
@@ -144,6 +151,12 @@ struct VRArgs {
   const double *Vb, *t1, *fvo, *ovs, *t2s;  // ovs, t2s: pair-symmetrised blocks (OrbitArgs)
   int o, v, i, j, k, has_fvo;
   double *R;            // scratch: vr_scratch_doubles(v) (layout in kernels)
+  int parts;            // parts the sums are split into: kVRS, or 1 for a batch
+  // a batch when tri is set: nb triples tri[b], Vb one v^3 block and R r_stride
+  // doubles per triple
+  const int *tri;
+  int nb;
+  size_t r_stride;
 };
 
 // Per-triple gather of the adjoint pieces into the output cotangents.

@@ -28,6 +28,7 @@
 #include <mutex>
 #include "ccsdt_common.h"
 #include "gemm_desc.h"
+#include "walk64.h"
 #include "../../include/pyscfad_amd_ccsdt.h"
 #include "../../include/pyscfad_amd_debug.h"
 
@@ -483,6 +484,8 @@ static int build_w(const Ctx &c, int i, int j, int k, int nb = 1) {
 static int adjoint_vr(const Ctx &c, int i, int j, int k, hipStream_t st) {
   const double v3 = (double)c.v * c.v * c.v;
   VRArgs vr;
+  memset(&vr, 0, sizeof(vr));
+  vr.parts = kVRS;
   vr.Vb = c.Vb;
   vr.t1 = c.t1;
   vr.fvo = c.fvo;
@@ -1231,6 +1234,223 @@ static void bind_workspace(Ctx &c, const Layout &L, void *ws) {
 }
 
 // ---------------------------------------------------------------------------
+// Batched FP64 walk (walk64.h): nb triples per launch.
+// ---------------------------------------------------------------------------
+constexpr size_t kNoAllocScratchBytes = (size_t)128 << 20;
+
+struct WalkLayout {
+  WalkDims d;
+  int nb, S, G;
+  size_t r_stride, total;
+  size_t off_VT, off_TB, off_TBt, off_OVS, off_T2S, off_t1, off_fvo, off_mo, off_orb, off_tri_e, off_tab, off_wt,
+      off_W, off_part_t, off_Vb, off_VTb, off_R, off_part, off_vec, off_mo_rows, off_mo2;
+};
+
+static long long num_triples(int o) { return (long long)o * (o + 1) * (o + 2) / 6 - o; }
+
+static WalkLayout walk_layout(int o, int v, int vjp, int nb) {
+  WalkLayout L;
+  memset(&L, 0, sizeof(L));
+  L.d = walk_dims(o, v);
+  L.nb = nb;
+  const size_t vp = L.d.vp, up = L.d.up, v2 = vp * vp, n = (size_t)o + vp, oo = (size_t)o * o;
+  const size_t nt = vp / 8, norb = nt * (nt + 1) * (nt + 2) / 6;
+  size_t off = 0;
+  auto take = [&](size_t count) {
+    const size_t at = off;
+    off = align256(off + count * sizeof(double));
+    return at;
+  };
+  // parts of TB's adjoint: enough tiles for 16 rounds of the 1024 SIMDs, each
+  // part at least 8 outer steps
+  const long long tiles = 6LL * nb * ((vp + 15) / 16) * ((up + 15) / 16);
+  L.S = (int)std::max(1LL, std::min({(16 * 1024 + tiles - 1) / tiles, (long long)vp / 8, 8LL}));
+  // orbit epilogue: about four rounds of workgroups per launch
+  L.G = (int)std::max<size_t>(1, std::min<size_t>({(2048 + (size_t)nb - 1) / nb, norb, (size_t)kGmax}));
+  L.off_VT = take((size_t)o * vp * L.d.sp);
+  if (vjp) L.off_TB = take(oo * vp * up);
+  L.off_TBt = take(oo * vp * up);
+  L.off_OVS = take(oo * v2);
+  L.off_T2S = take(oo * v2);
+  L.off_t1 = take((size_t)o * vp);
+  L.off_fvo = take((size_t)o * vp);
+  L.off_mo = take(n);
+  L.off_orb = take(norb);
+  L.off_tri_e = take(oo * o);
+  // every shard's table fits: at most one run and one batch's round more
+  L.off_tab = take((size_t)(num_triples(o) + kWalkMaxBatch + 2 * kWalkRun) / 2 + 1);
+  L.off_wt = take(o);
+  L.off_W = take(vp * L.d.ws * nb);
+  L.off_part_t = take((size_t)nb * L.G);
+  if (vjp) {
+    L.off_Vb = take(v2 * vp * nb);
+    L.off_VTb = take((size_t)o * vp * L.d.sp);
+    L.r_stride = vr_col_blocks((int)vp) > 1 ? vr_scratch_doubles((int)vp) : 10 * v2 + 2 * vp;
+    L.off_R = take(L.r_stride * nb);
+    L.off_part = take((size_t)nb * 6 * L.S * vp * up);
+    L.off_vec = take((size_t)nb * 6 * vp);
+    L.off_mo_rows = take((size_t)nb * L.G * n);
+    L.off_mo2 = take((size_t)kWalkMoParts * n);
+  }
+  L.total = off;
+  return L;
+}
+
+// The batch of a call: as many triples as fit the library's own scratch
+// together with the rest when these are all, or 32 (so that the calls with and
+// without a workspace of their own split the walk alike and agree bit for bit),
+// else as many as 8 GB of blocks hold; fewer when `limit` bytes are there.
+// False when the walk does not apply: slabs beyond 32-bit offsets, not even one
+// run in `limit`, or a workspace noticeably larger than the one-triple walk's
+// where that is large itself.
+static bool walk_pick(int o, int v, int vjp, size_t limit, size_t one_triple_total, WalkLayout &L) {
+  if (!walk_dims_ok(walk_dims(o, v))) return false;
+  // batch sizes: whole runs
+  const int n = (int)std::min<long long>((num_triples(o) + kWalkRun - 1) / kWalkRun * kWalkRun, kWalkMaxBatch);
+  auto largest = [&](size_t bytes) {
+    int b = std::max(n, kWalkRun);
+    while (b > 0 && walk_layout(o, v, vjp, b).total > bytes) b -= kWalkRun;
+    return b;
+  };
+  int b = largest(kNoAllocScratchBytes);
+  if (b < std::min(n, 32))
+    b = std::max(kWalkRun, largest(walk_layout(o, v, vjp, kWalkRun).total + ((size_t)8 << 30)));
+  if (walk_layout(o, v, vjp, b).total > limit) b = largest(limit);
+  if (b < kWalkRun) return false;
+  L = walk_layout(o, v, vjp, walk_batches(num_triples(o), b).cap);
+  return L.total <= ((size_t)100 << 30) || L.total <= one_triple_total + one_triple_total / 20;
+}
+
+// One call's walk on its stream c.s: c.tri gets the triple energies, and with
+// c.vjp every cotangent is complete.
+static int run_walk(Ctx &c, const WalkLayout &L, void *ws, double *ovvv_bar, double *mo_bar) {
+  char *b = (char *)ws;
+  auto at = [&](size_t off) { return (double *)(b + off); };
+  const WalkDims &d = L.d;
+  const int o = d.o;
+  const hipStream_t s = c.s;
+  double *VT = at(L.off_VT), *TB = c.vjp ? at(L.off_TB) : nullptr, *TBt = at(L.off_TBt), *W = at(L.off_W);
+  int *tab = (int *)at(L.off_tab);
+  unsigned short *orb = (unsigned short *)at(L.off_orb);
+  c.tri = at(L.off_tri_e);
+  c.wt = at(L.off_wt);
+  PAMD_CHECK(launch_walk_inputs(d, c.mo, c.t1, c.t2, c.ovvv, c.packed, c.ovoo, c.ovov,
+                                c.has_fvo ? c.fvo : nullptr, VT, TB, TBt, at(L.off_OVS), at(L.off_T2S),
+                                at(L.off_t1), at(L.off_fvo), at(L.off_mo), s));
+  const long long n = (num_triples(o) - c.shard + c.nshards - 1) / c.nshards;
+  const WalkBatches wb = walk_batches(n, L.nb);
+  PAMD_CHECK(launch_walk_triples(o, c.shard, c.nshards, wb, tab, s));
+  PAMD_CHECK(launch_fill(c.tri, (size_t)o * o * o, 0.0, s));
+  const long long nt = d.vp / 8, norb = nt * (nt + 1) * (nt + 2) / 6;
+  PAMD_CHECK(launch_orbit_table(norb, orb, s));
+  const size_t rows = (size_t)L.nb * L.G;
+  if (c.vjp) PAMD_CHECK(launch_fill(at(L.off_mo_rows), rows * (o + d.vp), 0.0, s));
+  if (c.wt_host)
+    PAMD_CHECK(hipMemcpyAsync(c.wt, c.wt_host, sizeof(double) * (size_t)o, hipMemcpyHostToDevice, s));
+  const auto t_start = std::chrono::steady_clock::now();
+  const double v3 = (double)c.v * c.v * c.v, fl = 12.0 * v3 * (c.v + o);  // one family, per triple
+  long long reported = 0, t0 = 0;
+  // without triples one empty batch writes the (zero) cotangents
+  for (int bt = 0; bt < wb.count; t0 += wb.size(bt), ++bt) {
+    const int nb = wb.size(bt);
+    const int *tri = tab + (size_t)bt * wb.cap;
+    g_prof_on = g_prof_every > 0 && (t0 + g_prof_every - 1) / g_prof_every * g_prof_every < t0 + nb;
+    if (nb > 0) {
+      PAMD_CHECK(timed(s, kProfWBuild, fl * nb, 0.0, [&] { return launch_walk_w(d, VT, TBt, W, tri, nb, s); }));
+      OrbitArgs oa;
+      memset(&oa, 0, sizeof(oa));
+      oa.W = W;
+      oa.tab = orb;
+      oa.Vb = c.vjp ? at(L.off_Vb) : nullptr;
+      oa.t1 = at(L.off_t1);
+      oa.ovs = at(L.off_OVS);
+      oa.t2s = at(L.off_T2S);
+      oa.fvo = at(L.off_fvo);
+      oa.mo = at(L.off_mo);
+      oa.o = o;
+      oa.v = d.vp;
+      oa.has_fvo = c.has_fvo;
+      oa.vjp = c.vjp;
+      oa.norb = norb;
+      oa.ebar = c.ebar;
+      oa.part_t = at(L.off_part_t);
+      oa.part_mo = c.vjp ? at(L.off_mo_rows) : nullptr;
+      oa.tri = tri;
+      oa.nb = nb;
+      oa.ws = d.ws;
+      oa.wt = c.wt_host ? c.wt : nullptr;
+      const double ob = 8.0 * v3 * (c.vjp ? 3.0 : 1.0) * nb;
+      PAMD_CHECK(timed(s, kProfOrbit, 0.0, ob, [&] { return launch_orbit(oa, L.G, s, kOrbitBatch); }));
+    }
+    if (!c.vjp) {
+      PAMD_CHECK(launch_walk_energies(tri, nb, o, at(L.off_part_t), L.G, c.tri, s));
+    } else {
+      if (nb > 0) {
+        VRArgs vr;
+        memset(&vr, 0, sizeof(vr));
+        vr.Vb = at(L.off_Vb);
+        vr.t1 = at(L.off_t1);
+        vr.fvo = at(L.off_fvo);
+        vr.ovs = at(L.off_OVS);
+        vr.t2s = at(L.off_T2S);
+        vr.o = o;
+        vr.v = d.vp;
+        vr.has_fvo = c.has_fvo;
+        vr.R = at(L.off_R);
+        vr.parts = 1;
+        vr.tri = tri;
+        vr.nb = nb;
+        vr.r_stride = L.r_stride;
+        PAMD_CHECK(timed(s, kProfVR, 0.0, 16.0 * v3 * nb, [&] { return launch_vr(vr, s); }));
+      }
+      PAMD_CHECK(timed(s, kProfAdjOvvv, fl * nb, 0.0, [&] {
+        return launch_walk_vtb(d, W, TB, at(L.off_VTb), tri, nb, t0 == 0, s);
+      }));
+      if (nb > 0)
+        PAMD_CHECK(timed(s, kProfAdjT2P, fl * nb, 0.0, [&] {
+          return launch_walk_tbb(d, W, VT, at(L.off_part), tri, nb, L.S, s);
+        }));
+      WalkGather g;
+      g.d = d;
+      g.tri = tri;
+      g.nb = nb;
+      g.S = L.S;
+      g.G = L.G;
+      g.has_fvo = c.has_fvo;
+      g.first = t0 == 0;
+      g.part = at(L.off_part);
+      g.R = at(L.off_R);
+      g.r_stride = L.r_stride;
+      g.part_t = at(L.off_part_t);
+      g.vec = at(L.off_vec);
+      g.t1_bar = c.t1_bar;
+      g.t2_bar = c.t2_bar;
+      g.ovoo_bar = c.ovoo_bar;
+      g.ovov_bar = c.ovov_bar;
+      g.fvo_bar = c.fvo_bar;
+      g.tri_e = c.tri;
+      const double cb = 8.0 * 6.0 * L.S * (double)d.vp * d.up * nb;
+      PAMD_CHECK(timed(s, kProfCombine, 0.0, cb, [&] { return launch_walk_gather(g, s); }));
+    }
+    if (g_progress_every > 0 && (t0 + nb - reported >= g_progress_every || t0 + nb == n)) {
+      reported = t0 + nb;
+      PAMD_CHECK(hipStreamSynchronize(s));
+      const double el =
+          std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
+      fprintf(stderr, "pyscfad_amd: (T)%s triples %lld/%lld done, %.1f s\n", c.vjp ? "+VJP" : "", t0 + nb, n,
+              el);
+      fflush(stderr);
+    }
+  }
+  g_prof_on = false;
+  if (!g_prof_recs.empty()) PAMD_CHECK(prof_collect());
+  if (c.vjp)
+    PAMD_CHECK(launch_walk_finish(d, at(L.off_VTb), c.packed, ovvv_bar, c.t2_bar, at(L.off_mo_rows),
+                                  (int)rows, at(L.off_mo2), mo_bar, s));
+  return PAMD_OK;
+}
+
+// ---------------------------------------------------------------------------
 // Library-owned scratch for pamd_ccsdt_energy_vjp_noalloc: the workspace of
 // pamd_ccsdt_energy_vjp in a file-scope device array, so that call allocates
 // nothing.  Each GPU holds its own copy for the life of the process; its
@@ -1238,7 +1458,6 @@ static void bind_workspace(Ctx &c, const Layout &L, void *ws) {
 // current) and kept per device.  The host-side name `scratch` is never passed
 // to a kernel or a copy: only the looked-up address is.
 // ---------------------------------------------------------------------------
-constexpr size_t kNoAllocScratchBytes = (size_t)128 << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -1281,6 +1500,10 @@ const char *pamd_version(void) { return "pyscfad_amd 0.1.0 (gfx950)"; }
 int pamd_ccsdt_workspace_size(const pamd_ccsdt_config *cfg, int with_vjp, size_t *bytes) {
   if (!cfg || !bytes || cfg->nocc < 1 || cfg->nvir < 1) return PAMD_ERR_ARG;
   *bytes = make_layout(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, cfg->precision, true).total;
+  WalkLayout wl;
+  if (cfg->precision == PAMD_PREC_FP64 &&
+      walk_pick(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, (size_t)-1, *bytes, wl))
+    *bytes = std::max(*bytes, wl.total);
   return PAMD_OK;
 }
 
@@ -1309,6 +1532,9 @@ static int energy_impl(const pamd_ccsdt_config *cfg, const double *mo, const dou
   c.fvo = fvo;
   c.shard = shard;
   c.nshards = nshards;
+  WalkLayout wl;
+  if (c.prec == PAMD_PREC_FP64 && walk_pick(c.o, c.v, 0, ws_bytes, L.total, wl))
+    return run_walk(c, wl, ws, nullptr, nullptr);
   bind_workspace(c, L, ws);
   return run(c);
 }
@@ -1401,17 +1627,25 @@ static int vjp_impl(const pamd_ccsdt_config *cfg, const double *mo_energy, const
   c.fvo_bar = fvo_bar;
   c.shard = shard;
   c.nshards = nshards;
-  bind_workspace(c, L, workspace);
-  st = run(c);
+  WalkLayout wl;
+  const bool walk = c.prec == PAMD_PREC_FP64 && walk_pick(c.o, c.v, 1, workspace_bytes, L.total, wl);
+  if (walk) {
+    st = run_walk(c, wl, workspace, ovvv_bar, mo_energy_bar);
+  } else {
+    bind_workspace(c, L, workspace);
+    st = run(c);
+  }
   if (st != PAMD_OK) return st;
   const int o = c.o, v = c.v;
   if (wt_host) {
-    PAMD_CHECK(hipMemcpyAsync(c.wt, wt_host, sizeof(double) * (size_t)o, hipMemcpyHostToDevice,
-                              c.s));
+    if (!walk)
+      PAMD_CHECK(hipMemcpyAsync(c.wt, wt_host, sizeof(double) * (size_t)o, hipMemcpyHostToDevice,
+                                c.s));
     PAMD_CHECK(launch_weighted_energy(c.tri, o, c.wt, et_bar, e_out, wt_bar, c.s));
   } else {
     PAMD_CHECK(launch_total_energy(c.tri, o, e_out, c.s));
   }
+  if (walk) return PAMD_OK;
   PAMD_CHECK(launch_reduce_rows(c.part_mo, c.G, o + v, mo_energy_bar, 0, c.s));
   PAMD_CHECK(launch_fold_ovvv(c.Vpb, o, v, c.packed, ovvv_bar, c.s));
   PAMD_CHECK(launch_fold_t2m(c.T2mb, o, v, t2_bar, c.s));

@@ -19,6 +19,7 @@
 #include "ccsdt_common.h"
 #include "engine_staging.h"
 #include "bf16_split.h"
+#include "vr_layout.h"
 
 namespace pamd {
 
@@ -556,6 +557,8 @@ hipError_t launch_orbit_table(long long norb, unsigned short *tab, hipStream_t s
 // tile axes reduce within the wave; the per-wave sums are then added over the
 // waves in a fixed order (no atomics), so every output is bitwise reproducible.
 // Modes: kOrbitPlain -- energy, and for the adjoint the Wbar/Vbar/dE/de seeds;
+// kOrbitBatch -- the plain mode for the nb triples of A.tri, grid row y taking
+// triple y with its own W and Vbar blocks and rows of part_t and part_mo;
 // kOrbitProjAcc -- accA[f] += u_f W, accB[f] += u_f Z/D (projected walk);
 // kOrbitProjVjp -- seeds of the projected energy from the finished accA, accB
 // of the pair: Q = g sum_f u_f accA[f] (dE/dY), P = g sum_f u_f accB[f]
@@ -574,10 +577,22 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int o = A.o, v = A.v, n = o + v;
-  const int i = A.i, j = A.j, k = A.k;
+  int i = A.i, j = A.j, k = A.k;
+  double omega = A.omega;
+  if constexpr (MODE == kOrbitBatch) {
+    const int t = A.tri[blockIdx.y];
+    i = t & 1023;
+    j = (t >> 10) & 1023;
+    k = t >> 20;
+    omega = (i == j || j == k) ? 1.0 : 2.0;
+    if (A.wt) omega *= (A.wt[i] + A.wt[j] + A.wt[k]) / 3.0;
+    A.W += (size_t)blockIdx.y * v * A.ws;
+    if (A.vjp) A.Vb += (size_t)blockIdx.y * v * v * v;
+  }
+  const size_t row = MODE == kOrbitBatch ? (size_t)blockIdx.y * gridDim.x + blockIdx.x : blockIdx.x;
   const double eo = A.mo[i] + A.mo[j] + A.mo[k];
   const double *ev = A.mo + o;
-  const double g = A.ebar * A.omega;
+  const double g = A.ebar * omega;
   for (int x = tid; x < v; x += 512) vir[x] = 0.0;
   __syncthreads();
 
@@ -627,7 +642,7 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
       const int ps = p < pq.np ? p : 0;
       const int ar = min(vq[pq.sel[ps][0]] * OT + al, v - 1), br = min(vq[pq.sel[ps][1]] * OT + be, v - 1),
                 cr = min(vq[pq.sel[ps][2]] * OT + ga, v - 1);
-      w[p] = A.W[((long long)ar * v + br) * v + cr];
+      w[p] = A.W[MODE == kOrbitBatch ? ar * A.ws + br * v + cr : ((long long)ar * v + br) * v + cr];
     }
   };
   double wnext[6];
@@ -769,7 +784,7 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
             else if (A.Wb8)
               A.Wb8[idx] = split2(wbar).u;
             else
-              A.W[idx] = wbar;
+              A.W[MODE == kOrbitBatch ? a * A.ws + b * v + c : idx] = wbar;
             A.Vb[idx] = vbar;
             dbar = -g * w0 * Z * rD * rD;
             occ += dbar;
@@ -842,7 +857,7 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
   __syncthreads();
   double otot = 0.0;
   for (int w = 0; w < 8; ++w) otot += red[w];
-  if (tid == 0) A.part_t[blockIdx.x] = etot;
+  if (tid == 0) A.part_t[row] = etot;
   if constexpr (MODE == kOrbitProjVjp) {
     // per-workgroup sums of <W, accB[f]> + <accA[f], Z/D>, wave order fixed
 #pragma unroll
@@ -859,8 +874,8 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
       A.part_u[(size_t)blockIdx.x * kMaxFrag + tid] = s_;
     }
   }
-  if (MODE == kOrbitProjVjp || (MODE == kOrbitPlain && A.vjp)) {
-    double *pm = A.part_mo + (size_t)blockIdx.x * n;
+  if (MODE == kOrbitProjVjp || ((MODE == kOrbitPlain || MODE == kOrbitBatch) && A.vjp)) {
+    double *pm = A.part_mo + row * n;
     for (int x = tid; x < v; x += 512) pm[o + x] += vir[x];
     if (tid == 0) {
       pm[i] += otot;
@@ -896,6 +911,8 @@ hipError_t launch_orbit(const OrbitArgs &a, int grid, hipStream_t s, int mode) {
     hipLaunchKernelGGL(k_orbit<kOrbitProjAcc>, dim3(grid), dim3(512), sizeof(double) * a.v, s, a);
   else if (mode == kOrbitProjVjp)
     hipLaunchKernelGGL(k_orbit<kOrbitProjVjp>, dim3(grid), dim3(512), sizeof(double) * a.v, s, a);
+  else if (mode == kOrbitBatch)
+    hipLaunchKernelGGL(k_orbit<kOrbitBatch>, dim3(grid, a.nb), dim3(512), sizeof(double) * a.v, s, a);
   else
     hipLaunchKernelGGL(k_orbit<kOrbitPlain>, dim3(grid), dim3(512), sizeof(double) * a.v, s, a);
   return hipGetLastError();
@@ -975,49 +992,6 @@ __device__ double block_sum_vr(double x, double *scratch) {
   return r;
 }
 
-// Part s of kVRS of the b-sums (k_vr_a) and a-sums (k_vr_b): arrays that are
-// sums over the split index are written per part; part 0 uses the slots of R
-// listed above, parts 1.. an extension after them (vr_part, vr_part_vec).  The
-// vectors have kVRS x ncb parts (index cb * kVRS + s); blocks 0, 1, 8, 9 have
-// ncb parts (vr_cpart), column block cb >= 1 in a second extension.
-__device__ __forceinline__ double *vr_part(double *R, int v, int s, int q) {
-  const size_t vv = (size_t)v * v;
-  if (s == 0) return R + (size_t)q * vv;
-  return R + 10 * vv + 2 * (size_t)v + ((size_t)(s - 1) * 6 + (q - 2)) * vv;
-}
-__device__ __forceinline__ double *vr_part_vec(double *R, int v, int s, int which) {
-  const size_t vv = (size_t)v * v;
-  if (s == 0) return R + 10 * vv + (size_t)which * v;
-  return R + 10 * vv + 2 * (size_t)v + (size_t)(kVRS - 1) * 6 * vv + ((size_t)(s - 1) * 2 + which) * v;
-}
-__device__ __forceinline__ double *vr_cpart(double *R, int v, int cb, int q) {
-  const size_t vv = (size_t)v * v;
-  if (cb == 0) return R + (size_t)q * vv;
-  const int slot = q < 2 ? q : q - 6;  // 0, 1, 8, 9 -> 0, 1, 2, 3
-  return R + 10 * vv + 2 * (size_t)v + (size_t)(kVRS - 1) * 6 * vv +
-         (size_t)(kVRS * vr_col_blocks(v) - 1) * 2 * v + ((size_t)(cb - 1) * 4 + slot) * vv;
-}
-
-// sums over the parts, in part order
-__device__ __forceinline__ double vr_sum(const double *R, int v, int q, size_t idx) {
-  double x = 0.0;
-#pragma unroll
-  for (int s = 0; s < kVRS; ++s) x += vr_part(const_cast<double *>(R), v, s, q)[idx];
-  return x;
-}
-__device__ __forceinline__ double vr_sum_vec(const double *R, int v, int which, int idx) {
-  double x = 0.0;
-  const int np = kVRS * vr_col_blocks(v);
-  for (int s = 0; s < np; ++s) x += vr_part_vec(const_cast<double *>(R), v, s, which)[idx];
-  return x;
-}
-__device__ __forceinline__ double vr_csum(const double *R, int v, int q, size_t idx) {
-  double x = 0.0;
-  const int ncb = vr_col_blocks(v);
-  for (int cb = 0; cb < ncb; ++cb) x += vr_cpart(const_cast<double *>(R), v, cb, q)[idx];
-  return x;
-}
-
 // LDS of the V-bar reductions (one launch runs both kinds of workgroup)
 struct VRLds {
   double red[kVRW * kVRC];
@@ -1050,7 +1024,7 @@ __device__ __forceinline__ void vr_a_block(const VRArgs &A, VRLds &L, int a, int
   for (int qq = 0; qq < kMaxVQ; ++qq) r3[qq] = r4[qq] = pk[qq] = fk[qq] = 0.0;
   double t1i = 0.0, fvoi = 0.0;
   double *R = A.R;
-  for (int b = wave + kVRW * part; b < v; b += kVRW * kVRS) {
+  for (int b = wave + kVRW * part; b < v; b += kVRW * A.parts) {
     const double t1j = t1[j * v + b];
     const double S1 = SYM(ovs, i, j, a, b);
     const double fvj = FVO ? fvo[b * o + j] : 0.0;
@@ -1110,7 +1084,7 @@ __device__ __forceinline__ void vr_b_block(const VRArgs &A, VRLds &L, int b, int
   double r5[kMaxVQ], r6[kMaxVQ];
 #pragma unroll
   for (int qq = 0; qq < kMaxVQ; ++qq) r5[qq] = r6[qq] = 0.0;
-  for (int a = wave + kVRW * part; a < v; a += kVRW * kVRS) {
+  for (int a = wave + kVRW * part; a < v; a += kVRW * A.parts) {
     const double t1a = A.t1[i * v + a];
     const double fa = FVO ? A.fvo[a * o + i] : 0.0;
     const double *row = A.Vb + (size_t)a * vv + (size_t)b * v + c0;
@@ -1129,20 +1103,31 @@ __device__ __forceinline__ void vr_b_block(const VRArgs &A, VRLds &L, int b, int
 }
 #undef PAMD_WAVE_COMBINE
 
-// both V-bar reductions in one launch: blockIdx.y < kVRS runs part y of the
-// b-sums, the rest part y - kVRS of the a-sums
+// both V-bar reductions in one launch: blockIdx.y < parts runs part y of the
+// b-sums, the rest part y - parts of the a-sums
 template <bool FVO>
 __global__ __launch_bounds__(64 * kVRW) void k_vr(VRArgs A) {
   __shared__ VRLds L;
   const int y = blockIdx.y;
-  if (y < kVRS)
-    vr_a_block<FVO>(A, L, blockIdx.x, y, blockIdx.z);
+  int cb = blockIdx.z;
+  if (A.tri) {  // a batch: grid z runs over (triple, column block)
+    const int ncb = vr_col_blocks(A.v), b = cb / ncb;
+    cb -= b * ncb;
+    const int t = A.tri[b];
+    A.i = t & 1023;
+    A.j = (t >> 10) & 1023;
+    A.k = t >> 20;
+    A.Vb += (size_t)b * A.v * A.v * A.v;
+    A.R += b * A.r_stride;
+  }
+  if (y < A.parts)
+    vr_a_block<FVO>(A, L, blockIdx.x, y, cb);
   else
-    vr_b_block<FVO>(A, L, blockIdx.x, y - kVRS, blockIdx.z);
+    vr_b_block<FVO>(A, L, blockIdx.x, y - A.parts, cb);
 }
 
 hipError_t launch_vr(const VRArgs &a, hipStream_t s) {
-  const dim3 grid(a.v, 2 * kVRS, vr_col_blocks(a.v)), block(64 * kVRW);
+  const dim3 grid(a.v, 2 * a.parts, vr_col_blocks(a.v) * (a.tri ? a.nb : 1)), block(64 * kVRW);
   if (a.has_fvo)
     hipLaunchKernelGGL(k_vr<true>, grid, block, 0, s, a);
   else

@@ -1,0 +1,113 @@
+// The batched FP64 walk: many occupied triples per launch.
+//
+// Joined arrays.  The particle and the hole term of w_abc[ijk]
+// (pyscfadlib/pyscfadlib/vjp/cc/ccsd_t.c:121-142) contract over f (virtual) and m
+// (occupied) alike, so with
+//   VT[x][p][q][f] = ovvv[x,p,f,q],  VT[x][p][q][v + m] = t2[x,m,p,q]
+//   TB[z][y][r][f] = t2[z,y,r,f],    TB[z][y][r][v + m] = -ovoo[z,r,m,y]
+// the twelve terms of W_ijk are six products over one index k < v + o:
+//   W[a,b,c] = VT[i][a][b] TB[k,j][c] + VT[i][a][c] TB[j,k][b] + VT[j][b][a] TB[k,i][c]
+//            + VT[j][b][c] TB[i,k][a] + VT[k][c][a] TB[j,i][b] + VT[k][c][b] TB[i,j][a],
+// the adjoint of VT collects dE/d ovvv with the hole-term part of dE/d t2, and
+// that of TB the particle-term part of dE/d t2 with dE/d ovoo.
+//
+// Padded space.  Virtual extents are padded to vp = 8 ceil(v / 8), the joined
+// one to up = 8 ceil((v + o) / 8), with zeros: W and Wbar vanish there by
+// themselves, every extent is a multiple of 8, rows are 16-byte aligned, and
+// no kernel has a tail.
+#pragma once
+#include "ccsdt_common.h"
+
+namespace pamd {
+
+constexpr int kWalkMaxBatch = 256;  // triples per batch: 10 bits of slot would do for 1024
+
+//
+// Slabs: VT[x][p] (vp x up) and W[a] (vp x vp) start an odd multiple of 256
+// bytes apart (sp, ws elements).  L2 interleaves its 16 channels every 256
+// bytes, and the walk reads 16 rows one slab apart at once: with vp = 160 a
+// slab is a multiple of 4096 bytes, and all 16 rows would come from one channel.
+struct WalkDims {
+  int o, v, vp, up;
+  long long sp, ws;
+};
+inline WalkDims walk_dims(int o, int v) {
+  const int vp = (v + 7) / 8 * 8, up = (v + o + 7) / 8 * 8;
+  auto odd = [](long long n) { return ((n + 31) / 32 | 1) * 32; };
+  return {o, v, vp, up, odd((long long)vp * up), odd((long long)vp * vp)};
+}
+// 32-bit byte offsets within one occupied slab of VT
+inline bool walk_dims_ok(const WalkDims &d) {
+  return (d.vp + 8) * d.sp * 8 < (1LL << 32);
+}
+
+// padded inputs of the walk (TBt[z][y][k][r] = TB[z][y][r][k])
+hipError_t launch_walk_inputs(const WalkDims &d, const double *mo, const double *t1, const double *t2,
+                              const double *ovvv, int packed, const double *ovoo, const double *ovov,
+                              const double *fvo, double *VT, double *TB, double *TBt, double *OVS,
+                              double *T2S, double *t1p, double *fvop, double *mop, hipStream_t s);
+// Batches.  The call's triples (walk order i <= j <= k without i == j == k, every
+// nshards-th from shard on) are cut into runs of 8, dealt to the batches in
+// turn: a run shares i, j and so its slabs of VT, while every batch has about
+// the same number of triples with each x, over which the adjoint of VT[x]
+// sums.  (Batches of consecutive triples hold one i nearly throughout: that
+// adjoint took 288 instead of 63 ms at o16/v160.)
+constexpr int kWalkRun = 8;
+struct WalkBatches {
+  int cap;          // slots of a batch in the table (a multiple of 8)
+  int count;        // batches
+  long long n;      // triples
+  int size(int b) const {
+    const long long runs = (n + kWalkRun - 1) / kWalkRun;
+    if (b >= runs) return 0;
+    const long long mine = (runs - b + count - 1) / count, last = b + (mine - 1) * count;
+    const long long cut = last == runs - 1 ? runs * kWalkRun - n : 0;
+    return (int)(mine * kWalkRun - cut);
+  }
+};
+inline WalkBatches walk_batches(long long n, int nb) {
+  const long long runs = (n + kWalkRun - 1) / kWalkRun, per = nb / kWalkRun > 0 ? nb / kWalkRun : 1;
+  const int count = (int)(runs > 0 ? (runs + per - 1) / per : 1);
+  const int cap = (int)((runs + count - 1) / count) * kWalkRun;
+  return {cap > 0 ? cap : kWalkRun, count, n};
+}
+// tri[b cap + slot] = i | j << 10 | k << 20
+hipError_t launch_walk_triples(int o, int shard, int nshards, const WalkBatches &wb, int *tri, hipStream_t s);
+
+// W of nb triples (tri[0 .. nb)), each a block of vp ws elements
+hipError_t launch_walk_w(const WalkDims &d, const double *VT, const double *TBt, double *W, const int *tri,
+                         int nb, hipStream_t s);
+// VTb += dE/dVT of nb triples (Wb: their Wbar blocks); first: VTb is overwritten
+hipError_t launch_walk_vtb(const WalkDims &d, const double *Wb, const double *TB, double *VTb,
+                           const int *tri, int nb, bool first, hipStream_t s);
+// part[b][pr][sp]: part sp of S of the vp x up block that triple b adds to TB's
+// adjoint at [k,j], [j,k], [k,i], [i,k], [j,i], [i,j] (pr = 0 .. 5)
+hipError_t launch_walk_tbb(const WalkDims &d, const double *Wb, const double *VT, double *part,
+                           const int *tri, int nb, int S, hipStream_t s);
+
+// gather of a batch into the cotangents (overwritten when first)
+struct WalkGather {
+  WalkDims d;
+  const int *tri;
+  int nb, S, G, has_fvo, first;
+  const double *part;       // launch_walk_tbb
+  const double *R;          // V-bar reductions, r_stride doubles per triple
+  size_t r_stride;
+  const double *part_t;     // [nb][G] energy sums of the orbit epilogue
+  double *vec;              // scratch [nb][6][vp]
+  double *t1_bar, *t2_bar, *ovoo_bar, *ovov_bar, *fvo_bar, *tri_e;
+};
+hipError_t launch_walk_gather(const WalkGather &g, hipStream_t s);
+// tri_e of nb triples from the orbit epilogue's G sums each
+hipError_t launch_walk_energies(const int *tri, int nb, int o, const double *part_t, int G, double *tri_e,
+                                hipStream_t s);
+
+// at exit: ovvv_bar from VTb, its hole part added to t2_bar, and
+// mo_energy_bar from the rows of part_mo (o + vp columns; part2: scratch of
+// kWalkMoParts (o + vp))
+constexpr int kWalkMoParts = 64;
+hipError_t launch_walk_finish(const WalkDims &d, const double *VTb, int packed, double *ovvv_bar,
+                              double *t2_bar, const double *part_mo, int rows, double *part2,
+                              double *mo_bar, hipStream_t s);
+
+}  // namespace pamd
