@@ -128,8 +128,12 @@ struct OrbitArgs {
   // part_mo G rows per triple; wt: occupied weights of a diagonal projector or null
   const int *tri;
   int nb;
-  long long ws;  // element stride of W's first index (v^2 otherwise)
+  long long ws;  // element stride of W's first index (v^2 in the plain mode)
   const double *wt;
+  // projected modes: with tri set a batch of pairs (see k_orbit), ulo on the
+  // device; acc_first: accA, accB are overwritten
+  const double *udev;
+  int acc_first;
 };
 
 enum OrbitMode { kOrbitPlain = 0, kOrbitProjAcc = 1, kOrbitProjVjp = 2, kOrbitBatch = 3 };

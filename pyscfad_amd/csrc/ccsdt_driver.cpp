@@ -827,6 +827,7 @@ static int run_projected(Ctx &c, const double *ulo, int nfrag, double *accA, dou
         st = build_w(c, l, j, k);
         if (st != PAMD_OK) return st;
         OrbitArgs oa = orbit_args(c, l, j, k, norb);
+        oa.ws = (long long)c.v * c.v;
         oa.accA = accA;
         oa.accB = accB;
         oa.nfrag = nfrag;
@@ -850,6 +851,7 @@ static int run_projected(Ctx &c, const double *ulo, int nfrag, double *accA, dou
         wbar_out(c, fmt, oa);
         oa.vjp = 1;
         oa.ebar = g;
+        oa.ws = (long long)c.v * c.v;
         oa.accA = accA;
         oa.accB = accB;
         oa.nfrag = nfrag;
@@ -1321,133 +1323,296 @@ static bool walk_pick(int o, int v, int vjp, size_t limit, size_t one_triple_tot
   return L.total <= ((size_t)100 << 30) || L.total <= one_triple_total + one_triple_total / 20;
 }
 
+// Inputs, orbit table and zeroed row sums of a call; returns the orbit count.
+static int walk_setup(Ctx &c, const WalkLayout &L, char *b, long long &norb) {
+  auto at = [&](size_t off) { return (double *)(b + off); };
+  const WalkDims &d = L.d;
+  c.tri = at(L.off_tri_e);
+  c.wt = at(L.off_wt);
+  PAMD_CHECK(launch_walk_inputs(d, c.mo, c.t1, c.t2, c.ovvv, c.packed, c.ovoo, c.ovov,
+                                c.has_fvo ? c.fvo : nullptr, at(L.off_VT), c.vjp ? at(L.off_TB) : nullptr,
+                                at(L.off_TBt), at(L.off_OVS), at(L.off_T2S), at(L.off_t1), at(L.off_fvo),
+                                at(L.off_mo), c.s));
+  const long long nt = d.vp / 8;
+  norb = nt * (nt + 1) * (nt + 2) / 6;
+  PAMD_CHECK(launch_orbit_table(norb, (unsigned short *)at(L.off_orb), c.s));
+  if (c.vjp)
+    PAMD_CHECK(launch_fill(at(L.off_mo_rows), (size_t)L.nb * L.G * (d.o + d.vp), 0.0, c.s));
+  return PAMD_OK;
+}
+
+static OrbitArgs walk_orbit_args(const Ctx &c, const WalkLayout &L, char *b, const int *tri, int nb,
+                                 long long norb) {
+  auto at = [&](size_t off) { return (double *)(b + off); };
+  OrbitArgs oa;
+  memset(&oa, 0, sizeof(oa));
+  oa.W = at(L.off_W);
+  oa.tab = (const unsigned short *)at(L.off_orb);
+  oa.Vb = c.vjp ? at(L.off_Vb) : nullptr;
+  oa.t1 = at(L.off_t1);
+  oa.ovs = at(L.off_OVS);
+  oa.t2s = at(L.off_T2S);
+  oa.fvo = at(L.off_fvo);
+  oa.mo = at(L.off_mo);
+  oa.o = c.o;
+  oa.v = L.d.vp;
+  oa.has_fvo = c.has_fvo;
+  oa.vjp = c.vjp;
+  oa.norb = norb;
+  oa.ebar = c.ebar;
+  oa.part_t = at(L.off_part_t);
+  oa.part_mo = c.vjp ? at(L.off_mo_rows) : nullptr;
+  oa.tri = tri;
+  oa.nb = nb;
+  oa.ws = L.d.ws;
+  return oa;
+}
+
+// algorithmic flops of one contraction family (W build or an adjoint) of a triple
+static double walk_flops(const Ctx &c) { return 12.0 * c.v * (double)c.v * c.v * (c.v + c.o); }
+
+static int walk_build(const Ctx &c, const WalkLayout &L, char *b, const int *tri, int nb) {
+  auto at = [&](size_t off) { return (double *)(b + off); };
+  PAMD_CHECK(timed(c.s, kProfWBuild, walk_flops(c) * nb, 0.0, [&] {
+    return launch_walk_w(L.d, at(L.off_VT), at(L.off_TBt), at(L.off_W), tri, nb, c.s);
+  }));
+  return PAMD_OK;
+}
+
+// adjoint of a batch whose Wbar and Vbar blocks are written; tri_e: also the
+// triple energies
+static int walk_adjoint(const Ctx &c, const WalkLayout &L, char *b, const int *tri, int nb, bool first,
+                        double *tri_e) {
+  auto at = [&](size_t off) { return (double *)(b + off); };
+  const WalkDims &d = L.d;
+  const hipStream_t s = c.s;
+  const double v3 = (double)c.v * c.v * c.v, fl = walk_flops(c) * nb;
+  if (nb > 0) {
+    VRArgs vr;
+    memset(&vr, 0, sizeof(vr));
+    vr.Vb = at(L.off_Vb);
+    vr.t1 = at(L.off_t1);
+    vr.fvo = at(L.off_fvo);
+    vr.ovs = at(L.off_OVS);
+    vr.t2s = at(L.off_T2S);
+    vr.o = d.o;
+    vr.v = d.vp;
+    vr.has_fvo = c.has_fvo;
+    vr.R = at(L.off_R);
+    vr.parts = 1;
+    vr.tri = tri;
+    vr.nb = nb;
+    vr.r_stride = L.r_stride;
+    PAMD_CHECK(timed(s, kProfVR, 0.0, 16.0 * v3 * nb, [&] { return launch_vr(vr, s); }));
+  }
+  PAMD_CHECK(timed(s, kProfAdjOvvv, fl, 0.0, [&] {
+    return launch_walk_vtb(d, at(L.off_W), at(L.off_TB), at(L.off_VTb), tri, nb, first, s);
+  }));
+  if (nb > 0)
+    PAMD_CHECK(timed(s, kProfAdjT2P, fl, 0.0, [&] {
+      return launch_walk_tbb(d, at(L.off_W), at(L.off_VT), at(L.off_part), tri, nb, L.S, s);
+    }));
+  WalkGather g;
+  g.d = d;
+  g.tri = tri;
+  g.nb = nb;
+  g.S = L.S;
+  g.G = L.G;
+  g.has_fvo = c.has_fvo;
+  g.first = first;
+  g.part = at(L.off_part);
+  g.R = at(L.off_R);
+  g.r_stride = L.r_stride;
+  g.part_t = at(L.off_part_t);
+  g.vec = at(L.off_vec);
+  g.t1_bar = c.t1_bar;
+  g.t2_bar = c.t2_bar;
+  g.ovoo_bar = c.ovoo_bar;
+  g.ovov_bar = c.ovov_bar;
+  g.fvo_bar = c.fvo_bar;
+  g.tri_e = tri_e;
+  const double cb = 8.0 * 6.0 * L.S * (double)d.vp * d.up * nb;
+  PAMD_CHECK(timed(s, kProfCombine, 0.0, cb, [&] { return launch_walk_gather(g, s); }));
+  return PAMD_OK;
+}
+
+static int walk_finish(const Ctx &c, const WalkLayout &L, char *b, double *ovvv_bar, double *mo_bar) {
+  auto at = [&](size_t off) { return (double *)(b + off); };
+  PAMD_CHECK(launch_walk_finish(L.d, at(L.off_VTb), c.packed, ovvv_bar, c.t2_bar, at(L.off_mo_rows),
+                                L.nb * L.G, at(L.off_mo2), mo_bar, c.s));
+  return PAMD_OK;
+}
+
+// progress lines (pamd_profile_progress) and launch sampling of a batched walk
+struct WalkMeter {
+  const char *what;
+  long long n, reported;
+  std::chrono::steady_clock::time_point start;
+  explicit WalkMeter(const char *w, long long total)
+      : what(w), n(total), reported(0), start(std::chrono::steady_clock::now()) {}
+  void sample(long long t0, int nb) const {
+    g_prof_on = g_prof_every > 0 && (t0 + g_prof_every - 1) / g_prof_every * g_prof_every < t0 + nb;
+  }
+  hipError_t report(long long done, hipStream_t s) {
+    if (g_progress_every <= 0 || (done - reported < g_progress_every && done != n)) return hipSuccess;
+    reported = done;
+    const hipError_t e = hipStreamSynchronize(s);
+    if (e != hipSuccess) return e;
+    fprintf(stderr, "pyscfad_amd: %s triples %lld/%lld done, %.1f s\n", what, done, n,
+            std::chrono::duration<double>(std::chrono::steady_clock::now() - start).count());
+    fflush(stderr);
+    return hipSuccess;
+  }
+};
+
 // One call's walk on its stream c.s: c.tri gets the triple energies, and with
 // c.vjp every cotangent is complete.
 static int run_walk(Ctx &c, const WalkLayout &L, void *ws, double *ovvv_bar, double *mo_bar) {
   char *b = (char *)ws;
   auto at = [&](size_t off) { return (double *)(b + off); };
-  const WalkDims &d = L.d;
-  const int o = d.o;
+  const int o = c.o;
   const hipStream_t s = c.s;
-  double *VT = at(L.off_VT), *TB = c.vjp ? at(L.off_TB) : nullptr, *TBt = at(L.off_TBt), *W = at(L.off_W);
+  long long norb = 0;
+  int st = walk_setup(c, L, b, norb);
+  if (st != PAMD_OK) return st;
   int *tab = (int *)at(L.off_tab);
-  unsigned short *orb = (unsigned short *)at(L.off_orb);
-  c.tri = at(L.off_tri_e);
-  c.wt = at(L.off_wt);
-  PAMD_CHECK(launch_walk_inputs(d, c.mo, c.t1, c.t2, c.ovvv, c.packed, c.ovoo, c.ovov,
-                                c.has_fvo ? c.fvo : nullptr, VT, TB, TBt, at(L.off_OVS), at(L.off_T2S),
-                                at(L.off_t1), at(L.off_fvo), at(L.off_mo), s));
   const long long n = (num_triples(o) - c.shard + c.nshards - 1) / c.nshards;
   const WalkBatches wb = walk_batches(n, L.nb);
   PAMD_CHECK(launch_walk_triples(o, c.shard, c.nshards, wb, tab, s));
   PAMD_CHECK(launch_fill(c.tri, (size_t)o * o * o, 0.0, s));
-  const long long nt = d.vp / 8, norb = nt * (nt + 1) * (nt + 2) / 6;
-  PAMD_CHECK(launch_orbit_table(norb, orb, s));
-  const size_t rows = (size_t)L.nb * L.G;
-  if (c.vjp) PAMD_CHECK(launch_fill(at(L.off_mo_rows), rows * (o + d.vp), 0.0, s));
   if (c.wt_host)
     PAMD_CHECK(hipMemcpyAsync(c.wt, c.wt_host, sizeof(double) * (size_t)o, hipMemcpyHostToDevice, s));
-  const auto t_start = std::chrono::steady_clock::now();
-  const double v3 = (double)c.v * c.v * c.v, fl = 12.0 * v3 * (c.v + o);  // one family, per triple
-  long long reported = 0, t0 = 0;
+  const double v3 = (double)c.v * c.v * c.v;
+  WalkMeter meter(c.vjp ? "(T)+VJP" : "(T)", n);
+  long long t0 = 0;
   // without triples one empty batch writes the (zero) cotangents
-  for (int bt = 0; bt < wb.count; t0 += wb.size(bt), ++bt) {
+  for (int bt = 0; bt < wb.count; ++bt) {
     const int nb = wb.size(bt);
     const int *tri = tab + (size_t)bt * wb.cap;
-    g_prof_on = g_prof_every > 0 && (t0 + g_prof_every - 1) / g_prof_every * g_prof_every < t0 + nb;
+    meter.sample(t0, nb);
     if (nb > 0) {
-      PAMD_CHECK(timed(s, kProfWBuild, fl * nb, 0.0, [&] { return launch_walk_w(d, VT, TBt, W, tri, nb, s); }));
-      OrbitArgs oa;
-      memset(&oa, 0, sizeof(oa));
-      oa.W = W;
-      oa.tab = orb;
-      oa.Vb = c.vjp ? at(L.off_Vb) : nullptr;
-      oa.t1 = at(L.off_t1);
-      oa.ovs = at(L.off_OVS);
-      oa.t2s = at(L.off_T2S);
-      oa.fvo = at(L.off_fvo);
-      oa.mo = at(L.off_mo);
-      oa.o = o;
-      oa.v = d.vp;
-      oa.has_fvo = c.has_fvo;
-      oa.vjp = c.vjp;
-      oa.norb = norb;
-      oa.ebar = c.ebar;
-      oa.part_t = at(L.off_part_t);
-      oa.part_mo = c.vjp ? at(L.off_mo_rows) : nullptr;
-      oa.tri = tri;
-      oa.nb = nb;
-      oa.ws = d.ws;
+      st = walk_build(c, L, b, tri, nb);
+      if (st != PAMD_OK) return st;
+      OrbitArgs oa = walk_orbit_args(c, L, b, tri, nb, norb);
       oa.wt = c.wt_host ? c.wt : nullptr;
       const double ob = 8.0 * v3 * (c.vjp ? 3.0 : 1.0) * nb;
       PAMD_CHECK(timed(s, kProfOrbit, 0.0, ob, [&] { return launch_orbit(oa, L.G, s, kOrbitBatch); }));
     }
-    if (!c.vjp) {
-      PAMD_CHECK(launch_walk_energies(tri, nb, o, at(L.off_part_t), L.G, c.tri, s));
+    if (c.vjp) {
+      st = walk_adjoint(c, L, b, tri, nb, bt == 0, c.tri);
+      if (st != PAMD_OK) return st;
     } else {
-      if (nb > 0) {
-        VRArgs vr;
-        memset(&vr, 0, sizeof(vr));
-        vr.Vb = at(L.off_Vb);
-        vr.t1 = at(L.off_t1);
-        vr.fvo = at(L.off_fvo);
-        vr.ovs = at(L.off_OVS);
-        vr.t2s = at(L.off_T2S);
-        vr.o = o;
-        vr.v = d.vp;
-        vr.has_fvo = c.has_fvo;
-        vr.R = at(L.off_R);
-        vr.parts = 1;
-        vr.tri = tri;
-        vr.nb = nb;
-        vr.r_stride = L.r_stride;
-        PAMD_CHECK(timed(s, kProfVR, 0.0, 16.0 * v3 * nb, [&] { return launch_vr(vr, s); }));
-      }
-      PAMD_CHECK(timed(s, kProfAdjOvvv, fl * nb, 0.0, [&] {
-        return launch_walk_vtb(d, W, TB, at(L.off_VTb), tri, nb, t0 == 0, s);
-      }));
-      if (nb > 0)
-        PAMD_CHECK(timed(s, kProfAdjT2P, fl * nb, 0.0, [&] {
-          return launch_walk_tbb(d, W, VT, at(L.off_part), tri, nb, L.S, s);
-        }));
-      WalkGather g;
-      g.d = d;
-      g.tri = tri;
-      g.nb = nb;
-      g.S = L.S;
-      g.G = L.G;
-      g.has_fvo = c.has_fvo;
-      g.first = t0 == 0;
-      g.part = at(L.off_part);
-      g.R = at(L.off_R);
-      g.r_stride = L.r_stride;
-      g.part_t = at(L.off_part_t);
-      g.vec = at(L.off_vec);
-      g.t1_bar = c.t1_bar;
-      g.t2_bar = c.t2_bar;
-      g.ovoo_bar = c.ovoo_bar;
-      g.ovov_bar = c.ovov_bar;
-      g.fvo_bar = c.fvo_bar;
-      g.tri_e = c.tri;
-      const double cb = 8.0 * 6.0 * L.S * (double)d.vp * d.up * nb;
-      PAMD_CHECK(timed(s, kProfCombine, 0.0, cb, [&] { return launch_walk_gather(g, s); }));
+      PAMD_CHECK(launch_walk_energies(tri, nb, o, at(L.off_part_t), L.G, c.tri, s));
     }
-    if (g_progress_every > 0 && (t0 + nb - reported >= g_progress_every || t0 + nb == n)) {
-      reported = t0 + nb;
-      PAMD_CHECK(hipStreamSynchronize(s));
-      const double el =
-          std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
-      fprintf(stderr, "pyscfad_amd: (T)%s triples %lld/%lld done, %.1f s\n", c.vjp ? "+VJP" : "", t0 + nb, n,
-              el);
-      fflush(stderr);
-    }
+    t0 += nb;
+    PAMD_CHECK(meter.report(t0, s));
   }
   g_prof_on = false;
   if (!g_prof_recs.empty()) PAMD_CHECK(prof_collect());
-  if (c.vjp)
-    PAMD_CHECK(launch_walk_finish(d, at(L.off_VTb), c.packed, ovvv_bar, c.t2_bar, at(L.off_mo_rows),
-                                  (int)rows, at(L.off_mo2), mo_bar, s));
-  return PAMD_OK;
+  return c.vjp ? walk_finish(c, L, b, ovvv_bar, mo_bar) : PAMD_OK;
+}
+
+// (o10/v64, two fragment orbitals, E + VJP: 335 -> 27.0 ms against the one-triple walk.)
+// Batched projected walk: np pairs (j, k) at a time, the o triples (l, j, k) of
+// each in one batch, whose W blocks stay for the adjoint (the one-triple walk
+// builds every W twice).
+struct ProjWalkLayout {
+  WalkLayout L;
+  int np;
+  size_t off_tab, off_a, off_b, off_pair, off_dot, off_u, off_ulo, total;
+};
+
+static ProjWalkLayout proj_walk_layout(int o, int v, int nfrag, int vjp, int np) {
+  ProjWalkLayout P;
+  P.L = walk_layout(o, v, vjp, np * o);
+  P.np = np;
+  const size_t vp = P.L.d.vp, v3 = vp * vp * vp, pairs = (size_t)o * (o + 1) / 2;
+  size_t off = P.L.total;
+  auto take = [&](size_t count) {
+    const size_t at = off;
+    off = align256(off + count * sizeof(double));
+    return at;
+  };
+  P.off_tab = take((pairs * o + 1) / 2);
+  P.off_a = take(np * nfrag * v3);
+  P.off_b = take(np * nfrag * v3);
+  P.off_pair = take((size_t)o * o);
+  P.off_dot = take((size_t)np * kWalkDotParts);
+  P.off_u = take(vjp ? (size_t)np * o * P.L.G * kMaxFrag : 0);
+  P.off_ulo = take((size_t)nfrag * o);
+  P.total = off;
+  return P;
+}
+
+// Pairs per batch: all, or as many as a batch of kWalkMaxBatch triples, 8 GB more
+// than one pair needs, and `limit` hold.  False as in walk_pick, or when one pair
+// has more triples than a batch.
+static bool proj_walk_pick(int o, int v, int nfrag, int vjp, size_t limit, size_t one_triple_total,
+                           ProjWalkLayout &P) {
+  if (!walk_dims_ok(walk_dims(o, v)) || o > kWalkMaxBatch) return false;
+  const size_t cap = std::min(limit, proj_walk_layout(o, v, nfrag, vjp, 1).total + ((size_t)8 << 30));
+  int np = std::min(o * (o + 1) / 2, kWalkMaxBatch / o);
+  while (np > 0 && proj_walk_layout(o, v, nfrag, vjp, np).total > cap) --np;
+  if (np < 1) return false;
+  const int pairs = o * (o + 1) / 2, batches = (pairs + np - 1) / np;
+  P = proj_walk_layout(o, v, nfrag, vjp, (pairs + batches - 1) / batches);
+  if (P.total > cap) P = proj_walk_layout(o, v, nfrag, vjp, np);
+  return P.total <= ((size_t)100 << 30) || P.total <= one_triple_total + one_triple_total / 20;
+}
+
+static int run_projected_walk(Ctx &c, const ProjWalkLayout &P, void *ws, const double *ulo, int nfrag,
+                              double *e_out, double *ovvv_bar, double *mo_bar, double *ulo_bar) {
+  const WalkLayout &L = P.L;
+  char *b = (char *)ws;
+  auto at = [&](size_t off) { return (double *)(b + off); };
+  const int o = c.o;
+  const hipStream_t s = c.s;
+  long long norb = 0;
+  int st = walk_setup(c, L, b, norb);
+  if (st != PAMD_OK) return st;
+  int *tab = (int *)at(P.off_tab);
+  PAMD_CHECK(launch_walk_pairs(o, tab, s));
+  PAMD_CHECK(launch_walk_upload(ulo, (size_t)nfrag * o, at(P.off_ulo), s));
+  PAMD_CHECK(launch_fill(at(P.off_pair), (size_t)o * o, 0.0, s));
+  const double v3 = (double)c.v * c.v * c.v;
+  const size_t vp3 = (size_t)L.d.vp * L.d.vp * L.d.vp;
+  const int pairs = o * (o + 1) / 2;
+  WalkMeter meter(c.vjp ? "projected (T)+VJP" : "projected (T)", (long long)pairs * o);
+  for (int p0 = 0; p0 < pairs; p0 += P.np) {
+    const int np = std::min(P.np, pairs - p0), nb = np * o;
+    const int *tri = tab + (size_t)p0 * o;
+    meter.sample((long long)p0 * o, nb);
+    st = walk_build(c, L, b, tri, nb);
+    if (st != PAMD_OK) return st;
+    OrbitArgs oa = walk_orbit_args(c, L, b, tri, nb, norb);
+    oa.accA = at(P.off_a);
+    oa.accB = at(P.off_b);
+    oa.nfrag = nfrag;
+    oa.udev = at(P.off_ulo);
+    for (int l = 0; l < o; ++l) {
+      OrbitArgs ol = oa;
+      ol.i = l;
+      ol.nb = np;
+      ol.acc_first = l == 0;
+      PAMD_CHECK(timed(s, kProfOrbit, 0.0, 8.0 * v3 * (1.0 + 4.0 * nfrag) * np,
+                       [&] { return launch_orbit(ol, L.G, s, kOrbitProjAcc); }));
+    }
+    PAMD_CHECK(launch_walk_dots(at(P.off_a), at(P.off_b), nfrag * vp3, tri, np, o, at(P.off_dot),
+                                at(P.off_pair), s));
+    if (c.vjp) {
+      oa.part_u = at(P.off_u);
+      PAMD_CHECK(timed(s, kProfOrbit, 0.0, 8.0 * v3 * (3.0 + 2.0 * nfrag) * nb,
+                       [&] { return launch_orbit(oa, L.G, s, kOrbitProjVjp); }));
+      PAMD_CHECK(launch_walk_ulo(at(P.off_u), L.G, nfrag, c.ebar, tri, np, o, p0 == 0, ulo_bar, s));
+      st = walk_adjoint(c, L, b, tri, nb, p0 == 0, nullptr);
+      if (st != PAMD_OK) return st;
+    }
+    PAMD_CHECK(meter.report((long long)(p0 + np) * o, s));
+  }
+  g_prof_on = false;
+  if (!g_prof_recs.empty()) PAMD_CHECK(prof_collect());
+  PAMD_CHECK(launch_projected_total(at(P.off_pair), o, e_out, s));
+  return c.vjp ? walk_finish(c, L, b, ovvv_bar, mo_bar) : PAMD_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -1748,6 +1913,10 @@ int pamd_ccsdt_projected_workspace_size(const pamd_ccsdt_config *cfg, int nfrag,
   if (!cfg || !bytes || cfg->nocc < 1 || cfg->nvir < 1 || nfrag < 1 || nfrag > kMaxFrag)
     return PAMD_ERR_ARG;
   *bytes = projected_layout(cfg->nocc, cfg->nvir, nfrag, with_vjp ? 1 : 0, cfg->precision).total;
+  ProjWalkLayout pw;
+  if (cfg->precision == PAMD_PREC_FP64 &&
+      proj_walk_pick(cfg->nocc, cfg->nvir, nfrag, with_vjp ? 1 : 0, (size_t)-1, *bytes, pw))
+    *bytes = std::max(*bytes, pw.total);
   return PAMD_OK;
 }
 
@@ -1788,6 +1957,11 @@ static int projected_impl(const pamd_ccsdt_config *cfg, const double *mo_energy,
   c.ovoo_bar = ovoo_bar;
   c.ovov_bar = ovov_bar;
   c.fvo_bar = fvo_bar;
+  ProjWalkLayout pw;
+  if (c.prec == PAMD_PREC_FP64 && proj_walk_pick(c.o, c.v, nfrag, vjp, workspace_bytes, P.total, pw)) {
+    c.nshards = 1;
+    return run_projected_walk(c, pw, workspace, ulo, nfrag, e_out, ovvv_bar, mo_energy_bar, ulo_bar);
+  }
   bind_workspace(c, P.L, workspace);
   char *b = (char *)workspace;
   double *pair_e = (double *)(b + P.off_p);

@@ -95,12 +95,28 @@ struct WalkGather {
   size_t r_stride;
   const double *part_t;     // [nb][G] energy sums of the orbit epilogue
   double *vec;              // scratch [nb][6][vp]
-  double *t1_bar, *t2_bar, *ovoo_bar, *ovov_bar, *fvo_bar, *tri_e;
+  double *t1_bar, *t2_bar, *ovoo_bar, *ovov_bar, *fvo_bar;
+  double *tri_e;            // triple energies (null: not wanted)
 };
 hipError_t launch_walk_gather(const WalkGather &g, hipStream_t s);
 // tri_e of nb triples from the orbit epilogue's G sums each
 hipError_t launch_walk_energies(const int *tri, int nb, int o, const double *part_t, int G, double *tri_e,
                                 hipStream_t s);
+
+// Projected walk: slot p o + l of the table is the triple (l, j, k) of the p-th
+// pair j <= k (every first index l of the pair; nothing is left out)
+hipError_t launch_walk_pairs(int o, int *tri, hipStream_t s);
+// dst[0 .. n) = src (host), through kernel arguments: no copy to wait for or to
+// record in a captured graph
+hipError_t launch_walk_upload(const double *src, size_t n, double *dst, hipStream_t s);
+// pair_e[j o + k] = sum_f <accA[f], accB[f]> of np pairs (n doubles each;
+// part: scratch of kWalkDotParts np)
+constexpr int kWalkDotParts = 32;
+hipError_t launch_walk_dots(const double *accA, const double *accB, size_t n, const int *tri, int np, int o,
+                            double *part, double *pair_e, hipStream_t s);
+// ulo_bar[f][l] (+)= sum over np pairs of g_jk sum of the G part_u rows of (l, j, k)
+hipError_t launch_walk_ulo(const double *part_u, int G, int nfrag, double ebar, const int *tri, int np, int o,
+                           bool first, double *ulo_bar, hipStream_t s);
 
 // at exit: ovvv_bar from VTb, its hole part added to t2_bar, and
 // mo_energy_bar from the rows of part_mo (o + vp columns; part2: scratch of

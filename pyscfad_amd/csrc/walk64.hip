@@ -689,7 +689,102 @@ hipError_t launch_walk_gather(const WalkGather &g, hipStream_t s) {
   hipLaunchKernelGGL(k_walk_t1, dim3((g.d.v + 255) / 256, o), dim3(256), 0, s, g);
   const int nblk = (v * g.d.up + 255) / 256;
   hipLaunchKernelGGL(k_walk_gather, dim3((unsigned)(nblk * o * o)), dim3(256), 0, s, g, nblk);
+  if (!g.tri_e) return hipGetLastError();
   return launch_walk_energies(g.tri, g.nb, o, g.part_t, g.G, g.tri_e, s);
+}
+
+// ---------------------------------------------------------------------------
+// projected walk
+// ---------------------------------------------------------------------------
+__global__ void k_walk_pairs(int o, int *tri) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= o * o) return;
+  const int j = t / o, k = t % o;
+  if (k < j) return;
+  int *p = tri + (size_t)(j * o - j * (j - 1) / 2 + k - j) * o;
+  for (int l = 0; l < o; ++l) p[l] = l | (j << 10) | (k << 20);
+}
+
+hipError_t launch_walk_pairs(int o, int *tri, hipStream_t s) {
+  hipLaunchKernelGGL(k_walk_pairs, dim3((o * o + 255) / 256), dim3(256), 0, s, o, tri);
+  return hipGetLastError();
+}
+
+struct WalkUpload {
+  double v[256];
+};
+__global__ void k_walk_upload(WalkUpload u, int n, double *dst) {
+  if ((int)threadIdx.x < n) dst[threadIdx.x] = u.v[threadIdx.x];
+}
+
+hipError_t launch_walk_upload(const double *src, size_t n, double *dst, hipStream_t s) {
+  for (size_t at = 0; at < n; at += 256) {
+    WalkUpload u;
+    const int m = (int)std::min<size_t>(256, n - at);
+    for (int q = 0; q < m; ++q) u.v[q] = src[at + q];
+    hipLaunchKernelGGL(k_walk_upload, dim3(1), dim3(256), 0, s, u, m, dst + at);
+  }
+  return hipGetLastError();
+}
+
+// sum over the workgroup's 256 threads, in a fixed order, on thread 0
+__device__ __forceinline__ double walk_block_sum(double x, double *red) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  return red[0] + red[1] + red[2] + red[3];
+}
+
+__global__ __launch_bounds__(256) void k_walk_dot(const double *a, const double *b, size_t n, double *part) {
+  __shared__ double red[4];
+  a += blockIdx.y * n;
+  b += blockIdx.y * n;
+  double s = 0.0;
+  for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (size_t)gridDim.x * 256) s += a[t] * b[t];
+  s = walk_block_sum(s, red);
+  if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = s;
+}
+
+__global__ void k_walk_dot_sum(const double *part, const int *tri, int np, int o, double *pair_e) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= np) return;
+  double s = 0.0;
+  for (int q = 0; q < kWalkDotParts; ++q) s += part[p * kWalkDotParts + q];
+  const int w = tri[(size_t)p * o];
+  pair_e[((w >> 10) & 1023) * o + (w >> 20)] = s;
+}
+
+hipError_t launch_walk_dots(const double *accA, const double *accB, size_t n, const int *tri, int np, int o,
+                            double *part, double *pair_e, hipStream_t s) {
+  hipLaunchKernelGGL(k_walk_dot, dim3(kWalkDotParts, np), dim3(256), 0, s, accA, accB, n, part);
+  hipLaunchKernelGGL(k_walk_dot_sum, dim3((np + 63) / 64), dim3(64), 0, s, part, tri, np, o, pair_e);
+  return hipGetLastError();
+}
+
+// one workgroup per (l, f)
+__global__ __launch_bounds__(256) void k_walk_ulo(const double *part_u, int G, double ebar, const int *tri, int np,
+                                                  int o, int first, double *ulo_bar) {
+  __shared__ double red[4];
+  const int l = blockIdx.x, f = blockIdx.y;
+  double s = 0.0;
+  for (int t = threadIdx.x; t < np * G; t += 256) {
+    const int p = t / G, g = t - p * G, w = tri[(size_t)p * o];
+    const double x = part_u[(((size_t)p * o + l) * G + g) * kMaxFrag + f];
+    s += x * (((w >> 10) & 1023) == (w >> 20) ? 1.0 : 2.0);
+  }
+  s = walk_block_sum(s, red);
+  if (threadIdx.x == 0) {
+    double *d = ulo_bar + (size_t)f * o + l;
+    *d = ebar * s / 3.0 + (first ? 0.0 : *d);
+  }
+}
+
+hipError_t launch_walk_ulo(const double *part_u, int G, int nfrag, double ebar, const int *tri, int np, int o,
+                           bool first, double *ulo_bar, hipStream_t s) {
+  hipLaunchKernelGGL(k_walk_ulo, dim3(o, nfrag), dim3(256), 0, s, part_u, G, ebar, tri, np, o, first ? 1 : 0,
+                     ulo_bar);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------

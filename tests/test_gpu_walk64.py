@@ -16,9 +16,19 @@ from pyscfad_amd.gen import make_problem
 pytestmark = pytest.mark.gpu
 
 
+def _least(call, full):
+    """The least byte count (a multiple of 256) that ``call(nbytes)`` accepts."""
+    lo, hi = 0, full
+    while hi - lo > 256:
+        mid = (lo + hi) // 512 * 256
+        if call(mid) == _lib.PAMD_OK:
+            hi = mid
+        else:
+            lo = mid
+    return hi
+
+
 def _smallest_workspace(inp):
-    """The least byte count that pamd_ccsdt_energy_vjp accepts (no GPU work: a
-    refused call returns before it, an accepted one is only made at the end)."""
     lib = _lib.load()
     full = _lib.workspace_size(inp.cfg, True)
     ws = torch.empty(full, dtype=torch.uint8, device=inp.device)
@@ -30,14 +40,7 @@ def _smallest_workspace(inp):
                                          _ops._ptr(ws), n, _ops._ptr(e), *_ops._cotangent_ptrs(out),
                                          _ops._stream(inp.device))
 
-    lo, hi = 0, full  # sizes are multiples of 256
-    while hi - lo > 256:
-        mid = (lo + hi) // 512 * 256
-        if call(mid) == _lib.PAMD_OK:
-            hi = mid
-        else:
-            lo = mid
-    return ws, hi
+    return ws, _least(call, full)
 
 
 @pytest.mark.parametrize('o,v,fvo,packed', [(2, 7, 1e-3, True), (3, 9, 0.0, False), (4, 16, 1e-3, True),
@@ -55,3 +58,31 @@ def test_batched_walk_matches_the_one_triple_walk(o, v, fvo, packed, cuda):
         ref = float(g1[k].norm())
         assert float((g[k] - g1[k]).norm()) <= 1e-12 * ref + 1e-18, k
     assert torch.allclose(_ops.energy(inp), e1, rtol=1e-12, atol=1e-18)
+
+
+@pytest.mark.parametrize('o,v,nfrag,fvo', [(2, 9, 1, 1e-3), (5, 31, 2, 0.0), (3, 48, 3, 1e-3),
+                                           (4, 17, 8, 1e-3), (17, 8, 2, 0.0)])
+def test_batched_projected_walk_matches_the_one_triple_walk(o, v, nfrag, fvo, cuda):
+    p = make_problem(o, v, 3 * v, seed=o * 10 + v, fvo_scale=fvo)
+    inp = _ops.Inputs(p.mo_energy, p.t1, p.t2, p.ovvv_packed(), p.ovoo, p.ovov, p.fvo, device=cuda)
+    u = torch.randn((nfrag, o), generator=torch.Generator().manual_seed(o), dtype=torch.float64)
+    e, g = _ops.projected_energy_vjp(inp, u, et_bar=0.7)
+    lib = _lib.load()
+    un = u.numpy()
+    ws, full = _ops._projected_ws(inp, nfrag, True)
+    out = _ops._cotangent_outputs(inp)
+    out['ulo_bar'] = torch.empty((nfrag, o), dtype=torch.float64, device=cuda)
+    e1 = torch.zeros((), dtype=torch.float64, device=cuda)
+
+    def call(n):
+        return lib.pamd_ccsdt_projected_energy_vjp(
+            ctypes.byref(inp.cfg), *inp.args(), un.ctypes.data_as(ctypes.c_void_p), nfrag,
+            ctypes.c_double(0.7), _ops._ptr(ws), n, _ops._ptr(e1), *_ops._cotangent_ptrs(out),
+            _ops._ptr(out['ulo_bar']), _ops._stream(inp.device))
+
+    assert call(_least(call, full)) == _lib.PAMD_OK
+    torch.cuda.synchronize()
+    assert torch.allclose(e, e1, rtol=1e-12, atol=1e-18)
+    for k in out:
+        assert float((g[k] - out[k]).norm()) <= 1e-12 * float(out[k].norm()) + 1e-18, k
+    assert torch.allclose(_ops.projected_energy(inp, u), e1, rtol=1e-12, atol=1e-18)
