@@ -123,20 +123,17 @@ struct OrbitArgs {
   int nfrag;
   double u[kMaxFrag];
   double *part_u;       // [G][kMaxFrag] per-workgroup dE/du_f sums (projected adjoint)
-  // kOrbitBatch: triple b = tri[b] (i | j << 10 | k << 20), b < nb, in place of
-  // i, j, k and omega: W and Vb hold one v^3 block per triple, part_t and
-  // part_mo G rows per triple; wt: occupied weights of a diagonal projector or null
+  // batched walk (walk64_orbit.hip): triple b = tri[b] (i | j << 10 | k << 20),
+  // b < nb, in place of i, j, k and omega; W and Vb hold one block per triple,
+  // part_t and part_mo G rows per triple
   const int *tri;
   int nb;
-  long long ws;  // element stride of W's first index (v^2 in the plain mode)
-  const double *wt;
-  // projected modes: with tri set a batch of pairs (see k_orbit), ulo on the
-  // device; acc_first: accA, accB are overwritten
-  const double *udev;
-  int acc_first;
+  long long ws;        // element stride of W's first index
+  const double *wt;    // occupied weights of a diagonal projector or null
+  const double *udev;  // projected walk: ulo[f][l] on the device
 };
 
-enum OrbitMode { kOrbitPlain = 0, kOrbitProjAcc = 1, kOrbitProjVjp = 2, kOrbitBatch = 3 };
+enum OrbitMode { kOrbitPlain = 0, kOrbitProjAcc = 1, kOrbitProjVjp = 2 };
 
 // V-bar reductions: the sums over one virtual index are split into kVRS parts
 // (more workgroups in flight), and the last virtual index is processed in

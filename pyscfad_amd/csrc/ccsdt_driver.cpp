@@ -1496,7 +1496,7 @@ static int run_walk(Ctx &c, const WalkLayout &L, void *ws, double *ovvv_bar, dou
       OrbitArgs oa = walk_orbit_args(c, L, b, tri, nb, norb);
       oa.wt = c.wt_host ? c.wt : nullptr;
       const double ob = 8.0 * v3 * (c.vjp ? 3.0 : 1.0) * nb;
-      PAMD_CHECK(timed(s, kProfOrbit, 0.0, ob, [&] { return launch_orbit(oa, L.G, s, kOrbitBatch); }));
+      PAMD_CHECK(timed(s, kProfOrbit, 0.0, ob, [&] { return launch_walk_orbit(oa, L.G, s); }));
     }
     if (c.vjp) {
       st = walk_adjoint(c, L, b, tri, nb, bt == 0, c.tri);
@@ -1518,15 +1518,17 @@ static int run_walk(Ctx &c, const WalkLayout &L, void *ws, double *ovvv_bar, dou
 // builds every W twice).
 struct ProjWalkLayout {
   WalkLayout L;
-  int np;
-  size_t off_tab, off_a, off_b, off_pair, off_dot, off_u, off_ulo, total;
+  int np, Ga;  // pairs per batch, workgroups per pair of launch_walk_acc
+  size_t off_tab, off_a, off_pair, off_u, off_ulo, total;
 };
 
 static ProjWalkLayout proj_walk_layout(int o, int v, int nfrag, int vjp, int np) {
   ProjWalkLayout P;
   P.L = walk_layout(o, v, vjp, np * o);
   P.np = np;
-  const size_t vp = P.L.d.vp, v3 = vp * vp * vp, pairs = (size_t)o * (o + 1) / 2;
+  const size_t nt = P.L.d.vp / 8, norb = nt * (nt + 1) * (nt + 2) / 6, pairs = (size_t)o * (o + 1) / 2;
+  // (part_t holds G sums per triple: at least Ga per pair)
+  P.Ga = (int)std::min<size_t>({(2048 + (size_t)np - 1) / np, norb, (size_t)P.L.G * o});
   size_t off = P.L.total;
   auto take = [&](size_t count) {
     const size_t at = off;
@@ -1534,10 +1536,8 @@ static ProjWalkLayout proj_walk_layout(int o, int v, int nfrag, int vjp, int np)
     return at;
   };
   P.off_tab = take((pairs * o + 1) / 2);
-  P.off_a = take(np * nfrag * v3);
-  P.off_b = take(np * nfrag * v3);
+  P.off_a = take(np * nfrag * walk_acc_doubles(P.L.d));
   P.off_pair = take((size_t)o * o);
-  P.off_dot = take((size_t)np * kWalkDotParts);
   P.off_u = take(vjp ? (size_t)np * o * P.L.G * kMaxFrag : 0);
   P.off_ulo = take((size_t)nfrag * o);
   P.total = off;
@@ -1575,7 +1575,6 @@ static int run_projected_walk(Ctx &c, const ProjWalkLayout &P, void *ws, const d
   PAMD_CHECK(launch_walk_upload(ulo, (size_t)nfrag * o, at(P.off_ulo), s));
   PAMD_CHECK(launch_fill(at(P.off_pair), (size_t)o * o, 0.0, s));
   const double v3 = (double)c.v * c.v * c.v;
-  const size_t vp3 = (size_t)L.d.vp * L.d.vp * L.d.vp;
   const int pairs = o * (o + 1) / 2;
   WalkMeter meter(c.vjp ? "projected (T)+VJP" : "projected (T)", (long long)pairs * o);
   for (int p0 = 0; p0 < pairs; p0 += P.np) {
@@ -1586,23 +1585,14 @@ static int run_projected_walk(Ctx &c, const ProjWalkLayout &P, void *ws, const d
     if (st != PAMD_OK) return st;
     OrbitArgs oa = walk_orbit_args(c, L, b, tri, nb, norb);
     oa.accA = at(P.off_a);
-    oa.accB = at(P.off_b);
     oa.nfrag = nfrag;
     oa.udev = at(P.off_ulo);
-    for (int l = 0; l < o; ++l) {
-      OrbitArgs ol = oa;
-      ol.i = l;
-      ol.nb = np;
-      ol.acc_first = l == 0;
-      PAMD_CHECK(timed(s, kProfOrbit, 0.0, 8.0 * v3 * (1.0 + 4.0 * nfrag) * np,
-                       [&] { return launch_orbit(ol, L.G, s, kOrbitProjAcc); }));
-    }
-    PAMD_CHECK(launch_walk_dots(at(P.off_a), at(P.off_b), nfrag * vp3, tri, np, o, at(P.off_dot),
-                                at(P.off_pair), s));
+    PAMD_CHECK(timed(s, kProfOrbit, 0.0, 8.0 * v3 * nb, [&] { return launch_walk_acc(oa, P.Ga, np, s); }));
+    PAMD_CHECK(launch_walk_pair_energies(at(L.off_part_t), P.Ga, tri, np, o, at(P.off_pair), s));
     if (c.vjp) {
       oa.part_u = at(P.off_u);
       PAMD_CHECK(timed(s, kProfOrbit, 0.0, 8.0 * v3 * (3.0 + 2.0 * nfrag) * nb,
-                       [&] { return launch_orbit(oa, L.G, s, kOrbitProjVjp); }));
+                       [&] { return launch_walk_proj(oa, L.G, s); }));
       PAMD_CHECK(launch_walk_ulo(at(P.off_u), L.G, nfrag, c.ebar, tri, np, o, p0 == 0, ulo_bar, s));
       st = walk_adjoint(c, L, b, tri, nb, p0 == 0, nullptr);
       if (st != PAMD_OK) return st;

@@ -557,8 +557,6 @@ hipError_t launch_orbit_table(long long norb, unsigned short *tab, hipStream_t s
 // tile axes reduce within the wave; the per-wave sums are then added over the
 // waves in a fixed order (no atomics), so every output is bitwise reproducible.
 // Modes: kOrbitPlain -- energy, and for the adjoint the Wbar/Vbar/dE/de seeds;
-// kOrbitBatch -- the plain mode for the nb triples of A.tri, grid row y taking
-// triple y with its own W and Vbar blocks and rows of part_t and part_mo;
 // kOrbitProjAcc -- accA[f] += u_f W, accB[f] += u_f Z/D (projected walk);
 // kOrbitProjVjp -- seeds of the projected energy from the finished accA, accB
 // of the pair: Q = g sum_f u_f accA[f] (dE/dY), P = g sum_f u_f accB[f]
@@ -577,47 +575,10 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int o = A.o, v = A.v, n = o + v;
-  int i = A.i, j = A.j, k = A.k;
-  double omega = A.omega;
-  if constexpr (MODE == kOrbitBatch) {
-    const int t = A.tri[blockIdx.y];
-    i = t & 1023;
-    j = (t >> 10) & 1023;
-    k = t >> 20;
-    omega = (i == j || j == k) ? 1.0 : 2.0;
-    if (A.wt) omega *= (A.wt[i] + A.wt[j] + A.wt[k]) / 3.0;
-    A.W += (size_t)blockIdx.y * v * A.ws;
-    if (A.vjp) A.Vb += (size_t)blockIdx.y * v * v * v;
-  }
-  // projector rows u_f of this triple's first index, and the adjoint's seed g
-  double uf[MODE == kOrbitProjAcc || MODE == kOrbitProjVjp ? kMaxFrag : 1];
-  double gproj = A.ebar;
-  if constexpr (MODE == kOrbitProjAcc || MODE == kOrbitProjVjp) {
-    if (A.tri) {
-      // a batch of pairs (j, k), o triples (l, j, k) each: grid row = pair at
-      // fixed l = A.i (kOrbitProjAcc), or triple (kOrbitProjVjp)
-      const int t_ = MODE == kOrbitProjAcc ? blockIdx.y * A.o + A.i : blockIdx.y;
-      const int t = A.tri[t_];
-      i = t & 1023;
-      j = (t >> 10) & 1023;
-      k = t >> 20;
-      const size_t v3_ = (size_t)v * v * v, pair = t_ / A.o;
-      A.W += (size_t)t_ * v * A.ws;
-      if (MODE == kOrbitProjVjp) A.Vb += (size_t)t_ * v3_;
-      A.accA += pair * A.nfrag * v3_;
-      A.accB += pair * A.nfrag * v3_;
-      gproj *= (j == k ? 1.0 : 2.0) / 3.0;
-#pragma unroll
-      for (int f = 0; f < kMaxFrag; ++f) uf[f] = f < A.nfrag ? A.udev[f * A.o + i] : 0.0;
-    } else {
-#pragma unroll
-      for (int f = 0; f < kMaxFrag; ++f) uf[f] = A.u[f];
-    }
-  }
-  const size_t row = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+  const int i = A.i, j = A.j, k = A.k;
   const double eo = A.mo[i] + A.mo[j] + A.mo[k];
   const double *ev = A.mo + o;
-  const double g = A.ebar * omega;
+  const double g = A.ebar * A.omega;
   for (int x = tid; x < v; x += 512) vir[x] = 0.0;
   __syncthreads();
 
@@ -667,7 +628,7 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
       const int ps = p < pq.np ? p : 0;
       const int ar = min(vq[pq.sel[ps][0]] * OT + al, v - 1), br = min(vq[pq.sel[ps][1]] * OT + be, v - 1),
                 cr = min(vq[pq.sel[ps][2]] * OT + ga, v - 1);
-      w[p] = A.W[MODE != kOrbitPlain ? ar * A.ws + br * v + cr : ((long long)ar * v + br) * v + cr];
+      w[p] = A.W[((long long)ar * v + br) * v + cr];
     }
   };
   double wnext[6];
@@ -724,11 +685,9 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
         double qv = 0.0;
         if (A0 + al < v && B0 + be < v && C0 + ga < v) {
           const long long tile_w = ((long long)A0 * v + B0) * v + C0;
-          #pragma unroll
-          for (int f = 0; f < kMaxFrag; ++f)
-            if (f < A.nfrag) qv += uf[f] * A.accA[f * v3 + tile_w + thr_w];
+          for (int f = 0; f < A.nfrag; ++f) qv += A.u[f] * A.accA[f * v3 + tile_w + thr_w];
         }
-        Qs[p][l_id] = gproj * qv;
+        Qs[p][l_id] = A.ebar * qv;
       }
     }
 #pragma unroll
@@ -772,12 +731,9 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
         const long long idx = ((long long)A0 * v + B0) * v + C0 + thr_w;
         if constexpr (MODE == kOrbitProjAcc) {
           const double y = Z * rD;
-#pragma unroll
-          for (int f = 0; f < kMaxFrag; ++f) {
-            if (f >= A.nfrag) continue;
-            double *pa = A.accA + f * v3 + idx, *pb = A.accB + f * v3 + idx;
-            *pa = uf[f] * w0 + (A.acc_first ? 0.0 : *pa);
-            *pb = uf[f] * y + (A.acc_first ? 0.0 : *pb);
+          for (int f = 0; f < A.nfrag; ++f) {
+            A.accA[f * v3 + idx] += A.u[f] * w0;
+            A.accB[f * v3 + idx] += A.u[f] * y;
           }
         } else if constexpr (MODE == kOrbitProjVjp) {
           const double q0 = Qs[p][l_id];
@@ -789,18 +745,18 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
           for (int f = 0; f < kMaxFrag; ++f) {
             if (f < A.nfrag) {
               const double bf = A.accB[f * v3 + idx];
-              pw += uf[f] * bf;
+              pw += A.u[f] * bf;
               udot[f] += w0 * bf + A.accA[f * v3 + idx] * y;
             }
           }
           const double vbar = r3Q * rD;
-          const double wbar = gproj * pw + vbar;
+          const double wbar = A.ebar * pw + vbar;
           if (A.Wb3)
             put3(A.Wb3, v3, idx, wbar);
           else if (A.Wb8)
             A.Wb8[idx] = split2(wbar).u;
           else
-            A.W[a * A.ws + b * v + c] = wbar;
+            A.W[idx] = wbar;
           A.Vb[idx] = vbar;
           dbar = -q0 * Z * rD * rD;
           occ += dbar;
@@ -814,7 +770,7 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
             else if (A.Wb8)
               A.Wb8[idx] = split2(wbar).u;
             else
-              A.W[MODE == kOrbitBatch ? a * A.ws + b * v + c : idx] = wbar;
+              A.W[idx] = wbar;
             A.Vb[idx] = vbar;
             dbar = -g * w0 * Z * rD * rD;
             occ += dbar;
@@ -887,7 +843,7 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
   __syncthreads();
   double otot = 0.0;
   for (int w = 0; w < 8; ++w) otot += red[w];
-  if (tid == 0) A.part_t[row] = etot;
+  if (tid == 0) A.part_t[blockIdx.x] = etot;
   if constexpr (MODE == kOrbitProjVjp) {
     // per-workgroup sums of <W, accB[f]> + <accA[f], Z/D>, wave order fixed
 #pragma unroll
@@ -901,11 +857,11 @@ __global__ __launch_bounds__(512) void k_orbit(OrbitArgs A) {
     if (tid < A.nfrag) {
       double s_ = 0.0;
       for (int w = 0; w < 8; ++w) s_ += ured[tid * 8 + w];
-      A.part_u[row * kMaxFrag + tid] = s_;
+      A.part_u[(size_t)blockIdx.x * kMaxFrag + tid] = s_;
     }
   }
-  if (MODE == kOrbitProjVjp || ((MODE == kOrbitPlain || MODE == kOrbitBatch) && A.vjp)) {
-    double *pm = A.part_mo + row * n;
+  if (MODE == kOrbitProjVjp || (MODE == kOrbitPlain && A.vjp)) {
+    double *pm = A.part_mo + (size_t)blockIdx.x * n;
     for (int x = tid; x < v; x += 512) pm[o + x] += vir[x];
     if (tid == 0) {
       pm[i] += otot;
@@ -937,13 +893,10 @@ int orbit_grid(int v) {
 }
 
 hipError_t launch_orbit(const OrbitArgs &a, int grid, hipStream_t s, int mode) {
-  const unsigned ny = a.tri ? a.nb : 1;
   if (mode == kOrbitProjAcc)
-    hipLaunchKernelGGL(k_orbit<kOrbitProjAcc>, dim3(grid, ny), dim3(512), sizeof(double) * a.v, s, a);
+    hipLaunchKernelGGL(k_orbit<kOrbitProjAcc>, dim3(grid), dim3(512), sizeof(double) * a.v, s, a);
   else if (mode == kOrbitProjVjp)
-    hipLaunchKernelGGL(k_orbit<kOrbitProjVjp>, dim3(grid, ny), dim3(512), sizeof(double) * a.v, s, a);
-  else if (mode == kOrbitBatch)
-    hipLaunchKernelGGL(k_orbit<kOrbitBatch>, dim3(grid, ny), dim3(512), sizeof(double) * a.v, s, a);
+    hipLaunchKernelGGL(k_orbit<kOrbitProjVjp>, dim3(grid), dim3(512), sizeof(double) * a.v, s, a);
   else
     hipLaunchKernelGGL(k_orbit<kOrbitPlain>, dim3(grid), dim3(512), sizeof(double) * a.v, s, a);
   return hipGetLastError();

@@ -77,6 +77,18 @@ hipError_t launch_walk_triples(int o, int shard, int nshards, const WalkBatches 
 // W of nb triples (tri[0 .. nb)), each a block of vp ws elements
 hipError_t launch_walk_w(const WalkDims &d, const double *VT, const double *TBt, double *W, const int *tri,
                          int nb, hipStream_t s);
+// epilogue (OrbitArgs' batch fields, grid rows of G workgroups; walk64_orbit.hip):
+// energies and, with vjp, Wbar over W, Vbar and the mo_energy_bar rows
+hipError_t launch_walk_orbit(const OrbitArgs &a, int G, hipStream_t s);
+// projected walk: the sums over l of np pairs into accA (walk_acc_doubles per
+// pair and fragment orbital), their energies into part_t; then the seeds of all
+// nb triples
+inline size_t walk_acc_doubles(const WalkDims &d) {
+  const size_t nt = d.vp / 8;
+  return nt * (nt + 1) * (nt + 2) / 6 * 6 * 512 * 2;
+}
+hipError_t launch_walk_acc(const OrbitArgs &a, int G, int np, hipStream_t s);
+hipError_t launch_walk_proj(const OrbitArgs &a, int G, hipStream_t s);
 // VTb += dE/dVT of nb triples (Wb: their Wbar blocks); first: VTb is overwritten
 hipError_t launch_walk_vtb(const WalkDims &d, const double *Wb, const double *TB, double *VTb,
                            const int *tri, int nb, bool first, hipStream_t s);
@@ -109,11 +121,9 @@ hipError_t launch_walk_pairs(int o, int *tri, hipStream_t s);
 // dst[0 .. n) = src (host), through kernel arguments: no copy to wait for or to
 // record in a captured graph
 hipError_t launch_walk_upload(const double *src, size_t n, double *dst, hipStream_t s);
-// pair_e[j o + k] = sum_f <accA[f], accB[f]> of np pairs (n doubles each;
-// part: scratch of kWalkDotParts np)
-constexpr int kWalkDotParts = 32;
-hipError_t launch_walk_dots(const double *accA, const double *accB, size_t n, const int *tri, int np, int o,
-                            double *part, double *pair_e, hipStream_t s);
+// pair_e[j o + k] of np pairs from their G part_t sums (launch_walk_acc)
+hipError_t launch_walk_pair_energies(const double *part_t, int G, const int *tri, int np, int o,
+                                     double *pair_e, hipStream_t s);
 // ulo_bar[f][l] (+)= sum over np pairs of g_jk sum of the G part_u rows of (l, j, k)
 hipError_t launch_walk_ulo(const double *part_u, int G, int nfrag, double ebar, const int *tri, int np, int o,
                            bool first, double *ulo_bar, hipStream_t s);

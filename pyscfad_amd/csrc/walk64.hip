@@ -736,29 +736,19 @@ __device__ __forceinline__ double walk_block_sum(double x, double *red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 
-__global__ __launch_bounds__(256) void k_walk_dot(const double *a, const double *b, size_t n, double *part) {
+__global__ __launch_bounds__(256) void k_walk_pair_energies(const double *part_t, int G, const int *tri, int o,
+                                                            double *pair_e) {
   __shared__ double red[4];
-  a += blockIdx.y * n;
-  b += blockIdx.y * n;
   double s = 0.0;
-  for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (size_t)gridDim.x * 256) s += a[t] * b[t];
+  for (int r = threadIdx.x; r < G; r += 256) s += part_t[(size_t)blockIdx.x * G + r];
   s = walk_block_sum(s, red);
-  if (threadIdx.x == 0) part[blockIdx.y * gridDim.x + blockIdx.x] = s;
+  const int w = tri[(size_t)blockIdx.x * o];
+  if (threadIdx.x == 0) pair_e[((w >> 10) & 1023) * o + (w >> 20)] = s;
 }
 
-__global__ void k_walk_dot_sum(const double *part, const int *tri, int np, int o, double *pair_e) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= np) return;
-  double s = 0.0;
-  for (int q = 0; q < kWalkDotParts; ++q) s += part[p * kWalkDotParts + q];
-  const int w = tri[(size_t)p * o];
-  pair_e[((w >> 10) & 1023) * o + (w >> 20)] = s;
-}
-
-hipError_t launch_walk_dots(const double *accA, const double *accB, size_t n, const int *tri, int np, int o,
-                            double *part, double *pair_e, hipStream_t s) {
-  hipLaunchKernelGGL(k_walk_dot, dim3(kWalkDotParts, np), dim3(256), 0, s, accA, accB, n, part);
-  hipLaunchKernelGGL(k_walk_dot_sum, dim3((np + 63) / 64), dim3(64), 0, s, part, tri, np, o, pair_e);
+hipError_t launch_walk_pair_energies(const double *part_t, int G, const int *tri, int np, int o,
+                                     double *pair_e, hipStream_t s) {
+  hipLaunchKernelGGL(k_walk_pair_energies, dim3(np), dim3(256), 0, s, part_t, G, tri, o, pair_e);
   return hipGetLastError();
 }
 
