@@ -41,6 +41,29 @@ int pamd_mse(int n, const float *pred, const float *y, float *dpred, float *loss
 int pamd_f32_to_bf16(size_t n, const float *x, uint16_t *y, int M, int N, uint16_t *yt,
                      void *stream);
 
+/* Whole-network forms (two launches and one): widths sizes[0..nlayers] multiples of 8,
+ * at most 4 layers whose activations of 16 rows fit 64 KB of LDS, SiLU between
+ * layers, at most 8 members, rows % 8 == 0 when training, every matrix contiguous
+ * and 16-byte aligned; PAMD_ERR_UNSUPPORTED for anything else, before any GPU work.
+ *
+ * One training step: forward of x [rows][sizes[0]] (bf16, with its transpose xt),
+ * MSE against y [rows][sizes[nlayers]] (fp32), backward and Adam.  ptrs: per layer
+ * the device pointers w, b, m_w, v_w, m_b, v_b, wb, wt (masters and moments fp32,
+ * bf16 copies [N][K] and [K][N]); bias entries have no weight decay. */
+int pamd_mlp_train_scratch(int nlayers, const int *sizes, int rows, size_t *bytes);
+int pamd_mlp_train_step(int nlayers, const int *sizes, int rows, void *const *ptrs, const uint16_t *x,
+                        const uint16_t *xt, const float *y, float lr, float beta1, float beta2, float eps,
+                        float wd, int step, void *scratch, size_t scratch_bytes, float *loss, void *stream);
+
+/* out[member][row][sizes[nlayers]] (fp32) of every member on x; ptrs: wb, b of every
+ * layer of every member. */
+int pamd_mlp_forward(int members, int nlayers, const int *sizes, int rows, void *const *ptrs, const uint16_t *x,
+                     float *out, void *stream);
+
+/* out[row][p] = bf16((x[row][p] - mean[p]) / stddev[p]), p < n, and 0 for n <= p < ld. */
+int pamd_standardise_bf16(int rows, int n, int ld, const double *x, const double *mean, const double *stddev,
+                          uint16_t *out, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -34,7 +34,8 @@ EXPORTS = ('pamd_version', 'pamd_ccsdt_workspace_size', 'pamd_ccsdt_energy',
            'pamd_debug_paired_adjoint_descriptors', 'pamd_debug_split_factors',
            'pamd_debug_split_factors_prec', 'pamd_debug_gemm_direct_ok', 'pamd_debug_gemm_b3p_ok',
            'pamd_bf16_gemm_tn', 'pamd_bf16_act_fwd', 'pamd_bf16_act_bwd', 'pamd_adam_step',
-           'pamd_mse', 'pamd_f32_to_bf16', 'pamd_mp2_init_amps', 'pamd_df_eris_workspace_size',
+           'pamd_mse', 'pamd_f32_to_bf16', 'pamd_mlp_train_scratch', 'pamd_mlp_train_step',
+           'pamd_mlp_forward', 'pamd_standardise_bf16', 'pamd_mp2_init_amps', 'pamd_df_eris_workspace_size',
            'pamd_df_eris', 'pamd_df_eris_vjp', 'pamd_debug_df_descriptors')
 
 

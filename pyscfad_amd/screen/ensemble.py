@@ -15,7 +15,7 @@ import time
 import numpy as np
 import torch
 
-from .mlp import MLP, to_bf16
+from .mlp import MLP, forward_members, standardise, to_bf16
 
 SPREAD_TOL = 1e-5  # Eh
 
@@ -42,6 +42,15 @@ class Screen:
     def _xin(self, X):
         Xn = ((X - self.x_mean) / self.x_std).float()
         return to_bf16(_pad_cols(Xn, self.p_in).contiguous(), with_t=True)
+
+    def _x16(self, X):
+        """bf16 inputs without their transpose (prediction)."""
+        stats = (X, self.x_mean, self.x_std)
+        if X.dim() == 2 and X.shape[0] > 0 and all(
+                t.dtype == torch.float64 and t.device == X.device and t.is_contiguous() for t in stats) \
+                and X.is_cuda and self.x_mean.shape == self.x_std.shape == (X.shape[1],):
+            return standardise(X, self.x_mean, self.x_std, self.p_in)
+        return self._xin(X)[0]
 
     def fit(self, X, Y, epochs=300, batch=128, lr=2e-3, wd=1e-5, seed=0, bootstrap=True,
             log=None):
@@ -78,12 +87,11 @@ class Screen:
         return hist
 
     def predict_pairs(self, X):
-        x16, _ = self._xin(X)
-        outs = []
-        for net in self.members:
-            z = net.forward(x16)[:, :self.n_out].double()
-            outs.append(z * self.y_std + self.y_mean)
-        return torch.stack(outs)          # [members, n, n_out]
+        x16 = self._x16(X)
+        z = forward_members(self.members, x16)
+        if z is None:
+            z = torch.stack([net.forward(x16) for net in self.members])
+        return z[:, :, :self.n_out].double() * self.y_std + self.y_mean   # [members, n, n_out]
 
     def predict(self, X):
         e = self.predict_pairs(X).sum(-1)  # [members, n]

@@ -27,14 +27,25 @@ _SIGS = {
     'pamd_mse': [ctypes.c_int] + [ctypes.c_void_p] * 5,
     'pamd_f32_to_bf16': [ctypes.c_size_t, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                          ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p],
+    'pamd_mlp_train_scratch': [ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p],
+    'pamd_mlp_train_step': [ctypes.c_int, ctypes.c_void_p, ctypes.c_int] + [ctypes.c_void_p] * 4 +
+                           [ctypes.c_float] * 5 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t,
+                                                   ctypes.c_void_p, ctypes.c_void_p],
+    'pamd_mlp_forward': [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_int] +
+                        [ctypes.c_void_p] * 4,
+    'pamd_standardise_bf16': [ctypes.c_int] * 3 + [ctypes.c_void_p] * 5,
 }
+
+_FNS = {}
 
 
 def _fn(name):
-    lib = _lib.load()
-    f = getattr(lib, name)
-    f.argtypes = _SIGS[name]
-    f.restype = ctypes.c_int
+    f = _FNS.get(name)
+    if f is None:
+        f = getattr(_lib.load(), name)
+        f.argtypes = _SIGS[name]
+        f.restype = ctypes.c_int
+        _FNS[name] = f
     return f
 
 
@@ -71,6 +82,44 @@ def to_bf16(x, with_t=False):
 def bf16_to_f32(b):
     """bf16 bit patterns (int16) -> float32 values (exact)."""
     return (b.to(torch.int32) & 0xFFFF).bitwise_left_shift(16).view(torch.float32)
+
+
+def standardise(X, mean, std, width):
+    """bf16 bit patterns of (X - mean) / std, zero-padded to ``width`` columns (X,
+    mean, std: float64 on one device)."""
+    n, m = X.shape
+    out = torch.empty((n, width), dtype=torch.int16, device=X.device)
+    st = _fn('pamd_standardise_bf16')(n, m, width, _p(X), _p(mean), _p(std), _p(out), _s(X.device))
+    _lib.check(st, 'pamd_standardise_bf16')
+    return out
+
+
+def _plain(t, shape, dtype, dev):
+    return t.shape == shape and t.dtype == dtype and t.device == dev and t.is_contiguous()
+
+
+def forward_members(nets, X16):
+    """fp32 [members, B, out] of several networks of the same widths in one launch,
+    or None where the whole-network kernel does not apply."""
+    sizes, dev = nets[0].sizes, X16.device
+    n = X16.shape[0]
+    if n < 1 or not _plain(X16, (n, sizes[0]), torch.int16, dev) or \
+            any(net.sizes != sizes for net in nets):
+        return None
+    ptrs = []
+    for net in nets:
+        for L, k, o in zip(net.layers, sizes[:-1], sizes[1:]):
+            if not (_plain(L['wb'], (o, k), torch.int16, dev) and
+                    _plain(L['b'], (o,), torch.float32, dev)):
+                return None
+            ptrs += (L['wb'].data_ptr(), L['b'].data_ptr())
+    out = torch.empty((len(nets), n, sizes[-1]), dtype=torch.float32, device=dev)
+    st = _fn('pamd_mlp_forward')(len(nets), len(sizes) - 1, (ctypes.c_int * len(sizes))(*sizes), n,
+                                 (ctypes.c_void_p * len(ptrs))(*ptrs), _p(X16), _p(out), _s(dev))
+    if st == _lib.PAMD_ERR_UNSUPPORTED:
+        return None
+    _lib.check(st, 'pamd_mlp_forward')
+    return out
 
 
 class MLP:
@@ -163,6 +212,42 @@ class MLP:
         return pred, loss, self.backward(d)
 
     def train_step(self, X16, X16_t, y, lr, wd=0.0):
-        _, loss, g = self.grads(X16, X16_t, y)
-        self.adam(g, lr=lr, wd=wd)
+        loss = self._fused_step(X16, X16_t, y, lr, wd)
+        if loss is None:
+            _, loss, g = self.grads(X16, X16_t, y)
+            self.adam(g, lr=lr, wd=wd)
+        return loss
+
+    def _fused_step(self, X16, X16_t, y, lr, wd, b1=0.9, b2=0.999, eps=1e-8):
+        """``grads`` and ``adam`` in two launches; None (and nothing done) where the
+        whole-network kernels do not apply."""
+        sizes, dev, n = self.sizes, X16.device, X16.shape[0]
+        if not (_plain(X16, (n, sizes[0]), torch.int16, dev) and
+                _plain(X16_t, (sizes[0], n), torch.int16, dev) and
+                _plain(y, (n, sizes[-1]), torch.float32, dev)):
+            return None
+        ptrs = []
+        for L, k, o in zip(self.layers, sizes[:-1], sizes[1:]):
+            for key, shape, dtype in (('w', (o, k), torch.float32), ('b', (o,), torch.float32),
+                                      ('m_w', (o, k), torch.float32), ('v_w', (o, k), torch.float32),
+                                      ('m_b', (o,), torch.float32), ('v_b', (o,), torch.float32),
+                                      ('wb', (o, k), torch.int16), ('wt', (k, o), torch.int16)):
+                t = L[key]
+                if not _plain(t, shape, dtype, dev):
+                    return None
+                ptrs.append(t.data_ptr())
+        csizes = (ctypes.c_int * len(sizes))(*sizes)
+        need = ctypes.c_size_t(0)
+        st = _fn('pamd_mlp_train_scratch')(len(sizes) - 1, csizes, n, ctypes.byref(need))
+        if st != _lib.PAMD_OK:
+            return None
+        scratch = torch.empty(need.value, dtype=torch.uint8, device=dev)
+        loss = torch.empty((), dtype=torch.float32, device=dev)
+        st = _fn('pamd_mlp_train_step')(
+            len(sizes) - 1, csizes, n, (ctypes.c_void_p * len(ptrs))(*ptrs), _p(X16), _p(X16_t), _p(y),
+            lr, b1, b2, eps, wd, self.step_count + 1, _p(scratch), need.value, _p(loss), _s(dev))
+        if st == _lib.PAMD_ERR_UNSUPPORTED:
+            return None
+        _lib.check(st, 'pamd_mlp_train_step')
+        self.step_count += 1
         return loss
