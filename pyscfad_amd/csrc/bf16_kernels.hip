@@ -20,22 +20,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-// x (n doubles) -> three bf16 planes of n at out, out + n, out + 2 n
-__global__ void k_split_bf16x3(const double *__restrict__ x, size_t n,
-                               unsigned short *__restrict__ out) {
-  for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n;
-       t += (size_t)gridDim.x * blockDim.x)
-    put3(out, (long long)n, t, x[t]);
-}
-
-hipError_t launch_split_bf16x3(const double *x, size_t n, unsigned short *out, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  size_t b = (n + 255) / 256;
-  if (b > 262144) b = 262144;
-  hipLaunchKernelGGL(k_split_bf16x3, dim3((unsigned)b), dim3(256), 0, s, x, n, out);
-  return hipGetLastError();
-}
-
 // VpT[x][f][p][q] (mode 0) or VpU[x][f][q][p] (mode 1) from Vp[x][p][q][f]; all
 // three are planar split-BF16x3 arrays of o v^3 elements (plane stride o v^3).
 // One 64 x 64 tile transpose through LDS per block: y is the index that keeps
@@ -668,14 +652,14 @@ static const int kB3Shape[kB3Num][3] = {{128, 80, 2}, {80, 128, 2}, {128, 48, 2}
                                         {48, 128, 2}, {256, 64, 1}, {64, 256, 1}};
 constexpr int kB3Wide = 4;  // configurations 0 .. 3 are the 16x16-MFMA ones
 
-static int b3_pick(int M, int N) {
+static int b3_pick(int M, int N, int sums = kSumsAuto) {
   double best_eff = 0.0;
   for (int c = 0; c < kB3Wide; ++c)
     best_eff = std::max(best_eff, tile_eff(M, N, kB3Shape[c][0], kB3Shape[c][1]));
-  const int ncand = best_eff >= 0.5 ? kB3Wide : kB3Num;
+  const int ncand = sums == kSumsWhole || (sums == kSumsAuto && best_eff >= 0.5) ? kB3Wide : kB3Num;
   int best = 0;
   double bs = -1.0;
-  for (int c = 0; c < ncand; ++c) {
+  for (int c = sums == kSumsFlushed ? (int)kB3Wide : 0; c < ncand; ++c) {
     const int MT = kB3Shape[c][0], NT = kB3Shape[c][1];
     const double sc = tile_eff(M, N, MT, NT) * (double)MT * NT / (MT + NT);
     if (sc > bs + 1e-9) {
@@ -685,6 +669,8 @@ static int b3_pick(int M, int N) {
   }
   return best;
 }
+
+B3Sums gemm_b3_sums(int M, int N) { return b3_pick(M, N) < kB3Wide ? kSumsWhole : kSumsFlushed; }
 
 // (sides that are multiples of 8 normally run on the direct engine, with its own tiles)
 int gemm_tiles_b3(int M, int N) {
@@ -706,8 +692,8 @@ hipError_t launch_gemm_b3(const GemmDesc &d0, hipStream_t s, const GemmBatch &bt
   d.chunk_start[0] = 0;
   for (int q = 0; q < d.nseg; ++q) d.chunk_start[q + 1] = d.chunk_start[q] + (d.seg[q].L + BKC - 1) / BKC;
   for (int q = d.nseg + 1; q <= kMaxSeg; ++q) d.chunk_start[q] = d.chunk_start[d.nseg];
-  if (gemm_b3p_enabled() && gemm_b3p_ok(d, bt)) return launch_gemm_b3p(d, s, bt);
-  const int c = b3_pick(d.M, d.N);
+  if (gemm_b3p_enabled() && d.sums != kSumsFlushed && gemm_b3p_ok(d, bt)) return launch_gemm_b3p(d, s, bt);
+  const int c = b3_pick(d.M, d.N, d.sums);
   const int MT = kB3Shape[c][0], NT = kB3Shape[c][1];
   const unsigned grid =
       (unsigned)((long long)((d.M + MT - 1) / MT) * ((d.N + NT - 1) / NT) * d.splits * bt.nb);

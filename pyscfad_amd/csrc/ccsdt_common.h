@@ -54,7 +54,7 @@ struct GemmDesc {
   int M, N, nseg, mode;
   int chunk_start[kMaxSeg + 1];  // prefix sums of ceil(L_s / KC) in K chunks
   int splits;                    // split-K factor (grid z); partial mode only when > 1
-  int pad_;
+  int sums;                      // B3Sums
   SegDesc seg[kMaxSeg];
   OutDesc C;
   double *partial;               // kPartial: partial[(split * M + m) * N + n]
@@ -166,7 +166,8 @@ struct CombineArgs {
   double *part_p;                 // [6][S][v][v] particle t2_bar partials (reduced in place)
   double *part_h;                 // [6][S][v][o] hole ovoo_bar partials (reduced in place)
   int S_p, S_h;
-  int o, v, i, j, k, has_fvo;
+  int o, v, i, j, k, has_fvo;     // v: extent of the outputs and partials
+  int vp;                         // extent that R is laid out with
   double *t2_bar, *ovov_bar, *ovoo_bar, *t1_bar, *fvo_bar;
   // when part_t is set: *tri_dst = sum of the orbit epilogue's G per-workgroup
   // energy sums (fixed order), in the same launch
@@ -179,12 +180,14 @@ struct CombineArgs {
 hipError_t launch_fill(double *p, size_t n, double val, hipStream_t s);
 hipError_t launch_orbit_table(long long norb, unsigned short *tab, hipStream_t s);
 hipError_t launch_prep_sym(const double *src, int o, int v, int kind, double *dst, hipStream_t s);
+// op, vp: extents the arrays are laid out with (zeros past o and v)
 hipError_t launch_prepare(const double *ovvv, int packed, const double *t2, const double *ovoo,
-                          int o, int v, double *Vp, double *T2m, double *OOt, int split,
+                          int o, int v, int op, int vp, double *Vp, double *T2m, double *OOt, int split,
                           hipStream_t s);
+// three bf16 planes of t2[x][y][p][q] laid out [x][y][vp][vp]
+hipError_t launch_split_t2(const double *t2, int o, int v, int vp, unsigned short *out, hipStream_t s);
 hipError_t launch_split_f32x2(const double *x, size_t n, unsigned long long *out, hipStream_t s);
 hipError_t launch_gemm_f32x2(const GemmDesc &d, hipStream_t s, const GemmBatch &bt = no_batch());
-hipError_t launch_split_bf16x3(const double *x, size_t n, unsigned short *out, hipStream_t s);
 // planar split-BF16x3 VpT[x][f][p][q] and VpU[x][f][q][p] from Vp[x][p][q][f]
 hipError_t launch_vp_transposes(const unsigned short *Vp, int o, int v, unsigned short *VpT,
                                 unsigned short *VpU, hipStream_t s);
@@ -193,6 +196,13 @@ hipError_t launch_gemm_bf16x3(const GemmDesc &d, hipStream_t s, const GemmBatch 
 // descriptors whose chunk_start counts stages of 32; launch_gemm_bf16x3 picks
 // it when gemm_b3p_ok(d)
 bool gemm_b3p_ok(const GemmDesc &d, const GemmBatch &bt = no_batch());
+// How a split-BF16x3 product sums over K: one FP32 sum per part (direct engine and
+// register-staged 16x16-MFMA tiles: the same products in the same order, so the
+// same bits), FP32 sums of 128 k added up in FP64 (32x32-MFMA tiles), or
+// whichever the sizes pick.  Walks on zero-padded arrays ask for what the
+// unpadded extents would pick: gradients then do not depend on the padding.
+enum B3Sums { kSumsAuto = 0, kSumsWhole = 1, kSumsFlushed = 2 };
+B3Sums gemm_b3_sums(int M, int N);  // of the register-staged engine
 bool gemm_b3p_enabled();  // env PYSCFAD_AMD_B3_DIRECT=0 turns it off
 int gemm_b3p_tiles(int M, int N);  // workgroup tiles of one split
 hipError_t launch_gemm_b3p(const GemmDesc &d, hipStream_t s, const GemmBatch &bt = no_batch());
@@ -217,9 +227,11 @@ int gemm_wgs_per_cu_b3(int M, int N);  // split-BF16x3 engine: resident workgrou
 hipError_t launch_orbit(const OrbitArgs &a, int grid, hipStream_t s, int mode = kOrbitPlain);
 hipError_t launch_vr(const VRArgs &a, hipStream_t s);
 hipError_t launch_combine(const CombineArgs &a, hipStream_t s);
-hipError_t launch_fold_ovvv(const double *Vpb, int o, int v, int packed, double *out, hipStream_t s);
-hipError_t launch_fold_t2m(const double *T2mb, int o, int v, double *t2_bar, hipStream_t s);
-hipError_t launch_reduce_rows(const double *part, int rows, int cols, double *out, int accumulate,
+hipError_t launch_fold_ovvv(const double *Vpb, int o, int v, int vp, int packed, double *out, hipStream_t s);
+// op, vp: extents the accumulators are laid out with
+hipError_t launch_fold_t2m(const double *T2mb, int o, int v, int op, int vp, double *t2_bar, hipStream_t s);
+// (ld: row stride of part)
+hipError_t launch_reduce_rows(const double *part, int rows, int cols, int ld, double *out, int accumulate,
                               hipStream_t s);
 hipError_t launch_triple_energy(const double *part_t, int G, double *dst, hipStream_t s);
 int orbit_grid(int v);

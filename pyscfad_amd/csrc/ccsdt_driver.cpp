@@ -22,6 +22,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <algorithm>
+#include <climits>
 #include <vector>
 #include <atomic>
 #include <chrono>
@@ -140,7 +141,13 @@ static hipError_t timed(hipStream_t s, int kind, double flops, double bytes, F &
   return prof_end(s, r);
 }
 
+static long long num_triples(int o) { return (long long)o * (o + 1) * (o + 2) / 6 - o; }
+
 struct Layout {
+  // extents the operand arrays are laid out with: (o, v), or with pad their
+  // multiples of 8
+  int pad, op, vp;
+  size_t off_t1, off_fvo, off_mo, off_tab;
   size_t off_Vp, off_T2m, off_OOt, off_OVS, off_T2S, off_orb, off_W, off_tri, off_part_t, off_T2g, off_W8;
   int wbatch;  // W blocks of the energy walk's batched W build (1 with the adjoint)
   size_t off_Vb, off_Vpb, off_T2mb, off_part_mo, off_R, off_part_p, off_part_h, off_wt;
@@ -212,20 +219,32 @@ static int energy_batch(int o, int v, int prec) {
 // split-BF16x3 W build row-contiguous, the faster of the direct engine's two
 // staging forms (the big operand of all three passes).  They take two o v^3
 // arrays; held when the direct engine runs the W build (nocc and nvir
-// multiples of 8) and the copies stay within 48 GB.
-static bool vpt_fits(int o, int v, int prec) {
+// multiples of 8, or padded to them) and the copies stay within 48 GB.
+static bool vpt_fits(int o, int op, int v, int prec) {
   const double bytes = 2.0 * 8.0 * o * (double)v * v * v;
-  return prec == PAMD_PREC_BF16X3 && o % 8 == 0 && v % 8 == 0 && bytes <= 48e9 &&
+  return prec == PAMD_PREC_BF16X3 && op % 8 == 0 && v % 8 == 0 && bytes <= 48e9 &&
          gemm_b3p_enabled();
 }
 
 // pipe: the adjoint walk runs two triples in flight (run_vjp_pipelined) and
 // needs second copies of W, Wbar, the V-bar scratch and the split-K partials
-static Layout make_layout(int o, int v, int vjp, int prec, bool pipe = false) {
+// pad: split-BF16x3 operands with both extents padded to multiples of 8 by zeros.
+// Every operand is then 16-byte aligned, so the W build and the ovvv adjoints run
+// on the direct engine at every size, and the epilogue is the batched walk's
+// (walk64_orbit.hip), which needs whole 8 x 8 x 8 tiles.  Measured, E + VJP at
+// o6/v400 (nocc padded): 910 -> 790 ms; at o16/v160 (epilogue alone): 660 -> 636;
+// energy at o24/v240 (epilogue alone, 153 -> 65 us per triple): 1601 -> 1479.
+// The split-K products keep the unpadded extents: padding would cut their sums
+// over (p, q) differently.
+static Layout make_layout(int o, int v, int vjp, int prec, bool pipe = false, bool pad = false) {
   Layout L;
   memset(&L, 0, sizeof(L));
+  L.pad = pad ? 1 : 0;
+  L.op = pad ? (o + 7) / 8 * 8 : o;
+  L.vp = pad ? (v + 7) / 8 * 8 : v;
   const size_t d = sizeof(double);
-  const size_t v2 = (size_t)v * v, v3 = v2 * v, n = (size_t)o + v;
+  const size_t vp = L.vp, v2 = vp * vp, v3 = v2 * vp, n = (size_t)o + vp, t2m = o * v2 * L.op;
+  const size_t vv = (size_t)v * v;
   size_t off = 0;
   auto take = [&](size_t count) {
     size_t at = off;
@@ -233,36 +252,40 @@ static Layout make_layout(int o, int v, int vjp, int prec, bool pipe = false) {
     return at;
   };
   L.off_Vp = take((size_t)o * v3);
-  L.off_T2m = take((size_t)o * o * v2);
-  L.off_OOt = take((size_t)o * o * o * v);
+  L.off_T2m = take(t2m);
+  L.off_OOt = take((size_t)o * o * L.op * vp);
   L.off_OVS = take((size_t)o * o * v2);
   L.off_T2S = take((size_t)o * o * v2);
-  {
-    const size_t nt = (v + 7) / 8;
-    L.off_orb = take(nt * (nt + 1) * (nt + 2) / 6);  // 4 x uint16 per orbit = one double
-  }
-  L.wbatch = vjp ? 1 : energy_batch(o, v, prec);
+  const size_t nt = (v + 7) / 8, norb = nt * (nt + 1) * (nt + 2) / 6;
+  L.off_orb = take(norb);  // 4 x uint16 per orbit = one double
+  L.wbatch = vjp ? 1 : energy_batch(o, L.vp, prec);
   L.off_W = take(v3 * L.wbatch);
   L.off_tri = take((size_t)o * o * o);
-  L.off_part_t = take(kGmax);
+  L.off_part_t = take((size_t)kGmax * (pad ? L.wbatch : 1));
   L.off_wt = take((size_t)o);
+  if (pad) {
+    L.off_t1 = take((size_t)o * vp);
+    L.off_fvo = take((size_t)o * vp);
+    L.off_mo = take(n);
+    L.off_tab = take((size_t)(num_triples(o) + kWalkRun) / 2 + 1);
+  }
   if (prec == PAMD_PREC_BF16X3 || prec == PAMD_PREC_FP32X2) {
     L.off_T2g = take((size_t)o * o * v2);
     if (vjp) L.off_W8 = take(v3);
   }
-  const int chunks = (int)((v2 + KC - 1) / KC);
+  const int chunks = (int)((vv + KC - 1) / KC);
   L.S_p = splits_for(v, v, chunks, prec);
   L.S_h = splits_for(v, o, chunks, prec);
   if (vjp) {
     L.off_Vb = take(v3);
     L.off_Vpb = take((size_t)o * v3);
-    L.off_T2mb = take((size_t)o * o * v2);
+    L.off_T2mb = take(t2m);
     L.off_part_mo = take((size_t)kGmax * n);
-    L.off_R = take(vr_scratch_doubles(v));
-    L.off_part_p = take((size_t)6 * L.S_p * v2);
+    L.off_R = take(vr_scratch_doubles(L.vp));
+    L.off_part_p = take((size_t)6 * L.S_p * vv);
     L.off_part_h = take((size_t)6 * L.S_h * v * o);
   }
-  L.vpt = vpt_fits(o, v, prec) ? 1 : 0;
+  L.vpt = vpt_fits(o, L.op, L.vp, prec) ? 1 : 0;
   if (L.vpt) {
     L.off_VpT = take((size_t)o * v3);
     L.off_VpU = take((size_t)o * v3);
@@ -271,12 +294,24 @@ static Layout make_layout(int o, int v, int vjp, int prec, bool pipe = false) {
   if (L.pipe) {
     L.off_W2 = take(v3);
     if (prec == PAMD_PREC_BF16X3 || prec == PAMD_PREC_FP32X2) L.off_W8b = take(v3);
-    L.off_R2 = take(vr_scratch_doubles(v));
-    L.off_part_p2 = take((size_t)6 * L.S_p * v2);
+    L.off_R2 = take(vr_scratch_doubles(L.vp));
+    L.off_part_p2 = take((size_t)6 * L.S_p * vv);
     L.off_part_h2 = take((size_t)6 * L.S_h * v * o);
   }
   L.total = off;
   return L;
+}
+
+// The layout of a plain walk: padded for the split-BF16x3 engine (`plain`, the
+// unpadded one, stays where the direct engine is off, `limit` bytes do not hold
+// the padded arrays or these are noticeably larger in a workspace that is large
+// itself).
+static Layout b3_layout(int o, int v, int vjp, int prec, bool pipe, size_t limit, const Layout &plain) {
+  const long long vp = (v + 7) / 8 * 8;
+  if (prec != PAMD_PREC_BF16X3 || !gemm_b3p_enabled() || vp * vp * vp >= (1LL << 31)) return plain;
+  const Layout P = make_layout(o, v, vjp, prec, pipe, true);
+  const bool big = P.total > ((size_t)100 << 30) && P.total > plain.total + plain.total / 20;
+  return P.total > limit || big ? plain : P;
 }
 
 // Planar split-BF16x3 operands: the arrays the walk's descriptors point into
@@ -293,6 +328,9 @@ struct PlanarMap {
 
 struct Ctx {
   int o, v, packed, has_fvo, vjp, prec;
+  int pad, op, vp;    // extents the arrays are laid out with (Layout)
+  double *t1p, *fvop, *mop;  // padded copies (pad)
+  int *tab;                  // triples in walk order (pad)
   const double *gT2;  // t2 as a GEMM operand (FP64, or its split copy)
   unsigned short *orb;  // orbit table
   double *gW;         // Wbar as a GEMM operand (= W, or its split copy)
@@ -403,14 +441,20 @@ static hipError_t run_gemm_group(const Ctx &c, const GemmDesc *ds, int n, int ki
 // ---------------------------------------------------------------------------
 // W build for one triple
 // ---------------------------------------------------------------------------
+// sums of a product on padded arrays whose unpadded extents are M x N; aligned:
+// the direct engine would take it unpadded too
+static int b3_sums(const Ctx &c, int M, int N, bool aligned) {
+  return c.pad && !aligned ? (int)gemm_b3_sums(M, N) : (int)kSumsAuto;
+}
+
 // nb > 1: the W blocks of triples (i, j, k), (i, j, k + 1), ..., (i, j, k + nb - 1)
 // in one launch per pass, written to W + b v^3 (every operand slab that names
 // k moves by a fixed stride per step of k).
 static int build_w(const Ctx &c, int i, int j, int k, int nb = 1) {
-  const long long o = c.o, v = c.v;
-  const long long v2 = v * v, v3 = v2 * v, vo = v * o;
+  const long long o = c.o, os = c.op, v = c.vp;
+  const long long v2 = v * v, v3 = v2 * v, vo = v * os;
   // element strides per step of k of: Vp(k), T2(k, x), T2(x, k), OOt(k, x), OOt(x, k), T2m(k)
-  const long long sVp = v3, sT2k_ = o * v2, sT2_k = v2, sOOk_ = o * vo, sOO_k = vo, sT2m = v2 * o;
+  const long long sVp = v3, sT2k_ = o * v2, sT2_k = v2, sOOk_ = o * vo, sOO_k = vo, sT2m = v2 * os;
   auto batch = [&](std::initializer_list<long long> a, std::initializer_list<long long> bo) {
     GemmBatch bt = no_batch();
     int q = 0;
@@ -423,9 +467,12 @@ static int build_w(const Ctx &c, int i, int j, int k, int nb = 1) {
   };
   auto Vp = [&](int x) { return c.Vp + x * v3; };
   auto T2 = [&](int x, int y) { return c.gT2 + (x * o + y) * v2; };
-  auto T2m = [&](int x) { return c.T2m + x * v2 * o; };
+  auto T2m = [&](int x) { return c.T2m + x * v2 * os; };
   auto OOt = [&](int x, int y) { return c.OOt + (x * o + y) * vo; };
-  const int V = c.v, O = c.o;
+  const int V = c.vp, O = c.op;
+  const bool whole = c.v % 8 == 0 && c.o % 8 == 0;
+  // (an energy takes the direct engine wherever it can: only FP32 roundings differ)
+  const int sumsC = c.vjp ? b3_sums(c, c.v * c.v, c.v, whole) : 0, sumsR = c.vjp ? b3_sums(c, c.v, c.v * c.v, whole) : 0;
   // the ovvv slab of a particle term with its row pair (q, s) read as
   // Vp(x)[q][s][f] ("qs") or Vp(x)[s][q][f] ("sq"), K = f: from Vp itself
   // (K-contiguous), or, when the call holds the transposed copies, from
@@ -441,9 +488,10 @@ static int build_w(const Ctx &c, int i, int j, int k, int nb = 1) {
     GemmDesc d = gemm(V * V, V, kStore,
                       {seg(Pqs(i), op1(T2(k, j), v, 1, 0), V, 1.0),      // P1
                        seg(Psq(j), op1(T2(k, i), v, 1, 0), V, 1.0),      // P3
-                       seg(opR(T2m(j), o, vo, V, 1, 0), op1(OOt(k, i), o, 1, 0), O, -1.0),   // H5
-                       seg(opR(T2m(i), vo, o, V, 1, 0), op1(OOt(k, j), o, 1, 0), O, -1.0)},  // H6
+                       seg(opR(T2m(j), os, vo, V, 1, 0), op1(OOt(k, i), os, 1, 0), O, -1.0),   // H5
+                       seg(opR(T2m(i), vo, os, V, 1, 0), op1(OOt(k, j), os, 1, 0), O, -1.0)},  // H6
                       out(c.W, v2, v, V, 0, 1, kBig));
+    d.sums = sumsC;
     // P1: T2(k,j), P3: T2(k,i), H5: OOt(k,i), H6: OOt(k,j)
     PAMD_CHECK(run_gemm(c, d, kProfWBuild,
                         batch({0, 0, 0, 0}, {sT2k_, sT2k_, sOOk_, sOOk_})));
@@ -453,9 +501,10 @@ static int build_w(const Ctx &c, int i, int j, int k, int nb = 1) {
     GemmDesc d = gemm(V, V * V, kAccumulate,
                       {seg(op1(T2(j, k), v, 1, 0), Pqs(i), V, 1.0),      // P2
                        seg(op1(T2(j, i), v, 1, 0), Psq(k), V, 1.0),      // P5
-                       seg(op1(OOt(j, i), o, 1, 0), opR(T2m(k), o, vo, V, 1, 0), O, -1.0),   // H3
-                       seg(op1(OOt(j, k), o, 1, 0), opR(T2m(i), vo, o, V, 1, 0), O, -1.0)},  // H4
+                       seg(op1(OOt(j, i), os, 1, 0), opR(T2m(k), os, vo, V, 1, 0), O, -1.0),   // H3
+                       seg(op1(OOt(j, k), os, 1, 0), opR(T2m(i), vo, os, V, 1, 0), O, -1.0)},  // H4
                       out(c.W, 0, v, kBig, v2, 1, V));
+    d.sums = sumsR;
     // P2: T2(j,k) | Vp(i), P5: T2(j,i) | Vp(k), H3: OOt(j,i) | T2m(k), H4: OOt(j,k) | T2m(i)
     PAMD_CHECK(run_gemm(c, d, kProfWBuild,
                         batch({sT2_k, 0, 0, sOO_k}, {0, sVp, sT2m, 0})));
@@ -465,9 +514,10 @@ static int build_w(const Ctx &c, int i, int j, int k, int nb = 1) {
     GemmDesc d = gemm(V, V * V, kAccumulate,
                       {seg(op1(T2(i, k), v, 1, 0), Pqs(j), V, 1.0),      // P4
                        seg(op1(T2(i, j), v, 1, 0), Psq(k), V, 1.0),      // P6
-                       seg(op1(OOt(i, j), o, 1, 0), opR(T2m(k), o, vo, V, 1, 0), O, -1.0),   // H1
-                       seg(op1(OOt(i, k), o, 1, 0), opR(T2m(j), vo, o, V, 1, 0), O, -1.0)},  // H2
+                       seg(op1(OOt(i, j), os, 1, 0), opR(T2m(k), os, vo, V, 1, 0), O, -1.0),   // H1
+                       seg(op1(OOt(i, k), os, 1, 0), opR(T2m(j), vo, os, V, 1, 0), O, -1.0)},  // H2
                       out(c.W, 0, v2, kBig, v, 1, V));
+    d.sums = sumsR;
     // P4: T2(i,k) | Vp(j), P6: T2(i,j) | Vp(k), H1: OOt(i,j) | T2m(k), H2: OOt(i,k) | T2m(j)
     PAMD_CHECK(run_gemm(c, d, kProfWBuild,
                         batch({sT2_k, 0, 0, sOO_k}, {0, sVp, sT2m, 0})));
@@ -487,12 +537,12 @@ static int adjoint_vr(const Ctx &c, int i, int j, int k, hipStream_t st) {
   memset(&vr, 0, sizeof(vr));
   vr.parts = kVRS;
   vr.Vb = c.Vb;
-  vr.t1 = c.t1;
-  vr.fvo = c.fvo;
+  vr.t1 = c.pad ? c.t1p : c.t1;
+  vr.fvo = c.pad ? c.fvop : c.fvo;
   vr.ovs = c.OVS;
   vr.t2s = c.T2S;
   vr.o = c.o;
-  vr.v = c.v;
+  vr.v = c.vp;
   vr.i = i;
   vr.j = j;
   vr.k = k;
@@ -513,15 +563,17 @@ static int adjoint_vr(const Ctx &c, int i, int j, int k, hipStream_t st) {
 // ones into Vpb[k] and T2mb[k]
 static int adjoint_gemms(const Ctx &c, int i, int j, int k, int pair = 0, const Ctx *prev = nullptr,
                          int kp = 0) {
-  const long long o = c.o, v = c.v;
-  const long long v2 = v * v, v3 = v2 * v, vo = v * o;
-  const int V = c.v, O = c.o;
+  const long long o = c.o, os = c.op, v = c.vp;
+  const long long v2 = v * v, v3 = v2 * v, vo = v * os;
+  const int V = c.vp, O = c.op, V0 = c.v, O0 = c.o;
+  const int sums_v = b3_sums(c, V0 * V0, V0, V0 % 8 == 0),
+            sums_h = b3_sums(c, V0 * V0, O0, V0 % 8 == 0 && O0 % 8 == 0);
   const double *Wb = c.gW;
   auto Vp = [&](int x) { return c.Vp + x * v3; };
   auto Vpb = [&](int x) { return c.Vpb + x * v3; };
   auto T2 = [&](int x, int y) { return c.gT2 + (x * o + y) * v2; };
-  auto T2m = [&](int x) { return c.T2m + x * v2 * o; };
-  auto T2mb = [&](int x) { return c.T2mb + x * v2 * o; };
+  auto T2m = [&](int x) { return c.T2m + x * v2 * os; };
+  auto T2mb = [&](int x) { return c.T2mb + x * v2 * os; };
   auto OOt = [&](int x, int y) { return c.OOt + (x * o + y) * vo; };
 
   // the three adjoints into Vpb[i], Vpb[j], Vpb[k] and into T2mb[i], T2mb[j],
@@ -550,9 +602,12 @@ static int adjoint_gemms(const Ctx &c, int i, int j, int k, int pair = 0, const 
                    {seg(opR(Wb, v2, 1, V, v, 1), op1(T2(j, i), 1, v, 1), V, 1.0),
                     seg(opR(Wb, v, 1, V, v2, 1), op1(T2(i, j), 1, v, 1), V, 1.0)},
                    out(Vpb(k), v, v2, V, 0, 1, kBig));
-    for (int q = 0; q < n; ++q) PAMD_CHECK(run_gemm(c, ds[q], kProfAdjOvvv));
+    for (int q = 0; q < n; ++q) {
+      ds[q].sums = sums_v;
+      PAMD_CHECK(run_gemm(c, ds[q], kProfAdjOvvv));
+    }
   } else {
-    const GemmDesc ds[3] = {
+    GemmDesc ds[3] = {
         // Vpb[i][a][b|c][f]: P1 (K=c), P2 (K=b)
         gemm(V * V, V, kAccumulate,
              {seg(opR(Wb, v2, v, V, 1, 0), op1(T2(k, j), 1, v, 1), V, 1.0),
@@ -569,55 +624,56 @@ static int adjoint_gemms(const Ctx &c, int i, int j, int k, int pair = 0, const 
               seg(opR(Wb, v, 1, V, v2, 1), op1(T2(i, j), 1, v, 1), V, 1.0)},
              out(Vpb(k), v, v2, V, 0, 1, kBig)),
     };
+    for (GemmDesc &d : ds) d.sums = sums_v;
     PAMD_CHECK(run_gemm_group(c, ds, 3, kProfAdjOvvv, distinct));
   }
 
   // particle t2_bar pieces: split-K over the virtual pair, partials per problem
-  const size_t pp = (size_t)c.S_p * v2;
+  const size_t pp = (size_t)c.S_p * V0 * V0;
   {
     const GemmDesc ds[6] = {
         // P1: t2_bar[k,j][c][f] = sum_(a,b) Wb[a,b,c] Vp(i)[a][b][f]
-        gemm(V, V, kPartial, {seg(opK(Wb, 1, v2, v, V, 1), opK(Vp(i), 1, v2, v, V, 1), V * V, 1.0)},
+        gemm(V0, V0, kPartial, {seg(opK(Wb, 1, v2, v, V0, 1), opK(Vp(i), 1, v2, v, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 0 * pp),
         // P2: t2_bar[j,k][b][f] = sum_(a,c) Wb[a,b,c] Vp(i)[a][c][f]
-        gemm(V, V, kPartial, {seg(opK(Wb, v, v2, 1, V, 0), opK(Vp(i), 1, v2, v, V, 1), V * V, 1.0)},
+        gemm(V0, V0, kPartial, {seg(opK(Wb, v, v2, 1, V0, 0), opK(Vp(i), 1, v2, v, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 1 * pp),
         // P3: t2_bar[k,i][c][f] = sum_(a,b) Wb[a,b,c] Vp(j)[b][a][f]
-        gemm(V, V, kPartial, {seg(opK(Wb, 1, v2, v, V, 1), opK(Vp(j), 1, v, v2, V, 1), V * V, 1.0)},
+        gemm(V0, V0, kPartial, {seg(opK(Wb, 1, v2, v, V0, 1), opK(Vp(j), 1, v, v2, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 2 * pp),
         // P4: t2_bar[i,k][a][f] = sum_(b,c) Wb[a,b,c] Vp(j)[b][c][f]
-        gemm(V, V, kPartial, {seg(opK(Wb, v2, v, 1, V, 0), opK(Vp(j), 1, v2, v, V, 1), V * V, 1.0)},
+        gemm(V0, V0, kPartial, {seg(opK(Wb, v2, v, 1, V0, 0), opK(Vp(j), 1, v2, v, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 3 * pp),
         // P5: t2_bar[j,i][b][f] = sum_(a,c) Wb[a,b,c] Vp(k)[c][a][f]
-        gemm(V, V, kPartial, {seg(opK(Wb, v, v2, 1, V, 0), opK(Vp(k), 1, v, v2, V, 1), V * V, 1.0)},
+        gemm(V0, V0, kPartial, {seg(opK(Wb, v, v2, 1, V0, 0), opK(Vp(k), 1, v, v2, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 4 * pp),
         // P6: t2_bar[i,j][a][f] = sum_(b,c) Wb[a,b,c] Vp(k)[c][b][f]
-        gemm(V, V, kPartial, {seg(opK(Wb, v2, v, 1, V, 0), opK(Vp(k), 1, v, v2, V, 1), V * V, 1.0)},
+        gemm(V0, V0, kPartial, {seg(opK(Wb, v2, v, 1, V0, 0), opK(Vp(k), 1, v, v2, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 5 * pp),
     };
     PAMD_CHECK(run_gemm_group(c, ds, 6, kProfAdjT2P, true));
   }
   // hole ovoo_bar pieces: split-K over the virtual pair
-  const size_t ph = (size_t)c.S_h * v * o;
+  const size_t ph = (size_t)c.S_h * V0 * O0;
   {
     const GemmDesc ds[6] = {
         // H1: ovoo_bar[i,a,m,j] = -sum_(b,c) Wb[a,b,c] T2m(k)[c][b][m]
-        gemm(V, O, kPartial, {seg(opK(Wb, v2, v, 1, V, 0), opK(T2m(k), 1, o, vo, V, 1), V * V, -1.0)},
+        gemm(V0, O0, kPartial, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 0 * ph),
         // H2: ovoo_bar[i,a,m,k] = -sum_(b,c) Wb[a,b,c] T2m(j)[b][c][m]
-        gemm(V, O, kPartial, {seg(opK(Wb, v2, v, 1, V, 0), opK(T2m(j), 1, vo, o, V, 1), V * V, -1.0)},
+        gemm(V0, O0, kPartial, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(j), 1, vo, os, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 1 * ph),
         // H3: ovoo_bar[j,b,m,i] = -sum_(a,c) Wb[a,b,c] T2m(k)[c][a][m]
-        gemm(V, O, kPartial, {seg(opK(Wb, v, v2, 1, V, 0), opK(T2m(k), 1, o, vo, V, 1), V * V, -1.0)},
+        gemm(V0, O0, kPartial, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 2 * ph),
         // H4: ovoo_bar[j,b,m,k] = -sum_(a,c) Wb[a,b,c] T2m(i)[a][c][m]
-        gemm(V, O, kPartial, {seg(opK(Wb, v, v2, 1, V, 0), opK(T2m(i), 1, vo, o, V, 1), V * V, -1.0)},
+        gemm(V0, O0, kPartial, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 3 * ph),
         // H5: ovoo_bar[k,c,m,i] = -sum_(a,b) Wb[a,b,c] T2m(j)[b][a][m]
-        gemm(V, O, kPartial, {seg(opK(Wb, 1, v2, v, V, 1), opK(T2m(j), 1, o, vo, V, 1), V * V, -1.0)},
+        gemm(V0, O0, kPartial, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(j), 1, os, vo, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 4 * ph),
         // H6: ovoo_bar[k,c,m,j] = -sum_(a,b) Wb[a,b,c] T2m(i)[a][b][m]
-        gemm(V, O, kPartial, {seg(opK(Wb, 1, v2, v, V, 1), opK(T2m(i), 1, vo, o, V, 1), V * V, -1.0)},
+        gemm(V0, O0, kPartial, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 5 * ph),
     };
     PAMD_CHECK(run_gemm_group(c, ds, 6, kProfAdjOvoo, true));
@@ -629,41 +685,45 @@ static int adjoint_gemms(const Ctx &c, int i, int j, int k, int pair = 0, const 
     int n = 0;
     if (pair == 2) {
       ds[n++] = gemm(V * V, O, kAccumulate,
-                     {seg(opR(Wq, v2, 1, V, v, 1), op1(OOt(j, kp), 1, o, 1), V, -1.0),
-                      seg(opR(Wq, v2, v, V, 1, 0), op1(OOt(kp, j), 1, o, 1), V, -1.0),
-                      seg(opR(Wb, v2, 1, V, v, 1), op1(OOt(j, k), 1, o, 1), V, -1.0),
-                      seg(opR(Wb, v2, v, V, 1, 0), op1(OOt(k, j), 1, o, 1), V, -1.0)},
-                     out(T2mb(i), vo, o, V, 0, 1, kBig));
+                     {seg(opR(Wq, v2, 1, V, v, 1), op1(OOt(j, kp), 1, os, 1), V, -1.0),
+                      seg(opR(Wq, v2, v, V, 1, 0), op1(OOt(kp, j), 1, os, 1), V, -1.0),
+                      seg(opR(Wb, v2, 1, V, v, 1), op1(OOt(j, k), 1, os, 1), V, -1.0),
+                      seg(opR(Wb, v2, v, V, 1, 0), op1(OOt(k, j), 1, os, 1), V, -1.0)},
+                     out(T2mb(i), vo, os, V, 0, 1, kBig));
       ds[n++] = gemm(V * V, O, kAccumulate,
-                     {seg(opR(Wq, v, 1, V, v2, 1), op1(OOt(i, kp), 1, o, 1), V, -1.0),
-                      seg(opR(Wq, v, v2, V, 1, 0), op1(OOt(kp, i), 1, o, 1), V, -1.0),
-                      seg(opR(Wb, v, 1, V, v2, 1), op1(OOt(i, k), 1, o, 1), V, -1.0),
-                      seg(opR(Wb, v, v2, V, 1, 0), op1(OOt(k, i), 1, o, 1), V, -1.0)},
-                     out(T2mb(j), vo, o, V, 0, 1, kBig));
+                     {seg(opR(Wq, v, 1, V, v2, 1), op1(OOt(i, kp), 1, os, 1), V, -1.0),
+                      seg(opR(Wq, v, v2, V, 1, 0), op1(OOt(kp, i), 1, os, 1), V, -1.0),
+                      seg(opR(Wb, v, 1, V, v2, 1), op1(OOt(i, k), 1, os, 1), V, -1.0),
+                      seg(opR(Wb, v, v2, V, 1, 0), op1(OOt(k, i), 1, os, 1), V, -1.0)},
+                     out(T2mb(j), vo, os, V, 0, 1, kBig));
     }
     ds[n++] = gemm(V * V, O, kAccumulate,
-                   {seg(opR(Wb, v, 1, V, v2, 1), op1(OOt(i, j), 1, o, 1), V, -1.0),
-                    seg(opR(Wb, v2, 1, V, v, 1), op1(OOt(j, i), 1, o, 1), V, -1.0)},
-                   out(T2mb(k), o, vo, V, 0, 1, kBig));
-    for (int q = 0; q < n; ++q) PAMD_CHECK(run_gemm(c, ds[q], kProfAdjT2H));
+                   {seg(opR(Wb, v, 1, V, v2, 1), op1(OOt(i, j), 1, os, 1), V, -1.0),
+                    seg(opR(Wb, v2, 1, V, v, 1), op1(OOt(j, i), 1, os, 1), V, -1.0)},
+                   out(T2mb(k), os, vo, V, 0, 1, kBig));
+    for (int q = 0; q < n; ++q) {
+      ds[q].sums = sums_h;
+      PAMD_CHECK(run_gemm(c, ds[q], kProfAdjT2H));
+    }
   } else {
-    const GemmDesc ds[3] = {
+    GemmDesc ds[3] = {
         // T2mb[i]: H4 (p=a,q=c,K=b), H6 (p=a,q=b,K=c)
         gemm(V * V, O, kAccumulate,
-             {seg(opR(Wb, v2, 1, V, v, 1), op1(OOt(j, k), 1, o, 1), V, -1.0),
-              seg(opR(Wb, v2, v, V, 1, 0), op1(OOt(k, j), 1, o, 1), V, -1.0)},
-             out(T2mb(i), vo, o, V, 0, 1, kBig)),
+             {seg(opR(Wb, v2, 1, V, v, 1), op1(OOt(j, k), 1, os, 1), V, -1.0),
+              seg(opR(Wb, v2, v, V, 1, 0), op1(OOt(k, j), 1, os, 1), V, -1.0)},
+             out(T2mb(i), vo, os, V, 0, 1, kBig)),
         // T2mb[j]: H2 (p=b,q=c,K=a), H5 (p=b,q=a,K=c)
         gemm(V * V, O, kAccumulate,
-             {seg(opR(Wb, v, 1, V, v2, 1), op1(OOt(i, k), 1, o, 1), V, -1.0),
-              seg(opR(Wb, v, v2, V, 1, 0), op1(OOt(k, i), 1, o, 1), V, -1.0)},
-             out(T2mb(j), vo, o, V, 0, 1, kBig)),
+             {seg(opR(Wb, v, 1, V, v2, 1), op1(OOt(i, k), 1, os, 1), V, -1.0),
+              seg(opR(Wb, v, v2, V, 1, 0), op1(OOt(k, i), 1, os, 1), V, -1.0)},
+             out(T2mb(j), vo, os, V, 0, 1, kBig)),
         // T2mb[k]: rows m = q*v + p with p = c: H1 (q=b,K=a), H3 (q=a,K=b)
         gemm(V * V, O, kAccumulate,
-             {seg(opR(Wb, v, 1, V, v2, 1), op1(OOt(i, j), 1, o, 1), V, -1.0),
-              seg(opR(Wb, v2, 1, V, v, 1), op1(OOt(j, i), 1, o, 1), V, -1.0)},
-             out(T2mb(k), o, vo, V, 0, 1, kBig)),
+             {seg(opR(Wb, v, 1, V, v2, 1), op1(OOt(i, j), 1, os, 1), V, -1.0),
+              seg(opR(Wb, v2, 1, V, v, 1), op1(OOt(j, i), 1, os, 1), V, -1.0)},
+             out(T2mb(k), os, vo, V, 0, 1, kBig)),
     };
+    for (GemmDesc &d : ds) d.sums = sums_h;
     PAMD_CHECK(run_gemm_group(c, ds, 3, kProfAdjT2H, distinct));
   }
   return PAMD_OK;
@@ -682,6 +742,7 @@ static int adjoint_combine(const Ctx &c, int i, int j, int k, hipStream_t st,
   ca.S_h = c.S_h;
   ca.o = c.o;
   ca.v = c.v;
+  ca.vp = c.vp;
   ca.i = i;
   ca.j = j;
   ca.k = k;
@@ -724,10 +785,10 @@ static void wbar_out(const Ctx &c, int fmt, OrbitArgs &oa) {
 // Zero the adjoint accumulators and the cotangent outputs of one call.
 static int zero_vjp(const Ctx &c) {
   const int o = c.o, v = c.v;
-  const size_t v2 = (size_t)v * v;
-  PAMD_CHECK(launch_fill(c.Vpb, (size_t)o * v2 * v, 0.0, c.s));
-  PAMD_CHECK(launch_fill(c.T2mb, (size_t)o * o * v2, 0.0, c.s));
-  PAMD_CHECK(launch_fill(c.part_mo, (size_t)kGmax * (o + v), 0.0, c.s));
+  const size_t v2 = (size_t)v * v, vp2 = (size_t)c.vp * c.vp;
+  PAMD_CHECK(launch_fill(c.Vpb, (size_t)o * vp2 * c.vp, 0.0, c.s));
+  PAMD_CHECK(launch_fill(c.T2mb, (size_t)o * c.op * vp2, 0.0, c.s));
+  PAMD_CHECK(launch_fill(c.part_mo, (size_t)kGmax * (o + c.vp), 0.0, c.s));
   PAMD_CHECK(launch_fill(c.t1_bar, (size_t)o * v, 0.0, c.s));
   PAMD_CHECK(launch_fill(c.t2_bar, (size_t)o * o * v2, 0.0, c.s));
   PAMD_CHECK(launch_fill(c.ovoo_bar, (size_t)o * v * o * o, 0.0, c.s));
@@ -740,21 +801,31 @@ static int zero_vjp(const Ctx &c) {
 static int setup(Ctx &c, long long &norb) {
   const int o = c.o, v = c.v;
   const int fmt = split_format(c.prec);
-  PAMD_CHECK(launch_prepare(c.ovvv, c.packed, c.t2, c.ovoo, o, v, c.Vp, c.T2m, c.OOt, fmt, c.s));
-  PAMD_CHECK(launch_prep_sym(c.ovov, o, v, 0, c.OVS, c.s));
-  PAMD_CHECK(launch_prep_sym(c.t2, o, v, 1, c.T2S, c.s));
+  const int nt = (v + 7) / 8;
+  norb = (long long)nt * (nt + 1) * (nt + 2) / 6;
+  PAMD_CHECK(launch_prepare(c.ovvv, c.packed, c.t2, c.ovoo, o, v, c.op, c.vp, c.Vp, c.T2m, c.OOt, fmt, c.s));
+  if (c.pad) {
+    PAMD_CHECK(launch_walk_small_inputs(walk_dims(o, v), c.mo, c.t1, c.t2, c.ovov, c.has_fvo ? c.fvo : nullptr,
+                                        c.OVS, c.T2S, c.t1p, c.fvop, c.mop, c.s));
+    const long long n = (num_triples(o) - c.shard + c.nshards - 1) / c.nshards;
+    PAMD_CHECK(launch_walk_triples(o, c.shard, c.nshards, walk_batches(n, INT_MAX), c.tab, c.s));
+    if (c.wt_host) PAMD_CHECK(launch_walk_upload(c.wt_host, o, c.wt, c.s));
+  } else {
+    PAMD_CHECK(launch_prep_sym(c.ovov, o, v, 0, c.OVS, c.s));
+    PAMD_CHECK(launch_prep_sym(c.t2, o, v, 1, c.T2S, c.s));
+  }
   if (fmt == kSplitBf16x3)
-    PAMD_CHECK(launch_split_bf16x3(c.t2, (size_t)o * o * v * v, (unsigned short *)c.gT2, c.s));
+    PAMD_CHECK(launch_split_t2(c.t2, o, v, c.vp, (unsigned short *)c.gT2, c.s));
   if (c.VpT)
-    PAMD_CHECK(launch_vp_transposes((const unsigned short *)c.Vp, o, v, (unsigned short *)c.VpT,
+    PAMD_CHECK(launch_vp_transposes((const unsigned short *)c.Vp, o, c.vp, (unsigned short *)c.VpT,
                                     (unsigned short *)c.VpU, c.s));
   if (fmt == kSplitF32x2)
     PAMD_CHECK(launch_split_f32x2(c.t2, (size_t)o * o * v * v, (unsigned long long *)c.gT2, c.s));
   PAMD_CHECK(launch_fill(c.tri, (size_t)o * o * o, 0.0, c.s));
-  const int nt = (v + 7) / 8;
-  norb = (long long)nt * (nt + 1) * (nt + 2) / 6;
   PAMD_CHECK(launch_orbit_table(norb, c.orb, c.s));
-  c.G = std::min(orbit_grid(v), kGmax);
+  // padded: two workgroups per CU, four without the adjoint (LDS)
+  c.G = c.pad ? (int)std::min<long long>({norb, (long long)(c.vjp ? 2 : 4) * device_cus(), (long long)kGmax})
+              : std::min(orbit_grid(v), kGmax);
   return PAMD_OK;
 }
 
@@ -779,6 +850,37 @@ static OrbitArgs orbit_args(const Ctx &c, int i, int j, int k, long long norb) {
   oa.part_t = c.part_t;
   oa.part_mo = c.part_mo;
   return oa;
+}
+
+// Epilogue of the t-th triple (i, j, k) of the call's walk on stream st; W: its
+// block.  nb > 1 (padded, energy only): also of the nb - 1 triples after it.
+static int walk_epilogue(const Ctx &c, long long t, int i, int j, int k, double *W, int nb, long long norb,
+                         hipStream_t st) {
+  const double v3 = (double)c.v * c.v * c.v;
+  const double ob = 8.0 * v3 * (c.vjp ? 3.0 : 1.0) * nb;  // W read (+ Wbar, Vbar written)
+  OrbitArgs oa = orbit_args(c, i, j, k, norb);
+  oa.W = W;
+  if (c.vjp) wbar_out(c, split_format(c.prec), oa);
+  oa.vjp = c.vjp;
+  oa.ebar = c.ebar;
+  if (c.pad) {
+    oa.t1 = c.t1p;
+    oa.fvo = c.fvop;
+    oa.mo = c.mop;
+    oa.v = c.vp;
+    oa.ws = (long long)c.vp * c.vp;
+    oa.tri = c.tab + t;
+    oa.nb = nb;
+    oa.wt = c.wt_host ? c.wt : nullptr;
+    PAMD_CHECK(timed(st, kProfOrbit, 0.0, ob, [&] { return launch_walk_orbit(oa, c.G, st); }));
+    return PAMD_OK;
+  }
+  oa.omega = (i == j || j == k) ? 1.0 : 2.0;
+  // a diagonal occupied projector diag(m) weighs the whole triple by
+  // (m_i + m_j + m_k) / 3 (the triple energy is symmetric in i, j, k)
+  if (c.wt_host) oa.ebar = c.ebar * ((c.wt_host[i] + c.wt_host[j] + c.wt_host[k]) / 3.0);
+  PAMD_CHECK(timed(st, kProfOrbit, 0.0, ob, [&] { return launch_orbit(oa, c.G, st); }));
+  return PAMD_OK;
 }
 
 // Projected walk: for every unordered occupied pair (j, k), all o triples
@@ -913,7 +1015,7 @@ static PipeRes *pipe_resources() {
 // on G; the cotangents, triple energies and dE/de partials on E) are each
 // written by one stream, in walk order, so the sums are the sequential walk's.
 static int run_vjp_pipelined(Ctx &c, long long norb, PipeRes &pr) {
-  const int o = c.o, fmt = split_format(c.prec);
+  const int o = c.o;
   std::vector<int> tr;  // triples of this call in walk order, i | j << 10 | k << 20
   {
     long long windex = -1;
@@ -953,7 +1055,7 @@ static int run_vjp_pipelined(Ctx &c, long long norb, PipeRes &pr) {
   }();
   const bool pair_on = pair_env && c.gW != c.W && c.gW2 != nullptr;
   if (pair_on && c.prec == PAMD_PREC_BF16X3) {
-    const long long v3 = (long long)c.v * c.v * c.v;
+    const long long v3 = (long long)c.vp * c.vp * c.vp;
     for (int p = 0; p < 2; ++p) {
       PlanarMap &pm = cx[p].planes;
       if (pm.count >= 8) return PAMD_ERR_ARG;
@@ -991,15 +1093,8 @@ static int run_vjp_pipelined(Ctx &c, long long norb, PipeRes &pr) {
       ijk(t, i, j, k);
       // E: epilogue and V-bar reductions of t
       PAMD_CHECK(hipStreamWaitEvent(E, wb[p], 0));
-      OrbitArgs oa = orbit_args(C, i, j, k, norb);
-      wbar_out(C, fmt, oa);
-      oa.vjp = 1;
-      oa.omega = (i == j || j == k) ? 1.0 : 2.0;
-      oa.ebar = c.wt_host ? c.ebar * ((c.wt_host[i] + c.wt_host[j] + c.wt_host[k]) / 3.0) : c.ebar;
-      {
-        const double ob = 8.0 * (double)c.v * c.v * c.v * 3.0;  // W read, Wbar and Vbar written
-        PAMD_CHECK(timed(E, kProfOrbit, 0.0, ob, [&] { return launch_orbit(oa, C.G, E); }));
-      }
+      st = walk_epilogue(C, t, i, j, k, C.W, 1, norb, E);
+      if (st != PAMD_OK) return st;
       st = adjoint_vr(C, i, j, k, E);
       if (st != PAMD_OK) return st;
       PAMD_CHECK(hipEventRecord(vr[p], E));
@@ -1057,8 +1152,7 @@ static int run_vjp_pipelined(Ctx &c, long long norb, PipeRes &pr) {
 }
 
 static int run(Ctx &c) {
-  const int o = c.o, v = c.v;
-  const int fmt = split_format(c.prec);
+  const int o = c.o;
   long long norb = 0;
   {
     const int st0 = setup(c, norb);
@@ -1084,7 +1178,7 @@ static int run(Ctx &c) {
     // pair (i, j) are built by one launch per pass; each triple's epilogue then
     // reads its own block.  Same triples, same per-triple arithmetic and the
     // same fixed-order sum over tri as the walk below.
-    const size_t v3 = (size_t)v * v * v;
+    const size_t v3 = (size_t)c.vp * c.vp * c.vp;
     for (int i = 0; i < o; ++i)
       for (int j = i; j < o; ++j)
         for (int kb = (i == j ? j + 1 : j); kb < o; kb += c.wbatch) {
@@ -1092,16 +1186,19 @@ static int run(Ctx &c) {
           g_prof_on = g_prof_every > 0 && (tcount % g_prof_every) < nb;
           int st = build_w(c, i, j, kb, nb);
           if (st != PAMD_OK) return st;
+          if (c.pad) {
+            st = walk_epilogue(c, tcount, i, j, kb, c.W, nb, norb, c.s);
+            if (st != PAMD_OK) return st;
+            PAMD_CHECK(launch_walk_energies(c.tab + tcount, nb, o, c.part_t, c.G, c.tri, c.s));
+          }
           for (int b = 0; b < nb; ++b) {
             const int k = kb + b;
+            if (!c.pad) {
+              st = walk_epilogue(c, tcount, i, j, k, c.W + b * v3, 1, norb, c.s);
+              if (st != PAMD_OK) return st;
+              PAMD_CHECK(launch_triple_energy(c.part_t, c.G, c.tri + ((size_t)i * o + j) * o + k, c.s));
+            }
             ++tcount;
-            OrbitArgs oa = orbit_args(c, i, j, k, norb);
-            oa.W = c.W + b * v3;
-            oa.omega = (i == j || j == k) ? 1.0 : 2.0;
-            oa.ebar = c.ebar;
-            const double ob = 8.0 * (double)v3;  // W read
-            PAMD_CHECK(timed(c.s, kProfOrbit, 0.0, ob, [&] { return launch_orbit(oa, c.G, c.s); }));
-            PAMD_CHECK(launch_triple_energy(c.part_t, c.G, c.tri + ((size_t)i * o + j) * o + k, c.s));
             if (g_progress_every > 0 && tcount % g_progress_every == 0) {
               PAMD_CHECK(hipStreamSynchronize(c.s));
               const double el = std::chrono::duration<double>(std::chrono::steady_clock::now() -
@@ -1127,18 +1224,8 @@ static int run(Ctx &c) {
         ++tcount;
         int st = build_w(c, i, j, k);
         if (st != PAMD_OK) return st;
-        OrbitArgs oa = orbit_args(c, i, j, k, norb);
-        if (c.vjp) wbar_out(c, fmt, oa);
-        oa.vjp = c.vjp;
-        oa.omega = (i == j || j == k) ? 1.0 : 2.0;
-        // a diagonal occupied projector diag(m) weighs the whole triple by
-        // (m_i + m_j + m_k) / 3 (the triple energy is symmetric in i, j, k)
-        oa.ebar = c.wt_host ? c.ebar * ((c.wt_host[i] + c.wt_host[j] + c.wt_host[k]) / 3.0) : c.ebar;
-        {
-          const double v3 = (double)v * v * v;
-          const double ob = 8.0 * v3 * (c.vjp ? 3.0 : 1.0);  // W read (+ Wbar, Vbar written)
-          PAMD_CHECK(timed(c.s, kProfOrbit, 0.0, ob, [&] { return launch_orbit(oa, c.G, c.s); }));
-        }
+        st = walk_epilogue(c, tcount - 1, i, j, k, c.W, 1, norb, c.s);
+        if (st != PAMD_OK) return st;
         if (!c.vjp)
           PAMD_CHECK(launch_triple_energy(c.part_t, c.G, c.tri + ((size_t)i * o + j) * o + k, c.s));
         if (c.vjp) {
@@ -1185,6 +1272,15 @@ static void bind_workspace(Ctx &c, const Layout &L, void *ws) {
   c.orb = (unsigned short *)(b + L.off_orb);
   c.W = (double *)(b + L.off_W);
   c.wbatch = L.wbatch;
+  c.pad = L.pad;
+  c.op = L.op;
+  c.vp = L.vp;
+  if (L.pad) {
+    c.t1p = (double *)(b + L.off_t1);
+    c.fvop = (double *)(b + L.off_fvo);
+    c.mop = (double *)(b + L.off_mo);
+    c.tab = (int *)(b + L.off_tab);
+  }
   c.tri = (double *)(b + L.off_tri);
   c.part_t = (double *)(b + L.off_part_t);
   c.wt = (double *)(b + L.off_wt);
@@ -1194,7 +1290,7 @@ static void bind_workspace(Ctx &c, const Layout &L, void *ws) {
   c.VpT = L.vpt ? (double *)(b + L.off_VpT) : nullptr;
   c.VpU = L.vpt ? (double *)(b + L.off_VpU) : nullptr;
   {
-    const long long o = c.o, v = c.v, v3 = v * v * v;
+    const long long o = c.o, op = c.op, v = c.vp, v3 = v * v * v;
     PlanarMap &pm = c.planes;
     pm.count = 0;
     auto add = [&](const void *p, long long n) {
@@ -1203,8 +1299,8 @@ static void bind_workspace(Ctx &c, const Layout &L, void *ws) {
       ++pm.count;
     };
     add(c.Vp, o * v3);
-    add(c.T2m, o * o * v * v);
-    add(c.OOt, o * o * o * v);
+    add(c.T2m, o * op * v * v);
+    add(c.OOt, o * o * op * v);
     add(c.gT2, o * o * v * v);
     if (c.vjp) add(c.gW, v3);
     if (c.VpT) {
@@ -1247,8 +1343,6 @@ struct WalkLayout {
   size_t off_VT, off_TB, off_TBt, off_OVS, off_T2S, off_t1, off_fvo, off_mo, off_orb, off_tri_e, off_tab, off_wt,
       off_W, off_part_t, off_Vb, off_VTb, off_R, off_part, off_vec, off_mo_rows, off_mo2;
 };
-
-static long long num_triples(int o) { return (long long)o * (o + 1) * (o + 2) / 6 - o; }
 
 static WalkLayout walk_layout(int o, int v, int vjp, int nb) {
   WalkLayout L;
@@ -1654,7 +1748,9 @@ const char *pamd_version(void) { return "pyscfad_amd 0.1.0 (gfx950)"; }
 
 int pamd_ccsdt_workspace_size(const pamd_ccsdt_config *cfg, int with_vjp, size_t *bytes) {
   if (!cfg || !bytes || cfg->nocc < 1 || cfg->nvir < 1) return PAMD_ERR_ARG;
-  *bytes = make_layout(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, cfg->precision, true).total;
+  const Layout L = make_layout(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, cfg->precision, true);
+  *bytes = std::max(L.total, b3_layout(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, cfg->precision, true,
+                                       (size_t)-1, L).total);
   WalkLayout wl;
   if (cfg->precision == PAMD_PREC_FP64 &&
       walk_pick(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, (size_t)-1, *bytes, wl))
@@ -1690,7 +1786,7 @@ static int energy_impl(const pamd_ccsdt_config *cfg, const double *mo, const dou
   WalkLayout wl;
   if (c.prec == PAMD_PREC_FP64 && walk_pick(c.o, c.v, 0, ws_bytes, L.total, wl))
     return run_walk(c, wl, ws, nullptr, nullptr);
-  bind_workspace(c, L, ws);
+  bind_workspace(c, b3_layout(c.o, c.v, 0, c.prec, false, ws_bytes, L), ws);
   return run(c);
 }
 
@@ -1787,13 +1883,13 @@ static int vjp_impl(const pamd_ccsdt_config *cfg, const double *mo_energy, const
   if (walk) {
     st = run_walk(c, wl, workspace, ovvv_bar, mo_energy_bar);
   } else {
-    bind_workspace(c, L, workspace);
+    bind_workspace(c, b3_layout(c.o, c.v, 1, c.prec, pipe, workspace_bytes, L), workspace);
     st = run(c);
   }
   if (st != PAMD_OK) return st;
   const int o = c.o, v = c.v;
   if (wt_host) {
-    if (!walk)
+    if (!walk && !c.pad)
       PAMD_CHECK(hipMemcpyAsync(c.wt, wt_host, sizeof(double) * (size_t)o, hipMemcpyHostToDevice,
                                 c.s));
     PAMD_CHECK(launch_weighted_energy(c.tri, o, c.wt, et_bar, e_out, wt_bar, c.s));
@@ -1801,9 +1897,9 @@ static int vjp_impl(const pamd_ccsdt_config *cfg, const double *mo_energy, const
     PAMD_CHECK(launch_total_energy(c.tri, o, e_out, c.s));
   }
   if (walk) return PAMD_OK;
-  PAMD_CHECK(launch_reduce_rows(c.part_mo, c.G, o + v, mo_energy_bar, 0, c.s));
-  PAMD_CHECK(launch_fold_ovvv(c.Vpb, o, v, c.packed, ovvv_bar, c.s));
-  PAMD_CHECK(launch_fold_t2m(c.T2mb, o, v, t2_bar, c.s));
+  PAMD_CHECK(launch_reduce_rows(c.part_mo, c.G, o + v, o + c.vp, mo_energy_bar, 0, c.s));
+  PAMD_CHECK(launch_fold_ovvv(c.Vpb, o, v, c.vp, c.packed, ovvv_bar, c.s));
+  PAMD_CHECK(launch_fold_t2m(c.T2mb, o, v, c.op, c.vp, t2_bar, c.s));
   return PAMD_OK;
 }
 
@@ -1961,9 +2057,9 @@ static int projected_impl(const pamd_ccsdt_config *cfg, const double *mo_energy,
   PAMD_CHECK(launch_projected_total(pair_e, c.o, e_out, c.s));
   if (vjp) {
     const int o = c.o, v = c.v;
-    PAMD_CHECK(launch_reduce_rows(c.part_mo, c.G, o + v, mo_energy_bar, 0, c.s));
-    PAMD_CHECK(launch_fold_ovvv(c.Vpb, o, v, c.packed, ovvv_bar, c.s));
-    PAMD_CHECK(launch_fold_t2m(c.T2mb, o, v, t2_bar, c.s));
+    PAMD_CHECK(launch_reduce_rows(c.part_mo, c.G, o + v, o + c.vp, mo_energy_bar, 0, c.s));
+    PAMD_CHECK(launch_fold_ovvv(c.Vpb, o, v, c.vp, c.packed, ovvv_bar, c.s));
+    PAMD_CHECK(launch_fold_t2m(c.T2mb, o, v, c.op, c.vp, t2_bar, c.s));
   }
   return PAMD_OK;
 }
@@ -2019,8 +2115,8 @@ int pamd_debug_gemm_descriptors(int nocc, int nvir, int i, int j, int k, int wit
   Layout L = make_layout(nocc, nvir, with_vjp ? 1 : 0, PAMD_PREC_FP64);
   Ctx c;
   memset(&c, 0, sizeof(c));
-  c.o = nocc;
-  c.v = nvir;
+  c.o = c.op = nocc;
+  c.v = c.vp = nvir;
   c.vjp = with_vjp ? 1 : 0;
   c.Vp = (double *)bases[0];
   c.T2m = (double *)bases[1];
@@ -2059,8 +2155,8 @@ int pamd_debug_paired_adjoint_descriptors(int nocc, int nvir, int i, int j, int 
   Layout L = make_layout(nocc, nvir, 1, PAMD_PREC_FP64);
   Ctx c1;
   memset(&c1, 0, sizeof(c1));
-  c1.o = nocc;
-  c1.v = nvir;
+  c1.o = c1.op = nocc;
+  c1.v = c1.vp = nvir;
   c1.vjp = 1;
   c1.Vp = (double *)bases[0];
   c1.T2m = (double *)bases[1];

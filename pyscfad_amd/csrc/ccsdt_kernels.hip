@@ -69,49 +69,62 @@ __device__ double block_sum256(double x, double *scratch) {
 //   OOt[x][y][p][m] = ovoo[x,p,m,y]
 // ---------------------------------------------------------------------------
 template <class T>
-__global__ void k_prep_vp(const double *__restrict__ ovvv, int packed, int o, int v, T Vp) {
-  const size_t total = (size_t)o * v * v * v;
+__global__ void k_prep_vp(const double *__restrict__ ovvv, int packed, int o, int v, int vp, T Vp) {
+  const size_t total = (size_t)o * vp * vp * vp;
   const size_t vv = (size_t)v * v;
   const size_t npair = (size_t)v * (v + 1) / 2;
   for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
        t += (size_t)gridDim.x * blockDim.x) {
-    size_t f = t % v;
-    size_t q = (t / v) % v;
-    size_t xp = t / vv;  // x * v + p
-    double val;
-    if (packed) {
-      size_t hi = f > q ? f : q, lo = f > q ? q : f;
-      val = ovvv[xp * npair + hi * (hi + 1) / 2 + lo];
-    } else {
-      val = ovvv[xp * vv + f * v + q];
+    size_t f = t % vp;
+    size_t q = (t / vp) % vp;
+    size_t p = (t / ((size_t)vp * vp)) % vp, x = t / ((size_t)vp * vp * vp);
+    double val = 0.0;
+    if (p < (size_t)v && q < (size_t)v && f < (size_t)v) {
+      const size_t xp = x * v + p;
+      if (packed) {
+        size_t hi = f > q ? f : q, lo = f > q ? q : f;
+        val = ovvv[xp * npair + hi * (hi + 1) / 2 + lo];
+      } else {
+        val = ovvv[xp * vv + f * v + q];
+      }
     }
     put(Vp, t, val);
   }
 }
 
 template <class T>
-__global__ void k_prep_t2m(const double *__restrict__ t2, int o, int v, T T2m) {
-  const size_t total = (size_t)o * o * v * v;
+__global__ void k_prep_t2m(const double *__restrict__ t2, int o, int v, int op, int vp, T T2m) {
+  const size_t total = (size_t)o * vp * vp * op;
   for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
        t += (size_t)gridDim.x * blockDim.x) {
-    size_t m = t % o;
-    size_t q = (t / o) % v;
-    size_t p = (t / ((size_t)o * v)) % v;
-    size_t x = t / ((size_t)o * v * v);
-    put(T2m, t, t2[((x * o + m) * v + p) * v + q]);
+    size_t m = t % op;
+    size_t q = (t / op) % vp;
+    size_t p = (t / ((size_t)op * vp)) % vp;
+    size_t x = t / ((size_t)op * vp * vp);
+    const bool in = m < (size_t)o && q < (size_t)v && p < (size_t)v;
+    put(T2m, t, in ? t2[((x * o + m) * v + p) * v + q] : 0.0);
   }
 }
 
 template <class T>
-__global__ void k_prep_oot(const double *__restrict__ ovoo, int o, int v, T OOt) {
-  const size_t total = (size_t)o * o * v * o;
+__global__ void k_prep_oot(const double *__restrict__ ovoo, int o, int v, int op, int vp, T OOt) {
+  const size_t total = (size_t)o * o * vp * op;
   for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
        t += (size_t)gridDim.x * blockDim.x) {
-    size_t m = t % o;
-    size_t p = (t / o) % v;
-    size_t y = (t / ((size_t)o * v)) % o;
-    size_t x = t / ((size_t)o * v * o);
-    put(OOt, t, ovoo[((x * v + p) * o + m) * o + y]);
+    size_t m = t % op;
+    size_t p = (t / op) % vp;
+    size_t y = (t / ((size_t)op * vp)) % o;
+    size_t x = t / ((size_t)op * vp * o);
+    put(OOt, t, m < (size_t)o && p < (size_t)v ? ovoo[((x * v + p) * o + m) * o + y] : 0.0);
+  }
+}
+
+__global__ void k_split_t2(const double *__restrict__ t2, int o, int v, int vp, Planar3 out) {
+  const size_t total = (size_t)o * o * vp * vp;
+  for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
+       t += (size_t)gridDim.x * blockDim.x) {
+    const size_t q = t % vp, p = (t / vp) % vp, xy = t / ((size_t)vp * vp);
+    put(out, t, q < (size_t)v && p < (size_t)v ? t2[(xy * v + p) * v + q] : 0.0);
   }
 }
 
@@ -125,32 +138,38 @@ static unsigned grid_for(size_t n) {
 // T: the store sink (a pointer, or Planar3)
 template <class T>
 static hipError_t prepare_as(const double *ovvv, int packed, const double *t2, const double *ovoo,
-                             int o, int v, T Vp, T T2m, T OOt, hipStream_t s) {
-  hipLaunchKernelGGL(k_prep_vp<T>, dim3(grid_for((size_t)o * v * v * v)), dim3(256), 0, s, ovvv,
-                     packed, o, v, Vp);
-  hipLaunchKernelGGL(k_prep_t2m<T>, dim3(grid_for((size_t)o * o * v * v)), dim3(256), 0, s, t2, o,
-                     v, T2m);
-  hipLaunchKernelGGL(k_prep_oot<T>, dim3(grid_for((size_t)o * o * v * o)), dim3(256), 0, s, ovoo, o,
-                     v, OOt);
+                             int o, int v, int op, int vp, T Vp, T T2m, T OOt, hipStream_t s) {
+  hipLaunchKernelGGL(k_prep_vp<T>, dim3(grid_for((size_t)o * vp * vp * vp)), dim3(256), 0, s, ovvv,
+                     packed, o, v, vp, Vp);
+  hipLaunchKernelGGL(k_prep_t2m<T>, dim3(grid_for((size_t)o * op * vp * vp)), dim3(256), 0, s, t2, o,
+                     v, op, vp, T2m);
+  hipLaunchKernelGGL(k_prep_oot<T>, dim3(grid_for((size_t)o * o * vp * op)), dim3(256), 0, s, ovoo, o,
+                     v, op, vp, OOt);
+  return hipGetLastError();
+}
+
+hipError_t launch_split_t2(const double *t2, int o, int v, int vp, unsigned short *out, hipStream_t s) {
+  const size_t n = (size_t)o * o * vp * vp;
+  hipLaunchKernelGGL(k_split_t2, dim3(grid_for(n)), dim3(256), 0, s, t2, o, v, vp, Planar3{out, (long long)n});
   return hipGetLastError();
 }
 
 // split == kSplitBf16x3: three bf16 planes (hi, mid, lo) per array, each plane
 // as long as the array (in the first 6 of the 8 bytes per element allocated)
 hipError_t launch_prepare(const double *ovvv, int packed, const double *t2, const double *ovoo,
-                          int o, int v, double *Vp, double *T2m, double *OOt, int split,
+                          int o, int v, int op, int vp, double *Vp, double *T2m, double *OOt, int split,
                           hipStream_t s) {
   if (split == kSplitBf16x3) {
-    const long long n_vp = (long long)o * v * v * v, n_t2m = (long long)o * o * v * v,
-                    n_oot = (long long)o * o * v * o;
-    return prepare_as<Planar3>(ovvv, packed, t2, ovoo, o, v,
+    const long long n_vp = (long long)o * vp * vp * vp, n_t2m = (long long)o * op * vp * vp,
+                    n_oot = (long long)o * o * vp * op;
+    return prepare_as<Planar3>(ovvv, packed, t2, ovoo, o, v, op, vp,
                                Planar3{(unsigned short *)Vp, n_vp},
                                Planar3{(unsigned short *)T2m, n_t2m},
                                Planar3{(unsigned short *)OOt, n_oot}, s);
   }
   if (split == kSplitF32x2)
-    return prepare_as<F2 *>(ovvv, packed, t2, ovoo, o, v, (F2 *)Vp, (F2 *)T2m, (F2 *)OOt, s);
-  return prepare_as<double *>(ovvv, packed, t2, ovoo, o, v, Vp, T2m, OOt, s);
+    return prepare_as<F2 *>(ovvv, packed, t2, ovoo, o, v, op, vp, (F2 *)Vp, (F2 *)T2m, (F2 *)OOt, s);
+  return prepare_as<double *>(ovvv, packed, t2, ovoo, o, v, op, vp, Vp, T2m, OOt, s);
 }
 
 __global__ void k_split_f32x2(const double *__restrict__ x, size_t n, F2 *__restrict__ out) {
@@ -1150,22 +1169,22 @@ __global__ void k_splitk_reduce(double *part_p, int S_p, size_t T_p, double *par
 }
 
 __device__ __forceinline__ void combine_block(const CombineArgs &A, size_t t) {
-  const int o = A.o, v = A.v, i = A.i, j = A.j, k = A.k;
+  const int o = A.o, v = A.v, vr = A.vp, i = A.i, j = A.j, k = A.k;
   const size_t vv = (size_t)v * v;
   const double *R = A.R;
   if (t < vv) {
     const int p = (int)(t / v), q = (int)(t % v);
-    const size_t pq = (size_t)p * v + q, qp = (size_t)q * v + p;
+    const size_t pq = (size_t)p * vr + q, qp = (size_t)q * vr + p;
     // ovov_bar[x,p,y,q]
     auto ob = [&](int x, int y) -> double & {
       return A.ovov_bar[(((size_t)x * v + p) * o + y) * v + q];
     };
-    ob(i, j) += 0.5 * vr_csum(R, v, 0, pq);
-    ob(j, i) += 0.5 * vr_csum(R, v, 0, qp);
-    ob(i, k) += 0.5 * vr_sum(R, v, 2, pq);
-    ob(k, i) += 0.5 * vr_sum(R, v, 2, qp);
-    ob(j, k) += 0.5 * vr_sum(R, v, 4, pq);
-    ob(k, j) += 0.5 * vr_sum(R, v, 4, qp);
+    ob(i, j) += 0.5 * vr_csum(R, vr, 0, pq);
+    ob(j, i) += 0.5 * vr_csum(R, vr, 0, qp);
+    ob(i, k) += 0.5 * vr_sum(R, vr, 2, pq);
+    ob(k, i) += 0.5 * vr_sum(R, vr, 2, qp);
+    ob(j, k) += 0.5 * vr_sum(R, vr, 4, pq);
+    ob(k, j) += 0.5 * vr_sum(R, vr, 4, qp);
     // t2_bar[x,y,p,q]: particle split-K partials (problem order P1..P6) + V terms
     auto tb = [&](int x, int y) -> double & {
       return A.t2_bar[(((size_t)x * o + y) * v + p) * v + q];
@@ -1173,15 +1192,15 @@ __device__ __forceinline__ void combine_block(const CombineArgs &A, size_t t) {
     const int xs[6] = {k, j, k, i, j, i};
     const int ys[6] = {j, k, i, k, i, j};
     for (int pr = 0; pr < 6; ++pr) {
-      double s = A.part_p[(size_t)pr * A.S_p * vv + pq];  // split-K sum (k_splitk_reduce)
+      double s = A.part_p[(size_t)pr * A.S_p * vv + t];  // split-K sum (k_splitk_reduce)
       if (A.has_fvo) {
         switch (pr) {
-          case 0: s += 0.5 * vr_sum(R, v, 5, qp); break;  // t2_bar[k,j,c,b] += R6[b,c]/2
-          case 1: s += 0.5 * vr_sum(R, v, 5, pq); break;  // t2_bar[j,k,b,c] += R6[b,c]/2
-          case 2: s += 0.5 * vr_sum(R, v, 3, qp); break;  // t2_bar[k,i,c,a] += R4[a,c]/2
-          case 3: s += 0.5 * vr_sum(R, v, 3, pq); break;  // t2_bar[i,k,a,c] += R4[a,c]/2
-          case 4: s += 0.5 * vr_csum(R, v, 1, qp); break;  // t2_bar[j,i,b,a] += R2[a,b]/2
-          case 5: s += 0.5 * vr_csum(R, v, 1, pq); break;  // t2_bar[i,j,a,b] += R2[a,b]/2
+          case 0: s += 0.5 * vr_sum(R, vr, 5, qp); break;  // t2_bar[k,j,c,b] += R6[b,c]/2
+          case 1: s += 0.5 * vr_sum(R, vr, 5, pq); break;  // t2_bar[j,k,b,c] += R6[b,c]/2
+          case 2: s += 0.5 * vr_sum(R, vr, 3, qp); break;  // t2_bar[k,i,c,a] += R4[a,c]/2
+          case 3: s += 0.5 * vr_sum(R, vr, 3, pq); break;  // t2_bar[i,k,a,c] += R4[a,c]/2
+          case 4: s += 0.5 * vr_csum(R, vr, 1, qp); break;  // t2_bar[j,i,b,a] += R2[a,b]/2
+          case 5: s += 0.5 * vr_csum(R, vr, 1, pq); break;  // t2_bar[i,j,a,b] += R2[a,b]/2
         }
       }
       tb(xs[pr], ys[pr]) += s;
@@ -1203,18 +1222,18 @@ __device__ __forceinline__ void combine_block(const CombineArgs &A, size_t t) {
 // t1_bar / fvo_bar pieces of one triple: column sums over a of four v x v
 // slices of R, one block per 64 columns (the 4 waves split the rows).
 __device__ __forceinline__ void colsums_block(const CombineArgs &A, int blk, double (*red)[4][64]) {
-  const int o = A.o, v = A.v, i = A.i, j = A.j, k = A.k;
+  const int o = A.o, v = A.v, vr = A.vp, i = A.i, j = A.j, k = A.k;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = blk * 64 + lane;
   const double *R = A.R;
   double sk = 0.0, sj = 0.0, fk = 0.0, fj = 0.0;
   if (c < v) {
     for (int a = wave; a < v; a += 4) {
-      const size_t ac = (size_t)a * v + c;
-      sk += vr_sum(R, v, 6, ac);
-      sj += vr_csum(R, v, 8, ac);
-      fk += vr_sum(R, v, 7, ac);
-      fj += vr_csum(R, v, 9, ac);
+      const size_t ac = (size_t)a * vr + c;
+      sk += vr_sum(R, vr, 6, ac);
+      sj += vr_csum(R, vr, 8, ac);
+      fk += vr_sum(R, vr, 7, ac);
+      fj += vr_csum(R, vr, 9, ac);
     }
   }
   red[0][wave][lane] = sk;
@@ -1228,10 +1247,10 @@ __device__ __forceinline__ void colsums_block(const CombineArgs &A, int blk, dou
     for (int q = 0; q < 4; ++q) s[q] = red[q][0][lane] + red[q][1][lane] + red[q][2][lane] + red[q][3][lane];
     A.t1_bar[k * v + c] += 0.5 * s[0];
     A.t1_bar[j * v + c] += 0.5 * s[1];
-    A.t1_bar[i * v + c] += 0.5 * vr_sum_vec(R, v, 0, c);
+    A.t1_bar[i * v + c] += 0.5 * vr_sum_vec(R, vr, 0, c);
     A.fvo_bar[(size_t)c * o + k] += 0.5 * s[2];
     A.fvo_bar[(size_t)c * o + j] += 0.5 * s[3];
-    A.fvo_bar[(size_t)c * o + i] += 0.5 * vr_sum_vec(R, v, 1, c);
+    A.fvo_bar[(size_t)c * o + i] += 0.5 * vr_sum_vec(R, vr, 1, c);
   }
 }
 
@@ -1280,7 +1299,7 @@ hipError_t launch_combine(const CombineArgs &a, hipStream_t s) {
 // ovvv_bar from Vpb[x][p][q][f] (= dE/d ovvv[x,p,f,q]):
 //   full:   out[x,p,f,q] = Vpb[x][p][q][f]
 //   packed: out[x,p,f(f+1)/2+q] = g[f,q] + g[q,f] (q < f), g[f,f] (q == f)
-__global__ void k_fold_ovvv(const double *__restrict__ Vpb, int o, int v, int packed,
+__global__ void k_fold_ovvv(const double *__restrict__ Vpb, int o, int v, int vp, int packed,
                             double *__restrict__ out) {
   const size_t vv = (size_t)v * v;
   const size_t npair = (size_t)v * (v + 1) / 2;
@@ -1293,54 +1312,54 @@ __global__ void k_fold_ovvv(const double *__restrict__ Vpb, int o, int v, int pa
       while (f * (f + 1) / 2 > r) --f;
       while ((f + 1) * (f + 2) / 2 <= r) ++f;
       const size_t q = r - f * (f + 1) / 2;
-      const double *base = Vpb + xp * vv;
-      double val = base[q * v + f];
-      if (q != f) val += base[f * v + q];
+      const double *base = Vpb + ((xp / v) * vp + xp % v) * vp * vp;
+      double val = base[q * vp + f];
+      if (q != f) val += base[f * vp + q];
       out[t] = val;
     } else {
       const size_t xp = t / vv, r = t % vv;
       const size_t f = r / v, q = r % v;
-      out[t] = Vpb[xp * vv + q * v + f];
+      out[t] = Vpb[((xp / v) * vp + xp % v) * vp * vp + q * vp + f];
     }
   }
 }
 
-hipError_t launch_fold_ovvv(const double *Vpb, int o, int v, int packed, double *out, hipStream_t s) {
+hipError_t launch_fold_ovvv(const double *Vpb, int o, int v, int vp, int packed, double *out, hipStream_t s) {
   size_t n = (size_t)o * v * (packed ? (size_t)v * (v + 1) / 2 : (size_t)v * v);
-  hipLaunchKernelGGL(k_fold_ovvv, dim3(grid_for(n)), dim3(256), 0, s, Vpb, o, v, packed, out);
+  hipLaunchKernelGGL(k_fold_ovvv, dim3(grid_for(n)), dim3(256), 0, s, Vpb, o, v, vp, packed, out);
   return hipGetLastError();
 }
 
 // t2_bar[x,m,p,q] += T2mb[x][p][q][m]
-__global__ void k_fold_t2m(const double *__restrict__ T2mb, int o, int v, double *__restrict__ t2_bar) {
+__global__ void k_fold_t2m(const double *__restrict__ T2mb, int o, int v, int op, int vp, double *__restrict__ t2_bar) {
   const size_t total = (size_t)o * o * v * v;
   for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
        t += (size_t)gridDim.x * blockDim.x) {
     const size_t q = t % v, p = (t / v) % v, m = (t / ((size_t)v * v)) % o,
                  x = t / ((size_t)v * v * o);
-    t2_bar[t] += T2mb[((x * v + p) * v + q) * o + m];
+    t2_bar[t] += T2mb[((x * vp + p) * vp + q) * op + m];
   }
 }
 
-hipError_t launch_fold_t2m(const double *T2mb, int o, int v, double *t2_bar, hipStream_t s) {
+hipError_t launch_fold_t2m(const double *T2mb, int o, int v, int op, int vp, double *t2_bar, hipStream_t s) {
   hipLaunchKernelGGL(k_fold_t2m, dim3(grid_for((size_t)o * o * v * v)), dim3(256), 0, s, T2mb, o,
-                     v, t2_bar);
+                     v, op, vp, t2_bar);
   return hipGetLastError();
 }
 
 // out[c] (+)= sum_r part[r][c], fixed order
-__global__ void k_reduce_rows(const double *part, int rows, int cols, double *out, int accumulate) {
+__global__ void k_reduce_rows(const double *part, int rows, int cols, int ld, double *out, int accumulate) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= cols) return;
   double s = 0.0;
-  for (int r = 0; r < rows; ++r) s += part[(size_t)r * cols + c];
+  for (int r = 0; r < rows; ++r) s += part[(size_t)r * ld + c];
   out[c] = accumulate ? out[c] + s : s;
 }
 
-hipError_t launch_reduce_rows(const double *part, int rows, int cols, double *out, int accumulate,
+hipError_t launch_reduce_rows(const double *part, int rows, int cols, int ld, double *out, int accumulate,
                               hipStream_t s) {
   hipLaunchKernelGGL(k_reduce_rows, dim3((cols + 255) / 256), dim3(256), 0, s, part, rows, cols,
-                     out, accumulate);
+                     ld, out, accumulate);
   return hipGetLastError();
 }
 

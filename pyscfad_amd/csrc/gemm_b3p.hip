@@ -582,7 +582,7 @@ bool gemm_b3p_group_ok(const GemmDesc *ds, int n) {
   for (int p = 0; p < n; ++p) {
     const GemmDesc &d = ds[p];
     if (d.nseg > 2 || d.M != ds[0].M || d.N != ds[0].N || d.splits != ds[0].splits ||
-        d.mode != ds[0].mode || !gemm_b3p_ok(d))
+        d.mode != ds[0].mode || d.sums == kSumsFlushed || !gemm_b3p_ok(d))
       return false;
   }
   const GemmDesc &d = ds[0];

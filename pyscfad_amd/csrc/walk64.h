@@ -46,6 +46,10 @@ hipError_t launch_walk_inputs(const WalkDims &d, const double *mo, const double 
                               const double *ovvv, int packed, const double *ovoo, const double *ovov,
                               const double *fvo, double *VT, double *TB, double *TBt, double *OVS,
                               double *T2S, double *t1p, double *fvop, double *mop, hipStream_t s);
+// of these, what the orbit epilogue and the V-bar reductions read
+hipError_t launch_walk_small_inputs(const WalkDims &d, const double *mo, const double *t1, const double *t2,
+                                    const double *ovov, const double *fvo, double *OVS, double *T2S, double *t1p,
+                                    double *fvop, double *mop, hipStream_t s);
 // Batches.  The call's triples (walk order i <= j <= k without i == j == k, every
 // nshards-th from shard on) are cut into runs of 8, dealt to the batches in
 // turn: a run shares i, j and so its slabs of VT, while every batch has about
@@ -78,7 +82,8 @@ hipError_t launch_walk_triples(int o, int shard, int nshards, const WalkBatches 
 hipError_t launch_walk_w(const WalkDims &d, const double *VT, const double *TBt, double *W, const int *tri,
                          int nb, hipStream_t s);
 // epilogue (OrbitArgs' batch fields, grid rows of G workgroups; walk64_orbit.hip):
-// energies and, with vjp, Wbar over W, Vbar and the mo_energy_bar rows
+// energies and, with vjp, Wbar (over W, or as bf16 planes when Wb3 is set), Vbar and
+// the mo_energy_bar rows
 hipError_t launch_walk_orbit(const OrbitArgs &a, int G, hipStream_t s);
 // projected walk: the sums over l of np pairs into accA (walk_acc_doubles per
 // pair and fragment orbital), their energies into part_t; then the seeds of all

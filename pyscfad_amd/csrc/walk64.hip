@@ -137,6 +137,13 @@ hipError_t launch_walk_inputs(const WalkDims &d, const double *mo, const double 
   const size_t ntb = (size_t)d.o * d.o * d.vp * d.up;
   hipLaunchKernelGGL(k_walk_tb, dim3((unsigned)std::min<size_t>((ntb + 255) / 256, 262144), TB ? 2 : 1), dim3(256),
                      0, s, d, t2, ovoo, TB, TBt);
+  return launch_walk_small_inputs(d, mo, t1, t2, ovov, fvo, OVS, T2S, t1p, fvop, mop, s);
+}
+
+hipError_t launch_walk_small_inputs(const WalkDims &d, const double *mo, const double *t1, const double *t2,
+                                    const double *ovov, const double *fvo, double *OVS, double *T2S, double *t1p,
+                                    double *fvop, double *mop, hipStream_t s) {
+  const int nq = (d.vp + 31) / 32;
   hipLaunchKernelGGL(k_walk_sym, dim3((unsigned)(d.o * d.o * nq * nq), 1, 2), dim3(256), 0, s, d, ovov, t2, OVS,
                      T2S, nq);
   hipLaunchKernelGGL(k_walk_small, dim3((d.o * d.vp + d.vp + d.o + 255) / 256), dim3(256), 0, s, d, mo, t1,
@@ -846,7 +853,7 @@ hipError_t launch_walk_finish(const WalkDims &d, const double *VTb, int packed, 
   hipLaunchKernelGGL(k_walk_fold_t2, dim3(nt, (d.o + 31) / 32, nz), dim3(256), 0, s, d, VTb, t2_bar);
   hipLaunchKernelGGL(k_walk_mo, dim3((d.o + d.vp + 63) / 64, kWalkMoParts), dim3(64), 0, s, part_mo, rows,
                      d.o + d.vp, part2);
-  return launch_reduce_rows(part2, kWalkMoParts, d.o + d.vp, mo_bar, 0, s);
+  return launch_reduce_rows(part2, kWalkMoParts, d.o + d.v, d.o + d.vp, mo_bar, 0, s);
 }
 
 }  // namespace pamd

@@ -20,6 +20,7 @@
 // Loads of the next orbit are in flight during the arithmetic of the current
 // one.  Measured, per launch of all triples: see launch_walk_orbit.
 #include <algorithm>
+#include "bf16_split.h"
 #include "engine_staging.h"
 #include "walk64.h"
 
@@ -281,8 +282,9 @@ __device__ __forceinline__ double image_weight(int pat, int al, int be, int ga) 
   return e1 && e2 ? 1.0 / 6.0 : (e1 || e2 ? 0.5 : 1.0);
 }
 
-// Energy (VJP false), or energy and seeds.  Grid (G, triples).
-template <bool VJP, bool FVO>
+// Energy (VJP false), or energy and seeds.  Grid (G, triples).  PL: Wbar leaves as
+// three bf16 planes (split-BF16x3; one triple), W is kept.
+template <bool VJP, bool FVO, bool PL>
 __global__ __launch_bounds__(512, 4) void k_walk_orbit(OrbitArgs A) {
   __shared__ double Ws[6][kT3];
   __shared__ double Vs[VJP ? 6 : 1][VJP ? kT3 : 1];
@@ -364,8 +366,12 @@ __global__ __launch_bounds__(512, 4) void k_walk_orbit(OrbitArgs A) {
 #pragma unroll
         for (int p = 0; p < 6; ++p) {
           if (p >= pt.np()) continue;
-          st64(W + tile_at(oc, pt, p, A.ws, v), off8, Ws[p][own]);
-          st64(Vb + tile_at(oc, pt, p, (long long)v * v, v), off8, Vs[p][own]);
+          const long long at = tile_at(oc, pt, p, (long long)v * v, v);
+          if (PL)
+            put3(A.Wb3, (long long)v * v * v, at + off8 / 8, Ws[p][own]);
+          else
+            st64(W + tile_at(oc, pt, p, A.ws, v), off8, Ws[p][own]);
+          st64(Vb + at, off8, Vs[p][own]);
         }
       }
     };
@@ -611,14 +617,19 @@ __global__ __launch_bounds__(512, 4) void k_walk_proj(OrbitArgs A) {
 hipError_t launch_walk_orbit(const OrbitArgs &a, int G, hipStream_t s) {
   const dim3 grid(G, a.nb), block(512);
   const size_t lds = a.vjp ? sizeof(double) * a.v : 0;
-  if (a.vjp && a.has_fvo)
-    hipLaunchKernelGGL((k_walk_orbit<true, true>), grid, block, lds, s, a);
+  if (a.vjp && a.Wb3 && a.nb != 1) return hipErrorInvalidValue;
+  if (a.vjp && a.Wb3 && a.has_fvo)
+    hipLaunchKernelGGL((k_walk_orbit<true, true, true>), grid, block, lds, s, a);
+  else if (a.vjp && a.Wb3)
+    hipLaunchKernelGGL((k_walk_orbit<true, false, true>), grid, block, lds, s, a);
+  else if (a.vjp && a.has_fvo)
+    hipLaunchKernelGGL((k_walk_orbit<true, true, false>), grid, block, lds, s, a);
   else if (a.vjp)
-    hipLaunchKernelGGL((k_walk_orbit<true, false>), grid, block, lds, s, a);
+    hipLaunchKernelGGL((k_walk_orbit<true, false, false>), grid, block, lds, s, a);
   else if (a.has_fvo)
-    hipLaunchKernelGGL((k_walk_orbit<false, true>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((k_walk_orbit<false, true, false>), grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((k_walk_orbit<false, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((k_walk_orbit<false, false, false>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 

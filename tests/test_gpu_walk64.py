@@ -86,3 +86,30 @@ def test_batched_projected_walk_matches_the_one_triple_walk(o, v, nfrag, fvo, cu
     for k in out:
         assert float((g[k] - out[k]).norm()) <= 1e-12 * float(out[k].norm()) + 1e-18, k
     assert torch.allclose(_ops.projected_energy(inp, u), e1, rtol=1e-12, atol=1e-18)
+
+
+# (v < 24: the 32x32-MFMA tiles, which sum in FP64; o = 6, 12 with v a multiple of
+# 8; one virtual below and above a multiple; nothing but padding changes at (8, 40))
+@pytest.mark.parametrize('o,v,fvo,packed', [(2, 7, 1e-3, True), (3, 17, 0.0, False), (6, 48, 1e-3, True),
+                                            (12, 40, 0.0, False), (8, 40, 1e-3, True), (5, 63, 1e-3, False),
+                                            (9, 81, 0.0, True), (1, 24, 1e-3, True)])
+def test_padded_walk_matches_the_unpadded_one(o, v, fvo, packed, cuda):
+    """The split-BF16x3 walk on operands padded to multiples of 8 against the same walk
+    on unpadded ones, which a call falls back to when its workspace does not hold
+    the padded arrays: the smallest workspace the entry point takes against the one
+    pamd_ccsdt_workspace_size asks for.  Padding keeps every FP32 sum (the same
+    products in the same order), so gradients differ by FP64 roundings (1e-12
+    relative) and by the few elements of Wbar whose last bf16 piece rounds the other
+    way: 2^-24 of one term of a sum each, below 1e-9 of a block's norm.  An energy
+    takes the direct engine at every size, FP32 sums in another order: 1e-8 of E."""
+    p = make_problem(o, v, 3 * v, seed=o * 100 + v, fvo_scale=fvo)
+    inp = _ops.Inputs(p.mo_energy, p.t1, p.t2, p.ovvv_packed() if packed else p.ovvv, p.ovoo, p.ovov,
+                      p.fvo, precision='bf16x3', device=cuda)
+    e, g = _ops.energy_vjp(inp, et_bar=0.7)
+    ws, least = _smallest_workspace(inp)
+    assert least < ws.numel()
+    e1, g1 = _ops.energy_vjp(inp, et_bar=0.7, workspace=(ws, least))
+    assert torch.allclose(e, e1, rtol=1e-12, atol=1e-18)
+    for k in g:
+        assert float((g[k] - g1[k]).norm()) <= 1e-9 * float(g1[k].norm()) + 1e-18, k
+    assert torch.allclose(_ops.energy(inp), e1, rtol=1e-8, atol=1e-18)
