@@ -1395,7 +1395,8 @@ static WalkLayout walk_layout(int o, int v, int vjp, int nb) {
 // The batch of a call: as many triples as fit the library's own scratch
 // together with the rest when these are all, or 32 (so that the calls with and
 // without a workspace of their own split the walk alike and agree bit for bit),
-// else as many as 8 GB of blocks hold; fewer when `limit` bytes are there.
+// else as many as 8 GB of blocks hold; fewer when `limit` bytes are there, or
+// when an adjoint would hold nearly every triple.
 // False when the walk does not apply: slabs beyond 32-bit offsets, not even one
 // run in `limit`, or a workspace noticeably larger than the one-triple walk's
 // where that is large itself.
@@ -1411,6 +1412,13 @@ static bool walk_pick(int o, int v, int vjp, size_t limit, size_t one_triple_tot
   int b = largest(kNoAllocScratchBytes);
   if (b < std::min(n, 32))
     b = std::max(kWalkRun, largest(walk_layout(o, v, vjp, kWalkRun).total + ((size_t)8 << 30)));
+  if (vjp) {
+    // an adjoint keeps no more than three quarters of what W and Wbar of all
+    // triples would take (where that is more than 8 MB)
+    const size_t all = (size_t)num_triples(o) * 2 * sizeof(double) * v * v * v;
+    const size_t most = std::max<size_t>(all / 4 * 3, (size_t)8 << 20);
+    if (walk_layout(o, v, vjp, b).total > most) b = std::max(kWalkRun, largest(most));
+  }
   if (walk_layout(o, v, vjp, b).total > limit) b = largest(limit);
   if (b < kWalkRun) return false;
   L = walk_layout(o, v, vjp, walk_batches(num_triples(o), b).cap);
