@@ -611,7 +611,7 @@ __global__ __launch_bounds__(512, MINW) void k_gemm_b3n(GemmDesc d, GemmBatch bt
       for (int r = 0; r < 4; ++r) {
         const int ml = wm * WTM + 16 * a + 4 * (lane >> 4) + r;
         const int nl = wn * WTN + 16 * b + (lane & 15);
-        const bool part = d.mode == kPartial;
+        const bool part = d.mode >= kPartial;
         const OutPos pm = out_pos<MT>(tm, ml, part ? (1 << 30) : d.C.mdiv);
         const OutPos pn = out_pos<NT>(tn, nl, part ? (1 << 30) : d.C.ndiv);
         const int m = pm.idx, n = pn.idx;
@@ -621,7 +621,9 @@ __global__ __launch_bounds__(512, MINW) void k_gemm_b3n(GemmDesc d, GemmBatch bt
           val = (double)fa[a][b][r];
         else
           val = acc[a][b][r];
-        if (part) {
+        if (d.mode == kPartialF32) {
+          ((float *)d.partial)[((size_t)split * d.M + m) * d.N + n] = (float)val;
+        } else if (part) {
           d.partial[((size_t)split * d.M + m) * d.N + n] = val;
         } else {
           double *c = d.C.p + batch * bt.c + (long long)pm.q * d.C.mx + (long long)pm.r * d.C.my +
@@ -687,13 +689,14 @@ int gemm_wgs_per_cu_b3(int M, int N) {
 
 hipError_t launch_gemm_b3(const GemmDesc &d0, hipStream_t s, const GemmBatch &bt) {
   if (d0.M <= 0 || d0.N <= 0) return hipSuccess;
-  if (bt.nb < 1 || (bt.nb > 1 && d0.mode == kPartial)) return hipErrorInvalidValue;
+  if (bt.nb < 1 || (bt.nb > 1 && d0.mode >= kPartial)) return hipErrorInvalidValue;
   GemmDesc d = d0;  // chunks of BKC
   d.chunk_start[0] = 0;
   for (int q = 0; q < d.nseg; ++q) d.chunk_start[q + 1] = d.chunk_start[q] + (d.seg[q].L + BKC - 1) / BKC;
   for (int q = d.nseg + 1; q <= kMaxSeg; ++q) d.chunk_start[q] = d.chunk_start[d.nseg];
   if (gemm_b3p_enabled() && d.sums != kSumsFlushed && gemm_b3p_ok(d, bt)) return launch_gemm_b3p(d, s, bt);
   const int c = b3_pick(d.M, d.N, d.sums);
+  if (c >= kB3Wide && d.mode == kPartialF32) return hipErrorInvalidValue;
   const int MT = kB3Shape[c][0], NT = kB3Shape[c][1];
   const unsigned grid =
       (unsigned)((long long)((d.M + MT - 1) / MT) * ((d.N + NT - 1) / NT) * d.splits * bt.nb);

@@ -48,7 +48,8 @@ struct OutDesc {
   int mdiv, ndiv;
 };
 
-enum GemmMode { kStore = 0, kAccumulate = 1, kPartial = 2 };
+// kPartialF32: FP32 parts (split-BF16x3 products of one FP32 sum per part: exact)
+enum GemmMode { kStore = 0, kAccumulate = 1, kPartial = 2, kPartialF32 = 3 };
 
 struct GemmDesc {
   int M, N, nseg, mode;
@@ -57,7 +58,7 @@ struct GemmDesc {
   int sums;                      // B3Sums
   SegDesc seg[kMaxSeg];
   OutDesc C;
-  double *partial;               // kPartial: partial[(split * M + m) * N + n]
+  double *partial;               // kPartial, kPartialF32: partial[(split * M + m) * N + n]
 };
 
 // A descriptor of at most two segments (same fields as GemmDesc), for group
@@ -166,6 +167,7 @@ struct CombineArgs {
   double *part_p;                 // [6][S][v][v] particle t2_bar partials (reduced in place)
   double *part_h;                 // [6][S][v][o] hole ovoo_bar partials (reduced in place)
   int S_p, S_h;
+  int f32_p, f32_h;               // parts are FP32 (kPartialF32)
   int o, v, i, j, k, has_fvo;     // v: extent of the outputs and partials
   int vp;                         // extent that R is laid out with
   double *t2_bar, *ovov_bar, *ovoo_bar, *t1_bar, *fvo_bar;
@@ -226,6 +228,9 @@ int gemm_tiles_b3(int M, int N);  // split-BF16x3 engine: workgroup tiles of one
 int gemm_wgs_per_cu_b3(int M, int N);  // split-BF16x3 engine: resident workgroups per CU
 hipError_t launch_orbit(const OrbitArgs &a, int grid, hipStream_t s, int mode = kOrbitPlain);
 hipError_t launch_vr(const VRArgs &a, hipStream_t s);
+// where the sum over S parts of T elements each goes: over part 0, or, of FP32
+// parts (S >= 2), behind them
+__host__ __device__ inline size_t part_sum_at(int S, size_t T, int f32) { return f32 ? (S * T + 1) / 2 : 0; }
 hipError_t launch_combine(const CombineArgs &a, hipStream_t s);
 hipError_t launch_fold_ovvv(const double *Vpb, int o, int v, int vp, int packed, double *out, hipStream_t s);
 // op, vp: extents the accumulators are laid out with

@@ -339,6 +339,7 @@ struct Ctx {
   double *Vp, *T2m, *OOt, *OVS, *T2S, *W, *tri, *part_t;
   double *Vb, *Vpb, *T2mb, *part_mo, *R, *part_p, *part_h;
   int S_p, S_h, G;
+  int f32_p, f32_h;   // the split-K parts are FP32 (kPartialF32)
   int wbatch;  // W blocks available to the energy walk's batched W build
   double ebar;
   int shard, nshards;     // this call covers walk triples with index % nshards == shard
@@ -631,51 +632,57 @@ static int adjoint_gemms(const Ctx &c, int i, int j, int k, int pair = 0, const 
   // particle t2_bar pieces: split-K over the virtual pair, partials per problem
   const size_t pp = (size_t)c.S_p * V0 * V0;
   {
-    const GemmDesc ds[6] = {
+    const int mode_p = c.f32_p ? kPartialF32 : kPartial;
+    GemmDesc ds[6] = {
         // P1: t2_bar[k,j][c][f] = sum_(a,b) Wb[a,b,c] Vp(i)[a][b][f]
-        gemm(V0, V0, kPartial, {seg(opK(Wb, 1, v2, v, V0, 1), opK(Vp(i), 1, v2, v, V0, 1), V0 * V0, 1.0)},
+        gemm(V0, V0, mode_p, {seg(opK(Wb, 1, v2, v, V0, 1), opK(Vp(i), 1, v2, v, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 0 * pp),
         // P2: t2_bar[j,k][b][f] = sum_(a,c) Wb[a,b,c] Vp(i)[a][c][f]
-        gemm(V0, V0, kPartial, {seg(opK(Wb, v, v2, 1, V0, 0), opK(Vp(i), 1, v2, v, V0, 1), V0 * V0, 1.0)},
+        gemm(V0, V0, mode_p, {seg(opK(Wb, v, v2, 1, V0, 0), opK(Vp(i), 1, v2, v, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 1 * pp),
         // P3: t2_bar[k,i][c][f] = sum_(a,b) Wb[a,b,c] Vp(j)[b][a][f]
-        gemm(V0, V0, kPartial, {seg(opK(Wb, 1, v2, v, V0, 1), opK(Vp(j), 1, v, v2, V0, 1), V0 * V0, 1.0)},
+        gemm(V0, V0, mode_p, {seg(opK(Wb, 1, v2, v, V0, 1), opK(Vp(j), 1, v, v2, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 2 * pp),
         // P4: t2_bar[i,k][a][f] = sum_(b,c) Wb[a,b,c] Vp(j)[b][c][f]
-        gemm(V0, V0, kPartial, {seg(opK(Wb, v2, v, 1, V0, 0), opK(Vp(j), 1, v2, v, V0, 1), V0 * V0, 1.0)},
+        gemm(V0, V0, mode_p, {seg(opK(Wb, v2, v, 1, V0, 0), opK(Vp(j), 1, v2, v, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 3 * pp),
         // P5: t2_bar[j,i][b][f] = sum_(a,c) Wb[a,b,c] Vp(k)[c][a][f]
-        gemm(V0, V0, kPartial, {seg(opK(Wb, v, v2, 1, V0, 0), opK(Vp(k), 1, v, v2, V0, 1), V0 * V0, 1.0)},
+        gemm(V0, V0, mode_p, {seg(opK(Wb, v, v2, 1, V0, 0), opK(Vp(k), 1, v, v2, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 4 * pp),
         // P6: t2_bar[i,j][a][f] = sum_(b,c) Wb[a,b,c] Vp(k)[c][b][f]
-        gemm(V0, V0, kPartial, {seg(opK(Wb, v2, v, 1, V0, 0), opK(Vp(k), 1, v, v2, V0, 1), V0 * V0, 1.0)},
+        gemm(V0, V0, mode_p, {seg(opK(Wb, v2, v, 1, V0, 0), opK(Vp(k), 1, v, v2, V0, 1), V0 * V0, 1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_p, c.part_p + 5 * pp),
     };
+    if (c.f32_p)
+      for (GemmDesc &d : ds) d.sums = kSumsWhole;
     PAMD_CHECK(run_gemm_group(c, ds, 6, kProfAdjT2P, true));
   }
   // hole ovoo_bar pieces: split-K over the virtual pair
   const size_t ph = (size_t)c.S_h * V0 * O0;
   {
-    const GemmDesc ds[6] = {
+    const int mode_h = c.f32_h ? kPartialF32 : kPartial;
+    GemmDesc ds[6] = {
         // H1: ovoo_bar[i,a,m,j] = -sum_(b,c) Wb[a,b,c] T2m(k)[c][b][m]
-        gemm(V0, O0, kPartial, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, O0, mode_h, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 0 * ph),
         // H2: ovoo_bar[i,a,m,k] = -sum_(b,c) Wb[a,b,c] T2m(j)[b][c][m]
-        gemm(V0, O0, kPartial, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(j), 1, vo, os, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, O0, mode_h, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(j), 1, vo, os, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 1 * ph),
         // H3: ovoo_bar[j,b,m,i] = -sum_(a,c) Wb[a,b,c] T2m(k)[c][a][m]
-        gemm(V0, O0, kPartial, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, O0, mode_h, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 2 * ph),
         // H4: ovoo_bar[j,b,m,k] = -sum_(a,c) Wb[a,b,c] T2m(i)[a][c][m]
-        gemm(V0, O0, kPartial, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, O0, mode_h, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 3 * ph),
         // H5: ovoo_bar[k,c,m,i] = -sum_(a,b) Wb[a,b,c] T2m(j)[b][a][m]
-        gemm(V0, O0, kPartial, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(j), 1, os, vo, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, O0, mode_h, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(j), 1, os, vo, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 4 * ph),
         // H6: ovoo_bar[k,c,m,j] = -sum_(a,b) Wb[a,b,c] T2m(i)[a][b][m]
-        gemm(V0, O0, kPartial, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, O0, mode_h, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 5 * ph),
     };
+    if (c.f32_h)
+      for (GemmDesc &d : ds) d.sums = kSumsWhole;
     PAMD_CHECK(run_gemm_group(c, ds, 6, kProfAdjOvoo, true));
   }
   // hole-term t2 reads: T2mb[x][p][q][m] (= dE/d t2[x,m,p,q])
@@ -740,6 +747,8 @@ static int adjoint_combine(const Ctx &c, int i, int j, int k, hipStream_t st,
   ca.part_h = c.part_h;
   ca.S_p = c.S_p;
   ca.S_h = c.S_h;
+  ca.f32_p = c.f32_p;
+  ca.f32_h = c.f32_h;
   ca.o = c.o;
   ca.v = c.v;
   ca.vp = c.vp;
@@ -1329,6 +1338,14 @@ static void bind_workspace(Ctx &c, const Layout &L, void *ws) {
   }
   c.S_p = L.S_p;
   c.S_h = L.S_h;
+  // FP32 parts (half the traffic of the reduction) wherever a part is one FP32
+  // sum, and two of them leave room for the FP64 result (part_sum_at)
+  auto whole = [&](int M, int N) {
+    return c.prec == PAMD_PREC_BF16X3 &&
+           ((gemm_b3p_enabled() && M % 8 == 0 && N % 8 == 0) || gemm_b3_sums(M, N) == kSumsWhole);
+  };
+  c.f32_p = L.S_p >= 2 && whole(c.v, c.v);
+  c.f32_h = L.S_h >= 2 && whole(c.v, c.o);
 }
 
 // ---------------------------------------------------------------------------

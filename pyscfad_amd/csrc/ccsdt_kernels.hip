@@ -1143,29 +1143,57 @@ hipError_t launch_vr(const VRArgs &a, hipStream_t s) {
 // of every slab it touches, so coinciding occupied indices (i == j etc.) are
 // summed sequentially in the same thread: no atomics, deterministic.
 // ---------------------------------------------------------------------------
-// Split-K partial sums of the six particle and six hole problems of a triple,
-// in place: part[pr][0][t] = sum_s part[pr][s][t], s = 0..S-1, in a fixed
-// order (four interleaved partial sums); blockIdx.y < 6 picks a particle
-// problem, the rest a hole problem.
-__global__ void k_splitk_reduce(double *part_p, int S_p, size_t T_p, double *part_h, int S_h,
-                                size_t T_h) {
-  const int y = blockIdx.y;
+// Split-K partial sums of the six particle and six hole problems of a triple:
+// part[pr][.][t] summed over the parts s = 0 .. S - 1 in a fixed order, to
+// part_sum_at; blockIdx.y < 6 picks a particle problem, the rest a hole
+// problem.  The kernel only streams the parts, so what counts is bytes in
+// flight: a workgroup takes 64 positions and splits the parts over its four
+// waves, eight loads at a time each (o16/v160, S = 128: 81 us with one thread
+// per position and FP64 parts).
+template <class T>
+__device__ __forceinline__ double part_sum(const T *p, size_t ld, int S, int wave) {
+  double a[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) a[u] = 0.0;
+  int s = wave;
+  for (; s + 28 < S; s += 32)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] += (double)p[(size_t)(s + 4 * u) * ld];
+  for (; s < S; s += 4) a[0] += (double)p[(size_t)s * ld];
+  return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+}
+
+__global__ __launch_bounds__(256) void k_splitk_reduce(double *part_p, int S_p, size_t T_p, int f32_p,
+                                                       double *part_h, int S_h, size_t T_h, int f32_h) {
+  __shared__ double red[4][64];
+  const int y = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const bool hole = y >= 6;
   const size_t T = hole ? T_h : T_p;
-  const int S = hole ? S_h : S_p;
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= T) return;
-  double *p = (hole ? part_h + (size_t)(y - 6) * S * T : part_p + (size_t)y * S * T) + t;
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-  int s = 0;
-  for (; s + 4 <= S; s += 4) {
-    a0 += p[(size_t)s * T];
-    a1 += p[(size_t)(s + 1) * T];
-    a2 += p[(size_t)(s + 2) * T];
-    a3 += p[(size_t)(s + 3) * T];
+  const int S = hole ? S_h : S_p, f32 = hole ? f32_h : f32_p;
+  const size_t t = (size_t)blockIdx.x * 64 + lane;
+  if ((size_t)blockIdx.x * 64 >= T) return;
+  double *p = hole ? part_h + (size_t)(y - 6) * S * T : part_p + (size_t)y * S * T;
+  double s = 0.0;
+  if (t < T) s = f32 ? part_sum((const float *)p + t, T, S, wave) : part_sum(p + t, T, S, wave);
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && t < T)
+    p[part_sum_at(S, T, f32) + t] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+}
+
+// slabs at coinciding occupied pairs (i == j, j == k) are one: the sum of a
+// later one moves to the first of them, which alone is read and written
+__device__ __forceinline__ void merge_slabs(const int (&x)[6], const int (&y)[6], double (&s)[6], bool (&own)[6]) {
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    own[q] = true;
+#pragma unroll
+    for (int r = 0; r < q; ++r)
+      if (own[q] && own[r] && x[r] == x[q] && y[r] == y[q]) {
+        s[r] += s[q];
+        own[q] = false;
+      }
   }
-  for (; s < S; ++s) a0 += p[(size_t)s * T];
-  p[0] = (a0 + a1) + (a2 + a3);
 }
 
 __device__ __forceinline__ void combine_block(const CombineArgs &A, size_t t) {
@@ -1175,60 +1203,75 @@ __device__ __forceinline__ void combine_block(const CombineArgs &A, size_t t) {
   if (t < vv) {
     const int p = (int)(t / v), q = (int)(t % v);
     const size_t pq = (size_t)p * vr + q, qp = (size_t)q * vr + p;
-    // ovov_bar[x,p,y,q]
-    auto ob = [&](int x, int y) -> double & {
-      return A.ovov_bar[(((size_t)x * v + p) * o + y) * v + q];
-    };
-    ob(i, j) += 0.5 * vr_csum(R, vr, 0, pq);
-    ob(j, i) += 0.5 * vr_csum(R, vr, 0, qp);
-    ob(i, k) += 0.5 * vr_sum(R, vr, 2, pq);
-    ob(k, i) += 0.5 * vr_sum(R, vr, 2, qp);
-    ob(j, k) += 0.5 * vr_sum(R, vr, 4, pq);
-    ob(k, j) += 0.5 * vr_sum(R, vr, 4, qp);
-    // t2_bar[x,y,p,q]: particle split-K partials (problem order P1..P6) + V terms
-    auto tb = [&](int x, int y) -> double & {
-      return A.t2_bar[(((size_t)x * o + y) * v + p) * v + q];
-    };
-    const int xs[6] = {k, j, k, i, j, i};
-    const int ys[6] = {j, k, i, k, i, j};
-    for (int pr = 0; pr < 6; ++pr) {
-      double s = A.part_p[(size_t)pr * A.S_p * vv + t];  // split-K sum (k_splitk_reduce)
-      if (A.has_fvo) {
-        switch (pr) {
-          case 0: s += 0.5 * vr_sum(R, vr, 5, qp); break;  // t2_bar[k,j,c,b] += R6[b,c]/2
-          case 1: s += 0.5 * vr_sum(R, vr, 5, pq); break;  // t2_bar[j,k,b,c] += R6[b,c]/2
-          case 2: s += 0.5 * vr_sum(R, vr, 3, qp); break;  // t2_bar[k,i,c,a] += R4[a,c]/2
-          case 3: s += 0.5 * vr_sum(R, vr, 3, pq); break;  // t2_bar[i,k,a,c] += R4[a,c]/2
-          case 4: s += 0.5 * vr_csum(R, vr, 1, qp); break;  // t2_bar[j,i,b,a] += R2[a,b]/2
-          case 5: s += 0.5 * vr_csum(R, vr, 1, pq); break;  // t2_bar[i,j,a,b] += R2[a,b]/2
-        }
-      }
-      tb(xs[pr], ys[pr]) += s;
+    // ovov_bar[x,p,y,q] (all old values are read at once: six dependent updates
+    // one after the other took 10 us)
+    const int xv[6] = {i, j, i, k, j, k}, yv[6] = {j, i, k, i, k, j};
+    double sv[6] = {0.5 * vr_csum(R, vr, 0, pq), 0.5 * vr_csum(R, vr, 0, qp), 0.5 * vr_sum(R, vr, 2, pq),
+                    0.5 * vr_sum(R, vr, 2, qp),  0.5 * vr_sum(R, vr, 4, pq),  0.5 * vr_sum(R, vr, 4, qp)};
+    bool own[6];
+    merge_slabs(xv, yv, sv, own);
+    auto ob = [&](int u) { return A.ovov_bar + (((size_t)xv[u] * v + p) * o + yv[u]) * v + q; };
+    double old[6];
+#pragma unroll
+    for (int u = 0; u < 6; ++u) old[u] = own[u] ? *ob(u) : 0.0;
+#pragma unroll
+    for (int u = 0; u < 6; ++u)
+      if (own[u]) *ob(u) = old[u] + sv[u];
+    // t2_bar[x,y,p,q]: particle split-K sums (problem order P1..P6) + V terms
+    const int xs[6] = {k, j, k, i, j, i}, ys[6] = {j, k, i, k, i, j};
+    double s[6];
+#pragma unroll
+    for (int pr = 0; pr < 6; ++pr)
+      s[pr] = A.part_p[(size_t)pr * A.S_p * vv + part_sum_at(A.S_p, vv, A.f32_p) + t];
+    if (A.has_fvo) {
+      s[0] += 0.5 * vr_sum(R, vr, 5, qp);   // t2_bar[k,j,c,b] += R6[b,c]/2
+      s[1] += 0.5 * vr_sum(R, vr, 5, pq);   // t2_bar[j,k,b,c] += R6[b,c]/2
+      s[2] += 0.5 * vr_sum(R, vr, 3, qp);   // t2_bar[k,i,c,a] += R4[a,c]/2
+      s[3] += 0.5 * vr_sum(R, vr, 3, pq);   // t2_bar[i,k,a,c] += R4[a,c]/2
+      s[4] += 0.5 * vr_csum(R, vr, 1, qp);  // t2_bar[j,i,b,a] += R2[a,b]/2
+      s[5] += 0.5 * vr_csum(R, vr, 1, pq);  // t2_bar[i,j,a,b] += R2[a,b]/2
     }
+    merge_slabs(xs, ys, s, own);
+    auto tb = [&](int u) { return A.t2_bar + (((size_t)xs[u] * o + ys[u]) * v + p) * v + q; };
+#pragma unroll
+    for (int u = 0; u < 6; ++u) old[u] = own[u] ? *tb(u) : 0.0;
+#pragma unroll
+    for (int u = 0; u < 6; ++u)
+      if (own[u]) *tb(u) = old[u] + s[u];
   }
   if (t < (size_t)v * o) {
-    // ovoo_bar[x,p,m,y] from the hole split-K partials H1..H6
+    // ovoo_bar[x,p,m,y] from the hole split-K sums H1..H6
     const int p = (int)(t / o), m = (int)(t % o);
     const int xs[6] = {i, i, j, j, k, k};
     const int ys[6] = {j, k, i, k, i, j};
     const size_t vo = (size_t)v * o;
-    for (int pr = 0; pr < 6; ++pr) {
-      const double s = A.part_h[(size_t)pr * A.S_h * vo + t];  // split-K sum (k_splitk_reduce)
-      A.ovoo_bar[(((size_t)xs[pr] * v + p) * o + m) * o + ys[pr]] += s;
-    }
+    double s[6], old[6];
+    bool own[6];
+#pragma unroll
+    for (int pr = 0; pr < 6; ++pr)
+      s[pr] = A.part_h[(size_t)pr * A.S_h * vo + part_sum_at(A.S_h, vo, A.f32_h) + t];
+    merge_slabs(xs, ys, s, own);
+    auto hb = [&](int u) { return A.ovoo_bar + (((size_t)xs[u] * v + p) * o + m) * o + ys[u]; };
+#pragma unroll
+    for (int u = 0; u < 6; ++u) old[u] = own[u] ? *hb(u) : 0.0;
+#pragma unroll
+    for (int u = 0; u < 6; ++u)
+      if (own[u]) *hb(u) = old[u] + s[u];
   }
 }
 
 // t1_bar / fvo_bar pieces of one triple: column sums over a of four v x v
-// slices of R, one block per 64 columns (the 4 waves split the rows).
-__device__ __forceinline__ void colsums_block(const CombineArgs &A, int blk, double (*red)[4][64]) {
+// slices of R, one block per 16 columns, its threads in 16 rows (64 columns and
+// four waves: a chain of v / 4 rows of dependent loads, 60 us at v = 160).
+__device__ __forceinline__ void colsums_block(const CombineArgs &A, int blk, double (*red)[16][17]) {
   const int o = A.o, v = A.v, vr = A.vp, i = A.i, j = A.j, k = A.k;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = blk * 64 + lane;
+  const int col = threadIdx.x & 15, row = threadIdx.x >> 4;
+  const int c = blk * 16 + col;
   const double *R = A.R;
   double sk = 0.0, sj = 0.0, fk = 0.0, fj = 0.0;
   if (c < v) {
-    for (int a = wave; a < v; a += 4) {
+#pragma unroll 2
+    for (int a = row; a < v; a += 16) {
       const size_t ac = (size_t)a * vr + c;
       sk += vr_sum(R, vr, 6, ac);
       sj += vr_csum(R, vr, 8, ac);
@@ -1236,15 +1279,19 @@ __device__ __forceinline__ void colsums_block(const CombineArgs &A, int blk, dou
       fj += vr_csum(R, vr, 9, ac);
     }
   }
-  red[0][wave][lane] = sk;
-  red[1][wave][lane] = sj;
-  red[2][wave][lane] = fk;
-  red[3][wave][lane] = fj;
+  red[0][row][col] = sk;
+  red[1][row][col] = sj;
+  red[2][row][col] = fk;
+  red[3][row][col] = fj;
   __syncthreads();
-  if (wave == 0 && c < v) {
+  if (row == 0 && c < v) {
     double s[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) s[q] = red[q][0][lane] + red[q][1][lane] + red[q][2][lane] + red[q][3][lane];
+    for (int q = 0; q < 4; ++q) {
+      s[q] = 0.0;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[q] += red[q][r][col];
+    }
     A.t1_bar[k * v + c] += 0.5 * s[0];
     A.t1_bar[j * v + c] += 0.5 * s[1];
     A.t1_bar[i * v + c] += 0.5 * vr_sum_vec(R, vr, 0, c);
@@ -1257,17 +1304,17 @@ __device__ __forceinline__ void colsums_block(const CombineArgs &A, int blk, dou
 // The gather of one triple in one launch (after k_splitk_reduce): blocks
 // [0, nc) gather the split-K sums and the V terms into t2_bar / ovov_bar /
 // ovoo_bar (one thread per
-// position), the next ceil(v / 64) the t1_bar / fvo_bar column sums, and,
+// position), the next ceil(v / 16) the t1_bar / fvo_bar column sums, and,
 // when A.part_t is set, one more the triple's energy from the orbit
 // epilogue's per-workgroup sums.
 __global__ __launch_bounds__(256) void k_gather(CombineArgs A, int nc) {
-  __shared__ double red[4][4][64];
+  __shared__ double red[4][16][17];
   const int blk = blockIdx.x;
   if (blk < nc) {
     combine_block(A, (size_t)blk * 256 + threadIdx.x);
     return;
   }
-  const int ncs = (A.v + 63) / 64;
+  const int ncs = (A.v + 15) / 16;
   if (blk < nc + ncs) {
     colsums_block(A, blk - nc, red);
     return;
@@ -1281,13 +1328,12 @@ __global__ __launch_bounds__(256) void k_gather(CombineArgs A, int nc) {
 hipError_t launch_combine(const CombineArgs &a, hipStream_t s) {
   {
     const size_t Tp = (size_t)a.v * a.v, Th = (size_t)a.v * a.o;
-    hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)((std::max(Tp, Th) + 255) / 256), 12),
-                       dim3(256), 0, s, const_cast<double *>(a.part_p), a.S_p, Tp,
-                       const_cast<double *>(a.part_h), a.S_h, Th);
+    hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)((std::max(Tp, Th) + 63) / 64), 12), dim3(256), 0, s,
+                       a.part_p, a.S_p, Tp, a.f32_p, a.part_h, a.S_h, Th, a.f32_h);
   }
   size_t n = (size_t)a.v * a.v;
   if ((size_t)a.v * a.o > n) n = (size_t)a.v * a.o;
-  const int nc = (int)((n + 255) / 256), ncs = (a.v + 63) / 64;
+  const int nc = (int)((n + 255) / 256), ncs = (a.v + 15) / 16;
   const int blocks = nc + ncs + (a.part_t ? 1 : 0);
   hipLaunchKernelGGL(k_gather, dim3((unsigned)blocks), dim3(256), 0, s, a, nc);
   return hipGetLastError();

@@ -27,6 +27,15 @@
 // in flight.  Each iteration waits for its own loads (s_waitcnt vmcnt(0)),
 // then one s_barrier (no memory fence) makes every wave's loads visible and
 // retires the stage read one iteration earlier, which the new loads overwrite.
+// The loads are issued from inline asm (lds_dma16): behind the builtin the
+// compiler takes every later ds_read_tr for a reader of the load in flight and
+// waits for it (vmcnt(0) in front of the fragments), which left no overlap.
+//
+// What bounds it (W build, M = 240^2, N = 240, K = 528): loads alone 97 us (about
+// 10 TB/s through L2), MFMA and LDS reads alone 90, the FP64 output 25 (50 when
+// it accumulates); 187 us (215) as first built, 171 (193) with these loads and
+// all old values of a tile row read at once in the epilogue, 150 (173) with the
+// 240-wide tile.
 //
 // Eligibility (gemm_b3p_ok): 8 consecutive elements along the fast index are
 // adjacent and 16-byte aligned for every row and k the kernel addresses: fast
@@ -36,6 +45,7 @@
 // that is.  Rows past M or N and k past L are clamped to valid elements
 // (finite inputs); k past L is zeroed in the fragments of one side, rows past
 // M or N are never stored.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include "ccsdt_common.h"
@@ -174,13 +184,20 @@ __device__ __forceinline__ bool pop_full(const POp &f, int kappa, int L) {
   return kappa + kPK <= L && (f.kdiv >= (1 << 30) || f.r + kPK <= f.kdiv);
 }
 
+// 16 bytes per lane from src to dst + 16 lane (dst: the wave's).  No register is
+// written; the waits are wait_vmcnt's.  M0 needs one wait state before its use.
+__device__ __forceinline__ void lds_dma16(const void *src, bf16_t *dst) {
+  const unsigned at = __builtin_amdgcn_readfirstlane((unsigned)(unsigned long long)(lds_ptr_t)dst);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(src)
+               : "memory", "m0");
+}
+
 template <int R, int T>
 __device__ __forceinline__ void pissue_full(const PPlan<R, T> &pl, long long kb, bf16_t *lds,
                                             int wave) {
 #pragma unroll
   for (int q = 0; q < PPlan<R, T>::NI; ++q)
-    __builtin_amdgcn_global_load_lds((const void *)(pl.ptr[q] + kb),
-                                     (lds_ptr_t)(lds + (q * T + wave * 64) * 8), 16, 0, 0);
+    lds_dma16(pl.ptr[q] + kb, lds + (q * T + wave * 64) * 8);
 }
 
 // the loads of a partial stage: each load's row and k recomputed, k clamped
@@ -194,8 +211,7 @@ __device__ __forceinline__ void pissue_part(const OpDesc &d, int Rtot, int r0, i
     int plane, rl, kl;
     pslot<R, T>(q, tid, rc, plane, rl, kl);
     const bf16_t *src = p + plane * d.ps + prow(d, rc, Rtot, r0 + rl) + pkoff(d, rc, L, kappa + kl);
-    __builtin_amdgcn_global_load_lds((const void *)src,
-                                     (lds_ptr_t)(lds + (q * T + wave * 64) * 8), 16, 0, 0);
+    lds_dma16(src, lds + (q * T + wave * 64) * 8);
   }
 }
 
@@ -235,14 +251,15 @@ __device__ __forceinline__ void frags(const bf16_t *T, int rc, int r16, int lane
   }
 }
 
-// WM x WN waves; two workgroups per CU (80 KB of LDS each at most)
+// WM x WN waves; two workgroups per CU (80 KB of LDS each at most), one of twelve
+// waves
 // LDS of one workgroup (bf16 elements): two stages of the A and B tiles
 template <int MT, int NT, int WM, int WN>
 struct B3pLds {
   static constexpr int T = 64 * WM * WN;
   static constexpr int SA = PPlan<MT, T>::SLOTS * 8, SB = PPlan<NT, T>::SLOTS * 8, SS = SA + SB;
   static constexpr int N = kPStages * SS;
-  static_assert(2 * N * 2 <= 160 * 1024, "LDS of two workgroups per CU");
+  static_assert((WM * WN > 8 ? 1 : 2) * N * 2 <= 160 * 1024, "LDS of a CU's workgroups");
 };
 
 // One workgroup's tile of one product: workgroup number `logical` of the
@@ -256,7 +273,7 @@ __device__ __forceinline__ void b3p_tile(const D &d, const GemmBatch &bt, int n_
   static_assert(TM * 16 == WTM && TN * 16 == WTN, "16x16 MFMA tiles");
   constexpr int SA = B3pLds<MT, NT, WM, WN>::SA, SS = B3pLds<MT, NT, WM, WN>::SS;
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
   const int mt = (d.M + MT - 1) / MT, nt = (d.N + NT - 1) / NT;
   const int per = mt * nt * d.splits;  // workgroups of one product of the batch
@@ -449,31 +466,61 @@ __device__ __forceinline__ void b3p_tile(const D &d, const GemmBatch &bt, int n_
   }
 
   // D layout of v_mfma_f32_16x16x32_bf16: lane l, element r -> row 4 (l / 16) + r, column l % 16
+  if (d.mode >= kPartial) {
+    const size_t part = (size_t)split * d.M * d.N;
 #pragma unroll
-  for (int a = 0; a < TM; ++a)
+    for (int a = 0; a < TM; ++a)
 #pragma unroll
-    for (int b = 0; b < TN; ++b)
+      for (int b = 0; b < TN; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int ml = wm * WTM + 16 * a + 4 * (lane >> 4) + r;
-        const int nl = wn * WTN + 16 * b + (lane & 15);
-        const bool part = d.mode == kPartial;
-        const OutPos pm = out_pos<MT>(tm, ml, part ? (1 << 30) : d.C.mdiv);
-        const OutPos pn = out_pos<NT>(tn, nl, part ? (1 << 30) : d.C.ndiv);
-        const int m = pm.idx, n = pn.idx;
-        if (m >= d.M || n >= d.N) continue;
-        const double val = (double)acc[a][b][r];
-        if (part) {
-          d.partial[((size_t)split * d.M + m) * d.N + n] = val;
-        } else {
-          double *c = d.C.p + batch * bt.c + (long long)pm.q * d.C.mx + (long long)pm.r * d.C.my +
-                      (long long)pn.q * d.C.nx + (long long)pn.r * d.C.ny;
-          if (d.mode == kAccumulate)
-            *c += val;
+        for (int r = 0; r < 4; ++r) {
+          const int m = m0 + wm * WTM + 16 * a + 4 * G + r, n = n0 + wn * WTN + 16 * b + (lane & 15);
+          if (m >= d.M || n >= d.N) continue;
+          const size_t at = part + (size_t)m * d.N + n;
+          if (d.mode == kPartialF32)
+            ((float *)d.partial)[at] = acc[a][b][r];
           else
-            *c = val;
+            d.partial[at] = (double)acc[a][b][r];
         }
-      }
+    return;
+  }
+  long long no[TN];
+  bool nok[TN];
+#pragma unroll
+  for (int b = 0; b < TN; ++b) {
+    const OutPos pn = out_pos<NT>(tn, wn * WTN + 16 * b + (lane & 15), d.C.ndiv);
+    nok[b] = pn.idx < d.N;
+    no[b] = (long long)pn.q * d.C.nx + (long long)pn.r * d.C.ny;
+  }
+#pragma unroll
+  for (int a = 0; a < TM; ++a) {
+    double *cp[4];
+    bool mok[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const OutPos pm = out_pos<MT>(tm, wm * WTM + 16 * a + 4 * G + r, d.C.mdiv);
+      mok[r] = pm.idx < d.M;
+      cp[r] = d.C.p + batch * bt.c + (long long)pm.q * d.C.mx + (long long)pm.r * d.C.my;
+    }
+    double old[TN][4];
+    if (d.mode == kAccumulate) {
+#pragma unroll
+      for (int b = 0; b < TN; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) old[b][r] = mok[r] && nok[b] ? cp[r][no[b]] : 0.0;
+#pragma unroll
+      for (int b = 0; b < TN; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (mok[r] && nok[b]) cp[r][no[b]] = old[b][r] + (double)acc[a][b][r];
+    } else {
+#pragma unroll
+      for (int b = 0; b < TN; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (mok[r] && nok[b]) cp[r][no[b]] = (double)acc[a][b][r];
+    }
+  }
 }
 
 template <int MT, int NT, int WM, int WN, int MINW>
@@ -554,12 +601,14 @@ static double b3p_eff(int M, int N, int MT, int NT) {
 // padded tiling's efficiency times the tile's flops per staged byte,
 // MT NT / (MT + NT).  (A 5-wave 80 x 80 tile for 400 x 400 was measured at
 // half the 128 x 80 rate: ten waves per CU instead of sixteen.)
-static const int kB3pShape[][2] = {{128, 80}, {80, 128}, {128, 48}, {48, 128}, {80, 48}, {48, 80}};
+constexpr int kB3pWide = 6;  // the 240-wide shapes (b3p_launch_shape)
+static const int kB3pShape[][2] = {{128, 80}, {80, 128}, {128, 48}, {48, 128}, {80, 48}, {48, 80},
+                                   {128, 240}, {240, 128}};
 
 int gemm_b3p_pick(int M, int N) {
   int best = 0;
   double bs = -1.0;
-  for (int c = 0; c < (int)(sizeof(kB3pShape) / sizeof(kB3pShape[0])); ++c) {
+  for (int c = 0; c < kB3pWide; ++c) {
     const int MT = kB3pShape[c][0], NT = kB3pShape[c][1];
     const double sc = b3p_eff(M, N, MT, NT) * (double)MT * NT / (MT + NT);
     if (sc > bs + 1e-9) {
@@ -570,9 +619,39 @@ int gemm_b3p_pick(int M, int N) {
   return best;
 }
 
+// (also sets the split-K factors, so it does not know of the 240-wide tiles below:
+// another number of parts would be other FP32 sums)
 int gemm_b3p_tiles(int M, int N) {
   const int c = gemm_b3p_pick(M, N);
   return ((M + kB3pShape[c][0] - 1) / kB3pShape[c][0]) * ((N + kB3pShape[c][1] - 1) / kB3pShape[c][1]);
+}
+
+// Tile shape of a launch of `count` products (or parts, or batch members).  128 x 240
+// (12 waves, one workgroup per CU) stages 29% fewer bytes per flop than 128 x 80
+// and ran 1.2 times as fast where both fill the GPU; a round of it is three
+// times as long, though, so the rounds decide: each shape costs its rounds of
+// workgroups times the time of one, 80 against 240 / (2 x 1.2) columns.
+// Measured, 128 x 80 against 128 x 240: W build v = 240 171 / 150 us, v = 200 104 / 125,
+// v = 320 411 / 517, v = 400 1007 / 990; split-K t2 adjoint v = 400 505 / 460.
+static int b3p_launch_shape(int M, int N, long long count) {
+  const int c = gemm_b3p_pick(M, N);
+  if (c > 1) return c;
+  static const int cus = [] {
+    int dev = 0;
+    hipDeviceProp_t prop;
+    return hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
+                   prop.multiProcessorCount > 0
+               ? prop.multiProcessorCount
+               : 256;
+  }();
+  auto rounds = [&](int mt, int nt, int slots) {
+    const long long t = (long long)((M + mt - 1) / mt) * ((N + nt - 1) / nt) * count;
+    return (double)((t + slots - 1) / slots);
+  };
+  const double narrow = rounds(kB3pShape[c][0], kB3pShape[c][1], 2 * cus) * 80;
+  const double wm = rounds(128, 240, cus) * 100, wn = rounds(240, 128, cus) * 100;
+  if (std::min(wm, wn) >= narrow) return c;
+  return wm < wn || (wm == wn && M >= N) ? kB3pWide : kB3pWide + 1;
 }
 
 // The products form a group: equal sizes, split-K factor and mode, at most two
@@ -586,7 +665,7 @@ bool gemm_b3p_group_ok(const GemmDesc *ds, int n) {
       return false;
   }
   const GemmDesc &d = ds[0];
-  const int c = gemm_b3p_pick(d.M, d.N);
+  const int c = gemm_b3p_pick(d.M, d.N);  // (the wider shapes have fewer workgroups)
   const long long per = (long long)((d.M + kB3pShape[c][0] - 1) / kB3pShape[c][0]) *
                         ((d.N + kB3pShape[c][1] - 1) / kB3pShape[c][1]) * d.splits;
   return per * n < (1LL << 31);
@@ -614,7 +693,7 @@ hipError_t launch_gemm_b3p_group(const GemmDesc *ds, int n, hipStream_t s) {
     e.partial = d.partial;
   }
   const GemmDesc &d = ds[0];
-  const int c = gemm_b3p_pick(d.M, d.N);
+  const int c = b3p_launch_shape(d.M, d.N, (long long)d.splits * n);
   const int MT = kB3pShape[c][0], NT = kB3pShape[c][1];
   const long long per = (long long)((d.M + MT - 1) / MT) * ((d.N + NT - 1) / NT) * d.splits;
   const unsigned grid = (unsigned)(per * n);
@@ -625,14 +704,16 @@ hipError_t launch_gemm_b3p_group(const GemmDesc *ds, int n, hipStream_t s) {
     case 2: hipLaunchKernelGGL((k_gemm_b3p_group<128, 48, 8, 1, 4>), dim3(grid), dim3(512), 0, s, g, n_fast); break;
     case 3: hipLaunchKernelGGL((k_gemm_b3p_group<48, 128, 1, 8, 4>), dim3(grid), dim3(512), 0, s, g, n_fast); break;
     case 4: hipLaunchKernelGGL((k_gemm_b3p_group<80, 48, 5, 1, 3>), dim3(grid), dim3(320), 0, s, g, n_fast); break;
-    default: hipLaunchKernelGGL((k_gemm_b3p_group<48, 80, 3, 1, 2>), dim3(grid), dim3(192), 0, s, g, n_fast); break;
+    case 5: hipLaunchKernelGGL((k_gemm_b3p_group<48, 80, 3, 1, 2>), dim3(grid), dim3(192), 0, s, g, n_fast); break;
+    case 6: hipLaunchKernelGGL((k_gemm_b3p_group<128, 240, 4, 3, 3>), dim3(grid), dim3(768), 0, s, g, n_fast); break;
+    default: hipLaunchKernelGGL((k_gemm_b3p_group<240, 128, 3, 4, 3>), dim3(grid), dim3(768), 0, s, g, n_fast); break;
   }
   return hipGetLastError();
 }
 
 // d: chunk_start in stages of 32
 hipError_t launch_gemm_b3p(const GemmDesc &d, hipStream_t s, const GemmBatch &bt) {
-  const int c = gemm_b3p_pick(d.M, d.N);
+  const int c = b3p_launch_shape(d.M, d.N, (long long)d.splits * bt.nb);
   const int MT = kB3pShape[c][0], NT = kB3pShape[c][1];
   const unsigned grid =
       (unsigned)((long long)((d.M + MT - 1) / MT) * ((d.N + NT - 1) / NT) * d.splits * bt.nb);
@@ -643,7 +724,9 @@ hipError_t launch_gemm_b3p(const GemmDesc &d, hipStream_t s, const GemmBatch &bt
     case 2: hipLaunchKernelGGL((k_gemm_b3p<128, 48, 8, 1, 4>), dim3(grid), dim3(512), 0, s, d, bt, n_fast); break;
     case 3: hipLaunchKernelGGL((k_gemm_b3p<48, 128, 1, 8, 4>), dim3(grid), dim3(512), 0, s, d, bt, n_fast); break;
     case 4: hipLaunchKernelGGL((k_gemm_b3p<80, 48, 5, 1, 3>), dim3(grid), dim3(320), 0, s, d, bt, n_fast); break;
-    default: hipLaunchKernelGGL((k_gemm_b3p<48, 80, 3, 1, 2>), dim3(grid), dim3(192), 0, s, d, bt, n_fast); break;
+    case 5: hipLaunchKernelGGL((k_gemm_b3p<48, 80, 3, 1, 2>), dim3(grid), dim3(192), 0, s, d, bt, n_fast); break;
+    case 6: hipLaunchKernelGGL((k_gemm_b3p<128, 240, 4, 3, 3>), dim3(grid), dim3(768), 0, s, d, bt, n_fast); break;
+    default: hipLaunchKernelGGL((k_gemm_b3p<240, 128, 3, 4, 3>), dim3(grid), dim3(768), 0, s, d, bt, n_fast); break;
   }
   return hipGetLastError();
 }

@@ -89,10 +89,11 @@ def test_batched_projected_walk_matches_the_one_triple_walk(o, v, nfrag, fvo, cu
 
 
 # (v < 24: the 32x32-MFMA tiles, which sum in FP64; o = 6, 12 with v a multiple of
-# 8; one virtual below and above a multiple; nothing but padding changes at (8, 40))
+# 8; one virtual below and above a multiple; nothing but padding changes at (8, 40);
+# v = 239: the direct engine's 240-wide tiles against the register-staged engine)
 @pytest.mark.parametrize('o,v,fvo,packed', [(2, 7, 1e-3, True), (3, 17, 0.0, False), (6, 48, 1e-3, True),
                                             (12, 40, 0.0, False), (8, 40, 1e-3, True), (5, 63, 1e-3, False),
-                                            (9, 81, 0.0, True), (1, 24, 1e-3, True)])
+                                            (9, 81, 0.0, True), (1, 24, 1e-3, True), (3, 239, 0.0, True)])
 def test_padded_walk_matches_the_unpadded_one(o, v, fvo, packed, cuda):
     """The split-BF16x3 walk on operands padded to multiples of 8 against the same walk
     on unpadded ones, which a call falls back to when its workspace does not hold
