@@ -29,7 +29,9 @@ int pamd_mp2_init_amps(int nocc, int nvir, const double *mo_energy, const double
 
 /* Device bytes of the workspace of pamd_df_eris (with_vjp = 0) or of
  * pamd_df_eris_vjp (with_vjp = 1): the packed virtual-virtual factors Lvv, and
- * for the adjoint also their cotangent. */
+ * for the adjoint also their cotangent, the symmetrised ovov cotangent and the
+ * parts of its split products (the adjoint also runs, more slowly, with a
+ * workspace for the first two alone). */
 int pamd_df_eris_workspace_size(int nocc, int nmo, int naux, int with_vjp, size_t *bytes);
 
 /* The (T) blocks of the in-core DF integrals, _make_df_eris_incore

@@ -10,7 +10,8 @@
 //             ovov[ia, jb] = sum_P Lov[P, ia] Lov[P, jb]          (M o v, N o v)
 //   adjoint   Loo_bar[P, jk] += sum_ia Lov[P, ia] ovoo_bar[ia, jk]
 //             Lov_bar[P, ia] += sum_bc Lvv[P, bc] ovvv_bar[ia, bc] + sum_jk Loo[P, jk] ovoo_bar[ia, jk]
-//                             + sum_jb Lov[P, jb] (ovov_bar[ia, jb] + ovov_bar[jb, ia])
+//                             + sum_jb Lov[P, jb] (ovov_bar[ia, jb] + ovov_bar[jb, ia])  (summed first when the
+//                               workspace holds it)
 //             Lvv_bar[P, bc]  = sum_ia Lov[P, ia] ovvv_bar[ia, bc]
 // The engine addresses operands with 32-bit element offsets from each
 // descriptor's base, so products that read ovvv_bar are blocked over the
@@ -76,7 +77,22 @@ struct DfPtrs {
   double *Lvv, *Lvv_bar;
   double *ovvv, *ovoo, *ovov;  // outputs (forward) or cotangents (adjoint; read only)
   double *Lpq_bar;
+  // adjoint with the large workspace: ovov_bar + ovov_bar^T, and room for split-K parts
+  double *ovov_sym, *part;
+  long long part_n;  // elements of part
 };
+
+// Split-K factor of an adjoint product into Lpq_bar: its M x N output has few
+// tiles (o16/v160, naux = 640: 160, and 20 for Loo_bar, for 512 resident
+// workgroups) but a long K (18256, 2560): one round of workgroups, each at
+// least 8 chunks.  Measured there, with the parts added up: Lov_bar 2.2 -> 1.13 ms, Loo_bar 0.27 -> 0.05.
+constexpr size_t kMaxPartBytes = (size_t)512 << 20;
+int df_splits(int M, int N, long long K) {
+  const long long slots = 512, tiles = std::max(1, gemm_tiles(M, N, false));
+  long long S = std::min(slots / tiles, K / (8 * KC));
+  S = std::min<long long>(S, (long long)(kMaxPartBytes / (8.0 * M * N)));
+  return (int)std::max(1LL, S);
+}
 
 void forward_descs(const DfShape &s, const DfPtrs &p, std::vector<GemmDesc> &out_d) {
   const int o = s.o, v = s.v, n = s.n;
@@ -103,9 +119,16 @@ void adjoint_descs(const DfShape &s, const DfPtrs &p, std::vector<GemmDesc> &out
   const OpDesc lovK = opK(p.Lpq + o, s.n2, n, 1, v, 0);    // A(P, ia) = Lpq[P, i, o + a]
   const OpDesc looK = opK(p.Lpq, s.n2, n, 1, o, 0);        // A(P, jk) = Lpq[P, j, k]
   // Loo_bar[P, jk] += sum_ia Lov[P, ia] ovoo_bar[ia, jk]
+  auto add = [&](int N, const std::vector<SegDesc> &sg, OutDesc C) {
+    long long K = 0;
+    for (const SegDesc &g : sg) K += g.L;
+    // (the last occupied block may be smaller, and would take more parts)
+    const int S = p.part ? (int)std::min<long long>(df_splits(naux, N, K), p.part_n / ((long long)naux * N)) : 1;
+    out_d.push_back(gemm(naux, N, S > 1 ? kPartial : kAccumulate, sg.data(), sg.data() + sg.size(), C, S,
+                         S > 1 ? p.part : nullptr));
+  };
   if (p.ovoo)
-    out_d.push_back(gemm(naux, OO, kAccumulate, {seg(lovK, op1(p.ovoo, 1, OO, 1), OV, 1.0)},
-                         out(p.Lpq_bar, 0, s.n2, kBig, n, 1, o)));
+    add(OO, {seg(lovK, op1(p.ovoo, 1, OO, 1), OV, 1.0)}, out(p.Lpq_bar, 0, s.n2, kBig, n, 1, o));
   const int ib = ovvv_block(s, forced_block);
   for (int i0 = 0; i0 < o; i0 += ib) {
     const int ni = std::min(ib, o - i0);
@@ -117,13 +140,13 @@ void adjoint_descs(const DfShape &s, const DfPtrs &p, std::vector<GemmDesc> &out
                        NP, 1.0));
     if (p.ovoo)
       sg.push_back(seg(looK, op1(p.ovoo + (long long)i0 * v * OO, OO, 1, 0), OO, 1.0));
-    if (p.ovov) {
+    if (p.ovov && p.ovov_sym) {
+      sg.push_back(seg(lovK, op1(p.ovov_sym + (long long)i0 * v * s.ov, s.ov, 1, 0), OV, 1.0));
+    } else if (p.ovov) {
       sg.push_back(seg(lovK, op1(p.ovov + (long long)i0 * v * s.ov, s.ov, 1, 0), OV, 1.0));
       sg.push_back(seg(lovK, op1(p.ovov + (long long)i0 * v, 1, s.ov, 1), OV, 1.0));
     }
-    if (!sg.empty())
-      out_d.push_back(gemm(naux, NB, kAccumulate, sg.data(), sg.data() + sg.size(),
-                           out(p.Lpq_bar + o + (long long)i0 * n, 0, s.n2, kBig, n, 1, v)));
+    if (!sg.empty()) add(NB, sg, out(p.Lpq_bar + o + (long long)i0 * n, 0, s.n2, kBig, n, 1, v));
     // Lvv_bar[P, bc] (+)= sum_{ia in block} Lov[P, ia] ovvv_bar[ia, bc]
     if (p.ovvv)
       out_d.push_back(gemm(naux, NP, i0 == 0 ? kStore : kAccumulate,
@@ -134,9 +157,26 @@ void adjoint_descs(const DfShape &s, const DfPtrs &p, std::vector<GemmDesc> &out
 }
 
 int run_descs(const std::vector<GemmDesc> &ds, hipStream_t st) {
-  for (const GemmDesc &d : ds) ERIS_CHECK(launch_gemm_f64(d, st));
+  for (const GemmDesc &d : ds) {
+    ERIS_CHECK(launch_gemm_f64(d, st));
+    if (d.mode == kPartial)
+      ERIS_CHECK(launch_add_parts(d.partial, d.splits, d.M, d.N, d.C.p, d.C.my, (int)d.C.nx, d.C.ndiv, st));
+  }
   return PAMD_OK;
 }
+
+size_t sym_bytes(const DfShape &s) { return ((size_t)s.ov * s.ov * 8 + 255) & ~(size_t)255; }
+
+// elements of the split-K parts, and the workspace of the adjoint with them (the
+// least it takes: 2 lvv_bytes)
+long long part_count(const DfShape &s) {
+  const int nb = ovvv_block(s, 0) * s.v;
+  const long long K = s.np + (long long)s.o * s.o + 2 * s.ov;
+  const long long lov = (long long)df_splits(s.naux, nb, K) * s.naux * nb;
+  const long long loo = (long long)df_splits(s.naux, s.o * s.o, s.ov) * s.naux * s.o * s.o;
+  return std::max(lov, loo);
+}
+size_t vjp_bytes(const DfShape &s) { return 2 * lvv_bytes(s) + sym_bytes(s) + 8 * (size_t)part_count(s); }
 
 }  // namespace
 }  // namespace pamd
@@ -157,7 +197,7 @@ int pamd_df_eris_workspace_size(int nocc, int nmo, int naux, int with_vjp, size_
   DfShape s;
   const int st = df_shape(nocc, nmo, naux, s);
   if (st != PAMD_OK) return st;
-  *bytes = lvv_bytes(s) * (with_vjp ? 2 : 1);
+  *bytes = with_vjp ? vjp_bytes(s) : lvv_bytes(s);
   return PAMD_OK;
 }
 
@@ -169,7 +209,7 @@ int pamd_df_eris(int nocc, int nmo, int naux, const double *Lpq, double *ovvv, d
   if (!Lpq) return PAMD_ERR_ARG;
   if (ovvv && (!workspace || workspace_bytes < lvv_bytes(s))) return PAMD_ERR_WORKSPACE;
   hipStream_t hs = (hipStream_t)stream;
-  DfPtrs p{Lpq, (double *)workspace, nullptr, ovvv, ovoo, ovov, nullptr};
+  DfPtrs p{Lpq, (double *)workspace, nullptr, ovvv, ovoo, ovov, nullptr, nullptr, nullptr, 0};
   if (ovvv) ERIS_CHECK(launch_pack_lvv(Lpq, nocc, nmo, naux, p.Lvv, hs));
   std::vector<GemmDesc> ds;
   forward_descs(s, p, ds);
@@ -187,7 +227,13 @@ int pamd_df_eris_vjp(int nocc, int nmo, int naux, const double *Lpq, const doubl
   hipStream_t hs = (hipStream_t)stream;
   DfPtrs p{Lpq, (double *)workspace, (double *)((char *)workspace + lvv_bytes(s)),
            const_cast<double *>(ovvv_bar), const_cast<double *>(ovoo_bar),
-           const_cast<double *>(ovov_bar), Lpq_bar};
+           const_cast<double *>(ovov_bar), Lpq_bar, nullptr, nullptr, 0};
+  if (workspace_bytes >= vjp_bytes(s)) {
+    p.ovov_sym = (double *)((char *)workspace + 2 * lvv_bytes(s));
+    p.part = (double *)((char *)p.ovov_sym + sym_bytes(s));
+    p.part_n = part_count(s);
+    if (ovov_bar) ERIS_CHECK(launch_add_transpose(ovov_bar, (int)s.ov, p.ovov_sym, hs));
+  }
   ERIS_CHECK(launch_zero_occ_rows(nocc, nmo, naux, Lpq_bar, hs));
   if (ovvv_bar) ERIS_CHECK(launch_pack_lvv(Lpq, nocc, nmo, naux, p.Lvv, hs));
   else ERIS_CHECK(launch_fill(p.Lvv_bar, (size_t)naux * s.np, 0.0, hs));
@@ -207,7 +253,7 @@ int pamd_debug_df_descriptors(int nocc, int nmo, int naux, int with_vjp, int blo
   const int st = df_shape(nocc, nmo, naux, s);
   if (st != PAMD_OK) return st;
   DfPtrs p{(const double *)bases[0], (double *)bases[1], (double *)bases[2], (double *)bases[3],
-           (double *)bases[4],       (double *)bases[5], (double *)bases[6]};
+           (double *)bases[4],       (double *)bases[5], (double *)bases[6], nullptr, nullptr, 0};
   std::vector<GemmDesc> ds;
   if (with_vjp) adjoint_descs(s, p, ds, block_i);
   else forward_descs(s, p, ds);

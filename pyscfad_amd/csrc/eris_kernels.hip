@@ -139,4 +139,45 @@ hipError_t launch_zero_occ_rows(int o, int n, int naux, double *Lpq_bar, hipStre
   return hipGetLastError();
 }
 
+// B + B^T, 32 x 32 tiles, the transposed one through LDS
+__global__ void __launch_bounds__(256) k_add_transpose(const double *__restrict__ B, int n,
+                                                       double *__restrict__ out) {
+  __shared__ double t[32][33];
+  const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  for (int r = ty; r < 32; r += 8)
+    if (x0 + r < n && y0 + tx < n) t[r][tx] = B[(size_t)(x0 + r) * n + y0 + tx];
+  __syncthreads();
+  for (int r = ty; r < 32; r += 8)
+    if (y0 + r < n && x0 + tx < n) {
+      const size_t at = (size_t)(y0 + r) * n + x0 + tx;
+      out[at] = B[at] + t[tx][r];
+    }
+}
+
+hipError_t launch_add_transpose(const double *B, int n, double *out, hipStream_t s) {
+  const unsigned g = (unsigned)((n + 31) / 32);
+  hipLaunchKernelGGL(k_add_transpose, dim3(g, g), dim3(256), 0, s, B, n, out);
+  return hipGetLastError();
+}
+
+// split-K parts into the occupied rows of Lpq_bar, in part order
+__global__ void __launch_bounds__(256) k_add_parts(const double *__restrict__ part, int S, int M, int N,
+                                                   double *__restrict__ out, long long ld, int n, int div) {
+  const int x = blockIdx.x * 256 + threadIdx.x, P = blockIdx.y;
+  if (x >= N) return;
+  const size_t MN = (size_t)M * N;
+  const double *p = part + (size_t)P * N + x;
+  double s = 0.0;
+#pragma unroll 4
+  for (int q = 0; q < S; ++q) s += p[q * MN];
+  out[P * ld + (long long)(x / div) * n + x % div] += s;
+}
+
+hipError_t launch_add_parts(const double *part, int S, int M, int N, double *out, long long ld, int n, int div,
+                            hipStream_t s) {
+  hipLaunchKernelGGL(k_add_parts, dim3((unsigned)((N + 255) / 256), (unsigned)M), dim3(256), 0, s, part, S, M, N,
+                     out, ld, n, div);
+  return hipGetLastError();
+}
+
 }  // namespace pamd
