@@ -1522,7 +1522,7 @@ static int walk_adjoint(const Ctx &c, const WalkLayout &L, char *b, const int *t
     vr.tri = tri;
     vr.nb = nb;
     vr.r_stride = L.r_stride;
-    PAMD_CHECK(timed(s, kProfVR, 0.0, 16.0 * v3 * nb, [&] { return launch_vr(vr, s); }));
+    PAMD_CHECK(timed(s, kProfVR, 0.0, 16.0 * v3 * nb, [&] { return launch_walk_vr(vr, s); }));
   }
   PAMD_CHECK(timed(s, kProfAdjOvvv, fl, 0.0, [&] {
     return launch_walk_vtb(d, at(L.off_W), at(L.off_TB), at(L.off_VTb), tri, nb, first, s);

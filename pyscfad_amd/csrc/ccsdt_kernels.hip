@@ -1397,8 +1397,15 @@ hipError_t launch_fold_t2m(const double *T2mb, int o, int v, int op, int vp, dou
 __global__ void k_reduce_rows(const double *part, int rows, int cols, int ld, double *out, int accumulate) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= cols) return;
-  double s = 0.0;
-  for (int r = 0; r < rows; ++r) s += part[(size_t)r * ld + c];
+  double a[8];  // eight loads in flight
+#pragma unroll
+  for (int u = 0; u < 8; ++u) a[u] = 0.0;
+  int r = 0;
+  for (; r + 8 <= rows; r += 8)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] += part[(size_t)(r + u) * ld + c];
+  for (; r < rows; ++r) a[0] += part[(size_t)r * ld + c];
+  const double s = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
   out[c] = accumulate ? out[c] + s : s;
 }
 

@@ -102,6 +102,9 @@ hipError_t launch_walk_vtb(const WalkDims &d, const double *Wb, const double *TB
 hipError_t launch_walk_tbb(const WalkDims &d, const double *Wb, const double *VT, double *part,
                            const int *tri, int nb, int S, hipStream_t s);
 
+// V-bar reductions of a batch (VRArgs with tri set, parts = 1)
+hipError_t launch_walk_vr(const VRArgs &a, hipStream_t s);
+
 // gather of a batch into the cotangents (overwritten when first)
 struct WalkGather {
   WalkDims d;

@@ -538,6 +538,179 @@ hipError_t launch_walk_tbb(const WalkDims &d, const double *Wb, const double *VT
 }
 
 // ---------------------------------------------------------------------------
+// V-bar reductions of a batch (the blocks are listed at k_vr, which a single
+// triple uses: there the sums must be split to fill the GPU).  Vbar is read
+// twice and little else, so the work is in not adding barriers and idle lanes to
+// that: one wave owns one a and walks the rows b, its sums over b stay in
+// registers, and rows of at most 64 (32) elements run two (four) to a wave, two
+// elements to a lane.  k_vr spends most of its time in the LDS combines of eight
+// waves that see v / 8 rows each.  Measured, o11/v77, 140 triples: 1380 -> 420 us.
+// ---------------------------------------------------------------------------
+typedef double vr_d2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ double vr_wave_sum(double x) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  return x;
+}
+
+// sums of four values over G lanes; lane G / 4 q of them ends up with value q
+template <int G>
+__device__ __forceinline__ double group_sum4(double v0, double v1, double v2, double v3) {
+  const int lane = threadIdx.x & 63;
+  const bool hi = (lane & (G / 2)) != 0, mid = (lane & (G / 4)) != 0;
+  double x = hi ? v2 : v0, y = hi ? v3 : v1;
+  x += __shfl_xor(hi ? v0 : v2, G / 2, 64);
+  y += __shfl_xor(hi ? v1 : v3, G / 2, 64);
+  double z = mid ? y : x;
+  z += __shfl_xor(mid ? x : y, G / 4, 64);
+#pragma unroll
+  for (int off = G / 8; off > 0; off >>= 1) z += __shfl_xor(z, off, 64);
+  return z;
+}
+
+// G lanes per row, Q pairs of columns per lane; all extents multiples of 8
+template <int G, int Q, bool FVO>
+__device__ __forceinline__ void vr_rows(const VRArgs &A, double *R, const double *Vb, int i, int j, int k, int a) {
+  constexpr int RP = 64 / G, U = Q > 2 ? 2 : (8 / RP < 4 ? 8 / RP : 4);
+  const int lane = threadIdx.x & 63, row = lane / G, l = lane % G;
+  const int o = A.o, v = A.v;
+  const size_t vv = (size_t)v * v;
+  auto pair = [&](const double *arr, int x, int y) { return arr + ((size_t)x * o + y) * vv; };
+  vr_d2 c1[Q], c2[Q], c3[Q], c4[FVO ? Q : 1], r3[Q], pk[Q], fk[Q], r4[FVO ? Q : 1];
+  int c[Q];
+  bool ok[Q];
+  const vr_d2 zero = {0.0, 0.0};
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int at = 2 * (l + G * q);
+    ok[q] = at < v;
+    c[q] = ok[q] ? at : v - 2;  // (lanes past the row read its end, times zero)
+    c1[q] = ok[q] ? *(const vr_d2 *)(A.t1 + (size_t)k * v + c[q]) : zero;
+    c2[q] = ok[q] ? *(const vr_d2 *)(pair(A.ovs, i, k) + (size_t)a * v + c[q]) : zero;
+    c3[q] = ok[q] ? *(const vr_d2 *)(pair(A.t2s, i, k) + (size_t)a * v + c[q]) : zero;
+    if (FVO) c4[q] = ok[q] ? vr_d2{A.fvo[(size_t)c[q] * o + k], A.fvo[(size_t)(c[q] + 1) * o + k]} : zero;
+    r3[q] = pk[q] = fk[q] = zero;
+    if (FVO) r4[q] = zero;
+  }
+  const double *sij = pair(A.ovs, i, j) + (size_t)a * v, *tij = pair(A.t2s, i, j) + (size_t)a * v;
+  const double *sjk = pair(A.ovs, j, k), *tjk = pair(A.t2s, j, k), *x0 = Vb + (size_t)a * vv;
+  double t1i = 0.0, fvoi = 0.0;
+  for (int b0 = 0; b0 < v; b0 += RP * U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int b = b0 + u * RP + row;
+      const double t1j = A.t1[(size_t)j * v + b], S1 = sij[b], T1 = tij[b];
+      const double fj = FVO ? A.fvo[(size_t)b * o + j] : 0.0;
+      double sr1 = 0.0, sr2 = 0.0, spj = 0.0, sfj = 0.0;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const size_t at = (size_t)b * v + c[q];
+        const vr_d2 x = *(const vr_d2 *)(x0 + at);
+        vr_d2 s = *(const vr_d2 *)(sjk + at), t = *(const vr_d2 *)(tjk + at);
+        s = ok[q] ? s : zero;
+        t = ok[q] ? t : zero;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          sr1 = fma(x[e], c1[q][e], sr1);
+          spj = fma(x[e], c2[q][e], spj);
+          sfj = fma(x[e], c3[q][e], sfj);
+          r3[q][e] = fma(x[e], t1j, r3[q][e]);
+          pk[q][e] = fma(x[e], S1, pk[q][e]);
+          fk[q][e] = fma(x[e], T1, fk[q][e]);
+          t1i = fma(x[e], s[e], t1i);
+          fvoi = fma(x[e], t[e], fvoi);
+          if (FVO) {
+            sr2 = fma(x[e], c4[q][e], sr2);
+            r4[q][e] = fma(x[e], fj, r4[q][e]);
+          }
+        }
+      }
+      const double z = group_sum4<G>(sr1, sr2, spj, sfj);
+      if (l % (G / 4) == 0) {
+        const int q = l / (G / 4);
+        if (FVO || q != 1) R[(size_t)(q < 2 ? q : q + 6) * vv + (size_t)a * v + b] = z;
+      }
+    }
+  }
+  // the rows of a wave's RP groups
+  auto across = [&](double x) {
+#pragma unroll
+    for (int off = 32; off >= G; off >>= 1) x += __shfl_xor(x, off, 64);
+    return x;
+  };
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    auto put2 = [&](int blk, const vr_d2 &s) {
+      const vr_d2 x = {across(s[0]), across(s[1])};
+      if (row == 0 && ok[q]) *(vr_d2 *)(R + (size_t)blk * vv + (size_t)a * v + c[q]) = x;
+    };
+    put2(2, r3[q]);
+    if (FVO) put2(3, r4[q]);
+    put2(6, pk[q]);
+    put2(7, fk[q]);
+  }
+  t1i = vr_wave_sum(t1i);
+  fvoi = vr_wave_sum(fvoi);
+  if (lane == 0) {
+    R[10 * vv + a] = t1i;
+    R[10 * vv + v + a] = fvoi;
+  }
+}
+
+// grid (row blocks: four a each; then sums over a: 256 positions (b, c) each), triples
+template <int G, int Q, bool FVO>
+__global__ __launch_bounds__(256) void k_walk_vr(VRArgs A) {
+  const int v = A.v, o = A.o, nrow = (v + 3) / 4;
+  const size_t vv = (size_t)v * v;
+  int i, j, k;
+  walk_ijk(A.tri, blockIdx.y, i, j, k);
+  const double *Vb = A.Vb + (size_t)blockIdx.y * vv * v;
+  double *R = A.R + (size_t)blockIdx.y * A.r_stride;
+  if ((int)blockIdx.x < nrow) {
+    const int a = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    vr_rows<G, Q, FVO>(A, R, Vb, i, j, k, a);  // (v is a multiple of 8: a < v)
+    return;
+  }
+  const size_t t = (size_t)(blockIdx.x - nrow) * 256 + threadIdx.x;
+  if (t >= vv) return;
+  const double *x = Vb + t, *t1 = A.t1 + (size_t)i * v;
+  double r5 = 0.0, r6 = 0.0;
+#pragma unroll 8
+  for (int a = 0; a < v; ++a) {
+    const double y = x[a * vv];
+    r5 = fma(y, t1[a], r5);
+    if (FVO) r6 = fma(y, A.fvo[(size_t)a * o + i], r6);
+  }
+  R[4 * vv + t] = r5;
+  if (FVO) R[5 * vv + t] = r6;
+}
+
+hipError_t launch_walk_vr(const VRArgs &a, hipStream_t s) {
+  if (a.v > 512) return launch_vr(a, s);
+  const size_t vv = (size_t)a.v * a.v;
+  const dim3 grid((unsigned)((a.v + 3) / 4 + (vv + 255) / 256), a.nb), block(256);
+#define WALK_VR(G, Q)                                                      \
+  if (a.has_fvo)                                                           \
+    hipLaunchKernelGGL((k_walk_vr<G, Q, true>), grid, block, 0, s, a);     \
+  else                                                                     \
+    hipLaunchKernelGGL((k_walk_vr<G, Q, false>), grid, block, 0, s, a)
+  if (a.v <= 32) {
+    WALK_VR(16, 1);
+  } else if (a.v <= 64) {
+    WALK_VR(32, 1);
+  } else if (a.v <= 128) {
+    WALK_VR(64, 1);
+  } else if (a.v <= 256) {
+    WALK_VR(64, 2);
+  } else {
+    WALK_VR(64, 4);
+  }
+#undef WALK_VR
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // gather
 // ---------------------------------------------------------------------------
 // more than one column block (v > 512): their parts of blocks 0, 1, 8, 9 and of
@@ -586,20 +759,30 @@ __global__ __launch_bounds__(256) void k_walk_cols(int v, const double *R, size_
   }
 }
 
-// t1_bar and fvo_bar of occupied orbital blockIdx.y from the batch's vectors
+// t1_bar and fvo_bar of occupied orbital blockIdx.y from the batch's vectors: 64
+// columns per workgroup, the four waves splitting the triples
 __global__ __launch_bounds__(256) void k_walk_t1(WalkGather G) {
+  __shared__ double red[2][4][64];
   const int v = G.d.v, vp = G.d.vp, o = G.d.o, x = blockIdx.y;
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= v) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = blockIdx.x * 64 + lane;
   double st = 0.0, sf = 0.0;
-  for (int b = 0; b < G.nb; ++b) {
-    const int w = G.tri[b];
-    const int i = w & 1023, j = (w >> 10) & 1023, k = w >> 20;
-    const double *d = G.vec + (size_t)b * 6 * vp + c;
-    if (k == x) st += d[0], sf += d[3 * (size_t)vp];
-    if (j == x) st += d[(size_t)vp], sf += d[4 * (size_t)vp];
-    if (i == x) st += d[2 * (size_t)vp], sf += d[5 * (size_t)vp];
-  }
+  if (c < v)
+#pragma unroll 4
+    for (int b = wave; b < G.nb; b += 4) {
+      const int w = G.tri[b];
+      const int i = w & 1023, j = (w >> 10) & 1023, k = w >> 20;
+      const double *d = G.vec + (size_t)b * 6 * vp + c;
+      if (k == x) st += d[0], sf += d[3 * (size_t)vp];
+      if (j == x) st += d[(size_t)vp], sf += d[4 * (size_t)vp];
+      if (i == x) st += d[2 * (size_t)vp], sf += d[5 * (size_t)vp];
+    }
+  red[0][wave][lane] = st;
+  red[1][wave][lane] = sf;
+  __syncthreads();
+  if (wave != 0 || c >= v) return;
+  st = (red[0][0][lane] + red[0][1][lane]) + (red[0][2][lane] + red[0][3][lane]);
+  sf = (red[1][0][lane] + red[1][1][lane]) + (red[1][2][lane] + red[1][3][lane]);
   double *t = G.t1_bar + (size_t)x * v + c, *f = G.fvo_bar + (size_t)c * o + x;
   *t = 0.5 * st + (G.first ? 0.0 : *t);
   *f = 0.5 * sf + (G.first ? 0.0 : *f);
@@ -693,7 +876,7 @@ hipError_t launch_walk_gather(const WalkGather &g, hipStream_t s) {
                        const_cast<double *>(g.R), g.r_stride, g.has_fvo);
     hipLaunchKernelGGL(k_walk_cols, dim3((v + 63) / 64, g.nb), dim3(256), 0, s, v, g.R, g.r_stride, g.vec);
   }
-  hipLaunchKernelGGL(k_walk_t1, dim3((g.d.v + 255) / 256, o), dim3(256), 0, s, g);
+  hipLaunchKernelGGL(k_walk_t1, dim3((g.d.v + 63) / 64, o), dim3(256), 0, s, g);
   const int nblk = (v * g.d.up + 255) / 256;
   hipLaunchKernelGGL(k_walk_gather, dim3((unsigned)(nblk * o * o)), dim3(256), 0, s, g, nblk);
   if (!g.tri_e) return hipGetLastError();

@@ -45,7 +45,8 @@ def _smallest_workspace(inp):
 
 @pytest.mark.parametrize('o,v,fvo,packed', [(2, 7, 1e-3, True), (3, 9, 0.0, False), (4, 16, 1e-3, True),
                                             (5, 47, 1e-3, False), (3, 81, 0.0, True),
-                                            (6, 49, 1e-3, True), (1, 12, 1e-3, False)])
+                                            (6, 49, 1e-3, True), (1, 12, 1e-3, False), (2, 33, 1e-3, True),
+                                            (2, 131, 1e-3, True), (2, 263, 0.0, True)])
 def test_batched_walk_matches_the_one_triple_walk(o, v, fvo, packed, cuda):
     p = make_problem(o, v, 3 * v, seed=o * 100 + v, fvo_scale=fvo)
     inp = _ops.Inputs(p.mo_energy, p.t1, p.t2, p.ovvv_packed() if packed else p.ovvv, p.ovoo, p.ovov,
