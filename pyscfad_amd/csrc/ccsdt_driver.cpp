@@ -806,6 +806,24 @@ static int zero_vjp(const Ctx &c) {
   return PAMD_OK;
 }
 
+// inputs of a call's WalkPrep; the caller adds the outputs
+static WalkPrep walk_prep(const Ctx &c, const WalkDims &d) {
+  WalkPrep w;
+  memset(&w, 0, sizeof(w));
+  w.d = d;
+  w.mo = c.mo;
+  w.t1 = c.t1;
+  w.t2 = c.t2;
+  w.ovvv = c.ovvv;
+  w.ovoo = c.ovoo;
+  w.ovov = c.ovov;
+  w.fvo = c.has_fvo ? c.fvo : nullptr;
+  w.packed = c.packed;
+  w.shard = c.shard;
+  w.nshards = c.nshards;
+  return w;
+}
+
 // Layout changes at entry, shared by every walk; returns the orbit count.
 static int setup(Ctx &c, long long &norb) {
   const int o = c.o, v = c.v;
@@ -814,14 +832,25 @@ static int setup(Ctx &c, long long &norb) {
   norb = (long long)nt * (nt + 1) * (nt + 2) / 6;
   PAMD_CHECK(launch_prepare(c.ovvv, c.packed, c.t2, c.ovoo, o, v, c.op, c.vp, c.Vp, c.T2m, c.OOt, fmt, c.s));
   if (c.pad) {
-    PAMD_CHECK(launch_walk_small_inputs(walk_dims(o, v), c.mo, c.t1, c.t2, c.ovov, c.has_fvo ? c.fvo : nullptr,
-                                        c.OVS, c.T2S, c.t1p, c.fvop, c.mop, c.s));
-    const long long n = (num_triples(o) - c.shard + c.nshards - 1) / c.nshards;
-    PAMD_CHECK(launch_walk_triples(o, c.shard, c.nshards, walk_batches(n, INT_MAX), c.tab, c.s));
+    WalkPrep w = walk_prep(c, walk_dims(o, v));
+    w.OVS = c.OVS;
+    w.T2S = c.T2S;
+    w.t1p = c.t1p;
+    w.fvop = c.fvop;
+    w.mop = c.mop;
+    w.orb = c.orb;
+    w.norb = norb;
+    w.tri = c.tab;
+    w.wb = walk_batches((num_triples(o) - c.shard + c.nshards - 1) / c.nshards, INT_MAX);
+    w.zero[0] = c.tri;
+    w.nzero[0] = (size_t)o * o * o;
+    PAMD_CHECK(launch_walk_prep(w, c.s));
     if (c.wt_host) PAMD_CHECK(launch_walk_upload(c.wt_host, o, c.wt, c.s));
   } else {
     PAMD_CHECK(launch_prep_sym(c.ovov, o, v, 0, c.OVS, c.s));
     PAMD_CHECK(launch_prep_sym(c.t2, o, v, 1, c.T2S, c.s));
+    PAMD_CHECK(launch_fill(c.tri, (size_t)o * o * o, 0.0, c.s));
+    PAMD_CHECK(launch_orbit_table(norb, c.orb, c.s));
   }
   if (fmt == kSplitBf16x3)
     PAMD_CHECK(launch_split_t2(c.t2, o, v, c.vp, (unsigned short *)c.gT2, c.s));
@@ -830,8 +859,6 @@ static int setup(Ctx &c, long long &norb) {
                                     (unsigned short *)c.VpU, c.s));
   if (fmt == kSplitF32x2)
     PAMD_CHECK(launch_split_f32x2(c.t2, (size_t)o * o * v * v, (unsigned long long *)c.gT2, c.s));
-  PAMD_CHECK(launch_fill(c.tri, (size_t)o * o * o, 0.0, c.s));
-  PAMD_CHECK(launch_orbit_table(norb, c.orb, c.s));
   // padded: two workgroups per CU, four without the adjoint (LDS)
   c.G = c.pad ? (int)std::min<long long>({norb, (long long)(c.vjp ? 2 : 4) * device_cus(), (long long)kGmax})
               : std::min(orbit_grid(v), kGmax);
@@ -1442,21 +1469,37 @@ static bool walk_pick(int o, int v, int vjp, size_t limit, size_t one_triple_tot
   return L.total <= ((size_t)100 << 30) || L.total <= one_triple_total + one_triple_total / 20;
 }
 
-// Inputs, orbit table and zeroed row sums of a call; returns the orbit count.
-static int walk_setup(Ctx &c, const WalkLayout &L, char *b, long long &norb) {
+// Inputs, tables and zeroed sums of a call: the triples of wb, or with pairs those
+// of the projected walk, in tab; zero[0 .. nzero) = 0.  Returns the orbit count.
+static int walk_setup(Ctx &c, const WalkLayout &L, char *b, const WalkBatches *wb, int *tab, double *zero,
+                      size_t nzero, long long &norb) {
   auto at = [&](size_t off) { return (double *)(b + off); };
   const WalkDims &d = L.d;
   c.tri = at(L.off_tri_e);
   c.wt = at(L.off_wt);
-  PAMD_CHECK(launch_walk_inputs(d, c.mo, c.t1, c.t2, c.ovvv, c.packed, c.ovoo, c.ovov,
-                                c.has_fvo ? c.fvo : nullptr, at(L.off_VT), c.vjp ? at(L.off_TB) : nullptr,
-                                at(L.off_TBt), at(L.off_OVS), at(L.off_T2S), at(L.off_t1), at(L.off_fvo),
-                                at(L.off_mo), c.s));
   const long long nt = d.vp / 8;
   norb = nt * (nt + 1) * (nt + 2) / 6;
-  PAMD_CHECK(launch_orbit_table(norb, (unsigned short *)at(L.off_orb), c.s));
-  if (c.vjp)
-    PAMD_CHECK(launch_fill(at(L.off_mo_rows), (size_t)L.nb * L.G * (d.o + d.vp), 0.0, c.s));
+  WalkPrep w = walk_prep(c, d);
+  w.VT = at(L.off_VT);
+  w.TB = c.vjp ? at(L.off_TB) : nullptr;
+  w.TBt = at(L.off_TBt);
+  w.OVS = at(L.off_OVS);
+  w.T2S = at(L.off_T2S);
+  w.t1p = at(L.off_t1);
+  w.fvop = at(L.off_fvo);
+  w.mop = at(L.off_mo);
+  w.orb = (unsigned short *)at(L.off_orb);
+  w.norb = norb;
+  w.tri = tab;
+  w.pairs = wb ? 0 : 1;
+  if (wb) w.wb = *wb;
+  w.zero[0] = zero;
+  w.nzero[0] = nzero;
+  if (c.vjp) {
+    w.zero[1] = at(L.off_mo_rows);
+    w.nzero[1] = (size_t)L.nb * L.G * (d.o + d.vp);
+  }
+  PAMD_CHECK(launch_walk_prep(w, c.s));
   return PAMD_OK;
 }
 
@@ -1592,13 +1635,11 @@ static int run_walk(Ctx &c, const WalkLayout &L, void *ws, double *ovvv_bar, dou
   const int o = c.o;
   const hipStream_t s = c.s;
   long long norb = 0;
-  int st = walk_setup(c, L, b, norb);
-  if (st != PAMD_OK) return st;
   int *tab = (int *)at(L.off_tab);
   const long long n = (num_triples(o) - c.shard + c.nshards - 1) / c.nshards;
   const WalkBatches wb = walk_batches(n, L.nb);
-  PAMD_CHECK(launch_walk_triples(o, c.shard, c.nshards, wb, tab, s));
-  PAMD_CHECK(launch_fill(c.tri, (size_t)o * o * o, 0.0, s));
+  int st = walk_setup(c, L, b, &wb, tab, at(L.off_tri_e), (size_t)o * o * o, norb);
+  if (st != PAMD_OK) return st;
   if (c.wt_host)
     PAMD_CHECK(hipMemcpyAsync(c.wt, c.wt_host, sizeof(double) * (size_t)o, hipMemcpyHostToDevice, s));
   const double v3 = (double)c.v * c.v * c.v;
@@ -1687,12 +1728,10 @@ static int run_projected_walk(Ctx &c, const ProjWalkLayout &P, void *ws, const d
   const int o = c.o;
   const hipStream_t s = c.s;
   long long norb = 0;
-  int st = walk_setup(c, L, b, norb);
-  if (st != PAMD_OK) return st;
   int *tab = (int *)at(P.off_tab);
-  PAMD_CHECK(launch_walk_pairs(o, tab, s));
+  int st = walk_setup(c, L, b, nullptr, tab, at(P.off_pair), (size_t)o * o, norb);
+  if (st != PAMD_OK) return st;
   PAMD_CHECK(launch_walk_upload(ulo, (size_t)nfrag * o, at(P.off_ulo), s));
-  PAMD_CHECK(launch_fill(at(P.off_pair), (size_t)o * o, 0.0, s));
   const double v3 = (double)c.v * c.v * c.v;
   const int pairs = o * (o + 1) / 2;
   WalkMeter meter(c.vjp ? "projected (T)+VJP" : "projected (T)", (long long)pairs * o);

@@ -508,18 +508,6 @@ int gemm_tiles(int M, int N, bool fx2) {
 // ---------------------------------------------------------------------------
 constexpr int OT = 8, OT3 = OT * OT * OT;
 
-__device__ __forceinline__ void decode_orbit(long long q, int &A, int &B, int &C) {
-  int a = 0;
-  while ((long long)(a + 1) * (a + 2) * (a + 3) / 6 <= q) ++a;
-  long long rem = q - (long long)a * (a + 1) * (a + 2) / 6;
-  int b = 0;
-  while ((long long)(b + 1) * (b + 2) / 2 <= rem) ++b;
-  A = a;
-  B = b;
-  C = (int)(rem - (long long)b * (b + 1) / 2);
-}
-
-
 // Distinct tiles of an orbit and where the five non-identity permutations of a
 // position land, for the four equality patterns of A >= B >= C: 0 all distinct,
 // 1 A == B > C, 2 A > B == C, 3 A == B == C.  sel[p] picks the tile indices of
@@ -547,18 +535,9 @@ __constant__ OrbitPattern kOrbitPat[4] = {
 
 typedef const __attribute__((address_space(4))) unsigned long long *OrbitEntryPtr;
 
-// Orbit table: entry q = (A, B, C, pattern) of the q-th tile triple A >= B >= C;
-// pattern = (A == B) + 2 (B == C) selects kOrbitPat.
 __global__ void k_orbit_table(long long norb, unsigned short *tab) {
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= norb) return;
-  int a, b, c;
-  decode_orbit(q, a, b, c);
-  unsigned short *e = tab + 4 * q;
-  e[0] = (unsigned short)a;
-  e[1] = (unsigned short)b;
-  e[2] = (unsigned short)c;
-  e[3] = (unsigned short)((a == b ? 1 : 0) + (b == c ? 2 : 0));
+  if (q < norb) put_orbit(q, tab);
 }
 
 hipError_t launch_orbit_table(long long norb, unsigned short *tab, hipStream_t s) {

@@ -28,6 +28,29 @@ struct OpStage {
   static_assert(KSTEP * E == R && RSTEP * E == GKC, "staging map covers the panel");
 };
 
+__device__ __forceinline__ void decode_orbit(long long q, int &A, int &B, int &C) {
+  int a = 0;
+  while ((long long)(a + 1) * (a + 2) * (a + 3) / 6 <= q) ++a;
+  long long rem = q - (long long)a * (a + 1) * (a + 2) / 6;
+  int b = 0;
+  while ((long long)(b + 1) * (b + 2) / 2 <= rem) ++b;
+  A = a;
+  B = b;
+  C = (int)(rem - (long long)b * (b + 1) / 2);
+}
+
+// Orbit table: entry q = (A, B, C, pattern) of the q-th tile triple A >= B >= C;
+// pattern = (A == B) + 2 (B == C) selects kOrbitPat.
+__device__ __forceinline__ void put_orbit(long long q, unsigned short *tab) {
+  int a, b, c;
+  decode_orbit(q, a, b, c);
+  unsigned short *e = tab + 4 * q;
+  e[0] = (unsigned short)a;
+  e[1] = (unsigned short)b;
+  e[2] = (unsigned short)c;
+  e[3] = (unsigned short)((a == b ? 1 : 0) + (b == c ? 2 : 0));
+}
+
 // Output coordinate of position w of tile t along one dimension: the index,
 // and its split (q, r) = divmod(index, div) for the output descriptor (no
 // division when div is the "no split" value 2^30).

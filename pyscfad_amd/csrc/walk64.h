@@ -41,15 +41,6 @@ inline bool walk_dims_ok(const WalkDims &d) {
   return (d.vp + 8) * d.sp * 8 < (1LL << 32);
 }
 
-// padded inputs of the walk (TBt[z][y][k][r] = TB[z][y][r][k])
-hipError_t launch_walk_inputs(const WalkDims &d, const double *mo, const double *t1, const double *t2,
-                              const double *ovvv, int packed, const double *ovoo, const double *ovov,
-                              const double *fvo, double *VT, double *TB, double *TBt, double *OVS,
-                              double *T2S, double *t1p, double *fvop, double *mop, hipStream_t s);
-// of these, what the orbit epilogue and the V-bar reductions read
-hipError_t launch_walk_small_inputs(const WalkDims &d, const double *mo, const double *t1, const double *t2,
-                                    const double *ovov, const double *fvo, double *OVS, double *T2S, double *t1p,
-                                    double *fvop, double *mop, hipStream_t s);
 // Batches.  The call's triples (walk order i <= j <= k without i == j == k, every
 // nshards-th from shard on) are cut into runs of 8, dealt to the batches in
 // turn: a run shares i, j and so its slabs of VT, while every batch has about
@@ -75,8 +66,25 @@ inline WalkBatches walk_batches(long long n, int nb) {
   const int cap = (int)((runs + count - 1) / count) * kWalkRun;
   return {cap > 0 ? cap : kWalkRun, count, n};
 }
-// tri[b cap + slot] = i | j << 10 | k << 20
-hipError_t launch_walk_triples(int o, int shard, int nshards, const WalkBatches &wb, int *tri, hipStream_t s);
+// Everything a call prepares, in one launch: padded inputs (TBt[z][y][k][r] =
+// TB[z][y][r][k]; VT null: only what the orbit epilogue and the V-bar reductions
+// read), the orbit table, the triple table (tri[b cap + slot] = i | j << 10 |
+// k << 20; pairs: slot p o + l is the triple (l, j, k) of the p-th pair j <= k, and
+// nothing is left out) and two arrays to be zeroed.
+struct WalkPrep {
+  WalkDims d;
+  const double *mo, *t1, *t2, *ovvv, *ovoo, *ovov, *fvo;
+  double *VT, *TB, *TBt, *OVS, *T2S, *t1p, *fvop, *mop;
+  unsigned short *orb;
+  int *tri;
+  double *zero[2];
+  size_t nzero[2];
+  long long norb;
+  WalkBatches wb;
+  int packed, shard, nshards, pairs;
+  unsigned blocks[4];  // of VT, TB, the symmetrised blocks and the rest (set by the launcher)
+};
+hipError_t launch_walk_prep(WalkPrep a, hipStream_t s);
 
 // W of nb triples (tri[0 .. nb)), each a block of vp ws elements
 hipError_t launch_walk_w(const WalkDims &d, const double *VT, const double *TBt, double *W, const int *tri,
@@ -123,9 +131,6 @@ hipError_t launch_walk_gather(const WalkGather &g, hipStream_t s);
 hipError_t launch_walk_energies(const int *tri, int nb, int o, const double *part_t, int G, double *tri_e,
                                 hipStream_t s);
 
-// Projected walk: slot p o + l of the table is the triple (l, j, k) of the p-th
-// pair j <= k (every first index l of the pair; nothing is left out)
-hipError_t launch_walk_pairs(int o, int *tri, hipStream_t s);
 // dst[0 .. n) = src (host), through kernel arguments: no copy to wait for or to
 // record in a captured graph
 hipError_t launch_walk_upload(const double *src, size_t n, double *dst, hipStream_t s);

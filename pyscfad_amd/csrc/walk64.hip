@@ -23,14 +23,14 @@ namespace pamd {
 // VT: a 32 x 32 tile (q, k) of one (x, p) per workgroup.  Full ovvv rows run
 // along q, VT rows along k, so the tile is turned in LDS; packed ovvv and the
 // t2 part are read along whichever index is contiguous.
-__global__ __launch_bounds__(256) void k_walk_vt(WalkDims d, const double *__restrict__ ovvv, int packed,
-                                                 const double *__restrict__ t2, double *__restrict__ VT) {
-  __shared__ double tile[32][33];
+__device__ __forceinline__ void prep_vt(const WalkDims &d, const double *__restrict__ ovvv, int packed,
+                                        const double *__restrict__ t2, double *__restrict__ VT, int bq, int bk,
+                                        int bz, int nz, double (*tile)[33]) {
   const int o = d.o, v = d.v, vp = d.vp, up = d.up;
-  const int q0 = blockIdx.x * 32, k0 = blockIdx.y * 32;
+  const int q0 = bq * 32, k0 = bk * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const size_t npair = (size_t)v * (v + 1) / 2;
-  for (int xp = blockIdx.z; xp < o * vp; xp += gridDim.z) {
+  for (int xp = bz; xp < o * vp; xp += nz) {
     const int x = xp / vp, p = xp - x * vp;
     // tile[k][q], lanes along q
     for (int r = ty; r < 32; r += 8) {
@@ -61,15 +61,14 @@ __global__ __launch_bounds__(256) void k_walk_vt(WalkDims d, const double *__res
   }
 }
 
-// TB, and TBt[z][y][k][r] = TB[z][y][r][k]
-__global__ __launch_bounds__(256) void k_walk_tb(WalkDims d, const double *__restrict__ t2,
-                                                 const double *__restrict__ ovoo, double *__restrict__ TB,
-                                                 double *__restrict__ TBt) {
+// TB (turned: TBt[z][y][k][r] = TB[z][y][r][k])
+__device__ __forceinline__ void prep_tb(const WalkDims &d, const double *__restrict__ t2,
+                                        const double *__restrict__ ovoo, double *__restrict__ out, bool turned,
+                                        unsigned blk, unsigned nblk) {
   const int o = d.o, v = d.v, vp = d.vp, up = d.up;
   const size_t total = (size_t)o * o * vp * up;
-  const bool turned = blockIdx.y != 0 || !TB;  // (no TB for an energy: grid y is 1)
   const int fast = turned ? vp : up, slow = turned ? up : vp;
-  for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (size_t)gridDim.x * 256) {
+  for (size_t t = (size_t)blk * 256 + threadIdx.x; t < total; t += (size_t)nblk * 256) {
     const int x = (int)(t % fast);
     const size_t u = t / fast, zy = u / slow;
     const int y = (int)(u % slow);
@@ -79,22 +78,20 @@ __global__ __launch_bounds__(256) void k_walk_tb(WalkDims d, const double *__res
       val = t2[(zy * v + r) * v + k];
     else if (r < v && k < v + o)
       val = -ovoo[(((zy / o) * v + r) * o + (k - v)) * o + zy % o];
-    (turned ? TBt : TB)[t] = val;
+    out[t] = val;
   }
 }
 
-// OVS[x][y][p][q] = ovov[x,p,y,q] + ovov[y,q,x,p], T2S[x][y][p][q] = t2[x,y,p,q] +
-// t2[y,x,q,p] (blockIdx.z 0 / 1): the transposed term goes through LDS.
-__global__ __launch_bounds__(256) void k_walk_sym(WalkDims d, const double *__restrict__ ovov,
-                                                  const double *__restrict__ t2, double *__restrict__ OVS,
-                                                  double *__restrict__ T2S, int ntile) {
-  __shared__ double tile[32][33];
+// OVS[x][y][p][q] = ovov[x,p,y,q] + ovov[y,q,x,p], or (amp) T2S[x][y][p][q] =
+// t2[x,y,p,q] + t2[y,x,q,p]: the transposed term goes through LDS.
+__device__ __forceinline__ void prep_sym(const WalkDims &d, const double *__restrict__ ovov,
+                                         const double *__restrict__ t2, double *__restrict__ dst, bool amp,
+                                         int ntile, int blk, double (*tile)[33]) {
   const int o = d.o, v = d.v, vp = d.vp;
-  const int xy = blockIdx.x / (ntile * ntile), tl = blockIdx.x - xy * ntile * ntile;
+  const int xy = blk / (ntile * ntile), tl = blk - xy * ntile * ntile;
   const int x = xy / o, y = xy % o;
   const int p0 = (tl / ntile) * 32, q0 = (tl % ntile) * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  const bool amp = blockIdx.z != 0;
   auto src = [&](int xx, int pp, int yy, int qq) {
     return amp ? t2[(((size_t)xx * o + yy) * v + pp) * v + qq]
                : ovov[(((size_t)xx * v + pp) * o + yy) * v + qq];
@@ -104,7 +101,6 @@ __global__ __launch_bounds__(256) void k_walk_sym(WalkDims d, const double *__re
     tile[r][tx] = (q < v && p < v) ? src(y, q, x, p) : 0.0;
   }
   __syncthreads();
-  double *dst = amp ? T2S : OVS;
   for (int r = ty; r < 32; r += 8) {
     const int p = p0 + r, q = q0 + tx;
     if (p >= vp || q >= vp) continue;
@@ -113,9 +109,8 @@ __global__ __launch_bounds__(256) void k_walk_sym(WalkDims d, const double *__re
   }
 }
 
-__global__ void k_walk_small(WalkDims d, const double *mo, const double *t1, const double *fvo, double *t1p,
-                             double *fvop, double *mop) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void prep_small(const WalkDims &d, const double *mo, const double *t1,
+                                           const double *fvo, double *t1p, double *fvop, double *mop, int t) {
   const int o = d.o, v = d.v, vp = d.vp;
   if (t < o * vp) {
     const int i = t / vp, a = t - i * vp;
@@ -127,34 +122,8 @@ __global__ void k_walk_small(WalkDims d, const double *mo, const double *t1, con
   if (t < o + vp) mop[t] = mo[min(t, o + v - 1)];
 }
 
-hipError_t launch_walk_inputs(const WalkDims &d, const double *mo, const double *t1, const double *t2,
-                              const double *ovvv, int packed, const double *ovoo, const double *ovov,
-                              const double *fvo, double *VT, double *TB, double *TBt, double *OVS,
-                              double *T2S, double *t1p, double *fvop, double *mop, hipStream_t s) {
-  const int nq = (d.vp + 31) / 32, nk = (d.up + 31) / 32;
-  hipLaunchKernelGGL(k_walk_vt, dim3(nq, nk, std::min(d.o * d.vp, 65535)), dim3(256), 0, s, d, ovvv, packed,
-                     t2, VT);
-  const size_t ntb = (size_t)d.o * d.o * d.vp * d.up;
-  hipLaunchKernelGGL(k_walk_tb, dim3((unsigned)std::min<size_t>((ntb + 255) / 256, 262144), TB ? 2 : 1), dim3(256),
-                     0, s, d, t2, ovoo, TB, TBt);
-  return launch_walk_small_inputs(d, mo, t1, t2, ovov, fvo, OVS, T2S, t1p, fvop, mop, s);
-}
-
-hipError_t launch_walk_small_inputs(const WalkDims &d, const double *mo, const double *t1, const double *t2,
-                                    const double *ovov, const double *fvo, double *OVS, double *T2S, double *t1p,
-                                    double *fvop, double *mop, hipStream_t s) {
-  const int nq = (d.vp + 31) / 32;
-  hipLaunchKernelGGL(k_walk_sym, dim3((unsigned)(d.o * d.o * nq * nq), 1, 2), dim3(256), 0, s, d, ovov, t2, OVS,
-                     T2S, nq);
-  hipLaunchKernelGGL(k_walk_small, dim3((d.o * d.vp + d.vp + d.o + 255) / 256), dim3(256), 0, s, d, mo, t1,
-                     fvo, t1p, fvop, mop);
-  return hipGetLastError();
-}
-
-// one thread per pair i <= j, in closed form: the triples before (i, j, j)
-__global__ void k_walk_triples(int o, int shard, int nshards, WalkBatches wb, int *tri) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= o * o) return;
+// the triples of pair t = i o + j, in closed form: the triples before (i, j, j)
+__device__ __forceinline__ void prep_triples(int o, int shard, int nshards, const WalkBatches &wb, int *tri, int t) {
   const int i = t / o, j = t % o;
   if (j < i) return;
   // triples with first index < i: sum_{x<i} ((o-x)(o-x+1)/2 - 1)
@@ -170,8 +139,83 @@ __global__ void k_walk_triples(int o, int shard, int nshards, WalkBatches wb, in
     }
 }
 
-hipError_t launch_walk_triples(int o, int shard, int nshards, const WalkBatches &wb, int *tri, hipStream_t s) {
-  hipLaunchKernelGGL(k_walk_triples, dim3((o * o + 255) / 256), dim3(256), 0, s, o, shard, nshards, wb, tri);
+__device__ __forceinline__ void prep_pairs(int o, int *tri, int t) {
+  const int j = t / o, k = t % o;
+  if (k < j) return;
+  int *p = tri + (size_t)(j * o - j * (j - 1) / 2 + k - j) * o;
+  for (int l = 0; l < o; ++l) p[l] = l | (j << 10) | (k << 20);
+}
+
+// The pieces do not depend on each other: a workgroup's number says which it
+// works on.  (Eight launches at o4/v16, each 3 us of a call that takes 100.)
+__global__ __launch_bounds__(256) void k_walk_prep(WalkPrep A) {
+  __shared__ double tile[32][33];
+  const WalkDims &d = A.d;
+  unsigned blk = blockIdx.x;
+  if (blk < A.blocks[0]) {
+    const unsigned nq = (d.vp + 31) / 32, nk = (d.up + 31) / 32, r = blk / nq;
+    prep_vt(d, A.ovvv, A.packed, A.t2, A.VT, (int)(blk - r * nq), (int)(r % nk), (int)(r / nk),
+            (int)(A.blocks[0] / (nq * nk)), tile);
+    return;
+  }
+  blk -= A.blocks[0];
+  if (blk < A.blocks[1]) {  // TBt, and with an adjoint TB
+    const unsigned n = A.TB ? A.blocks[1] / 2 : A.blocks[1];
+    const bool turned = blk < n;
+    prep_tb(d, A.t2, A.ovoo, turned ? A.TBt : A.TB, turned, turned ? blk : blk - n, n);
+    return;
+  }
+  blk -= A.blocks[1];
+  if (blk < A.blocks[2]) {
+    const unsigned n = A.blocks[2] / 2;
+    const bool amp = blk >= n;
+    prep_sym(d, A.ovov, A.t2, amp ? A.T2S : A.OVS, amp, (d.vp + 31) / 32, (int)(amp ? blk - n : blk), tile);
+    return;
+  }
+  blk -= A.blocks[2];
+  const int o = d.o, ns = o * d.vp + d.vp + o;
+  long long t = (long long)blk * 256 + threadIdx.x;
+  if (t < ns) {
+    prep_small(d, A.mo, A.t1, A.fvo, A.t1p, A.fvop, A.mop, (int)t);
+    return;
+  }
+  t -= ns;
+  if (t < A.norb) {
+    put_orbit(t, A.orb);
+    return;
+  }
+  t -= A.norb;
+  if (t < o * o) {
+    if (A.pairs)
+      prep_pairs(o, A.tri, (int)t);
+    else
+      prep_triples(o, A.shard, A.nshards, A.wb, A.tri, (int)t);
+    return;
+  }
+  t -= o * o;
+#pragma unroll
+  for (int z = 0; z < 2; ++z) {
+    if (t < (long long)A.nzero[z]) {
+      A.zero[z][t] = 0.0;
+      return;
+    }
+    t -= (long long)A.nzero[z];
+  }
+}
+
+hipError_t launch_walk_prep(WalkPrep a, hipStream_t s) {
+  const WalkDims &d = a.d;
+  const unsigned nq = (d.vp + 31) / 32, nk = (d.up + 31) / 32;
+  const size_t ntb = (size_t)d.o * d.o * d.vp * d.up;
+  a.blocks[0] = a.VT ? nq * nk * (unsigned)std::min(d.o * d.vp, 65535) : 0;
+  a.blocks[1] = a.TBt ? (unsigned)std::min<size_t>((ntb + 255) / 256, 262144) * (a.TB ? 2 : 1) : 0;
+  a.blocks[2] = 2u * (unsigned)(d.o * d.o) * nq * nq;
+  const long long rest = (long long)d.o * d.vp + d.vp + d.o + a.norb + (long long)d.o * d.o +
+                         (long long)(a.nzero[0] + a.nzero[1]);
+  a.blocks[3] = (unsigned)((rest + 255) / 256);
+  const long long total = (long long)a.blocks[0] + a.blocks[1] + a.blocks[2] + a.blocks[3];
+  if (total >= (1LL << 31)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_walk_prep, dim3((unsigned)total), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -733,11 +777,11 @@ __global__ __launch_bounds__(256) void k_walk_vrsum(int v, double *R, size_t r_s
 
 // column sums of a triple's blocks: vec[b] = {for t1[k], t1[j], t1[i], fvo[k],
 // fvo[j], fvo[i]}, 64 columns per workgroup, the four waves splitting the rows
-__global__ __launch_bounds__(256) void k_walk_cols(int v, const double *R, size_t r_stride, double *vec) {
-  __shared__ double red[4][4][64];
+__device__ __forceinline__ void walk_cols(int v, const double *R, size_t r_stride, double *vec, int bx, int by,
+                                          double (*red)[4][64]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + lane;
-  const double *r = R + blockIdx.y * r_stride;
+  const int c = bx * 64 + lane;
+  const double *r = R + by * r_stride;
   const size_t vv = (size_t)v * v;
   double s[4] = {0.0, 0.0, 0.0, 0.0};
   constexpr int blk[4] = {6, 8, 7, 9};
@@ -749,7 +793,7 @@ __global__ __launch_bounds__(256) void k_walk_cols(int v, const double *R, size_
   for (int q = 0; q < 4; ++q) red[q][wave][lane] = s[q];
   __syncthreads();
   if (wave == 0 && c < v) {
-    double *d = vec + (size_t)blockIdx.y * 6 * v;
+    double *d = vec + (size_t)by * 6 * v;
     constexpr int to[4] = {0, 1, 3, 4};
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -791,11 +835,9 @@ __global__ __launch_bounds__(256) void k_walk_t1(WalkGather G) {
 // t2_bar[x,y], ovov_bar[x,.,y,.] and ovoo_bar[x,.,.,y]: a workgroup holds 256
 // positions (p, k) of one pair (x, y) and walks the batch's triples that write
 // to it, so every position is summed by one thread in a fixed order.
-__global__ __launch_bounds__(256) void k_walk_gather(WalkGather G, int nblk) {
-  __shared__ int list[kWalkMaxBatch];
-  __shared__ int cnt[4];
+__device__ __forceinline__ void walk_gather(const WalkGather &G, int nblk, int blk, int *list, int *cnt) {
   const int o = G.d.o, v = G.d.v, vp = G.d.vp, up = G.d.up;
-  const int xy = blockIdx.x / nblk, x = xy / o, y = xy - x * o;
+  const int xy = blk / nblk, x = xy / o, y = xy - x * o;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // slots that write to (x, y), with the mask of their pieces
   int mask = 0;
@@ -815,11 +857,11 @@ __global__ __launch_bounds__(256) void k_walk_gather(WalkGather G, int nblk) {
   }
   if (mask) list[at + __popcll(m & ((1ULL << lane) - 1))] = threadIdx.x | (mask << 16);
   __syncthreads();
-  const int t = (blockIdx.x - xy * nblk) * 256 + threadIdx.x;
+  const int t = (blk - xy * nblk) * 256 + threadIdx.x;
   if (t >= vp * up) return;
   const int p = t / up, k = t - p * up;
   if (p >= v || k >= v + o) return;
-  const size_t vv = (size_t)vp * vp, blk = (size_t)vp * up;
+  const size_t vv = (size_t)vp * vp, slab = (size_t)vp * up;
   const size_t pq = (size_t)p * vp + k, qp = (size_t)k * vp + p;
   double s = 0.0, r = 0.0;
   for (int e = 0; e < n; ++e) {
@@ -827,8 +869,8 @@ __global__ __launch_bounds__(256) void k_walk_gather(WalkGather G, int nblk) {
     const double *R = G.R + b * G.r_stride;
     for (int pr = 0; pr < 6; ++pr) {
       if (!((mk >> pr) & 1)) continue;
-      const double *q = G.part + ((size_t)b * 6 + pr) * G.S * blk + t;
-      for (int sp = 0; sp < G.S; ++sp) s += q[sp * blk];
+      const double *q = G.part + ((size_t)b * 6 + pr) * G.S * slab + t;
+      for (int sp = 0; sp < G.S; ++sp) s += q[sp * slab];
       if (k < v) {
         // R5, R5, R3, R3, R1, R1 over (b,c), (a,c), (a,b), transposed for even pieces
         const size_t at_ = (pr & 1) ? pq : qp;
@@ -849,16 +891,21 @@ __global__ __launch_bounds__(256) void k_walk_gather(WalkGather G, int nblk) {
   }
 }
 
-// tri_e of every triple of the batch, one wave each
+// tri_e of the triple in slot b, by one wave
+__device__ __forceinline__ void walk_energy(const int *tri, int o, const double *part_t, int G, double *tri_e,
+                                            int b) {
+  const int lane = threadIdx.x & 63;
+  const double *p = part_t + (size_t)b * G;
+  double s = 0.0;
+  for (int r = lane; r < G; r += 64) s += p[r];
+  s = vr_wave_sum(s);
+  const int w = tri[b];
+  if (lane == 0) tri_e[((size_t)(w & 1023) * o + ((w >> 10) & 1023)) * o + (w >> 20)] = s;
+}
+
 __global__ __launch_bounds__(64) void k_walk_energies(const int *tri, int o, const double *part_t, int G,
                                                       double *tri_e) {
-  const double *p = part_t + (size_t)blockIdx.x * G;
-  double s = 0.0;
-  for (int r = threadIdx.x; r < G; r += 64) s += p[r];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  const int w = tri[blockIdx.x];
-  if (threadIdx.x == 0) tri_e[((size_t)(w & 1023) * o + ((w >> 10) & 1023)) * o + (w >> 20)] = s;
+  walk_energy(tri, o, part_t, G, tri_e, blockIdx.x);
 }
 
 hipError_t launch_walk_energies(const int *tri, int nb, int o, const double *part_t, int G, double *tri_e,
@@ -867,39 +914,44 @@ hipError_t launch_walk_energies(const int *tri, int nb, int o, const double *par
   return hipGetLastError();
 }
 
+// One launch: the column sums (ncol workgroups), the gather (o^2 nblk) and the
+// triple energies (four to a workgroup).
+__global__ __launch_bounds__(256) void k_walk_gather(WalkGather G, int ncol, int nblk) {
+  __shared__ double red[4][4][64];
+  __shared__ int list[kWalkMaxBatch];
+  __shared__ int cnt[4];
+  int blk = blockIdx.x;
+  if (blk < ncol) {
+    const int n = (G.d.vp + 63) / 64;
+    walk_cols(G.d.vp, G.R, G.r_stride, G.vec, blk % n, blk / n, red);
+    return;
+  }
+  blk -= ncol;
+  if (blk < nblk * G.d.o * G.d.o) {
+    walk_gather(G, nblk, blk, list, cnt);
+    return;
+  }
+  const int b = (blk - nblk * G.d.o * G.d.o) * 4 + (threadIdx.x >> 6);
+  if (b < G.nb) walk_energy(G.tri, G.d.o, G.part_t, G.G, G.tri_e, b);
+}
+
 hipError_t launch_walk_gather(const WalkGather &g, hipStream_t s) {
   const int v = g.d.vp, o = g.d.o;
   if (g.nb > kWalkMaxBatch) return hipErrorInvalidValue;
-  if (g.nb > 0) {
-    if (vr_col_blocks(v) > 1)
-      hipLaunchKernelGGL(k_walk_vrsum, dim3((v * v + 255) / 256, g.nb), dim3(256), 0, s, v,
+  if (g.nb > 0 && vr_col_blocks(v) > 1)
+    hipLaunchKernelGGL(k_walk_vrsum, dim3((v * v + 255) / 256, g.nb), dim3(256), 0, s, v,
                        const_cast<double *>(g.R), g.r_stride, g.has_fvo);
-    hipLaunchKernelGGL(k_walk_cols, dim3((v + 63) / 64, g.nb), dim3(256), 0, s, v, g.R, g.r_stride, g.vec);
-  }
+  const int ncol = (v + 63) / 64 * g.nb, nblk = (v * g.d.up + 255) / 256;
+  const long long total = ncol + (long long)nblk * o * o + (g.tri_e ? (g.nb + 3) / 4 : 0);
+  if (total >= (1LL << 31)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_walk_gather, dim3((unsigned)total), dim3(256), 0, s, g, ncol, nblk);
   hipLaunchKernelGGL(k_walk_t1, dim3((g.d.v + 63) / 64, o), dim3(256), 0, s, g);
-  const int nblk = (v * g.d.up + 255) / 256;
-  hipLaunchKernelGGL(k_walk_gather, dim3((unsigned)(nblk * o * o)), dim3(256), 0, s, g, nblk);
-  if (!g.tri_e) return hipGetLastError();
-  return launch_walk_energies(g.tri, g.nb, o, g.part_t, g.G, g.tri_e, s);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
 // projected walk
 // ---------------------------------------------------------------------------
-__global__ void k_walk_pairs(int o, int *tri) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= o * o) return;
-  const int j = t / o, k = t % o;
-  if (k < j) return;
-  int *p = tri + (size_t)(j * o - j * (j - 1) / 2 + k - j) * o;
-  for (int l = 0; l < o; ++l) p[l] = l | (j << 10) | (k << 20);
-}
-
-hipError_t launch_walk_pairs(int o, int *tri, hipStream_t s) {
-  hipLaunchKernelGGL(k_walk_pairs, dim3((o * o + 255) / 256), dim3(256), 0, s, o, tri);
-  return hipGetLastError();
-}
-
 struct WalkUpload {
   double v[256];
 };
@@ -972,14 +1024,14 @@ hipError_t launch_walk_ulo(const double *part_u, int G, int nfrag, double ebar, 
 // ---------------------------------------------------------------------------
 // ovvv_bar[x,p,f,q] = VTb[x][p][q][f], or packed g[f,q] + g[q,f] (q < f), g[f,f]:
 // a 32 x 32 tile (f, q) of one (x, p) per workgroup, turned in LDS
-__global__ __launch_bounds__(256) void k_walk_fold(WalkDims d, const double *__restrict__ VTb, int packed,
-                                                   double *__restrict__ out) {
-  __shared__ double tile[32][33];
-  const int f0 = blockIdx.x * 32, q0 = blockIdx.y * 32, v = d.v, vp = d.vp, up = d.up;
+__device__ __forceinline__ void fold_ovvv(const WalkDims &d, const double *__restrict__ VTb, int packed,
+                                          double *__restrict__ out, int bf, int bq, int bz, int nz,
+                                          double (*tile)[33]) {
+  const int f0 = bf * 32, q0 = bq * 32, v = d.v, vp = d.vp, up = d.up;
   if (packed && q0 > f0) return;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const size_t npair = (size_t)v * (v + 1) / 2;
-  for (int xp = blockIdx.z; xp < d.o * v; xp += gridDim.z) {
+  for (int xp = bz; xp < d.o * v; xp += nz) {
     const double *g = VTb + ((size_t)(xp / v) * vp + xp % v) * d.sp;
     for (int r = ty; r < 32; r += 8) {
       const int q = q0 + r, f = f0 + tx;
@@ -999,12 +1051,12 @@ __global__ __launch_bounds__(256) void k_walk_fold(WalkDims d, const double *__r
 }
 
 // t2_bar[x,m,p,q] += VTb[x][p][q][v + m], one (x, p) and 32 (m, q) per workgroup
-__global__ __launch_bounds__(256) void k_walk_fold_t2(WalkDims d, const double *__restrict__ VTb,
-                                                      double *__restrict__ t2_bar) {
-  __shared__ double tile[32][33];
-  const int q0 = blockIdx.x * 32, m0 = blockIdx.y * 32, o = d.o, v = d.v, vp = d.vp, up = d.up;
+__device__ __forceinline__ void fold_t2(const WalkDims &d, const double *__restrict__ VTb,
+                                        double *__restrict__ t2_bar, int bq, int bm, int bz, int nz,
+                                        double (*tile)[33]) {
+  const int q0 = bq * 32, m0 = bm * 32, o = d.o, v = d.v, vp = d.vp, up = d.up;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  for (int xp = blockIdx.z; xp < o * v; xp += gridDim.z) {
+  for (int xp = bz; xp < o * v; xp += nz) {
     const int x = xp / v, p = xp - x * v;
     const double *g = VTb + ((size_t)x * vp + p) * d.sp + v;
     for (int r = ty; r < 32; r += 8)
@@ -1018,24 +1070,49 @@ __global__ __launch_bounds__(256) void k_walk_fold_t2(WalkDims d, const double *
 }
 
 // column sums of part_mo: kWalkMoParts row ranges, then those in order
-__global__ void k_walk_mo(const double *part, int rows, int cols, double *part2) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void fold_mo(const double *part, int rows, int cols, double *part2, int c, int y) {
   if (c >= cols) return;
   const int per = (rows + kWalkMoParts - 1) / kWalkMoParts;
   double s = 0.0;
-  for (int r = blockIdx.y * per; r < min(rows, (int)(blockIdx.y + 1) * per); ++r) s += part[(size_t)r * cols + c];
-  part2[(size_t)blockIdx.y * cols + c] = s;
+  for (int r = y * per; r < min(rows, (y + 1) * per); ++r) s += part[(size_t)r * cols + c];
+  part2[(size_t)y * cols + c] = s;
+}
+
+// the three in one launch: n0 workgroups of fold_ovvv, n1 of fold_t2, then fold_mo
+__global__ __launch_bounds__(256) void k_walk_finish(WalkDims d, const double *__restrict__ VTb, int packed,
+                                                     double *__restrict__ ovvv_bar, double *__restrict__ t2_bar,
+                                                     const double *part_mo, int rows, double *part2, unsigned n0,
+                                                     unsigned n1, int nz) {
+  __shared__ double tile[32][33];
+  const unsigned nt = (d.v + 31) / 32, nm = (d.o + 31) / 32;
+  unsigned blk = blockIdx.x;
+  if (blk < n0) {
+    const unsigned r = blk / nt;
+    fold_ovvv(d, VTb, packed, ovvv_bar, (int)(blk - r * nt), (int)(r % nt), (int)(r / nt), nz, tile);
+    return;
+  }
+  blk -= n0;
+  if (blk < n1) {
+    const unsigned r = blk / nt;
+    fold_t2(d, VTb, t2_bar, (int)(blk - r * nt), (int)(r % nm), (int)(r / nm), nz, tile);
+    return;
+  }
+  blk -= n1;
+  const int cols = d.o + d.vp, nc = (cols + 63) / 64;
+  fold_mo(part_mo, rows, cols, part2, (int)(blk % nc) * 64 + (threadIdx.x & 63),
+          (int)(blk / nc) * 4 + (threadIdx.x >> 6));
 }
 
 hipError_t launch_walk_finish(const WalkDims &d, const double *VTb, int packed, double *ovvv_bar,
                               double *t2_bar, const double *part_mo, int rows, double *part2,
                               double *mo_bar, hipStream_t s) {
-  const int nt = (d.v + 31) / 32;
+  const unsigned nt = (d.v + 31) / 32, nm = (d.o + 31) / 32;
   const unsigned nz = (unsigned)std::min(d.o * d.v, 65535);
-  hipLaunchKernelGGL(k_walk_fold, dim3(nt, nt, nz), dim3(256), 0, s, d, VTb, packed, ovvv_bar);
-  hipLaunchKernelGGL(k_walk_fold_t2, dim3(nt, (d.o + 31) / 32, nz), dim3(256), 0, s, d, VTb, t2_bar);
-  hipLaunchKernelGGL(k_walk_mo, dim3((d.o + d.vp + 63) / 64, kWalkMoParts), dim3(64), 0, s, part_mo, rows,
-                     d.o + d.vp, part2);
+  static_assert(kWalkMoParts % 4 == 0, "four row ranges per workgroup");
+  const unsigned n0 = nt * nt * nz, n1 = nt * nm * nz, n2 = (d.o + d.vp + 63) / 64 * (kWalkMoParts / 4);
+  if ((long long)nt * (nt + nm) * nz + n2 >= (1LL << 31)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_walk_finish, dim3(n0 + n1 + n2), dim3(256), 0, s, d, VTb, packed, ovvv_bar, t2_bar, part_mo,
+                     rows, part2, n0, n1, (int)nz);
   return launch_reduce_rows(part2, kWalkMoParts, d.o + d.v, d.o + d.vp, mo_bar, 0, s);
 }
 
