@@ -55,7 +55,9 @@ class Inputs:
         self.ovvv = _dev(ovvv, self.device)
         self.ovoo = _dev(ovoo, self.device)
         self.ovov = _dev(ovov, self.device)
-        self.fvo = _dev(fvo, self.device)
+        # (a zero fvo, the canonical reference, is looked at where it lies and not copied)
+        self.fvo = fvo if fvo is None or isinstance(fvo, torch.Tensor) else \
+            torch.from_numpy(np.ascontiguousarray(np.asarray(fvo, dtype=np.float64)))
         o, v = self.nocc, self.nvir
         self.packed = self.ovvv.dim() == 3
         expect = {
@@ -70,9 +72,8 @@ class Inputs:
         for name, (t, shape) in expect.items():
             if tuple(t.shape) != shape:
                 raise ValueError(f'{name} has shape {tuple(t.shape)}, expected {shape}')
-        self.has_fvo = self.fvo is not None and bool(torch.count_nonzero(self.fvo).item() > 0)
-        if not self.has_fvo:
-            self.fvo = None
+        self.has_fvo = self.fvo is not None and bool(self.fvo.detach().any().item())
+        self.fvo = _dev(self.fvo, self.device) if self.has_fvo else None
         self.precision = precision
         self.cfg = _lib.make_config(o, v, self.packed, self.has_fvo, precision)
 
@@ -95,7 +96,7 @@ def energy(inp: Inputs):
     """E(T) as a 0-d float64 device tensor."""
     lib = _lib.load()
     ws, nbytes = inp.workspace(False)
-    e = torch.zeros((), dtype=torch.float64, device=inp.device)
+    e = torch.empty((), dtype=torch.float64, device=inp.device)
     st = lib.pamd_ccsdt_energy(ctypes.byref(inp.cfg), *inp.args(), _ptr(ws), nbytes, _ptr(e),
                                _stream(inp.device))
     _lib.check(st, 'pamd_ccsdt_energy')
@@ -151,7 +152,7 @@ def energy_vjp(inp: Inputs, et_bar=1.0, workspace=None):
     reused across calls."""
     lib = _lib.load()
     ws, nbytes = workspace if workspace is not None else inp.workspace(True)
-    e = torch.zeros((), dtype=torch.float64, device=inp.device)
+    e = torch.empty((), dtype=torch.float64, device=inp.device)
     out = _cotangent_outputs(inp)
     st = lib.pamd_ccsdt_energy_vjp(
         ctypes.byref(inp.cfg), *inp.args(), ctypes.c_double(float(et_bar)), _ptr(ws), nbytes,
