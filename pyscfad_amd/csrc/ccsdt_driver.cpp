@@ -472,8 +472,7 @@ static int build_w(const Ctx &c, int i, int j, int k, int nb = 1) {
   auto OOt = [&](int x, int y) { return c.OOt + (x * o + y) * vo; };
   const int V = c.vp, O = c.op;
   const bool whole = c.v % 8 == 0 && c.o % 8 == 0;
-  // (an energy takes the direct engine wherever it can: only FP32 roundings differ)
-  const int sumsC = c.vjp ? b3_sums(c, c.v * c.v, c.v, whole) : 0, sumsR = c.vjp ? b3_sums(c, c.v, c.v * c.v, whole) : 0;
+  const int sumsC = b3_sums(c, c.v * c.v, c.v, whole), sumsR = b3_sums(c, c.v, c.v * c.v, whole);
   // the ovvv slab of a particle term with its row pair (q, s) read as
   // Vp(x)[q][s][f] ("qs") or Vp(x)[s][q][f] ("sq"), K = f: from Vp itself
   // (K-contiguous), or, when the call holds the transposed copies, from
