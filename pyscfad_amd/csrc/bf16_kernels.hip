@@ -696,6 +696,8 @@ hipError_t launch_gemm_b3(const GemmDesc &d0, hipStream_t s, const GemmBatch &bt
   for (int q = d.nseg + 1; q <= kMaxSeg; ++q) d.chunk_start[q] = d.chunk_start[d.nseg];
   if (gemm_b3p_enabled() && d.sums != kSumsFlushed && gemm_b3p_ok(d, bt)) return launch_gemm_b3p(d, s, bt);
   const int c = b3_pick(d.M, d.N, d.sums);
+  if (c >= kB3Wide && d.N <= 32 && d.M >= d.N && gemm_b3p_enabled() && gemm_b3p_ok(d, bt))
+    return launch_gemm_b3p_narrow(d, s, bt);
   if (c >= kB3Wide && d.mode == kPartialF32) return hipErrorInvalidValue;
   const int MT = kB3Shape[c][0], NT = kB3Shape[c][1];
   const unsigned grid =

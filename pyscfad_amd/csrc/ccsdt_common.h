@@ -165,11 +165,11 @@ struct VRArgs {
 struct CombineArgs {
   const double *R;                // VR scratch
   double *part_p;                 // [6][S][v][v] particle t2_bar partials (reduced in place)
-  double *part_h;                 // [6][S][v][o] hole ovoo_bar partials (reduced in place)
+  double *part_h;                 // [6][S][v][op] hole ovoo_bar partials (reduced in place)
   int S_p, S_h;
   int f32_p, f32_h;               // parts are FP32 (kPartialF32)
   int o, v, i, j, k, has_fvo;     // v: extent of the outputs and partials
-  int vp;                         // extent that R is laid out with
+  int vp, op;                     // extents that R and part_h ([6][S][v][op]) are laid out with
   double *t2_bar, *ovov_bar, *ovoo_bar, *t1_bar, *fvo_bar;
   // when part_t is set: *tri_dst = sum of the orbit epilogue's G per-workgroup
   // energy sums (fixed order), in the same launch
@@ -208,6 +208,7 @@ B3Sums gemm_b3_sums(int M, int N);  // of the register-staged engine
 bool gemm_b3p_enabled();  // env PYSCFAD_AMD_B3_DIRECT=0 turns it off
 int gemm_b3p_tiles(int M, int N);  // workgroup tiles of one split
 hipError_t launch_gemm_b3p(const GemmDesc &d, hipStream_t s, const GemmBatch &bt = no_batch());
+hipError_t launch_gemm_b3p_narrow(const GemmDesc &d, hipStream_t s, const GemmBatch &bt);
 // n independent products in one launch of the direct engine (chunk_start in
 // stages of 32), when gemm_b3p_group_ok (see gemm_b3p.hip)
 bool gemm_b3p_group_ok(const GemmDesc *ds, int n);

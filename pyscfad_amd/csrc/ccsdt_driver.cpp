@@ -283,7 +283,7 @@ static Layout make_layout(int o, int v, int vjp, int prec, bool pipe = false, bo
     L.off_part_mo = take((size_t)kGmax * n);
     L.off_R = take(vr_scratch_doubles(L.vp));
     L.off_part_p = take((size_t)6 * L.S_p * vv);
-    L.off_part_h = take((size_t)6 * L.S_h * v * o);
+    L.off_part_h = take((size_t)6 * L.S_h * v * L.op);
   }
   L.vpt = vpt_fits(o, L.op, L.vp, prec) ? 1 : 0;
   if (L.vpt) {
@@ -296,7 +296,7 @@ static Layout make_layout(int o, int v, int vjp, int prec, bool pipe = false, bo
     if (prec == PAMD_PREC_BF16X3 || prec == PAMD_PREC_FP32X2) L.off_W8b = take(v3);
     L.off_R2 = take(vr_scratch_doubles(L.vp));
     L.off_part_p2 = take((size_t)6 * L.S_p * vv);
-    L.off_part_h2 = take((size_t)6 * L.S_h * v * o);
+    L.off_part_h2 = take((size_t)6 * L.S_h * v * L.op);
   }
   L.total = off;
   return L;
@@ -657,31 +657,32 @@ static int adjoint_gemms(const Ctx &c, int i, int j, int k, int pair = 0, const 
     PAMD_CHECK(run_gemm_group(c, ds, 6, kProfAdjT2P, true));
   }
   // hole ovoo_bar pieces: split-K over the virtual pair
-  const size_t ph = (size_t)c.S_h * V0 * O0;
+  const int N = c.pad ? c.op : O0;  // (padded: direct loads of T2m's rows)
+  const int sums_o = b3_sums(c, V0, O0, V0 % 8 == 0 && O0 % 8 == 0);
+  const size_t ph = (size_t)c.S_h * V0 * N;
   {
     const int mode_h = c.f32_h ? kPartialF32 : kPartial;
     GemmDesc ds[6] = {
         // H1: ovoo_bar[i,a,m,j] = -sum_(b,c) Wb[a,b,c] T2m(k)[c][b][m]
-        gemm(V0, O0, mode_h, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, N, mode_h, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 0 * ph),
         // H2: ovoo_bar[i,a,m,k] = -sum_(b,c) Wb[a,b,c] T2m(j)[b][c][m]
-        gemm(V0, O0, mode_h, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(j), 1, vo, os, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, N, mode_h, {seg(opK(Wb, v2, v, 1, V0, 0), opK(T2m(j), 1, vo, os, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 1 * ph),
         // H3: ovoo_bar[j,b,m,i] = -sum_(a,c) Wb[a,b,c] T2m(k)[c][a][m]
-        gemm(V0, O0, mode_h, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, N, mode_h, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(k), 1, os, vo, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 2 * ph),
         // H4: ovoo_bar[j,b,m,k] = -sum_(a,c) Wb[a,b,c] T2m(i)[a][c][m]
-        gemm(V0, O0, mode_h, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, N, mode_h, {seg(opK(Wb, v, v2, 1, V0, 0), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 3 * ph),
         // H5: ovoo_bar[k,c,m,i] = -sum_(a,b) Wb[a,b,c] T2m(j)[b][a][m]
-        gemm(V0, O0, mode_h, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(j), 1, os, vo, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, N, mode_h, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(j), 1, os, vo, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 4 * ph),
         // H6: ovoo_bar[k,c,m,j] = -sum_(a,b) Wb[a,b,c] T2m(i)[a][b][m]
-        gemm(V0, O0, mode_h, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
+        gemm(V0, N, mode_h, {seg(opK(Wb, 1, v2, v, V0, 1), opK(T2m(i), 1, vo, os, V0, 1), V0 * V0, -1.0)},
              out(nullptr, 0, 0, 1, 0, 0, 1), c.S_h, c.part_h + 5 * ph),
     };
-    if (c.f32_h)
-      for (GemmDesc &d : ds) d.sums = kSumsWhole;
+    for (GemmDesc &d : ds) d.sums = c.f32_h ? (int)kSumsWhole : sums_o;
     PAMD_CHECK(run_gemm_group(c, ds, 6, kProfAdjOvoo, true));
   }
   // hole-term t2 reads: T2mb[x][p][q][m] (= dE/d t2[x,m,p,q])
@@ -751,6 +752,7 @@ static int adjoint_combine(const Ctx &c, int i, int j, int k, hipStream_t st,
   ca.o = c.o;
   ca.v = c.v;
   ca.vp = c.vp;
+  ca.op = c.op;
   ca.i = i;
   ca.j = j;
   ca.k = k;
@@ -764,7 +766,7 @@ static int adjoint_combine(const Ctx &c, int i, int j, int k, hipStream_t st,
   ca.G = c.G;
   ca.tri_dst = with_energy ? c.tri + ((size_t)i * c.o + j) * c.o + k : nullptr;
   if (!g_record) {
-    const double cb = 8.0 * (6.0 * c.S_p * v2 + 6.0 * c.S_h * v * o + 12.0 * v2);
+    const double cb = 8.0 * (6.0 * c.S_p * v2 + 6.0 * c.S_h * v * c.op + 12.0 * v2);
     PAMD_CHECK(timed(st, kProfCombine, 0.0, cb, [&] { return launch_combine(ca, st); }));
   }
   return PAMD_OK;

@@ -1223,12 +1223,12 @@ __device__ __forceinline__ void combine_block(const CombineArgs &A, size_t t) {
     const int p = (int)(t / o), m = (int)(t % o);
     const int xs[6] = {i, i, j, j, k, k};
     const int ys[6] = {j, k, i, k, i, j};
-    const size_t vo = (size_t)v * o;
+    const size_t vo = (size_t)v * A.op, at = (size_t)p * A.op + m;
     double s[6], old[6];
     bool own[6];
 #pragma unroll
     for (int pr = 0; pr < 6; ++pr)
-      s[pr] = A.part_h[(size_t)pr * A.S_h * vo + part_sum_at(A.S_h, vo, A.f32_h) + t];
+      s[pr] = A.part_h[(size_t)pr * A.S_h * vo + part_sum_at(A.S_h, vo, A.f32_h) + at];
     merge_slabs(xs, ys, s, own);
     auto hb = [&](int u) { return A.ovoo_bar + (((size_t)xs[u] * v + p) * o + m) * o + ys[u]; };
 #pragma unroll
@@ -1306,7 +1306,7 @@ __global__ __launch_bounds__(256) void k_gather(CombineArgs A, int nc) {
 
 hipError_t launch_combine(const CombineArgs &a, hipStream_t s) {
   {
-    const size_t Tp = (size_t)a.v * a.v, Th = (size_t)a.v * a.o;
+    const size_t Tp = (size_t)a.v * a.v, Th = (size_t)a.v * a.op;
     hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned)((std::max(Tp, Th) + 63) / 64), 12), dim3(256), 0, s,
                        a.part_p, a.S_p, Tp, a.f32_p, a.part_h, a.S_h, Th, a.f32_h);
   }

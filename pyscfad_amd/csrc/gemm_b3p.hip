@@ -58,6 +58,7 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
@@ -251,6 +252,25 @@ __device__ __forceinline__ void frags(const bf16_t *T, int rc, int r16, int lane
   }
 }
 
+// the same for v_mfma_f32_32x32x16_bf16: rows r32 .. r32 + 31 (lane % 32), k
+// 16 step + 8 (lane / 32) .. + 7
+template <int R>
+__device__ __forceinline__ u32x4 frag32(const bf16_t *P, int rc, int r32, int step, int lane) {
+  if (!rc) {
+    const int r = r32 + (lane & 31);
+    return *(const u32x4 *)(P + r * kPK + 8 * ((2 * step + (lane >> 5)) ^ ksw(r)));
+  }
+  const int i = lane & 15, e = i >> 2, rr = r32 + 16 * ((lane >> 4) & 1) + 4 * (i & 3);
+  const int c = rr >> 3, half = rr & 7;
+  const int k0 = 16 * step + 8 * (lane >> 5) + e, k1 = k0 + 4;
+  const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (lds_v4i16 *)(P + k0 * R + 8 * (c ^ rsw<R>(k0)) + half));
+  const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (lds_v4i16 *)(P + k1 * R + 8 * (c ^ rsw<R>(k1)) + half));
+  const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+  return u32x4{l2[0], l2[1], h2[0], h2[1]};
+}
+
 // WM x WN waves; two workgroups per CU (80 KB of LDS each at most), one of twelve
 // waves
 // LDS of one workgroup (bf16 elements): two stages of the A and B tiles
@@ -264,7 +284,10 @@ struct B3pLds {
 
 // One workgroup's tile of one product: workgroup number `logical` of the
 // product's (or the batch's) grid.  D is GemmDesc or GemmDescS (same fields).
-template <int MT, int NT, int WM, int WN, class D>
+// FLUSH: sums as the register-staged engine's 32x32-MFMA tiles form them (FP32 over
+// four stages, those added up in FP64), for narrow products: one 32 x 32 tile per
+// wave.
+template <int MT, int NT, int WM, int WN, bool FLUSH, class D>
 __device__ __forceinline__ void b3p_tile(const D &d, const GemmBatch &bt, int n_fast, int logical,
                                          bf16_t *S) {
   constexpr int T = 64 * WM * WN;
@@ -290,10 +313,30 @@ __device__ __forceinline__ void b3p_tile(const D &d, const GemmBatch &bt, int n_
   const int g1 = min(total, g0 + cps);
 
   f32x4 acc[TM][TN];
+  f32x16 f32s;
+  double sum[FLUSH ? 16 : 1];
+  int nfl = 0;
+  if constexpr (FLUSH) {
+    static_assert(WTM == 32 && WTN == 32, "one 32x32 MFMA tile per wave");
 #pragma unroll
-  for (int a = 0; a < TM; ++a)
+    for (int r = 0; r < 16; ++r) {
+      f32s[r] = 0.f;
+      sum[r] = 0.0;
+    }
+  } else {
 #pragma unroll
-    for (int b = 0; b < TN; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+      for (int b = 0; b < TN; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  auto flush = [&]() {
+#pragma unroll
+    for (int r = 0; r < (FLUSH ? 16 : 0); ++r) {
+      sum[r] += (double)f32s[r];
+      f32s[r] = 0.f;
+    }
+    nfl = 0;
+  };
 
   // fetch tracker: segment, stage start and K position of the next stage to load
   int fs = 0;
@@ -391,7 +434,33 @@ __device__ __forceinline__ void b3p_tile(const D &d, const GemmBatch &bt, int n_
     // the fragments of the narrower side stay in registers; the other side is
     // read two tiles at a time, and the six products of those two tiles
     // alternate between their accumulators
-    if constexpr (TM <= TN) {
+    if constexpr (FLUSH) {
+#pragma unroll
+      for (int step = 0; step < 2; ++step) {
+        u32x4 a[3], b[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          a[q] = frag32<MT>(As + q * MT * kPK, la, wm * 32, step, lane);
+          b[q] = frag32<NT>(Bs + q * NT * kPK, lb, wn * 32, step, lane);
+        }
+        if (fix) {
+          u32x4 m;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const int k = 16 * step + 8 * (lane >> 5) + 2 * w;
+            m[w] = (k < kv ? 0xffffu : 0u) | (k + 1 < kv ? 0xffff0000u : 0u);
+          }
+#pragma unroll
+          for (int q = 0; q < 3; ++q) a[q] = (a[q] ^ sgn) & m;
+        }
+        constexpr int pa_[6] = {1, 0, 2, 0, 1, 0}, pb_[6] = {1, 2, 0, 1, 0, 0};  // smallest terms first
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+          f32s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[pa_[q]]),
+                                                         __builtin_bit_cast(bf16x8, b[pb_[q]]), f32s, 0, 0, 0);
+      }
+      if (++nfl == 4) flush();
+    } else if constexpr (TM <= TN) {
       u32x4 ah[TM], am[TM], al[TM];
 #pragma unroll
       for (int t = 0; t < TM; ++t) {
@@ -465,6 +534,29 @@ __device__ __forceinline__ void b3p_tile(const D &d, const GemmBatch &bt, int n_
     }
   }
 
+  if constexpr (FLUSH) {
+    flush();
+    // D layout of v_mfma_f32_32x32x16_bf16: lane l, element r -> row 8 (r / 4) + 4 (l / 32) + r % 4,
+    // column l % 32
+    const OutPos pn = out_pos<NT>(tn, wn * 32 + (lane & 31), d.mode == kPartial ? (1 << 30) : d.C.ndiv);
+    if (pn.idx >= d.N) return;
+    double old[16], *cp[16];
+    bool ok[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const OutPos pm = out_pos<MT>(tm, wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3),
+                                    d.mode == kPartial ? (1 << 30) : d.C.mdiv);
+      ok[r] = pm.idx < d.M;
+      cp[r] = d.mode == kPartial ? d.partial + ((size_t)split * d.M + pm.idx) * d.N + pn.idx
+                                 : d.C.p + batch * bt.c + (long long)pm.q * d.C.mx + (long long)pm.r * d.C.my +
+                                       (long long)pn.q * d.C.nx + (long long)pn.r * d.C.ny;
+      old[r] = d.mode == kAccumulate && ok[r] ? *cp[r] : 0.0;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (ok[r]) *cp[r] = d.mode == kAccumulate ? old[r] + sum[r] : sum[r];
+    return;
+  }
   // D layout of v_mfma_f32_16x16x32_bf16: lane l, element r -> row 4 (l / 16) + r, column l % 16
   if (d.mode >= kPartial) {
     const size_t part = (size_t)split * d.M * d.N;
@@ -526,7 +618,13 @@ __device__ __forceinline__ void b3p_tile(const D &d, const GemmBatch &bt, int n_
 template <int MT, int NT, int WM, int WN, int MINW>
 __global__ __launch_bounds__(64 * WM * WN, MINW) void k_gemm_b3p(GemmDesc d, GemmBatch bt, int n_fast) {
   __shared__ __align__(16) bf16_t S[B3pLds<MT, NT, WM, WN>::N];
-  b3p_tile<MT, NT, WM, WN>(d, bt, n_fast, xcd_remap(blockIdx.x, gridDim.x), S);
+  b3p_tile<MT, NT, WM, WN, false>(d, bt, n_fast, xcd_remap(blockIdx.x, gridDim.x), S);
+}
+
+// narrow products (N <= 32) of the flushed sums
+__global__ __launch_bounds__(256, 2) void k_gemm_b3p_narrow(GemmDesc d, GemmBatch bt) {
+  __shared__ __align__(16) bf16_t S[B3pLds<128, 32, 4, 1>::N];
+  b3p_tile<128, 32, 4, 1, true>(d, bt, 1, xcd_remap(blockIdx.x, gridDim.x), S);
 }
 
 // A group of up to kMaxGroup independent products with equal M, N, split-K
@@ -542,7 +640,7 @@ __global__ __launch_bounds__(64 * WM * WN, MINW) void k_gemm_b3p_group(GemmGroup
   for (int q = 0; q < kMaxSeg; ++q) bt.a[q] = bt.bo[q] = 0;
   bt.c = 0;
   bt.nb = 1;
-  b3p_tile<MT, NT, WM, WN>(g.d[p], bt, n_fast, logical - p * per, S);
+  b3p_tile<MT, NT, WM, WN, false>(g.d[p], bt, n_fast, logical - p * per, S);
 }
 
 // An operand can be staged with 16-byte direct loads of 8 bf16 along its fast
@@ -708,6 +806,15 @@ hipError_t launch_gemm_b3p_group(const GemmDesc *ds, int n, hipStream_t s) {
     case 6: hipLaunchKernelGGL((k_gemm_b3p_group<128, 240, 4, 3, 3>), dim3(grid), dim3(768), 0, s, g, n_fast); break;
     default: hipLaunchKernelGGL((k_gemm_b3p_group<240, 128, 3, 4, 3>), dim3(grid), dim3(768), 0, s, g, n_fast); break;
   }
+  return hipGetLastError();
+}
+
+// Flushed sums on direct loads: N <= 32, where the register-staged engine's 256 x 64
+// tile pads N and stages with one workgroup per CU.  Measured, M = 400, N = 6,
+// K = 400^2: 301 -> 131 us (87 us of reading Wbar).
+hipError_t launch_gemm_b3p_narrow(const GemmDesc &d, hipStream_t s, const GemmBatch &bt) {
+  const unsigned grid = (unsigned)((long long)((d.M + 127) / 128) * d.splits * bt.nb);
+  hipLaunchKernelGGL(k_gemm_b3p_narrow, dim3(grid), dim3(256), 0, s, d, bt);
   return hipGetLastError();
 }
 
