@@ -1,14 +1,14 @@
 // Kernels of the batched FP64 walk (walk64.h).
 //
 // Measured on one MI355X against the one-triple walk (25 launches and two
-// streams per triple): E(T) + VJP o4/v16 4.5 -> 0.45 ms, o8/v40 40.4 -> 1.35 ms,
-// o11/v77 160 -> 20.4 ms, o16/v160 1123 -> 537 ms; pair energies o16/v160 189 ->
-// 132 ms.  Small sizes were bound by launches, odd ones by the register-staged
-// engine, o16/v160 by short contractions (K = v) on padded tiles.  At o16/v160
-// the contractions now run at 57-62 TFLOP/s of their unpadded work (a large
-// rocBLAS product: 72.6; the FP64 MFMA rate at the clock it holds there, 2.2 GHz:
-// 72), W build 5 x 2 tiles, VT's adjoint 5 x 3 and TB's 5 x 4 (11 column tiles
-// padded to 12).
+// streams per triple): E(T) + VJP o4/v16 4.5 -> 0.35 ms, o8/v40 40.4 -> 1.19 ms,
+// o11/v77 160 -> 16.0 ms, o16/v160 1123 -> 490 ms; energy o5/v19 1.34 -> 0.096 ms;
+// pair energies o16/v160 189 -> 118 ms.  Small sizes were bound by launches, odd
+// ones by the register-staged engine, o16/v160 by short contractions (K = v) on
+// padded tiles.  At o16/v160 the contractions now run at 61-64 TFLOP/s of their
+// unpadded work (a large rocBLAS product: 72.6; the FP64 MFMA rate at the clock it
+// holds there, 2.2 GHz: 72), W build 5 x 2 tiles, VT's adjoint 5 x 3 and TB's 5 x 4
+// (11 column tiles padded to 12).
 #include <algorithm>
 #include "engine_staging.h"
 #include "vr_layout.h"
