@@ -110,7 +110,7 @@ def engine_roofline(prof, precision):
         # three fp32 MFMA products (hi*hi, hi*lo, lo*hi) per multiply-add
         kernel, mfma_factor, peak = 'k_gemm_f64 (FP32 hi/lo mode)', 3.0, PEAKS['fp32']
     else:
-        kernel, mfma_factor, peak = 'k_gemm_f64', 1.0, PEAKS['fp64']
+        kernel, mfma_factor, peak = 'k_walk_w, k_walk_vtb, k_walk_tbb (a batch of triples per launch)', 1.0, PEAKS['fp64']
     achieved = fp64_equiv * mfma_factor if fp64_equiv else None
     traffic, traffic_src = engine_traffic(precision)
     roofline = {'bound': 'mfma', 'achieved': achieved, 'peak': peak, 'unit': 'TFLOP/s',
@@ -126,13 +126,11 @@ def engine_roofline(prof, precision):
     return roofline
 
 
-# rocprofv3 FETCH_SIZE / WRITE_SIZE summaries of the engine launches: the
-# split-BF16x3 one at the default nocc=40 (its tile shapes for the occupied-side
-# contractions depend on nocc), the FP64 one at nocc=10 (the FP64 engine runs the
-# same two tile shapes at every size)
-TRAFFIC_FILES = {p: os.path.join(os.path.dirname(os.path.abspath(__file__)), 'profiles', f)
-                 for p, f in (('bf16x3', 'traffic_e_t_vjp_o40v400_bf16x3.json'),
-                              ('fp64', 'traffic_e_t_vjp_o10v400_fp64.json'))}
+# rocprofv3 FETCH_SIZE / WRITE_SIZE summary of the split-BF16x3 engine launches at
+# the default nocc=40 (its tile shapes for the occupied-side contractions depend
+# on nocc).  (The FP64 one in profiles/ is of the one-triple walk's engine.)
+TRAFFIC_FILES = {'bf16x3': os.path.join(os.path.dirname(os.path.abspath(__file__)), 'profiles',
+                                        'traffic_e_t_vjp_o40v400_bf16x3.json')}
 
 
 def engine_traffic(precision):
@@ -142,7 +140,7 @@ def engine_traffic(precision):
     path = TRAFFIC_FILES.get(precision)
     if path is None:
         return None, None
-    prefix = 'k_gemm_b3' if precision == 'bf16x3' else 'k_gemm_f64'
+    prefix = 'k_gemm_b3'
     if not os.path.exists(path):
         return None, None
     with open(path) as f:

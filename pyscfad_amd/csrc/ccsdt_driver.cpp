@@ -1641,8 +1641,7 @@ static int run_walk(Ctx &c, const WalkLayout &L, void *ws, double *ovvv_bar, dou
   const WalkBatches wb = walk_batches(n, L.nb);
   int st = walk_setup(c, L, b, &wb, tab, at(L.off_tri_e), (size_t)o * o * o, norb);
   if (st != PAMD_OK) return st;
-  if (c.wt_host)
-    PAMD_CHECK(hipMemcpyAsync(c.wt, c.wt_host, sizeof(double) * (size_t)o, hipMemcpyHostToDevice, s));
+  if (c.wt_host) PAMD_CHECK(launch_walk_upload(c.wt_host, o, c.wt, s));
   const double v3 = (double)c.v * c.v * c.v;
   WalkMeter meter(c.vjp ? "(T)+VJP" : "(T)", n);
   long long t0 = 0;
