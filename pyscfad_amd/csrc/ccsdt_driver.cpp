@@ -1672,7 +1672,7 @@ static int run_walk(Ctx &c, const WalkLayout &L, void *ws, double *ovvv_bar, dou
   return c.vjp ? walk_finish(c, L, b, ovvv_bar, mo_bar) : PAMD_OK;
 }
 
-// (o10/v64, two fragment orbitals, E + VJP: 335 -> 18.2 ms against the one-triple walk.)
+// (o10/v64, two fragment orbitals, E + VJP: 335 -> 17.6 ms against the one-triple walk.)
 // Batched projected walk: np pairs (j, k) at a time, the o triples (l, j, k) of
 // each in one batch, whose W blocks stay for the adjoint (the one-triple walk
 // builds every W twice).

@@ -493,8 +493,11 @@ __global__ __launch_bounds__(512, 2) void k_walk_acc(OrbitArgs A, int f0) {
 // Seeds of the projected energy, grid (G, triples (l, j, k)), from the pair's
 // finished sums: Q = g sum_f u_f A_f, Wbar = g sum_f u_f B_f + r3(Q) / D, Vbar =
 // r3(Q) / D, Dbar = -Q Z / D^2, and part_u[f] = <W, B_f> + <A_f, Z / D>.
+// Two waves per SIMD: at four the 128 registers spill 24 (o10/v64, two fragment
+// orbitals, 183 triples a launch: 877 us; 680 without spills; 819 with the next orbit's W in
+// flight as in k_walk_orbit).
 template <bool FVO>
-__global__ __launch_bounds__(512, 4) void k_walk_proj(OrbitArgs A) {
+__global__ __launch_bounds__(512, 2) void k_walk_proj(OrbitArgs A) {
   __shared__ double Ws[6][kT3];
   __shared__ double Vs[6][kT3];
   __shared__ StageLds<FVO> L;
