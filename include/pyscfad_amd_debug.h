@@ -30,6 +30,14 @@ int pamd_debug_paired_adjoint_descriptors(int nocc, int nvir, int i, int j, int 
                                           const unsigned long long *bases, void *out,
                                           int max_desc, int *n_desc, int *desc_bytes);
 
+/* Record the adjoint contractions of the triple (i, j, k), in any order of the
+ * occupied indices (the projected walk takes (l, j, k) with j <= k and any l),
+ * as the split-BF16x3 walks launch them: descriptors with the same launch[]
+ * number run concurrently, in one launch.  bases[10]: those of
+ * pamd_debug_gemm_descriptors; out and launch receive min(n, max_desc) entries. */
+int pamd_debug_adjoint_launches(int nocc, int nvir, int i, int j, int k, const unsigned long long *bases,
+                                void *out, int *launch, int max_desc, int *n_desc, int *desc_bytes);
+
 /* 1 when a recorded descriptor (one of pamd_debug_gemm_descriptors' outputs)
  * runs on the FP64 engine's direct-to-LDS path (16-byte element pairs: fast
  * strides 1, other strides and index divisors even, 16-byte aligned bases),

@@ -41,6 +41,8 @@ static const int kGmax = 1024;
 // kernels are skipped (host-only descriptor inspection, no GPU work).  Per host
 // thread, like every other piece of per-call state here.
 static thread_local std::vector<GemmDesc> *g_record = nullptr;
+// with it, when set: the launch that each recorded descriptor belongs to
+static thread_local std::vector<int> *g_record_launch = nullptr;
 
 // Sampled launch timing (pamd_profile_*): for one triple in g_prof_every, every
 // launch is bracketed by hipEvents on its own stream; the events are read after
@@ -372,6 +374,7 @@ static bool planarize(const PlanarMap &pm, OpDesc &o) {
 static hipError_t run_gemm(const Ctx &c, const GemmDesc &d0, int kind,
                            const GemmBatch &bt = no_batch()) {
   if (g_record) {
+    if (g_record_launch) g_record_launch->push_back((int)g_record->size());
     g_record->push_back(d0);
     return hipSuccess;
   }
@@ -410,11 +413,14 @@ constexpr double kGroupWbarBytes = 128.0 * (1 << 20);
 static hipError_t run_gemm_group(const Ctx &c, const GemmDesc *ds, int n, int kind,
                                  bool out_disjoint) {
   const int gm = group_mode();
-  const bool group = gm == 1 || (gm < 0 && 6.0 * c.v * (double)c.v * c.v <= kGroupWbarBytes);
-  if (g_record || c.prec != PAMD_PREC_BF16X3 || !out_disjoint || n > kMaxGroup || !group) {
+  const bool group = c.prec == PAMD_PREC_BF16X3 && out_disjoint && n <= kMaxGroup &&
+                     (gm == 1 || (gm < 0 && 6.0 * c.v * (double)c.v * c.v <= kGroupWbarBytes));
+  if (g_record || !group) {
+    const int first = g_record ? (int)g_record->size() : 0;
     for (int q = 0; q < n; ++q) {
       const hipError_t e = run_gemm(c, ds[q], kind);
       if (e != hipSuccess) return e;
+      if (g_record && g_record_launch && group) g_record_launch->back() = first;
     }
     return hipSuccess;
   }
@@ -577,8 +583,9 @@ static int adjoint_gemms(const Ctx &c, int i, int j, int k, int pair = 0, const 
   auto OOt = [&](int x, int y) { return c.OOt + (x * o + y) * vo; };
 
   // the three adjoints into Vpb[i], Vpb[j], Vpb[k] and into T2mb[i], T2mb[j],
-  // T2mb[k] write disjoint slabs unless two occupied indices coincide
-  const bool distinct = i != j && j != k;
+  // T2mb[k] write disjoint slabs unless two occupied indices coincide (any two: the
+  // projected walk's triples are not sorted, so i == k with another j occurs)
+  const bool distinct = i != j && j != k && i != k;
   // ovvv_bar, rows = virtual pairs, cols = f
   if (pair != 0) {
     const double *Wq = prev ? prev->gW : nullptr;
@@ -2208,6 +2215,44 @@ int pamd_debug_gemm_descriptors(int nocc, int nvir, int i, int j, int k, int wit
     const int n = std::min((int)rec.size(), max_desc);
     memcpy(out, rec.data(), sizeof(GemmDesc) * (size_t)n);
   }
+  return PAMD_OK;
+}
+
+int pamd_debug_adjoint_launches(int nocc, int nvir, int i, int j, int k, const unsigned long long *bases,
+                                void *out, int *launch, int max_desc, int *n_desc, int *desc_bytes) {
+  if (nocc < 1 || nvir < 1 || !bases || !out || !launch || !n_desc || !desc_bytes) return PAMD_ERR_ARG;
+  if (i < 0 || j < 0 || k < 0 || i >= nocc || j >= nocc || k >= nocc) return PAMD_ERR_ARG;
+  const Layout L = make_layout(nocc, nvir, 1, PAMD_PREC_BF16X3);
+  Ctx c;
+  memset(&c, 0, sizeof(c));
+  c.prec = PAMD_PREC_BF16X3;
+  c.o = c.op = nocc;
+  c.v = c.vp = nvir;
+  c.vjp = 1;
+  c.Vp = (double *)bases[0];
+  c.T2m = (double *)bases[1];
+  c.OOt = (double *)bases[2];
+  c.W = c.gW = (double *)bases[3];
+  c.t2 = c.gT2 = (const double *)bases[4];
+  c.Vpb = (double *)bases[6];
+  c.T2mb = (double *)bases[7];
+  c.part_p = (double *)bases[8];
+  c.part_h = (double *)bases[9];
+  c.S_p = L.S_p;
+  c.S_h = L.S_h;
+  std::vector<GemmDesc> rec;
+  std::vector<int> at;
+  g_record = &rec;
+  g_record_launch = &at;
+  const int st = adjoint_gemms(c, i, j, k);
+  g_record = nullptr;
+  g_record_launch = nullptr;
+  if (st != PAMD_OK) return st;
+  *desc_bytes = (int)sizeof(GemmDesc);
+  *n_desc = (int)rec.size();
+  const int n = std::min((int)rec.size(), max_desc);
+  memcpy(out, rec.data(), sizeof(GemmDesc) * (size_t)n);
+  memcpy(launch, at.data(), sizeof(int) * (size_t)n);
   return PAMD_OK;
 }
 
