@@ -52,6 +52,12 @@ typedef struct {
  * pamd_ccsdt_energy_vjp (with_vjp = 1).  Host-only call; no GPU work. */
 int pamd_ccsdt_workspace_size(const pamd_ccsdt_config *cfg, int with_vjp, size_t *bytes);
 
+/* The workspace these calls use when it is there, at least as large as the needed
+ * one: FP64 calls then work on many occupied triples per launch (some GB of
+ * blocks at nvir = 160), split-BF16x3 ones on operands padded to multiples of 8.
+ * A call takes any size in between and runs what fits.  Host-only call. */
+int pamd_ccsdt_preferred_workspace_size(const pamd_ccsdt_config *cfg, int with_vjp, size_t *bytes);
+
 /* E(T) -> *e_out (device, 1 double, overwritten).
  * Replaces the forward of the reference's (T) call: pyscf ccsd_t.kernel ->
  * libcc CCsd_t_contract at pyscfad/cc/ccsd_t.py:41, and its in-tree C sibling
@@ -182,9 +188,12 @@ int pamd_ccsdt_weighted_energy_vjp(const pamd_ccsdt_config *cfg,
  * (l, j, k): about three times the W builds of pamd_ccsdt_energy, and the
  * adjoint builds each W a second time.  Cotangents as pamd_ccsdt_energy_vjp,
  * plus ulo_bar (device, nfrag x nocc, overwritten) = ulo (mat_bar + mat_bar^T).
- * Workspace: pamd_ccsdt_projected_workspace_size(cfg, nfrag, with_vjp, ...). */
+ * Workspace: pamd_ccsdt_projected_workspace_size(cfg, nfrag, with_vjp, ...), or
+ * up to pamd_ccsdt_projected_preferred_workspace_size, as in the plain calls. */
 int pamd_ccsdt_projected_workspace_size(const pamd_ccsdt_config *cfg, int nfrag, int with_vjp,
                                         size_t *bytes);
+int pamd_ccsdt_projected_preferred_workspace_size(const pamd_ccsdt_config *cfg, int nfrag, int with_vjp,
+                                                  size_t *bytes);
 int pamd_ccsdt_projected_energy(const pamd_ccsdt_config *cfg,
                                 const double *mo_energy, const double *t1, const double *t2,
                                 const double *ovvv, const double *ovoo, const double *ovov,

@@ -22,7 +22,8 @@ STATUS_NAMES = {0: 'ok', 1: 'bad argument', 2: 'HIP runtime error', 3: 'workspac
 PRECISIONS = {'fp64': 0, 'bf16x3': 1, 'fp32x2': 2}
 
 # exported symbols of include/pyscfad_amd_ccsdt.h, _profile.h, _debug.h, _mlp.h and _eris.h
-EXPORTS = ('pamd_version', 'pamd_ccsdt_workspace_size', 'pamd_ccsdt_energy',
+EXPORTS = ('pamd_version', 'pamd_ccsdt_workspace_size', 'pamd_ccsdt_preferred_workspace_size',
+           'pamd_ccsdt_projected_preferred_workspace_size', 'pamd_ccsdt_energy',
            'pamd_ccsdt_energy_vjp', 'pamd_ccsdt_pair_energy', 'pamd_ccsdt_num_triples',
            'pamd_ccsdt_energy_shard', 'pamd_ccsdt_energy_vjp_shard',
            'pamd_ccsdt_energy_vjp_noalloc', 'pamd_ccsdt_noalloc_scratch_bytes',
@@ -63,6 +64,8 @@ def load():
     lib.pamd_version.argtypes = []
     lib.pamd_ccsdt_workspace_size.restype = i
     lib.pamd_ccsdt_workspace_size.argtypes = [cfgp, i, ctypes.POINTER(sz)]
+    lib.pamd_ccsdt_preferred_workspace_size.restype = i
+    lib.pamd_ccsdt_preferred_workspace_size.argtypes = [cfgp, i, ctypes.POINTER(sz)]
     lib.pamd_ccsdt_energy.restype = i
     lib.pamd_ccsdt_energy.argtypes = [cfgp] + [vp] * 7 + [vp, sz, vp, vp]
     lib.pamd_ccsdt_num_triples.restype = i
@@ -82,6 +85,8 @@ def load():
     lib.pamd_ccsdt_noalloc_scratch_bytes.argtypes = []
     lib.pamd_ccsdt_projected_workspace_size.restype = i
     lib.pamd_ccsdt_projected_workspace_size.argtypes = [cfgp, i, i, ctypes.POINTER(sz)]
+    lib.pamd_ccsdt_projected_preferred_workspace_size.restype = i
+    lib.pamd_ccsdt_projected_preferred_workspace_size.argtypes = [cfgp, i, i, ctypes.POINTER(sz)]
     lib.pamd_ccsdt_projected_energy_vjp.restype = i
     lib.pamd_ccsdt_projected_energy_vjp.argtypes = ([cfgp] + [vp] * 8 + [i, d, vp, sz] +
                                                     [vp] * 9 + [vp])
@@ -136,11 +141,12 @@ def make_config(nocc, nvir, ovvv_packed=False, has_fvo=False, precision='fp64'):
                   PRECISIONS[precision], 0)
 
 
-def workspace_size(cfg, with_vjp):
-    lib = load()
+def workspace_size(cfg, with_vjp, least=False):
+    """Device bytes a call uses when they are there (pamd_ccsdt_preferred_workspace_size),
+    or with ``least`` those it needs (pamd_ccsdt_workspace_size)."""
+    name = 'pamd_ccsdt_workspace_size' if least else 'pamd_ccsdt_preferred_workspace_size'
     out = ctypes.c_size_t(0)
-    check(lib.pamd_ccsdt_workspace_size(ctypes.byref(cfg), int(bool(with_vjp)), ctypes.byref(out)),
-          'pamd_ccsdt_workspace_size')
+    check(getattr(load(), name)(ctypes.byref(cfg), int(bool(with_vjp)), ctypes.byref(out)), name)
     return out.value
 
 

@@ -37,6 +37,22 @@ def _stream(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+def _scratch(preferred, least, device, what):
+    """A call's device workspace and its size: ``preferred`` bytes, or where the device
+    does not hold these, the first of their halves that fits, and at last ``least()``,
+    which every entry point takes (it then runs smaller batches)."""
+    # no device query before the allocation: a query can wait for the
+    # device, which would serialise calls issued on several streams
+    nbytes = preferred
+    while True:
+        try:
+            return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device), nbytes
+        except torch.OutOfMemoryError as exc:
+            if nbytes <= least():
+                raise type(exc)(f'{what}: {nbytes / 1e6:.0f} MB of device workspace needed') from exc
+        nbytes = max(nbytes // 512 * 256, least())
+
+
 class Inputs:
     """Device copies of the (T) inputs plus the C-ABI config."""
 
@@ -82,20 +98,22 @@ class Inputs:
                 _ptr(self.ovoo), _ptr(self.ovov), _ptr(self.fvo)]
 
     def workspace(self, with_vjp):
-        # no device query before the allocation: a query can wait for the
-        # device, which would serialise calls issued on several streams
-        nbytes = _lib.workspace_size(self.cfg, with_vjp)
-        try:
-            ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=self.device)
-        except torch.OutOfMemoryError as exc:
-            raise RuntimeError(f'(T): {nbytes / 1e6:.0f} MB of device workspace needed') from exc
-        return ws, nbytes
+        """(tensor, nbytes) for calls that take ``workspace``; room for the cotangents of
+        such a call is left."""
+        room = _cotangent_outputs(self) if with_vjp else None
+        ws = self._workspace(with_vjp)
+        del room
+        return ws
+
+    def _workspace(self, with_vjp):
+        return _scratch(_lib.workspace_size(self.cfg, with_vjp),
+                        lambda: _lib.workspace_size(self.cfg, with_vjp, least=True), self.device, '(T)')
 
 
 def energy(inp: Inputs):
     """E(T) as a 0-d float64 device tensor."""
     lib = _lib.load()
-    ws, nbytes = inp.workspace(False)
+    ws, nbytes = inp._workspace(False)
     e = torch.empty((), dtype=torch.float64, device=inp.device)
     st = lib.pamd_ccsdt_energy(ctypes.byref(inp.cfg), *inp.args(), _ptr(ws), nbytes, _ptr(e),
                                _stream(inp.device))
@@ -107,7 +125,7 @@ def energy_shard(inp: Inputs, shard, nshards):
     """E(T) of the round-robin shard ``shard`` of ``nshards`` over the occupied
     triples (the shards add up to ``energy``)."""
     lib = _lib.load()
-    ws, nbytes = inp.workspace(False)
+    ws, nbytes = inp._workspace(False)
     e = torch.zeros((), dtype=torch.float64, device=inp.device)
     st = lib.pamd_ccsdt_energy_shard(ctypes.byref(inp.cfg), *inp.args(), int(shard),
                                      int(nshards), _ptr(ws), nbytes, _ptr(e),
@@ -119,7 +137,7 @@ def energy_shard(inp: Inputs, shard, nshards):
 def pair_energy(inp: Inputs):
     """(o, o) occupied-pair resolved E(T); its sum is E(T)."""
     lib = _lib.load()
-    ws, nbytes = inp.workspace(False)
+    ws, nbytes = inp._workspace(False)
     e = torch.zeros((inp.nocc, inp.nocc), dtype=torch.float64, device=inp.device)
     st = lib.pamd_ccsdt_pair_energy(ctypes.byref(inp.cfg), *inp.args(), _ptr(ws), nbytes,
                                     _ptr(e), _stream(inp.device))
@@ -151,9 +169,9 @@ def energy_vjp(inp: Inputs, et_bar=1.0, workspace=None):
     ``workspace``: an optional (tensor, nbytes) from ``inp.workspace(True)``,
     reused across calls."""
     lib = _lib.load()
-    ws, nbytes = workspace if workspace is not None else inp.workspace(True)
     e = torch.empty((), dtype=torch.float64, device=inp.device)
     out = _cotangent_outputs(inp)
+    ws, nbytes = workspace if workspace is not None else inp._workspace(True)
     st = lib.pamd_ccsdt_energy_vjp(
         ctypes.byref(inp.cfg), *inp.args(), ctypes.c_double(float(et_bar)), _ptr(ws), nbytes,
         _ptr(e), *_cotangent_ptrs(out), _stream(inp.device))
@@ -166,9 +184,9 @@ def energy_vjp_shard(inp: Inputs, shard, nshards, et_bar=1.0, workspace=None):
     occupied triples; the shards' energies and cotangents add up to
     ``energy_vjp``'s."""
     lib = _lib.load()
-    ws, nbytes = workspace if workspace is not None else inp.workspace(True)
     e = torch.zeros((), dtype=torch.float64, device=inp.device)
     out = _cotangent_outputs(inp)
+    ws, nbytes = workspace if workspace is not None else inp._workspace(True)
     st = lib.pamd_ccsdt_energy_vjp_shard(
         ctypes.byref(inp.cfg), *inp.args(), ctypes.c_double(float(et_bar)), int(shard),
         int(nshards), _ptr(ws), nbytes, _ptr(e), *_cotangent_ptrs(out), _stream(inp.device))
@@ -188,7 +206,6 @@ def weighted_energy_vjp(inp: Inputs, occ_weight, et_bar=1.0):
     if m.shape != (o,):
         raise ValueError(f'occ_weight must have {o} entries, got {m.shape}')
     dev = inp.device
-    ws, nbytes = inp.workspace(True)
     f64 = dict(dtype=torch.float64, device=dev)
     e = torch.zeros((), **f64)
     out = dict(
@@ -201,6 +218,7 @@ def weighted_energy_vjp(inp: Inputs, occ_weight, et_bar=1.0):
         fvo_bar=torch.empty((v, o), **f64),
         occ_weight_bar=torch.empty(o, **f64),
     )
+    ws, nbytes = inp._workspace(True)
     st = lib.pamd_ccsdt_weighted_energy_vjp(
         ctypes.byref(inp.cfg), *inp.args(), m.ctypes.data_as(ctypes.c_void_p),
         ctypes.c_double(float(et_bar)), _ptr(ws), nbytes, _ptr(e), _ptr(out['mo_energy_bar']),
@@ -222,12 +240,13 @@ def _ulo_array(inp, ulo):
 
 
 def _projected_ws(inp, nfrag, with_vjp):
-    lib = _lib.load()
-    n = ctypes.c_size_t(0)
-    _lib.check(lib.pamd_ccsdt_projected_workspace_size(ctypes.byref(inp.cfg), nfrag,
-                                                       int(with_vjp), ctypes.byref(n)),
-               'pamd_ccsdt_projected_workspace_size')
-    return torch.empty(max(n.value, 1), dtype=torch.uint8, device=inp.device), n.value
+    def size(name):
+        n = ctypes.c_size_t(0)
+        _lib.check(getattr(_lib.load(), name)(ctypes.byref(inp.cfg), nfrag, int(with_vjp), ctypes.byref(n)), name)
+        return n.value
+
+    return _scratch(size('pamd_ccsdt_projected_preferred_workspace_size'),
+                    lambda: size('pamd_ccsdt_projected_workspace_size'), inp.device, 'projected (T)')
 
 
 # fragment orbitals per library call (nfrag <= 8 in pamd_ccsdt_projected_*); E is
@@ -248,8 +267,8 @@ def projected_energy(inp: Inputs, ulo):
     e = torch.zeros((), dtype=torch.float64, device=inp.device)
     for ug in _row_groups(u):
         ug = np.ascontiguousarray(ug)
-        ws, nb = _projected_ws(inp, ug.shape[0], False)
         eg = torch.zeros((), dtype=torch.float64, device=inp.device)
+        ws, nb = _projected_ws(inp, ug.shape[0], False)
         st = lib.pamd_ccsdt_projected_energy(ctypes.byref(inp.cfg), *inp.args(),
                                              ug.ctypes.data_as(ctypes.c_void_p), int(ug.shape[0]),
                                              _ptr(ws), nb, _ptr(eg), _stream(inp.device))
@@ -275,7 +294,6 @@ def projected_energy_vjp(inp: Inputs, ulo, et_bar=1.0):
     ulo_bar = []
     for ug in _row_groups(u):
         ug = np.ascontiguousarray(ug)
-        ws, nb = _projected_ws(inp, ug.shape[0], True)
         eg = torch.zeros((), **f64)
         g = dict(
             mo_energy_bar=torch.empty(o + v, **f64),
@@ -287,6 +305,7 @@ def projected_energy_vjp(inp: Inputs, ulo, et_bar=1.0):
             fvo_bar=torch.empty((v, o), **f64),
             ulo_bar=torch.empty(tuple(ug.shape), **f64),
         )
+        ws, nb = _projected_ws(inp, ug.shape[0], True)
         st = lib.pamd_ccsdt_projected_energy_vjp(
             ctypes.byref(inp.cfg), *inp.args(), ug.ctypes.data_as(ctypes.c_void_p),
             int(ug.shape[0]), ctypes.c_double(float(et_bar)), _ptr(ws), nb, _ptr(eg),

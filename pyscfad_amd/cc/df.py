@@ -21,7 +21,7 @@ import ctypes
 import torch
 
 from .. import _lib
-from ._ops import _dev, _ptr, _require_gpu, _stream
+from ._ops import _dev, _ptr, _require_gpu, _scratch, _stream
 from .eris import ChemistsERIs
 
 
@@ -35,11 +35,14 @@ def _shape(Lpq, nocc):
 
 
 def _workspace(nocc, nmo, naux, with_vjp, device):
-    lib = _lib.load()
-    n = ctypes.c_size_t(0)
-    _lib.check(lib.pamd_df_eris_workspace_size(nocc, nmo, naux, int(with_vjp), ctypes.byref(n)),
-               'pamd_df_eris_workspace_size')
-    return torch.empty(max(n.value, 1), dtype=torch.uint8, device=device), n.value
+    def size(vjp):
+        n = ctypes.c_size_t(0)
+        _lib.check(_lib.load().pamd_df_eris_workspace_size(nocc, nmo, naux, int(vjp), ctypes.byref(n)),
+                   'pamd_df_eris_workspace_size')
+        return n.value
+
+    # (an adjoint needs Lvv and its cotangent; with the full size it splits its products)
+    return _scratch(size(with_vjp), lambda: size(False) * (2 if with_vjp else 1), device, 'DF integrals')
 
 
 def df_eris(Lpq, nocc, blocks=('ovvv', 'ovoo', 'ovov')):

@@ -1819,12 +1819,17 @@ const char *pamd_version(void) { return "pyscfad_amd 0.1.0 (gfx950)"; }
 
 int pamd_ccsdt_workspace_size(const pamd_ccsdt_config *cfg, int with_vjp, size_t *bytes) {
   if (!cfg || !bytes || cfg->nocc < 1 || cfg->nvir < 1) return PAMD_ERR_ARG;
-  const Layout L = make_layout(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, cfg->precision, true);
-  *bytes = std::max(L.total, b3_layout(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, cfg->precision, true,
-                                       (size_t)-1, L).total);
+  *bytes = make_layout(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, cfg->precision, true).total;
+  return PAMD_OK;
+}
+
+int pamd_ccsdt_preferred_workspace_size(const pamd_ccsdt_config *cfg, int with_vjp, size_t *bytes) {
+  if (!cfg || !bytes || cfg->nocc < 1 || cfg->nvir < 1) return PAMD_ERR_ARG;
+  const int o = cfg->nocc, v = cfg->nvir, vjp = with_vjp ? 1 : 0;
+  const Layout L = make_layout(o, v, vjp, cfg->precision, true);
+  *bytes = std::max(L.total, b3_layout(o, v, vjp, cfg->precision, true, (size_t)-1, L).total);
   WalkLayout wl;
-  if (cfg->precision == PAMD_PREC_FP64 &&
-      walk_pick(cfg->nocc, cfg->nvir, with_vjp ? 1 : 0, (size_t)-1, *bytes, wl))
+  if (cfg->precision == PAMD_PREC_FP64 && walk_pick(o, v, vjp, (size_t)-1, *bytes, wl))
     *bytes = std::max(*bytes, wl.total);
   return PAMD_OK;
 }
@@ -2070,6 +2075,13 @@ int pamd_ccsdt_projected_workspace_size(const pamd_ccsdt_config *cfg, int nfrag,
   if (!cfg || !bytes || cfg->nocc < 1 || cfg->nvir < 1 || nfrag < 1 || nfrag > kMaxFrag)
     return PAMD_ERR_ARG;
   *bytes = projected_layout(cfg->nocc, cfg->nvir, nfrag, with_vjp ? 1 : 0, cfg->precision).total;
+  return PAMD_OK;
+}
+
+int pamd_ccsdt_projected_preferred_workspace_size(const pamd_ccsdt_config *cfg, int nfrag, int with_vjp,
+                                                  size_t *bytes) {
+  const int st = pamd_ccsdt_projected_workspace_size(cfg, nfrag, with_vjp, bytes);
+  if (st != PAMD_OK) return st;
   ProjWalkLayout pw;
   if (cfg->precision == PAMD_PREC_FP64 &&
       proj_walk_pick(cfg->nocc, cfg->nvir, nfrag, with_vjp ? 1 : 0, (size_t)-1, *bytes, pw))
