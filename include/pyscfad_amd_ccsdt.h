@@ -105,8 +105,8 @@ int pamd_ccsdt_energy_shard(const pamd_ccsdt_config *cfg,
                             double *e_out, void *stream);
 
 /* One shard of E(T) and of its VJP: the triples whose walk index t has
- * t % nshards == shard (the walk and rounding order of
- * pamd_ccsdt_energy_shard), with the outputs of pamd_ccsdt_energy_vjp for that
+ * t % nshards == shard (those of pamd_ccsdt_energy_shard, with the same energy to
+ * rounding), with the outputs of pamd_ccsdt_energy_vjp for that
  * share of the walk (overwritten; e_out is the shard's energy).  The shards'
  * cotangents add up to pamd_ccsdt_energy_vjp's.  Plays the role of the
  * reference's block-callable VJP, ccsd_t_energy_vjp(..., a0, a1, b0, b1, ...)
@@ -127,14 +127,19 @@ int pamd_ccsdt_energy_vjp_shard(const pamd_ccsdt_config *cfg,
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  The workspace is a library-owned device
  * array of pamd_ccsdt_noalloc_scratch_bytes() bytes (128 MiB), one per GPU,
- * held from the first call on that GPU until the process ends; problems whose
- * pamd_ccsdt_workspace_size(cfg, 1, ...) exceeds it are rejected with
- * PAMD_ERR_WORKSPACE (e.g. nocc=10/nvir=64 fits, nocc=16/nvir=64 does not).
+ * held from the first call on that GPU until the process ends; problems that need
+ * more (pamd_ccsdt_noalloc_workspace_size: one occupied triple at a time, on one
+ * stream) are rejected with PAMD_ERR_WORKSPACE (e.g. nocc=10/nvir=64 fits,
+ * nocc=16/nvir=64 does not).
  * Every call on one GPU shares that GPU's array: calls that overlap on one GPU
  * (several streams or host threads) race and must be serialised by the caller.
  * The call overwrites every part of the array it reads, so nothing carries
- * over from an earlier call.  Arguments, outputs and results are those of
- * pamd_ccsdt_energy_vjp; sampled profiling is not recorded for these calls. */
+ * over from an earlier call.  Arguments and outputs are those of
+ * pamd_ccsdt_energy_vjp; results agree to rounding, since the terms may be
+ * grouped otherwise: FP64 calls with a workspace can hold larger batches of
+ * triples (within 1e-12 relative per block, 1e-15 measured), split-BF16x3 ones pair
+ * triples that this call does not (ovvv_bar, t2_bar: within 1e-6, 1e-8 measured).
+ * Sampled profiling is not recorded for these calls. */
 int pamd_ccsdt_energy_vjp_noalloc(const pamd_ccsdt_config *cfg,
                                   const double *mo_energy, const double *t1, const double *t2,
                                   const double *ovvv, const double *ovoo, const double *ovov,
@@ -143,6 +148,8 @@ int pamd_ccsdt_energy_vjp_noalloc(const pamd_ccsdt_config *cfg,
                                   double *t2_bar, double *ovvv_bar, double *ovoo_bar,
                                   double *ovov_bar, double *fvo_bar, void *stream);
 size_t pamd_ccsdt_noalloc_scratch_bytes(void);
+/* What pamd_ccsdt_energy_vjp_noalloc needs of that array.  Host-only call. */
+int pamd_ccsdt_noalloc_workspace_size(const pamd_ccsdt_config *cfg, size_t *bytes);
 
 /* Occupied-pair resolved E(T): e_pair[i*o + j] = 1/3 sum_{k,abc} W Z / D,
  * sum(e_pair) = E(T).  Row sums are the occupied-weighted (T) of
@@ -185,8 +192,9 @@ int pamd_ccsdt_weighted_energy_vjp(const pamd_ccsdt_config *cfg,
  * mat = sum_f u_f u_f^T, so a larger fragment is the sum of calls on row groups
  * of ulo; pyscfad_amd.cc._ops does that).  e_out: device scalar.
  * The walk takes every unordered occupied pair (j, k) and all o triples
- * (l, j, k): about three times the W builds of pamd_ccsdt_energy, and the
- * adjoint builds each W a second time.  Cotangents as pamd_ccsdt_energy_vjp,
+ * (l, j, k): about three times the W builds of pamd_ccsdt_energy.  FP64 calls keep
+ * the W of several pairs for the adjoint; with less workspace than one pair's
+ * blocks, and in the split forms, the adjoint builds each W a second time.  Cotangents as pamd_ccsdt_energy_vjp,
  * plus ulo_bar (device, nfrag x nocc, overwritten) = ulo (mat_bar + mat_bar^T).
  * Workspace: pamd_ccsdt_projected_workspace_size(cfg, nfrag, with_vjp, ...), or
  * up to pamd_ccsdt_projected_preferred_workspace_size, as in the plain calls. */

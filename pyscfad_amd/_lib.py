@@ -23,7 +23,7 @@ PRECISIONS = {'fp64': 0, 'bf16x3': 1, 'fp32x2': 2}
 
 # exported symbols of include/pyscfad_amd_ccsdt.h, _profile.h, _debug.h, _mlp.h and _eris.h
 EXPORTS = ('pamd_version', 'pamd_ccsdt_workspace_size', 'pamd_ccsdt_preferred_workspace_size',
-           'pamd_ccsdt_projected_preferred_workspace_size', 'pamd_ccsdt_energy',
+           'pamd_ccsdt_projected_preferred_workspace_size', 'pamd_ccsdt_noalloc_workspace_size', 'pamd_ccsdt_energy',
            'pamd_ccsdt_energy_vjp', 'pamd_ccsdt_pair_energy', 'pamd_ccsdt_num_triples',
            'pamd_ccsdt_energy_shard', 'pamd_ccsdt_energy_vjp_shard',
            'pamd_ccsdt_energy_vjp_noalloc', 'pamd_ccsdt_noalloc_scratch_bytes',
@@ -66,6 +66,8 @@ def load():
     lib.pamd_ccsdt_workspace_size.argtypes = [cfgp, i, ctypes.POINTER(sz)]
     lib.pamd_ccsdt_preferred_workspace_size.restype = i
     lib.pamd_ccsdt_preferred_workspace_size.argtypes = [cfgp, i, ctypes.POINTER(sz)]
+    lib.pamd_ccsdt_noalloc_workspace_size.restype = i
+    lib.pamd_ccsdt_noalloc_workspace_size.argtypes = [cfgp, ctypes.POINTER(sz)]
     lib.pamd_ccsdt_energy.restype = i
     lib.pamd_ccsdt_energy.argtypes = [cfgp] + [vp] * 7 + [vp, sz, vp, vp]
     lib.pamd_ccsdt_num_triples.restype = i

@@ -1445,8 +1445,8 @@ static WalkLayout walk_layout(int o, int v, int vjp, int nb) {
 }
 
 // The batch of a call: as many triples as fit the library's own scratch
-// together with the rest when these are all, or 32 (so that the calls with and
-// without a workspace of their own split the walk alike and agree bit for bit),
+// together with the rest when these are all, or 32 (a call without a workspace of
+// its own then splits the walk like one with it),
 // else as many as 8 GB of blocks hold; fewer when `limit` bytes are there, or
 // when an adjoint would hold nearly every triple.
 // False when the walk does not apply: slabs beyond 32-bit offsets, not even one
@@ -2005,6 +2005,12 @@ int pamd_ccsdt_energy_vjp_shard(const pamd_ccsdt_config *cfg, const double *mo_e
 }
 
 size_t pamd_ccsdt_noalloc_scratch_bytes(void) { return kNoAllocScratchBytes; }
+
+int pamd_ccsdt_noalloc_workspace_size(const pamd_ccsdt_config *cfg, size_t *bytes) {
+  if (!cfg || !bytes || cfg->nocc < 1 || cfg->nvir < 1) return PAMD_ERR_ARG;
+  *bytes = make_layout(cfg->nocc, cfg->nvir, 1, cfg->precision).total;
+  return PAMD_OK;
+}
 
 int pamd_ccsdt_energy_vjp_noalloc(const pamd_ccsdt_config *cfg, const double *mo_energy,
                                   const double *t1, const double *t2, const double *ovvv,

@@ -39,6 +39,15 @@ def test_needed_projected_workspace_is_one_triples():
     assert _projected(cfg, 4, 'pamd_ccsdt_projected_preferred_workspace_size') > 429056000
 
 
+def test_noalloc_size_says_which_problems_fit():
+    lib = _lib.load()
+    n = ctypes.c_size_t(0)
+    for o, v, fits in ((10, 64, True), (8, 56, True), (16, 64, False), (11, 77, False)):
+        cfg = _lib.make_config(o, v)
+        assert lib.pamd_ccsdt_noalloc_workspace_size(ctypes.byref(cfg), ctypes.byref(n)) == _lib.PAMD_OK
+        assert (n.value <= lib.pamd_ccsdt_noalloc_scratch_bytes()) == fits, (o, v)
+
+
 def test_scratch_takes_what_fits(monkeypatch):
     asked, real = [], torch.empty
 
