@@ -687,6 +687,15 @@ int gemm_wgs_per_cu_b3(int M, int N) {
   return kB3Shape[b3_pick(M, N)][2];
 }
 
+// Products of one workgroup or two and at most four stages of K (nvir <= 16): the
+// direct engine's plan and first loads are then all of its time, and the
+// register-staged tiles start sooner.  Measured, one energy with padded operands:
+// o3/v8 380 -> 295 us, o8/v16 2.25 -> 2.05 ms; a gradient: o5/v7 7.35 -> 6.52 ms,
+// o8/v16 17.6 -> 16.2.  At nvir = 24 (576 x 24) both take the same.
+static bool b3_tiny(const GemmDesc &d) {
+  return (long long)d.M * d.N <= 4096 && d.chunk_start[d.nseg] <= 4 && d.mode < kPartial;
+}
+
 hipError_t launch_gemm_b3(const GemmDesc &d0, hipStream_t s, const GemmBatch &bt) {
   if (d0.M <= 0 || d0.N <= 0) return hipSuccess;
   if (bt.nb < 1 || (bt.nb > 1 && d0.mode >= kPartial)) return hipErrorInvalidValue;
@@ -694,7 +703,10 @@ hipError_t launch_gemm_b3(const GemmDesc &d0, hipStream_t s, const GemmBatch &bt
   d.chunk_start[0] = 0;
   for (int q = 0; q < d.nseg; ++q) d.chunk_start[q + 1] = d.chunk_start[q] + (d.seg[q].L + BKC - 1) / BKC;
   for (int q = d.nseg + 1; q <= kMaxSeg; ++q) d.chunk_start[q] = d.chunk_start[d.nseg];
-  if (gemm_b3p_enabled() && d.sums != kSumsFlushed && gemm_b3p_ok(d, bt)) return launch_gemm_b3p(d, s, bt);
+  if (gemm_b3p_enabled() && d.sums != kSumsFlushed && gemm_b3p_ok(d, bt)) {
+    if (!b3_tiny(d)) return launch_gemm_b3p(d, s, bt);
+    d.sums = kSumsWhole;  // (the direct engine's sums, the same bits)
+  }
   const int c = b3_pick(d.M, d.N, d.sums);
   if (c >= kB3Wide && d.N <= 32 && d.M >= d.N && gemm_b3p_enabled() && gemm_b3p_ok(d, bt))
     return launch_gemm_b3p_narrow(d, s, bt);

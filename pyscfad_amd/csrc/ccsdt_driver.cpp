@@ -1331,8 +1331,10 @@ static void bind_workspace(Ctx &c, const Layout &L, void *ws) {
   const bool packed_ops = c.prec == PAMD_PREC_BF16X3 || c.prec == PAMD_PREC_FP32X2;
   c.gT2 = packed_ops ? (const double *)(b + L.off_T2g) : c.t2;
   c.gW = (packed_ops && c.vjp) ? (double *)(b + L.off_W8) : c.W;
-  c.VpT = L.vpt ? (double *)(b + L.off_VpT) : nullptr;
-  c.VpU = L.vpt ? (double *)(b + L.off_VpU) : nullptr;
+  // (the tiny products are not run by the direct engine, which the copies are for: b3_tiny)
+  const bool vpt = L.vpt && L.vp > 16;
+  c.VpT = vpt ? (double *)(b + L.off_VpT) : nullptr;
+  c.VpU = vpt ? (double *)(b + L.off_VpU) : nullptr;
   {
     const long long o = c.o, op = c.op, v = c.vp, v3 = v * v * v;
     PlanarMap &pm = c.planes;
