@@ -222,6 +222,11 @@ class MLP:
         """``grads`` and ``adam`` in two launches; None (and nothing done) where the
         whole-network kernels do not apply."""
         sizes, dev, n = self.sizes, X16.device, X16.shape[0]
+        # (the widths first: networks too wide for the kernels pay for one call)
+        csizes = (ctypes.c_int * len(sizes))(*sizes)
+        need = ctypes.c_size_t(0)
+        if _fn('pamd_mlp_train_scratch')(len(sizes) - 1, csizes, n, ctypes.byref(need)) != _lib.PAMD_OK:
+            return None
         if not (_plain(X16, (n, sizes[0]), torch.int16, dev) and
                 _plain(X16_t, (sizes[0], n), torch.int16, dev) and
                 _plain(y, (n, sizes[-1]), torch.float32, dev)):
@@ -236,11 +241,6 @@ class MLP:
                 if not _plain(t, shape, dtype, dev):
                     return None
                 ptrs.append(t.data_ptr())
-        csizes = (ctypes.c_int * len(sizes))(*sizes)
-        need = ctypes.c_size_t(0)
-        st = _fn('pamd_mlp_train_scratch')(len(sizes) - 1, csizes, n, ctypes.byref(need))
-        if st != _lib.PAMD_OK:
-            return None
         scratch = torch.empty(need.value, dtype=torch.uint8, device=dev)
         loss = torch.empty((), dtype=torch.float32, device=dev)
         st = _fn('pamd_mlp_train_step')(
