@@ -1,10 +1,13 @@
 /*
- * Host-only inspection entry points of libpyscfad_amd_cc.so.  They run no GPU
- * work and have no counterpart in the reference: they let tests check, on the
- * CPU, every address the contraction engine will touch before a kernel runs.
+ * Inspection entry points of libpyscfad_amd_cc.so, with no counterpart in the
+ * reference.  All but the two pamd_debug_one_triple_* run no GPU work: they let
+ * tests check, on the CPU, every address the contraction engine will touch
+ * before a kernel runs.
  */
 #ifndef PYSCFAD_AMD_DEBUG_H
 #define PYSCFAD_AMD_DEBUG_H
+
+#include "pyscfad_amd_ccsdt.h"
 
 #ifdef __cplusplus
 extern "C" {
@@ -58,6 +61,28 @@ int pamd_debug_split_factors(int nocc, int nvir, int *S_p, int *S_h);
 /* The same for a given precision (PAMD_PREC_*): the split-BF16x3 engine sizes
  * its split-K for its own tile shapes and bounds the K range of one part. */
 int pamd_debug_split_factors_prec(int nocc, int nvir, int precision, int *S_p, int *S_h);
+
+/* Triples per batch that an FP64 call (nfrag = 0), or a projected one (nfrag > 0),
+ * works on with a workspace of workspace_bytes; 0: one triple at a time. */
+int pamd_debug_walk_batch(int nocc, int nvir, int nfrag, int with_vjp, size_t workspace_bytes, int *triples);
+
+/* pamd_ccsdt_energy_vjp and pamd_ccsdt_projected_energy_vjp, one triple at a time
+ * whatever the workspace holds: what an FP64 call does when it holds no batch, for
+ * tests that compare the walks.  two_streams: with the epilogue on the library's
+ * side stream (needs pamd_ccsdt_workspace_size bytes), or on the call's alone. */
+int pamd_debug_one_triple_vjp(const pamd_ccsdt_config *cfg, const double *mo_energy, const double *t1,
+                              const double *t2, const double *ovvv, const double *ovoo, const double *ovov,
+                              const double *fvo, double et_bar, int two_streams, void *workspace,
+                              size_t workspace_bytes, double *e_out, double *mo_energy_bar, double *t1_bar,
+                              double *t2_bar, double *ovvv_bar, double *ovoo_bar, double *ovov_bar,
+                              double *fvo_bar, void *stream);
+int pamd_debug_one_triple_projected_vjp(const pamd_ccsdt_config *cfg, const double *mo_energy, const double *t1,
+                                        const double *t2, const double *ovvv, const double *ovoo,
+                                        const double *ovov, const double *fvo, const double *ulo, int nfrag,
+                                        double et_bar, void *workspace, size_t workspace_bytes, double *e_out,
+                                        double *mo_energy_bar, double *t1_bar, double *t2_bar, double *ovvv_bar,
+                                        double *ovoo_bar, double *ovov_bar, double *fvo_bar, double *ulo_bar,
+                                        void *stream);
 
 #ifdef __cplusplus
 }

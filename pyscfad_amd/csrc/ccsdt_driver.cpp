@@ -1923,7 +1923,7 @@ static int vjp_impl(const pamd_ccsdt_config *cfg, const double *mo_energy, const
                     size_t workspace_bytes, double *e_out, double *mo_energy_bar, double *t1_bar,
                     double *t2_bar, double *ovvv_bar, double *ovoo_bar, double *ovov_bar,
                     double *fvo_bar, double *wt_bar, void *stream, int shard = 0,
-                    int nshards = 1, bool pipe = true) {
+                    int nshards = 1, bool pipe = true, bool batched = true) {
   int st = check_common(cfg, mo_energy, t1, t2, ovvv, ovoo, ovov, fvo);
   if (st != PAMD_OK) return st;
   if (!e_out || !mo_energy_bar || !t1_bar || !t2_bar || !ovvv_bar || !ovoo_bar || !ovov_bar ||
@@ -1957,7 +1957,8 @@ static int vjp_impl(const pamd_ccsdt_config *cfg, const double *mo_energy, const
   c.shard = shard;
   c.nshards = nshards;
   WalkLayout wl;
-  const bool walk = c.prec == PAMD_PREC_FP64 && walk_pick(c.o, c.v, 1, workspace_bytes, L.total, wl);
+  const bool walk =
+      batched && c.prec == PAMD_PREC_FP64 && walk_pick(c.o, c.v, 1, workspace_bytes, L.total, wl);
   if (walk) {
     st = run_walk(c, wl, workspace, ovvv_bar, mo_energy_bar);
   } else {
@@ -2103,7 +2104,7 @@ static int projected_impl(const pamd_ccsdt_config *cfg, const double *mo_energy,
                           int vjp, double et_bar, void *workspace, size_t workspace_bytes,
                           double *e_out, double *mo_energy_bar, double *t1_bar, double *t2_bar,
                           double *ovvv_bar, double *ovoo_bar, double *ovov_bar, double *fvo_bar,
-                          double *ulo_bar, void *stream) {
+                          double *ulo_bar, void *stream, bool batched = true) {
   int st = check_common(cfg, mo_energy, t1, t2, ovvv, ovoo, ovov, fvo);
   if (st != PAMD_OK) return st;
   if (!ulo || !e_out || nfrag < 1 || nfrag > kMaxFrag) return PAMD_ERR_ARG;
@@ -2135,7 +2136,8 @@ static int projected_impl(const pamd_ccsdt_config *cfg, const double *mo_energy,
   c.ovov_bar = ovov_bar;
   c.fvo_bar = fvo_bar;
   ProjWalkLayout pw;
-  if (c.prec == PAMD_PREC_FP64 && proj_walk_pick(c.o, c.v, nfrag, vjp, workspace_bytes, P.total, pw)) {
+  if (batched && c.prec == PAMD_PREC_FP64 &&
+      proj_walk_pick(c.o, c.v, nfrag, vjp, workspace_bytes, P.total, pw)) {
     c.nshards = 1;
     return run_projected_walk(c, pw, workspace, ulo, nfrag, e_out, ovvv_bar, mo_energy_bar, ulo_bar);
   }
@@ -2176,6 +2178,46 @@ int pamd_ccsdt_projected_energy_vjp(const pamd_ccsdt_config *cfg, const double *
   return projected_impl(cfg, mo_energy, t1, t2, ovvv, ovoo, ovov, fvo, ulo, nfrag, 1, et_bar,
                         workspace, workspace_bytes, e_out, mo_energy_bar, t1_bar, t2_bar,
                         ovvv_bar, ovoo_bar, ovov_bar, fvo_bar, ulo_bar, stream);
+}
+
+int pamd_debug_one_triple_vjp(const pamd_ccsdt_config *cfg, const double *mo_energy, const double *t1,
+                              const double *t2, const double *ovvv, const double *ovoo, const double *ovov,
+                              const double *fvo, double et_bar, int two_streams, void *workspace,
+                              size_t workspace_bytes, double *e_out, double *mo_energy_bar, double *t1_bar,
+                              double *t2_bar, double *ovvv_bar, double *ovoo_bar, double *ovov_bar,
+                              double *fvo_bar, void *stream) {
+  return vjp_impl(cfg, mo_energy, t1, t2, ovvv, ovoo, ovov, fvo, nullptr, et_bar, workspace, workspace_bytes,
+                  e_out, mo_energy_bar, t1_bar, t2_bar, ovvv_bar, ovoo_bar, ovov_bar, fvo_bar, nullptr, stream,
+                  0, 1, two_streams != 0, false);
+}
+
+int pamd_debug_one_triple_projected_vjp(const pamd_ccsdt_config *cfg, const double *mo_energy, const double *t1,
+                                        const double *t2, const double *ovvv, const double *ovoo,
+                                        const double *ovov, const double *fvo, const double *ulo, int nfrag,
+                                        double et_bar, void *workspace, size_t workspace_bytes, double *e_out,
+                                        double *mo_energy_bar, double *t1_bar, double *t2_bar, double *ovvv_bar,
+                                        double *ovoo_bar, double *ovov_bar, double *fvo_bar, double *ulo_bar,
+                                        void *stream) {
+  return projected_impl(cfg, mo_energy, t1, t2, ovvv, ovoo, ovov, fvo, ulo, nfrag, 1, et_bar, workspace,
+                        workspace_bytes, e_out, mo_energy_bar, t1_bar, t2_bar, ovvv_bar, ovoo_bar, ovov_bar,
+                        fvo_bar, ulo_bar, stream, false);
+}
+
+int pamd_debug_walk_batch(int nocc, int nvir, int nfrag, int with_vjp, size_t workspace_bytes, int *triples) {
+  if (nocc < 1 || nvir < 1 || nfrag < 0 || nfrag > kMaxFrag || !triples) return PAMD_ERR_ARG;
+  const int vjp = with_vjp ? 1 : 0;
+  *triples = 0;
+  if (nfrag) {
+    ProjWalkLayout pw;
+    if (proj_walk_pick(nocc, nvir, nfrag, vjp, workspace_bytes,
+                       projected_layout(nocc, nvir, nfrag, vjp, PAMD_PREC_FP64).total, pw))
+      *triples = pw.np * nocc;
+  } else {
+    WalkLayout wl;
+    if (walk_pick(nocc, nvir, vjp, workspace_bytes, make_layout(nocc, nvir, vjp, PAMD_PREC_FP64, true).total, wl))
+      *triples = wl.nb;
+  }
+  return PAMD_OK;
 }
 
 int pamd_debug_gemm_direct_ok(const void *desc) {
