@@ -1456,10 +1456,12 @@ static WalkLayout walk_layout(int o, int v, int vjp, int nb) {
 // where that is large itself.
 static bool walk_pick(int o, int v, int vjp, size_t limit, size_t one_triple_total, WalkLayout &L) {
   if (!walk_dims_ok(walk_dims(o, v))) return false;
-  // batch sizes: whole runs
-  const int n = (int)std::min<long long>((num_triples(o) + kWalkRun - 1) / kWalkRun * kWalkRun, kWalkMaxBatch);
+  // batch sizes: whole runs, one at least (one occupied orbital has no triples; its
+  // empty batch writes the zero cotangents)
+  const long long runs = std::max((num_triples(o) + kWalkRun - 1) / kWalkRun, 1LL);
+  const int n = (int)std::min<long long>(runs * kWalkRun, kWalkMaxBatch);
   auto largest = [&](size_t bytes) {
-    int b = std::max(n, kWalkRun);
+    int b = n;
     while (b > 0 && walk_layout(o, v, vjp, b).total > bytes) b -= kWalkRun;
     return b;
   };

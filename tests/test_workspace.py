@@ -27,6 +27,28 @@ def test_needed_workspace_is_one_triples(o, v, precision, fwd, vjp):
         assert _lib.workspace_size(cfg, w) >= n
 
 
+# (nvir = 100 and 112: where eight blocks of v^3 pass the library's 128 MiB, with and
+# without an adjoint)
+@pytest.mark.parametrize('v', [1, 40, 99, 100, 112, 300])
+def test_one_occupied_orbital_has_workspace_sizes(v):
+    cfg = _lib.make_config(1, v)
+    for w in (False, True):
+        assert 0 < _lib.workspace_size(cfg, w, least=True) <= _lib.workspace_size(cfg, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('v', [40, 112])
+def test_one_occupied_orbital_gives_zeros(v, cuda):
+    """There is no triple: E(T) and every cotangent are zero."""
+    p = make_problem(1, v, 2 * v, seed=v, fvo_scale=1e-3)
+    inp = _ops.Inputs(p.mo_energy, p.t1, p.t2, p.ovvv_packed(), p.ovoo, p.ovov, p.fvo, device=cuda)
+    assert float(_ops.energy(inp)) == 0.0
+    e, g = _ops.energy_vjp(inp, et_bar=0.7)
+    assert float(e) == 0.0
+    for k, x in g.items():
+        assert not bool(x.any()), k
+
+
 def _projected(cfg, nfrag, name):
     n = ctypes.c_size_t(0)
     assert getattr(_lib.load(), name)(ctypes.byref(cfg), nfrag, 1, ctypes.byref(n)) == _lib.PAMD_OK
