@@ -65,6 +65,8 @@ int pamd_debug_split_factors_prec(int nocc, int nvir, int precision, int *S_p, i
 /* Triples per batch that an FP64 call (nfrag = 0), or a projected one (nfrag > 0),
  * works on with a workspace of workspace_bytes; 0: one triple at a time. */
 int pamd_debug_walk_batch(int nocc, int nvir, int nfrag, int with_vjp, size_t workspace_bytes, int *triples);
+/* Bytes of that workspace which such a call uses (its batched walk; 0: none). */
+int pamd_debug_walk_bytes(int nocc, int nvir, int nfrag, int with_vjp, size_t workspace_bytes, size_t *bytes);
 
 /* pamd_ccsdt_energy_vjp and pamd_ccsdt_projected_energy_vjp, one triple at a time
  * whatever the workspace holds: what an FP64 call does when it holds no batch, for

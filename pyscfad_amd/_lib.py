@@ -32,7 +32,7 @@ EXPORTS = ('pamd_version', 'pamd_ccsdt_workspace_size', 'pamd_ccsdt_preferred_wo
            'pamd_ccsdt_projected_energy_vjp', 'pamd_profile_enable',
            'pamd_profile_reset', 'pamd_profile_progress', 'pamd_profile_num_kinds', 'pamd_profile_kind_name',
            'pamd_profile_read', 'pamd_debug_gemm_descriptors',
-           'pamd_debug_paired_adjoint_descriptors', 'pamd_debug_adjoint_launches', 'pamd_debug_walk_batch',
+           'pamd_debug_paired_adjoint_descriptors', 'pamd_debug_adjoint_launches', 'pamd_debug_walk_batch', 'pamd_debug_walk_bytes',
            'pamd_debug_one_triple_vjp', 'pamd_debug_one_triple_projected_vjp', 'pamd_debug_split_factors',
            'pamd_debug_split_factors_prec', 'pamd_debug_gemm_direct_ok', 'pamd_debug_gemm_b3p_ok',
            'pamd_bf16_gemm_tn', 'pamd_bf16_act_fwd', 'pamd_bf16_act_bwd', 'pamd_adam_step',
@@ -124,6 +124,8 @@ def load():
     lib.pamd_debug_gemm_b3p_ok.argtypes = [vp, ctypes.c_longlong]
     lib.pamd_debug_walk_batch.restype = i
     lib.pamd_debug_walk_batch.argtypes = [i, i, i, i, sz, ctypes.POINTER(i)]
+    lib.pamd_debug_walk_bytes.restype = i
+    lib.pamd_debug_walk_bytes.argtypes = [i, i, i, i, sz, ctypes.POINTER(sz)]
     lib.pamd_debug_one_triple_vjp.restype = i
     lib.pamd_debug_one_triple_vjp.argtypes = [cfgp] + [vp] * 7 + [d, i, vp, sz] + [vp] * 8 + [vp]
     lib.pamd_debug_one_triple_projected_vjp.restype = i

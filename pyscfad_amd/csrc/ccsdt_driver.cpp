@@ -1477,7 +1477,10 @@ static bool walk_pick(int o, int v, int vjp, size_t limit, size_t one_triple_tot
   }
   if (walk_layout(o, v, vjp, b).total > limit) b = largest(limit);
   if (b < kWalkRun) return false;
+  // batches of equal size, where these take no more than `limit` (fewer triples per
+  // batch may take more parts of TB's adjoint)
   L = walk_layout(o, v, vjp, walk_batches(num_triples(o), b).cap);
+  if (L.total > limit) L = walk_layout(o, v, vjp, b);
   return L.total <= ((size_t)100 << 30) || L.total <= one_triple_total + one_triple_total / 20;
 }
 
@@ -2218,6 +2221,23 @@ int pamd_debug_walk_batch(int nocc, int nvir, int nfrag, int with_vjp, size_t wo
     WalkLayout wl;
     if (walk_pick(nocc, nvir, vjp, workspace_bytes, make_layout(nocc, nvir, vjp, PAMD_PREC_FP64, true).total, wl))
       *triples = wl.nb;
+  }
+  return PAMD_OK;
+}
+
+int pamd_debug_walk_bytes(int nocc, int nvir, int nfrag, int with_vjp, size_t workspace_bytes, size_t *bytes) {
+  if (nocc < 1 || nvir < 1 || nfrag < 0 || nfrag > kMaxFrag || !bytes) return PAMD_ERR_ARG;
+  const int vjp = with_vjp ? 1 : 0;
+  *bytes = 0;
+  if (nfrag) {
+    ProjWalkLayout pw;
+    if (proj_walk_pick(nocc, nvir, nfrag, vjp, workspace_bytes,
+                       projected_layout(nocc, nvir, nfrag, vjp, PAMD_PREC_FP64).total, pw))
+      *bytes = pw.total;
+  } else {
+    WalkLayout wl;
+    if (walk_pick(nocc, nvir, vjp, workspace_bytes, make_layout(nocc, nvir, vjp, PAMD_PREC_FP64, true).total, wl))
+      *bytes = wl.total;
   }
   return PAMD_OK;
 }

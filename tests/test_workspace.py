@@ -61,6 +61,30 @@ def test_needed_projected_workspace_is_one_triples():
     assert _projected(cfg, 4, 'pamd_ccsdt_projected_preferred_workspace_size') > 429056000
 
 
+def _walk_bytes(o, v, vjp, limit, nfrag=0):
+    n = ctypes.c_size_t(0)
+    assert _lib.load().pamd_debug_walk_bytes(o, v, nfrag, vjp, limit, ctypes.byref(n)) == _lib.PAMD_OK
+    return n.value
+
+
+# (batches are cut to equal sizes, and a smaller batch can take more parts of an adjoint:
+# o13/v47 at 537679616 bytes, o15/v24 at 97909504)
+@pytest.mark.parametrize('o', [2, 5, 8, 13, 15, 17, 24, 33, 61, 100])
+def test_batches_stay_within_any_workspace(o):
+    lib = _lib.load()
+    for v in list(range(2, 60)) + [64, 72, 77, 96, 120, 160]:
+        for vjp in (0, 1):
+            top = _walk_bytes(o, v, vjp, 1 << 62)
+            limits = [lib.pamd_ccsdt_noalloc_scratch_bytes(), 537679616, 97909504, top // 2, top // 4]
+            for _ in range(20):   # every layout the rule can end at: just what the next smaller one takes
+                limits.append(top)
+                top = _walk_bytes(o, v, vjp, max(top - 1, 1))
+            for n in limits:
+                assert _walk_bytes(o, v, vjp, n) <= n, (v, vjp, n)
+                if o <= 17 and v % 8 == 0:
+                    assert _walk_bytes(o, v, vjp, n, nfrag=2) <= n, (v, vjp, n)
+
+
 def test_noalloc_size_says_which_problems_fit():
     lib = _lib.load()
     n = ctypes.c_size_t(0)
