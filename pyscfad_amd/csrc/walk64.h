@@ -20,9 +20,10 @@
 
 namespace pamd {
 
-constexpr int kWalkMaxBatch = 256;  // triples per batch: 10 bits of slot would do for 1024
+// triples per batch: the gather gives each slot of a batch to one of a workgroup's
+// 256 threads, and the adjoint of VT keeps the batch's entries in LDS
+constexpr int kWalkMaxBatch = 256;
 
-//
 // Slabs: VT[x][p] (vp x up) and W[a] (vp x vp) start an odd multiple of 256
 // bytes apart (sp, ws elements).  L2 interleaves its 16 channels every 256
 // bytes, and the walk reads 16 rows one slab apart at once: with vp = 160 a

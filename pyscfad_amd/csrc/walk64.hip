@@ -251,7 +251,7 @@ struct WalkArgs {
   const double *VT, *TB;
   double *W, *out;
   const int *tri;
-  int nb, S, pass;
+  int nb, S;
 };
 
 __device__ __forceinline__ void walk_ijk(const int *tri, int b, int &i, int &j, int &k) {
@@ -532,7 +532,7 @@ static hipError_t walk_launch(long long nprod, int M, int N, int most, F &&f) {
 
 hipError_t launch_walk_w(const WalkDims &d, const double *VT, const double *TBt, double *W, const int *tri,
                          int nb, hipStream_t s) {
-  WalkArgs A{d, VT, TBt, W, nullptr, tri, nb, 1, 0};
+  WalkArgs A{d, VT, TBt, W, nullptr, tri, nb, 1};
   const long long nprod = (long long)nb * d.vp;
   return walk_launch(nprod, d.vp, d.vp, 20, [&](WalkShape w, long long total, dim3 grid) {
 #define X(TM, TN)                                                                          \
@@ -548,7 +548,7 @@ hipError_t launch_walk_w(const WalkDims &d, const double *VT, const double *TBt,
 hipError_t launch_walk_vtb(const WalkDims &d, const double *Wb, const double *TB, double *VTb,
                            const int *tri, int nb, bool first, hipStream_t s) {
   if (nb > kWalkMaxBatch) return hipErrorInvalidValue;
-  WalkArgs A{d, nullptr, TB, const_cast<double *>(Wb), VTb, tri, nb, 1, 0};
+  WalkArgs A{d, nullptr, TB, const_cast<double *>(Wb), VTb, tri, nb, 1};
   const long long nprod = (long long)d.o * d.vp;
   return walk_launch(nprod, d.vp, d.up, 16, [&](WalkShape w, long long total, dim3 grid) {
 #define X(TM, TN)                                                                               \
@@ -563,7 +563,7 @@ hipError_t launch_walk_vtb(const WalkDims &d, const double *Wb, const double *TB
 
 hipError_t launch_walk_tbb(const WalkDims &d, const double *Wb, const double *VT, double *part,
                            const int *tri, int nb, int S, hipStream_t s) {
-  WalkArgs A{d, VT, nullptr, const_cast<double *>(Wb), part, tri, nb, S, 0};
+  WalkArgs A{d, VT, nullptr, const_cast<double *>(Wb), part, tri, nb, S};
   hipError_t e = walk_launch(2LL * nb * S, d.vp, d.up, 20, [&](WalkShape w, long long total, dim3 grid) {
 #define X(TM, TN)              \
   if (w.tm == TM && w.tn == TN) \
@@ -840,6 +840,7 @@ __device__ __forceinline__ void walk_gather(const WalkGather &G, int nblk, int b
   const int xy = blk / nblk, x = xy / o, y = xy - x * o;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // slots that write to (x, y), with the mask of their pieces
+  static_assert(kWalkMaxBatch <= 256, "one slot per thread");
   int mask = 0;
   if ((int)threadIdx.x < G.nb) {
     const int w = G.tri[threadIdx.x];
